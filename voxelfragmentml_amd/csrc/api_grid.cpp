@@ -569,7 +569,7 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
         g->buckets.ensure(relax_flag_bytes(g->dims[0], g->dims[1], g->dims[2]));  // two flag parities, brick liveness
         g->fctl.ensure(64 * 4);
         J.keys = g->keys.as<uint32_t>();
-        J.bflags = g->buckets.as<unsigned long long>();
+        J.bflags = g->buckets.as<uint8_t>();
         J.nbricks = nbricks;
         J.fctl = g->fctl.as<uint32_t>();
         J.key_bits = key_bits_for(S);
@@ -591,7 +591,7 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
         std::memset(g->pinned, 0, 128);
         g->pinned[1] = tasks;
         VF_HIP(hipMemcpyAsync(g->fctl.as<uint32_t>() + 32, g->pinned, 128, hipMemcpyHostToDevice, g->stream));
-        VF_HIP(hipMemsetAsync(J.bflags, 0, 16ull * relax_words_per_parity(nbricks), g->stream));  // both flag parities
+        VF_HIP(hipMemsetAsync(J.bflags, 0, 2ull * relax_parity_bytes(nbricks), g->stream));  // both flag parities
         VF_HIP(hipStreamSynchronize(g->stream));  // the pinned words are reused below
         launch_flood_init(L, W);
         launch_flood_seed(L, W);

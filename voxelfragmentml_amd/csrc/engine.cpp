@@ -21,7 +21,7 @@ constexpr size_t kAlign = 256;
 inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
 struct Layout {
-    size_t labels, occ, bits, seeds, hist, stats, fctl, keys, bricks, sub, erode, mask, mesh_xyz, mesh_tri, total;
+    size_t labels, occ, bits, seeds, hist, stats, fctl, keys, bricks, work, sub, erode, mask, mesh_xyz, mesh_tri, total;
     uint64_t V, words;
 };
 
@@ -65,6 +65,7 @@ Layout layout_of(const vf_job& j)
     L.fctl = o; o = align_up(o + 64 * 4);
     L.keys = o; if (flood) o = align_up(o + L.V * 4);
     L.bricks = o; if (flood) o = align_up(o + relax_flag_bytes(j.dims[0], j.dims[1], j.dims[2]));
+    L.work = o; if (flood) o = align_up(o + 8ull * kFloodWorkSlots * kFloodWorkStride);
     L.sub = o; if (needs_sub(j)) o = align_up(o + 8ull * seed_total(j));  // union-find parents + keep flags
     L.erode = o; if (j.erode) o = align_up(o + L.V * 2);                          // erosion output grid
     L.mask = o; if (j.erode) o = align_up(o + (size_t)kMaxErosionSide * kMaxErosionSide * kMaxErosionSide);
@@ -246,7 +247,8 @@ void Engine::alloc(EJob& e)
     d.bsize = j.erode ? 0 : j.boundary_size;  // erosion runs its own boundary detection
     if (j.algorithm == VF_FLOOD) {
         d.keys = reinterpret_cast<uint32_t*>(base + Lo.keys);
-        d.bflags = reinterpret_cast<unsigned long long*>(base + Lo.bricks);
+        d.bflags = base + Lo.bricks;
+        d.work = reinterpret_cast<unsigned long long*>(base + Lo.work);
         d.nbricks = relax_bricks(d.nx, d.ny, d.nz);
         d.sub = needs_sub(j) ? reinterpret_cast<uint32_t*>(base + Lo.sub) : nullptr;
     } else {

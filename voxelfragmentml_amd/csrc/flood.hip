@@ -75,11 +75,25 @@ constexpr uint32_t kZtWords = 100 * kSepStride;
 constexpr uint32_t kYtWords = 80 * kSepStride;
 static_assert(kYtWords <= kTileWords, "yt reuses the tile");
 constexpr uint32_t kRelaxLdsWords = kTileWords + kZtWords;
-// Consecutive worklist entries a relax workgroup takes at a time (batch step 11.47 ms with one run per
-// workgroup, 11.28 / 11.25 / 11.30 / 11.50 / 11.64 ms with runs of 2 / 3 / 4 / 5 / 6, 11.83 with 8)
+// Consecutive worklist entries a relax workgroup takes at a time, at most (batch step 11.47 ms with one run
+// per workgroup, 11.28 / 11.25 / 11.30 / 11.50 / 11.64 ms with runs of 2 / 3 / 4 / 5 / 6, 11.83 with 8).  A
+// list that has fewer entries than that for each workgroup is cut into shorter runs: a round of few bricks
+// then lasts one visit, about 8 us instead of 20 (the 203x150x177 6-neighbour flood's rounds: 19.3 -> 11.9 us).
 constexpr uint32_t kRelaxRun = 3;
+// A worklist entry: job << 32 | parity of its round << 31 | brick (a grid has fewer than 2^31 cells, 2^22 bricks).
+constexpr uint32_t kEntryParity = 1u << 31;
 constexpr uint32_t kMaxSweeps = 2048;              // a brick of 512 cells is stable after at most 513 sweeps
 constexpr uint32_t kXcds = kFloodXcds;             // XCDs of the device; workgroups are dealt round-robin
+
+// A job's brick flags of one round parity, and its liveness words after both parities.
+__device__ inline uint8_t* parity_flags(uint8_t* bflags, uint32_t nbricks, uint32_t par)
+{
+    return bflags + relax_parity_bytes(nbricks) * par;
+}
+__device__ inline unsigned long long* live_base(uint8_t* bflags, uint32_t nbricks)
+{
+    return reinterpret_cast<unsigned long long*>(bflags + 2u * relax_parity_bytes(nbricks));
+}
 
 __device__ inline uint32_t bdim(uint32_t n) { return (n + kRelaxBrick - 1) / kRelaxBrick; }
 
@@ -107,7 +121,7 @@ __global__ __launch_bounds__(256) void k_flood_seed(Launch L)
     if (!J->active || J->algo != VF_FLOOD) return;
     const uint32_t S = J->S, b = J->key_bits;
     const uint32_t nby = bdim(J->ny), nbz = bdim(J->nz);
-    unsigned long long* live = J->bflags + 2u * relax_words_per_parity(J->nbricks);
+    unsigned long long* live = live_base(J->bflags, J->nbricks);
     const uint32_t wpc = live_words_per_column(nbz);
     auto brick_of = [&](const uint4& q) {
         return ((q.x / kRelaxBrick) * nby + q.y / kRelaxBrick) * nbz + q.z / kRelaxBrick;
@@ -151,7 +165,7 @@ __global__ __launch_bounds__(256) void k_flood_seed(Launch L)
         atomicMax(J->keys + c, seed_key(s, c));
     }
     __syncthreads();
-    unsigned long long* flags1 = J->bflags + relax_words_per_parity(J->nbricks);  // round 1 consumes parity 1
+    uint8_t* flags1 = parity_flags(J->bflags, J->nbricks, 1u);  // round 1 consumes parity 1
     for (uint32_t s = threadIdx.x; s < S; s += blockDim.x) {
         const uint4 q = J->seeds[s];
         const size_t c = ((size_t)q.x * J->ny + q.y) * J->nz + q.z;
@@ -165,7 +179,7 @@ __global__ __launch_bounds__(256) void k_flood_seed(Launch L)
             for (uint32_t by = by0; by <= by1; ++by)
                 for (uint32_t bz = bz0; bz <= bz1; ++bz) {
                     const uint32_t id = (bx * nby + by) * nbz + bz;
-                    atomicOr(flags1 + (id >> 6), 1ull << (id & 63u));
+                    flags1[id] = 1u;
                 }
     }
     __syncthreads();
@@ -190,7 +204,7 @@ __global__ __launch_bounds__(256) void k_flood_nbr(Launch L, const uint32_t* tas
         const uint32_t id = (uint32_t)(g0 - (uint64_t)uni(task_prefix[j]) * 4096u) + threadIdx.x;
         const uint32_t nb = uni(J->nbricks);
         const uint32_t nbx = bdim(uni(J->nx)), nby = bdim(uni(J->ny)), nbz = bdim(uni(J->nz)), wpc = live_words_per_column(nbz);
-        unsigned long long* live = uni_ptr(J->bflags) + 2u * relax_words_per_parity(nb);
+        unsigned long long* live = live_base(uni_ptr(J->bflags), nb);
         const uint32_t idc = min(id, nb - 1u);
         const uint32_t bz = idc % nbz, t1 = idc / nbz, by = t1 % nby, bx = t1 / nby;
         const uint32_t q = bz & 63u, wi = bz >> 6;
@@ -231,12 +245,13 @@ __global__ __launch_bounds__(256) void k_flood_nbr(Launch L, const uint32_t* tas
 // Uniform per-job state of a round, held in scalar registers.
 struct RelaxJob {
     const JobDev* J;
-    uint32_t nx, ny, nz, nby, nbz, nbx, nb, b, amp, r;
-    uint64_t noise_seed;
+    uint32_t nx, ny, nz, nby, nbz, nbx, nb, b;
+    uint32_t par;               // parity of the round
     VF_AS_GLOBAL uint32_t* keys;
-    uint32_t nw;                // flag words per parity
-    VF_AS_GLOBAL unsigned long long* cur;  // brick flag bits consumed this round
-    VF_AS_GLOBAL unsigned long long* nxt;  // brick flag bits for the next round
+    VF_AS_GLOBAL uint32_t* ctl;  // the job's control words
+    unsigned long long* work;   // its work counters
+    uint8_t* flags;             // brick flags of both parities, then the liveness words and neighbour masks
+    VF_AS_GLOBAL uint8_t* nxt;  // brick flags for the next round
     const VF_AS_GLOBAL uint32_t* nmask;  // per brick: liveness of the brick and its 26 neighbours
     bool n26;
 };
@@ -512,7 +527,7 @@ __device__ inline uint32_t relax_brick(const RelaxJob& R, uint32_t brick, uint32
         if (qx >= 0 && qy >= 0 && qz >= 0 && (uint32_t)qx < R.nbx && (uint32_t)qy < R.nby && (uint32_t)qz < R.nbz)
         {
             const uint32_t id = ((uint32_t)qx * R.nby + (uint32_t)qy) * R.nbz + (uint32_t)qz;
-            __hip_atomic_fetch_or(R.nxt + (id >> 6), 1ull << (id & 63u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            R.nxt[id] = 1u;
         }
     }
     activated |= dirs != 0;
@@ -520,52 +535,57 @@ __device__ inline uint32_t relax_brick(const RelaxJob& R, uint32_t brick, uint32
     return sweeps;
 }
 
-// The round-independent part of a flood job's relaxation state, in scalar registers, read in one batch
-// of loads; returns the job's flag words (two parities, then the liveness words and neighbour masks).
-__device__ inline unsigned long long* load_relax_fields(const JobDev* J, RelaxJob& R)
+// The round-independent part of a flood job's relaxation state, in scalar registers, read in one batch of loads.
+__device__ inline void load_relax_fields(const JobDev* J, RelaxJob& R)
 {
     R.J = uni_ptr(J);
     R.nx = uni(J->nx); R.ny = uni(J->ny); R.nz = uni(J->nz);
     R.nbx = bdim(R.nx); R.nby = bdim(R.ny); R.nbz = bdim(R.nz);
     R.nb = uni(J->nbricks);
     R.b = uni(J->key_bits);
-    R.amp = uni(J->noise_amp);
-    R.noise_seed = ((uint64_t)uni((uint32_t)(J->noise_seed >> 32)) << 32) | uni((uint32_t)J->noise_seed);
     R.keys = gcast<uint32_t>(uni_ptr(J->keys));
-    R.nw = relax_words_per_parity(R.nb);
-    unsigned long long* flags = uni_ptr(J->bflags);
-    R.nmask = gcast<const uint32_t>(reinterpret_cast<const uint32_t*>(flags + (size_t)R.nw * 2u + live_words(R.nbx, R.nby, R.nbz)));
+    R.ctl = gcast<uint32_t>(uni_ptr(J->fctl));
+    R.flags = uni_ptr(J->bflags);
+    R.work = uni_ptr(J->work);
+    R.nmask = gcast<const uint32_t>(reinterpret_cast<const uint32_t*>(live_base(R.flags, R.nb) + live_words(R.nbx, R.nby, R.nbz)));
     R.n26 = uni((uint32_t)J->neighbourhood) != 6u;
-    return flags;
 }
 
-// Round r's flag words: round r consumes parity r & 1 and flags into the other.
-__device__ inline void set_relax_round(RelaxJob& R, unsigned long long* flags, uint32_t r)
+// A round of parity par consumes the flags of that parity and sets flags of the other.
+__device__ inline void set_relax_parity(RelaxJob& R, uint32_t par)
 {
-    R.r = r;
-    R.cur = gcast<unsigned long long>(flags + (size_t)R.nw * (r & 1u));
-    R.nxt = gcast<unsigned long long>(flags + (size_t)R.nw * ((r + 1u) & 1u));
+    R.par = par;
+    R.nxt = gcast<uint8_t>(parity_flags(R.flags, R.nb, par ^ 1u));
+}
+
+// The flags of 64 bricks, and as one bit per brick.
+struct FlagGroup {
+    uint4 q[4];
+};
+__device__ inline FlagGroup load_group(const uint8_t* flags, uint32_t w)
+{
+    FlagGroup g;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g.q[i] = gload4(flags + (size_t)w * 64u + 16u * i);
+    return g;
+}
+__device__ inline uint64_t group_bits(const FlagGroup& g)
+{
+    uint64_t m = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t v[4] = { g.q[i].x, g.q[i].y, g.q[i].z, g.q[i].w };
+#pragma unroll
+        for (int k = 0; k < 4; ++k)  // bytes are 0 or 1: byte b lands on bit 24 + b
+            m |= (uint64_t)((v[k] * 0x01020408u) >> 24) << (16 * i + 4 * k);
+    }
+    return m;
 }
 
 // A flood job is running and not drained: its record's flag (read with its fields, before any branch).
 __device__ inline uint32_t flood_job_active(const JobDev* J)
 {
     return uni((uint32_t)((J->active != 0) & (J->algo == VF_FLOOD)));
-}
-
-// A running job's state for the relaxation step (its round was set by this round's compaction): the job's
-// fields, then its control words, two dependent batches of loads.
-__device__ inline bool load_relax_job(const Launch& L, uint32_t j, RelaxJob& R)
-{
-    const JobDev* J = L.jobs + j;
-    const uint32_t act = flood_job_active(J);
-    const uint32_t* ctl = uni_ptr(J->fctl);
-    unsigned long long* flags = load_relax_fields(J, R);
-    if (!act) return false;
-    const uint32_t done = uni(ctl[1]), r = uni(ctl[0]);
-    if (done) return false;
-    set_relax_round(R, flags, r);
-    return true;
 }
 
 // Start job j's next round (in the compaction of chunk round i): the round the previous
@@ -575,17 +595,17 @@ __device__ inline bool load_relax_job(const Launch& L, uint32_t j, RelaxJob& R)
 // rp + 1's relaxation writes it for round rp + 2).  Every workgroup of the job computes the same
 // values from words no workgroup writes in this launch, and writes them: no ordering is needed.
 // The loads come in two dependent batches: the job's fields, then its control words together with
-// both parities' flag word w (lane w of the task), of which *m receives the new round's.
+// both parities' flag group w (lane w of the task), of which *m receives the new round's bits.
 __device__ inline bool start_round(const Launch& L, uint32_t j, uint32_t i, uint32_t w, RelaxJob& R, uint64_t& m)
 {
     const JobDev* J = L.jobs + j;
     const uint32_t act = flood_job_active(J);
-    uint32_t* ctl = uni_ptr(J->fctl);
-    unsigned long long* flags = load_relax_fields(J, R);
+    load_relax_fields(J, R);
     if (!act) return false;
+    VF_AS_GLOBAL uint32_t* ctl = R.ctl;
     const uint32_t done = uni(ctl[1]), s0 = uni(ctl[4]), s1 = uni(ctl[5]), f0 = uni(ctl[2]), f1 = uni(ctl[3]);
-    const bool in = w < R.nw;
-    const uint64_t m0 = in ? flags[w] : 0ull, m1 = in ? flags[(size_t)R.nw + w] : 0ull;
+    const uint32_t ng = relax_groups(R.nb), wc = min(w, ng - 1u);
+    const FlagGroup g0 = load_group(parity_flags(R.flags, R.nb, 0u), wc), g1 = load_group(parity_flags(R.flags, R.nb, 1u), wc);
     if (done) return false;
     const uint32_t rp = ((i + 1u) & 1u) ? s1 : s0;
     const bool lead = threadIdx.x == 0;
@@ -602,15 +622,15 @@ __device__ inline bool start_round(const Launch& L, uint32_t j, uint32_t i, uint
         ctl[0] = r;
         ctl[2 + (rp & 1u)] = 0u;
     }
-    set_relax_round(R, flags, r);
-    m = (r & 1u) ? m1 : m0;
+    set_relax_parity(R, r & 1u);
+    m = w < ng ? group_bits(R.par ? g1 : g0) : 0ull;
     return true;
 }
 
 // Round step 1: start every running job's next round (or find it drained) and
-// turn its flag bitmasks into worklists.
-// A task is 64 flag words (4096 bricks, one word per lane) of one job; each
-// lane clears its word and appends its flagged bricks as (job << 32 | brick)
+// turn its flags into worklists.
+// A task is 64 flag groups (4096 bricks, one group per lane) of one job; each
+// lane clears its group and appends its flagged bricks (with the job and the round's parity)
 // to the worklist of the task's XCD, with one list reservation per wave.
 // Tasks are dealt to the XCDs round-robin like workgroups, so the relax step,
 // which serves list x from the workgroups of XCD x, finds the halos of
@@ -648,7 +668,7 @@ __global__ __launch_bounds__(64) void k_flood_compact(Launch L, const uint32_t* 
             cur_job = j;
             running = start_round(L, j, i, w, R, m);
         } else if (running) {
-            m = w < R.nw ? R.cur[w] : 0ull;
+            m = w < relax_groups(R.nb) ? group_bits(load_group(parity_flags(R.flags, R.nb, R.par), w)) : 0ull;
         }
         if (!running) continue;
         const uint32_t n = (uint32_t)__popcll(m);
@@ -664,20 +684,25 @@ __global__ __launch_bounds__(64) void k_flood_compact(Launch L, const uint32_t* 
         if (lane == 0) base = atomicAdd(counts + xcd, total);
         base = __shfl(base, 0, 64) + inc - n;
         if (m) {
-            R.cur[w] = 0ull;  // consumed
+            uint8_t* cur = parity_flags(R.flags, R.nb, R.par) + (size_t)w * 64u;  // consumed
+#pragma unroll
+            for (int i = 0; i < 4; ++i) gstore4(cur + 16 * i, make_uint4(0u, 0u, 0u, 0u));
             uint64_t bits = m;
             unsigned long long* dst = lists + (size_t)xcd * list_cap;
             while (bits) {
                 const uint32_t bit = (uint32_t)__ffsll((long long)bits) - 1u;
                 bits &= bits - 1ull;
-                if (base < list_cap) dst[base] = ((unsigned long long)j << 32) | (w * 64u + bit);
+                if (base < list_cap) dst[base] = ((unsigned long long)j << 32) | (R.par ? kEntryParity : 0u) | (w * 64u + bit);
                 ++base;
             }
         }
     }
 }
 
-// Round step 2: relax the listed bricks; the workgroups of XCD x serve list x.
+// Round step 2: relax the listed bricks; the workgroups of XCD x serve list x.  Bound by the latency of a
+// visit's chain, and, before flags were bytes and the work counters spread, by same-address atomics at the
+// memory side.  Average of a flood's rounds: 256^3, 33 k visits, 20.3 -> 15.7 us; 512^3, 162 k visits, 34.5 ->
+// 23.8 us.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_flood_relax(Launch L, const unsigned long long* lists, uint32_t list_cap,
                                                     const uint32_t* counts)
 {
@@ -685,38 +710,51 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
     const uint32_t lane = threadIdx.x;
     const uint32_t xcd = blockIdx.x % kXcds, per_xcd = gridDim.x / kXcds, local = blockIdx.x / kXcds;
     if (local >= per_xcd) return;
-    const uint32_t n = min(uni(counts[xcd]), list_cap);
     const unsigned long long* list = lists + (size_t)xcd * list_cap;
+    // A round of few bricks is one visit's chain of dependent loads, so whatever the first visit may need is
+    // asked for together: the list's length, the entry this workgroup takes when runs are of one, and, where
+    // the table holds one job, its fields.
+    const uint32_t cnt = counts[xcd];
+    const unsigned long long spec = list[min(local, list_cap - 1u)];
     RelaxJob R{};
     uint32_t cur_job = 0xFFFFFFFFu;
+    if (L.njobs == 1u) {
+        cur_job = 0u;
+        load_relax_fields(L.jobs, R);
+    }
+    const uint32_t n = min(uni(cnt), list_cap);
     bool activated = false, error = false;
     unsigned long long work = 0;  // (sweeps << 32) + visits for cur_job
     auto flush = [&]() {
-        if (cur_job == 0xFFFFFFFFu) return;
+        if (!work) return;
         if (lane == 0) {
-            if (work) atomicAdd(R.J->stats + kStatFloodWork, work);
-            if (activated) R.J->fctl[2 + ((R.r + 1u) & 1u)] = 1u;
+            if (R.work) atomicAdd(R.work + (blockIdx.x % kFloodWorkSlots) * kFloodWorkStride, work);
+            if (activated) R.ctl[2 + (R.par ^ 1u)] = 1u;
             if (error) atomicOr(reinterpret_cast<unsigned int*>(R.J->stats + kStatError), (unsigned int)kDevErrRelax);
         }
         work = 0;
         activated = error = false;
     };
-    // the list is cut into runs of kRelaxRun consecutive entries, dealt round-robin to the workgroups: a
-    // run is mostly one job's (its state is loaded once per run) and neighbouring bricks of one flag word,
+    // the list is cut into runs of up to kRelaxRun consecutive entries, dealt round-robin to the workgroups: a
+    // run is mostly one job's (its state is loaded once per run) and neighbouring bricks of one flag group,
     // so a later brick of a run reads the cells an earlier one just dropped, while the bricks relaxed at
     // one time stay close together in the list and share their halos in L2 (longer runs, up to one run
-    // per workgroup, spread them over the whole list)
-    for (uint32_t e = local * kRelaxRun; e < n;
-         e = (e % kRelaxRun == kRelaxRun - 1u) ? e + 1u + (per_xcd - 1u) * kRelaxRun : e + 1u) {
-        const unsigned long long entry = list[e];
-        const uint32_t j = uni((uint32_t)(entry >> 32)), brick = uni((uint32_t)entry);
-        if (j != cur_job) {
-            flush();
-            cur_job = j;
-            load_relax_job(L, j, R);  // listed jobs are running
+    // per workgroup, spread them over the whole list).  A list shorter than kRelaxRun entries per workgroup
+    // is cut shorter, so that no workgroup takes several bricks one after another while others have none.
+    const uint32_t run = min(kRelaxRun, (n + per_xcd - 1u) / per_xcd);
+    for (uint32_t base = local * run; base < n; base += per_xcd * run) {
+        for (uint32_t e = base, end = min(base + run, n); e < end; ++e) {
+            const unsigned long long entry = run == 1u ? spec : list[e];
+            const uint32_t j = uni((uint32_t)(entry >> 32)), low = uni((uint32_t)entry);
+            if (j != cur_job) {
+                flush();
+                cur_job = j;
+                load_relax_fields(L.jobs + j, R);
+            }
+            set_relax_parity(R, low >> 31);
+            const uint32_t sw = relax_brick(R, low & ~kEntryParity, tile, activated, error);
+            work += ((unsigned long long)sw << 32) | 1ull;
         }
-        const uint32_t sw = relax_brick(R, brick, tile, activated, error);
-        work += ((unsigned long long)sw << 32) | 1ull;
     }
     flush();
 }
@@ -748,7 +786,7 @@ __global__ __launch_bounds__(1024) void k_flood_plan(Launch L)
 // bytes of one row, and packs its 512 occupancy bits into 16 words in LDS.  Then the live bricks are
 // written one after another, lane x * 8 + y writing row (x, y) of the brick from the packed bits.
 // Every word of the bitmap is written whole.  A job's words are dealt over the 64 slots of each of
-// its compaction tasks (a task is 64 flag words).
+// its compaction tasks (a task is 64 flag groups).
 constexpr uint32_t kInitBitStride = 65;  // LDS words between a wave's packed-bit planes (odd: no bank conflicts)
 
 // one bit per byte of v: bit k set iff byte k is not zero
@@ -778,7 +816,7 @@ __global__ __launch_bounds__(256) void k_flood_init(Launch L, const uint32_t* ta
         const VF_AS_GLOBAL uint8_t* occ = gcast<const uint8_t>(uni_ptr(J->occ));
         VF_AS_GLOBAL uint32_t* keys = gcast<uint32_t>(uni_ptr(J->keys));
         VF_AS_GLOBAL unsigned long long* live =
-            gcast<unsigned long long>(uni_ptr(J->bflags) + 2u * relax_words_per_parity(uni(J->nbricks)));
+            gcast<unsigned long long>(live_base(uni_ptr(J->bflags), uni(J->nbricks)));
         const bool quads = (nz & 3u) == 0u;  // rows of full bricks start on 4-cell boundaries
         for (uint32_t w = g - t0 * 64u; w < nwords; w += nslots) {
             const uint32_t chunk = w % wpc, col = w / wpc, by = col % nby, bx = col / nby;
@@ -1105,7 +1143,7 @@ __global__ __launch_bounds__(kCellThreads) void k_flood_sub_reseed(Launch L)
         if (c0 >= J.V) return;
         const uint32_t b = J.key_bits, mask = (1u << b) - 1u;
         const uint32_t nby = bdim(J.ny), nbz = bdim(J.nz);
-        unsigned long long* flags1 = J.bflags + relax_words_per_parity(J.nbricks);  // round 1 consumes parity 1
+        uint8_t* flags1 = parity_flags(J.bflags, J.nbricks, 1u);  // round 1 consumes parity 1
         uint32_t x, y, z, last = 0xFFFFFFFFu;
         decompose(c0, J, x, y, z);
         for (int k = 0; k < kCellsPerThread && c0 + k < J.V; ++k, advance(x, y, z, J)) {
@@ -1119,7 +1157,7 @@ __global__ __launch_bounds__(kCellThreads) void k_flood_sub_reseed(Launch L)
                 J.keys[c0 + k] = kUnreachedKey | (key & 3u);
                 const uint32_t id = ((x / kRelaxBrick) * nby + y / kRelaxBrick) * nbz + z / kRelaxBrick;
                 if (id != last) {
-                    atomicOr(flags1 + (id >> 6), 1ull << (id & 63u));
+                    flags1[id] = 1u;
                     last = id;
                 }
             }

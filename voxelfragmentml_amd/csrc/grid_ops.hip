@@ -525,9 +525,10 @@ __global__ __launch_bounds__(256) void k_job_init(Launch L)
     if (threadIdx.x < kStatCount) J->stats[threadIdx.x] = 0;
     if (J->fctl && threadIdx.x < 64) J->fctl[threadIdx.x] = 0;
     if (J->algo == VF_FLOOD && J->bflags) {  // both brick flag parities of the flood rounds
-        const uint32_t n = 2u * relax_words_per_parity(J->nbricks);
-        for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) J->bflags[i] = 0ull;
+        const size_t n = 2u * relax_parity_bytes(J->nbricks) / 16u;
+        for (size_t i = threadIdx.x; i < n; i += blockDim.x) gstore4(J->bflags + 16u * i, make_uint4(0u, 0u, 0u, 0u));
     }
+    if (J->work && threadIdx.x < kFloodWorkSlots) J->work[threadIdx.x * kFloodWorkStride] = 0ull;
 }
 
 // Block per job: stats and flood state into a compact table for one readback.
@@ -536,8 +537,10 @@ __global__ void k_gather(Launch L, uint32_t* out)
     const JobDev* J = L.jobs + blockIdx.x;
     uint32_t* o = out + 16 * (size_t)blockIdx.x;
     const uint32_t t = threadIdx.x;
+    static_assert(kFloodWorkSlots == 64, "one slot per lane");
+    const unsigned long long work = wave_sum_u64(J->active && J->work ? J->work[t * kFloodWorkStride] : 0ull);
     if (t < kStatCount) {
-        const unsigned long long v = J->active ? J->stats[t] : 0ull;
+        const unsigned long long v = t == kStatFloodWork ? work : J->active ? J->stats[t] : 0ull;
         o[2 * t] = (uint32_t)v;
         o[2 * t + 1] = (uint32_t)(v >> 32);
     }

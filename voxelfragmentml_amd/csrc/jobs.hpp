@@ -24,7 +24,7 @@ enum StatSlot : int {
     kStatShellPairs = 2, // (triangle, cell) SAT candidates
     kStatColPairs = 3,   // (triangle, column) parity candidates
     kStatError = 4,      // first error flag raised on the device
-    kStatFloodWork = 5,  // flood work: (sweeps << 32) + brick visits
+    kStatFloodWork = 5,  // flood work: (sweeps << 32) + brick visits (summed from JobDev::work when gathered)
     kStatFloodDone = 6,  // flood relaxation rounds run (0 while running)
     kStatLabels = 7,     // labels >= 2 with a nonzero count
     kStatCount = 8
@@ -80,8 +80,9 @@ struct JobDev {
     uint64_t seed_key;
     uint32_t* keys;         // flood keys, V: kFloodEmptyKey = EMPTY, else (K << 2) | weight (1..3), K = (distance << key_bits) | seed; kFloodUnreachedKey | weight unreached
     uint32_t* sub;          // sub-seed pass (null when the seeds carry one id per fragment): S union-find parents, S keep flags
-    unsigned long long* bflags;  // brick flag bits for even / odd rounds (relax_words_per_parity words each), then the brick liveness words
+    uint8_t* bflags;        // brick flags for even / odd rounds (relax_parity_bytes each, one byte per brick), then the brick liveness words
     uint32_t nbricks;       // relaxation bricks (kRelaxBrick^3 cells each)
+    unsigned long long* work;  // kFloodWorkSlots sums of (sweeps << 32) + brick visits, each on a cache line of its own (null: not counted)
     uint32_t* fctl;         // flood control: [0] round, [1] rounds run once drained (0 = running), [2..3] flags non-empty, [4..5] round started by the compaction of an even / odd round of a chunk
     unsigned long long* stats;  // kStatCount slots
     uint32_t* hist;         // 65536 counts
@@ -206,12 +207,18 @@ inline uint32_t relax_bricks(uint32_t nx, uint32_t ny, uint32_t nz)
     return ((nx + kRelaxBrick - 1) / kRelaxBrick) * ((ny + kRelaxBrick - 1) / kRelaxBrick) *
            ((nz + kRelaxBrick - 1) / kRelaxBrick);
 }
-// 64-bit brick flag words per round parity, and compaction tasks (64 words) of a job
-__host__ __device__ inline uint32_t relax_words_per_parity(uint32_t nbricks) { return (nbricks + 63u) / 64u; }
+// Brick flags: one byte per brick and round parity, in groups of 64 bricks (a lane's share of a compaction
+// task), and compaction tasks (64 groups) of a job.  Bytes, so that a visit flags its neighbours with plain
+// stores: bits needed an atomic each, executed at the memory side, and neighbours along z share a word.
+__host__ __device__ inline uint32_t relax_groups(uint32_t nbricks) { return (nbricks + 63u) / 64u; }
+__host__ __device__ inline size_t relax_parity_bytes(uint32_t nbricks) { return (size_t)relax_groups(nbricks) * 64u; }
 inline uint32_t relax_tasks(uint32_t nx, uint32_t ny, uint32_t nz)
 {
-    return (relax_words_per_parity(relax_bricks(nx, ny, nz)) + 63u) / 64u;
+    return (relax_groups(relax_bricks(nx, ny, nz)) + 63u) / 64u;
 }
+// Work counters of a flood job: a workgroup adds to slot workgroup % kFloodWorkSlots (one address for all of
+// them cost a round of 3000 visits about 30 us: same-address atomics execute one after another).
+constexpr uint32_t kFloodWorkSlots = 64, kFloodWorkStride = 8;  // stride in 64-bit words
 // Brick liveness (bricks holding an occupied cell, whose keys the init writes), after the two flag
 // parities: a bitmap with one 64-bit word per 64 bricks of a brick column (bx, by), bit bz % 64 of word
 // (bx * nby + by) * wpc + bz / 64, then one 32-bit word per brick with the liveness of the brick and its
@@ -225,7 +232,7 @@ inline uint64_t relax_flag_bytes(uint32_t nx, uint32_t ny, uint32_t nz)
 {
     const uint32_t nbx = (nx + kRelaxBrick - 1) / kRelaxBrick, nby = (ny + kRelaxBrick - 1) / kRelaxBrick,
                    nbz = (nz + kRelaxBrick - 1) / kRelaxBrick, nb = relax_bricks(nx, ny, nz);
-    return 16ull * relax_words_per_parity(nb) + 8ull * live_words(nbx, nby, nbz) + 4ull * nb;
+    return 2ull * relax_parity_bytes(nb) + 8ull * live_words(nbx, nby, nbz) + 4ull * nb;
 }
 // Device state of the flood rounds of one launch table.
 struct FloodRoundScratch {
