@@ -71,10 +71,10 @@ static void grid_setup_shape(vf_grid* g, const uint32_t dims[3], const float mn[
     }
     g->V = (uint64_t)dims[0] * dims[1] * dims[2];
     g->labels.ensure(g->V * 2 + 64);
-    g->occ.ensure(g->V + 64);
-    VF_HIP(hipMemsetAsync(g->labels.p, 0, g->V * 2, g->stream));
-    VF_HIP(hipMemsetAsync(g->occ.p, 0, g->V, g->stream));
-    g->labels_from_occ = false;
+    const uint64_t words = occ_words(dims);
+    g->occ.ensure(words * 4 + 64);
+    VF_HIP(hipMemsetAsync(g->occ.p, 0, words * 4, g->stream));
+    g->labels_from_occ = true;  // every cell EMPTY, written when something reads the cells
     g->clean = true;
     g->mc.valid = false;
     JobDev& J = g->job;
@@ -90,12 +90,13 @@ static void grid_setup_shape(vf_grid* g, const uint32_t dims[3], const float mn[
         J.cs[q] = g->cs[q];
     }
     J.labels = g->labels.as<uint16_t>();
-    J.occ = g->occ.as<uint8_t>();
+    J.occ = g->occ.as<uint32_t>();
+    J.inv_ny = 1.0f / (float)dims[1];
     J.stats = g->stats.as<unsigned long long>();
     J.hist = g->hist.as<uint32_t>();
     J.active = 1;
     g->job_dirty = true;
-    uint32_t pre[4] = { 0, grid_tiles(g), 0, brick_count(dims[0], dims[1], dims[2]) };
+    const uint32_t pre[6] = { 0, grid_tiles(g), 0, brick_count(dims[0], dims[1], dims[2]), 0, word_tiles(dims) };
     VF_HIP(hipMemcpyAsync(g->prefix.p, pre, sizeof pre, hipMemcpyHostToDevice, g->stream));
     VF_HIP(hipStreamSynchronize(g->stream));
 }
@@ -114,6 +115,10 @@ Launch grid_launch(vf_grid* g)
     L.njobs = 1;
     L.tile_prefix = g->prefix.as<uint32_t>();
     L.total_tiles = grid_tiles(g);
+    L.wtile_prefix = g->prefix.as<uint32_t>() + 4;
+    L.total_wtiles = word_tiles(g->dims);
+    L.bt_prefix = g->prefix.as<uint32_t>() + 2;
+    L.total_bricks = brick_count(g->dims[0], g->dims[1], g->dims[2]);
     L.s = g->stream;
     return L;
 }
@@ -273,7 +278,9 @@ int vf_occupancy_read(vf_grid* g, uint8_t* out)
     return guard([&] {
         checked(g);
         if (!out) fail(VF_ERR_INVALID_ARG, "out is NULL");
-        VF_HIP(hipMemcpyAsync(out, g->occ.p, g->V, hipMemcpyDeviceToHost, g->stream));
+        g->occ_tmp.ensure(g->V + 64);
+        launch_occ_bytes(grid_launch(g), g->occ_tmp.as<uint8_t>());
+        VF_HIP(hipMemcpyAsync(out, g->occ_tmp.p, g->V, hipMemcpyDeviceToHost, g->stream));
         VF_HIP(hipStreamSynchronize(g->stream));
     });
 }
@@ -315,9 +322,9 @@ int vf_voxelize_device(vf_grid* g, const float* d_xyz, uint32_t nv, const uint32
         if (nt && (!d_xyz || !d_tri)) fail(VF_ERR_INVALID_ARG, "mesh pointer is NULL");
         JobDev& J = g->job;
         const uint64_t words = (uint64_t)J.nx * J.ny * J.wp;
-        g->bits.ensure(words * 8 + 64);
-        J.shell_bits = g->bits.as<uint32_t>();
-        J.toggle_bits = g->bits.as<uint32_t>() + words;
+        g->bits.ensure(words * 4 + 64);
+        J.shell_bits = J.occ;  // the fill leaves the occupancy in place of the shell
+        J.toggle_bits = g->bits.as<uint32_t>();
         J.xyz = d_xyz;
         J.tri = d_tri;
         J.nt = nt;
@@ -326,8 +333,8 @@ int vf_voxelize_device(vf_grid* g, const float* d_xyz, uint32_t nv, const uint32
         // already holds values the new occupancy is merged afterwards.
         const bool merge = !g->clean;
         if (merge) {
-            g->occ_tmp.ensure(g->V + 64);
-            J.occ = g->occ_tmp.as<uint8_t>();
+            g->occ_tmp.ensure(words * 4 + 64);
+            J.shell_bits = g->occ_tmp.as<uint32_t>();
         }
         g->job_dirty = true;
         const uint32_t groups = ceil_div(words, 256);
@@ -351,19 +358,11 @@ int vf_voxelize_device(vf_grid* g, const float* d_xyz, uint32_t nv, const uint32
         launch_voxelize(L, X, g->ctl.as<uint32_t>() + 2, groups, nullptr);
         check_device_error(g, "voxelize");
         if (merge) {
-            // labels = new ? FREE : old, occupancy = old | new
-            std::vector<uint16_t> old(g->V);
-            std::vector<uint8_t> nw(g->V);
+            // labels = new ? FREE : old, occupancy as the labels then say
             grid_materialize(g);
-            VF_HIP(hipMemcpyAsync(old.data(), g->labels.p, g->V * 2, hipMemcpyDeviceToHost, g->stream));
-            VF_HIP(hipMemcpyAsync(nw.data(), g->occ_tmp.p, g->V, hipMemcpyDeviceToHost, g->stream));
-            VF_HIP(hipStreamSynchronize(g->stream));
-            for (uint64_t i = 0; i < g->V; ++i)
-                if (nw[i]) old[i] = kFree;
-            J.occ = g->occ.as<uint8_t>();
-            g->job_dirty = true;
-            VF_HIP(hipMemcpyAsync(g->labels.p, old.data(), g->V * 2, hipMemcpyHostToDevice, g->stream));
-            launch_labels_to_occ(grid_launch(g));
+            Launch M = grid_launch(g);
+            launch_occ_free(M, J.shell_bits);
+            launch_labels_to_occ(M);
             g->labels_from_occ = false;
         } else {
             g->labels_from_occ = true;
@@ -406,7 +405,7 @@ int vf_seed_uniform(vf_grid* g, uint32_t S, uint64_t seed, int location, vf_seed
         g->job.seed_key = seed;
         g->job.seed_location = location;
         g->job_dirty = true;
-        const uint32_t tiles = grid_tiles(g);
+        const uint32_t tiles = word_tiles(g->dims);
         g->seed_tile_cnt.ensure((size_t)tiles * 4 + 64);
         g->seed_tile_off.ensure(((size_t)tiles + 1) * 8 + 64);
         g->scan_tmp.ensure(scan_tmp_bytes(tiles) + 64);
@@ -504,7 +503,9 @@ int vf_fracture_naive(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
         g->job.algo = VF_NAIVE;
         g->job.naive_key64 = kf.key64;
         g->job_dirty = true;
-        launch_naive(grid_launch(g), key64);
+        Launch L = grid_launch(g);
+        launch_clear_labels(L);
+        launch_naive(L, key64);
         g->labels_from_occ = false;
         g->mc.valid = false;
         VF_HIP(hipStreamSynchronize(g->stream));
@@ -617,6 +618,7 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
             if (g->pinned[1] == 0) g->last_flood_levels += drain();  // regions were freed: second growth
         }
         check_device_error(g, "flood");
+        launch_clear_labels(L);
         launch_flood_finish(L);
         g->labels_from_occ = false;
         g->mc.valid = false;
@@ -635,8 +637,7 @@ int vf_detect_boundaries(vf_grid* g, int size)
             g->job_dirty = true;
         }
         Launch L = grid_launch(g);
-        if (size <= 1) launch_boundaries_tiled(L, g->prefix.as<uint32_t>() + 2, brick_count(g->dims[0], g->dims[1], g->dims[2]), false,
-                                              false);
+        if (size <= 1) launch_boundaries_tiled(L, false, false);
         else launch_boundaries(L, size, 0);
         g->mc.valid = false;
         VF_HIP(hipStreamSynchronize(g->stream));
@@ -674,9 +675,8 @@ int vf_erode(vf_grid* g, int convolution, uint32_t size, uint32_t iterations, fl
             g->job_dirty = true;
         }
         Launch L = grid_launch(g);
-        const uint32_t bricks = brick_count(g->dims[0], g->dims[1], g->dims[2]);
         for (uint32_t it = 0; it < iterations; ++it) {
-            launch_boundaries_tiled(L, g->prefix.as<uint32_t>() + 2, bricks, false, false);
+            launch_boundaries_tiled(L, false, false);
             launch_erode_step(L, g->erode_tmp.as<uint16_t>(), g->erode_mask.as<uint8_t>(), (uint32_t)side, limit,
                               probability, noise_seed, g->V);
             VF_HIP(hipMemcpyAsync(g->labels.p, g->erode_tmp.p, g->V * 2, hipMemcpyDeviceToDevice, g->stream));

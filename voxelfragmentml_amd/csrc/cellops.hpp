@@ -1,7 +1,7 @@
 // Device helpers for cell-parallel stages: each thread owns 8 consecutive
 // cells of one job's linear index range (x*ny*nz + y*nz + z), loaded and
-// stored as one 16-byte (uint16 labels) or 8-byte (uint8 occupancy) access
-// when the run is complete, element-wise at the tail.
+// stored as one 16-byte access when the run is complete, element-wise at the
+// tail; or 8 cells of a column, a byte of its occupancy words, in bricks (CellGroup).
 #pragma once
 
 #include <algorithm>
@@ -39,6 +39,16 @@ __device__ inline uint32_t sqrt_rn_bits(uint32_t n)
 }
 
 
+// x / d for x below 2^24, d below 2^16 and inv = 1 / d: a float estimate off by at most one, corrected.
+__device__ inline uint32_t small_div(uint32_t x, uint32_t d, float inv)
+{
+    uint32_t q = (uint32_t)((float)x * inv);
+    const int r = (int)x - (int)(q * d);
+    if (r < 0) --q;
+    else if (r >= (int)d) ++q;
+    return q;
+}
+
 constexpr uint32_t kCellThreads = 256;
 constexpr uint32_t kCellsPerThread = 8;
 static_assert(kCellThreads * kCellsPerThread == kTileCells, "tile shape");
@@ -75,24 +85,69 @@ __device__ inline void store8(uint16_t* p, uint64_t c0, uint64_t V, const uint16
     }
 }
 
-// 8 occupancy bytes packed little-endian into a uint64 (0 beyond V)
-__device__ inline uint64_t load8b(const uint8_t* p, uint64_t c0, uint64_t V)
+// Brick `id` of job J: its first cell.
+struct BrickAt {
+    uint32_t x, y, z;
+};
+__device__ inline BrickAt brick_at(const JobDev& J, uint32_t id)
 {
-    if (c0 + 8 <= V) return *gcast<const uint64_t>(p + c0);
-    uint64_t r = 0;
-    for (int k = 0; k < 8; ++k)
-        if (c0 + k < V) r |= (uint64_t)gcast<const uint8_t>(p)[c0 + k] << (8 * k);
-    return r;
+    const uint32_t tz = (J.nz + kBrickZ - 1u) / kBrickZ, ty = (J.ny + kBrickY - 1u) / kBrickY, t = id / tz;
+    return BrickAt{ t / ty * kBrickX, t % ty * kBrickY, id % tz * kBrickZ };
 }
 
-__device__ inline void store8b(uint8_t* p, uint64_t c0, uint64_t V, uint64_t r)
+// The cells of one thread in a brick: byte tid % 4 of the occupancy word of row tid / 4, i.e. cells z0 .. z0 + n - 1 of
+// column col (n = 8, less at the column's end, 0 outside the grid), linear index c0.
+static_assert(kBrickX * kBrickY * 4 == kCellThreads && kBrickZ == 32, "a thread owns a byte of occupancy");
+struct CellGroup {
+    uint64_t c0;
+    uint32_t col, z0, n;
+};
+__device__ inline CellGroup cell_group(const JobDev& J, const BrickAt& b)
 {
-    if (c0 + 8 <= V) {
-        *gcast<uint64_t>(p + c0) = r;
+    CellGroup g;
+    const uint32_t row = threadIdx.x >> 2, x = b.x + row / kBrickY, y = b.y + row % kBrickY;
+    g.col = x * J.ny + y;
+    g.z0 = b.z + (threadIdx.x & 3u) * 8u;
+    g.n = x < J.nx && y < J.ny && g.z0 < J.nz ? min(8u, J.nz - g.z0) : 0u;
+    g.c0 = (uint64_t)g.col * J.nz + g.z0;
+    return g;
+}
+__device__ inline CellGroup cell_group(const JobDev& J, uint32_t brick) { return cell_group(J, brick_at(J, brick)); }
+// the group's byte of an array of occupancy words
+__device__ inline size_t group_byte(const JobDev& J, const CellGroup& g) { return (size_t)g.col * J.wp * 4u + (g.z0 >> 3); }
+// the group's occupancy bits (0 for a group without cells)
+__device__ inline uint32_t group_occ(const JobDev& J, const CellGroup& g)
+{
+    return g.n ? gcast<const uint8_t>(J.occ)[group_byte(J, g)] : 0u;
+}
+__device__ inline void store_group(uint16_t* p, const CellGroup& g, uint4 q)
+{
+    if (g.n == 8u) {
+        gstore4_cells(p + g.c0, q);
     } else {
-        for (int k = 0; k < 8; ++k)
-            if (c0 + k < V) gcast<uint8_t>(p)[c0 + k] = (uint8_t)(r >> (8 * k));
+        const uint32_t w[4] = { q.x, q.y, q.z, q.w };
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k)
+            if (k < g.n) gcast<uint16_t>(p)[g.c0 + k] = (uint16_t)(w[k >> 1] >> (16u * (k & 1u)));
     }
+}
+__device__ inline uint4 load_group(const uint16_t* p, const CellGroup& g)
+{
+    if (g.n == 8u) return gload4_cells(p + g.c0);
+    uint32_t w[4] = { 0u, 0u, 0u, 0u };
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; ++k)
+        if (k < g.n) w[k >> 1] |= (uint32_t)gcast<const uint16_t>(p)[g.c0 + k] << (16u * (k & 1u));
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+__device__ inline uint4 pack_cells(const uint16_t v[8])
+{
+    return make_uint4((uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16),
+                      (uint32_t)v[4] | ((uint32_t)v[5] << 16), (uint32_t)v[6] | ((uint32_t)v[7] << 16));
+}
+__device__ inline bool occ_bit(const JobDev& J, uint32_t x, uint32_t y, uint32_t z)
+{
+    return (gcast<const uint32_t>(J.occ)[((size_t)x * J.ny + y) * J.wp + (z >> 5)] >> (z & 31u)) & 1u;
 }
 
 // Contiguous tile range of this block (keeps a block on one job for long
@@ -219,27 +274,6 @@ __device__ inline void walk_tile_runs_strided(const Launch& L, const uint32_t* p
             const uint32_t n = min(t1, sp[lo + 1]) - t;
             f(*sJ, lo, t - sp[lo], n);
             t += n;
-        }
-    }
-}
-
-__device__ inline void decompose(uint64_t c, const JobDev& J, uint32_t& x, uint32_t& y, uint32_t& z)
-{
-    uint32_t yz = J.ny * J.nz;
-    uint32_t cc = (uint32_t)c;
-    x = cc / yz;
-    uint32_t r = cc - x * yz;
-    y = r / J.nz;
-    z = r - y * J.nz;
-}
-
-__device__ inline void advance(uint32_t& x, uint32_t& y, uint32_t& z, const JobDev& J)
-{
-    if (++z == J.nz) {
-        z = 0;
-        if (++y == J.ny) {
-            y = 0;
-            ++x;
         }
     }
 }

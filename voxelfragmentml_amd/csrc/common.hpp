@@ -162,6 +162,28 @@ __device__ inline uint2 gload2(const void* p)
     const vf_u32x2 v = *(const VF_AS_GLOBAL vf_u32x2*)p;
     return make_uint2(v.x, v.y);
 }
+// the same at any cell's address: rows of uint16 cells start on 2-byte, rows of keys on 4-byte boundaries where
+// nz is odd (global accesses need no alignment on gfx950)
+typedef vf_u32x4 vf_u32x4_a2 __attribute__((aligned(2)));
+typedef vf_u32x4 vf_u32x4_a4 __attribute__((aligned(4)));
+__device__ inline void gstore4_cells(uint16_t* p, uint4 q)
+{
+    *(VF_AS_GLOBAL vf_u32x4_a2*)p = vf_u32x4_a2{ q.x, q.y, q.z, q.w };
+}
+__device__ inline uint4 gload4_cells(const uint16_t* p)
+{
+    const vf_u32x4 v = *(const VF_AS_GLOBAL vf_u32x4_a2*)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ inline uint4 gload4_words(const VF_AS_GLOBAL uint32_t* p)
+{
+    const vf_u32x4 v = *(const VF_AS_GLOBAL vf_u32x4_a4*)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ inline void gstore4_words(VF_AS_GLOBAL uint32_t* p, uint4 q)
+{
+    *(VF_AS_GLOBAL vf_u32x4_a4*)p = vf_u32x4_a4{ q.x, q.y, q.z, q.w };
+}
 __device__ inline void gstore2(void* p, uint2 q) { *(VF_AS_GLOBAL vf_u32x2*)p = vf_u32x2{ q.x, q.y }; }
 
 __host__ __device__ inline uint32_t fmix32(uint32_t h)

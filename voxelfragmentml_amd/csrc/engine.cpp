@@ -21,7 +21,7 @@ constexpr size_t kAlign = 256;
 inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
 struct Layout {
-    size_t labels, occ, bits, seeds, hist, stats, fctl, keys, bricks, work, sub, erode, mask, mesh_xyz, mesh_tri, total;
+    size_t labels, bits, seeds, hist, stats, fctl, keys, bricks, sums, sub, erode, mask, mesh_xyz, mesh_tri, total;
     uint64_t V, words;
 };
 
@@ -57,15 +57,14 @@ Layout layout_of(const vf_job& j)
     const bool flood = j.algorithm == VF_FLOOD;
     size_t o = 0;
     L.labels = o; o = align_up(o + L.V * 2);
-    L.occ = o; o = align_up(o + L.V);
-    L.bits = o; o = align_up(o + L.words * 8);
+    L.bits = o; o = align_up(o + L.words * 8);  // shell (then occupancy) and toggle bits
     L.seeds = o; o = align_up(o + (size_t)std::max<uint32_t>(seed_total(j), 1) * 16);
     L.hist = o; o = align_up(o + 65536 * 4);
     L.stats = o; o = align_up(o + kStatCount * 8);
     L.fctl = o; o = align_up(o + 64 * 4);
     L.keys = o; if (flood) o = align_up(o + L.V * 4);
     L.bricks = o; if (flood) o = align_up(o + relax_flag_bytes(j.dims[0], j.dims[1], j.dims[2]));
-    L.work = o; if (flood) o = align_up(o + 8ull * kFloodWorkSlots * kFloodWorkStride);
+    L.sums = o; o = align_up(o + kSumBytes);
     L.sub = o; if (needs_sub(j)) o = align_up(o + 8ull * seed_total(j));  // union-find parents + keep flags
     L.erode = o; if (j.erode) o = align_up(o + L.V * 2);                          // erosion output grid
     L.mask = o; if (j.erode) o = align_up(o + (size_t)kMaxErosionSide * kMaxErosionSide * kMaxErosionSide);
@@ -80,7 +79,7 @@ Layout layout_of(const vf_job& j)
 size_t job_footprint(const vf_job& j)
 {
     const Layout Lo = layout_of(j);
-    const uint64_t tiles = ceil_div(Lo.V, kTileCells);
+    const uint64_t tiles = ceil_div(Lo.words, kTileWords);
     // the job's share of the engine scratch its launches use: the voxelizer's per-triangle setup records,
     // work counts and their 64-bit scans, the seed-candidate counts per tile and their scan (each buffer
     // at least 256 bytes plus 64 bytes of slack), the launch table's descriptor and prefix entries (with
@@ -88,7 +87,7 @@ size_t job_footprint(const vf_job& j)
     // ceil(tasks / 8) x 4096 eight-byte entries: 64 KiB per task, plus one rounding step)
     const size_t front = (size_t)j.nt * (sizeof(TriSetup) + 8 + 16) + scan_tmp_bytes(2ull * j.nt) +
                          (size_t)tiles * 12 + scan_tmp_bytes(tiles) + 6 * (256 + 64);
-    const size_t table = sizeof(JobDev) + 16 * 4 + 6 * 4 + 9 * kAlign;
+    const size_t table = 3 * sizeof(JobDev) + 16 * 4 + 11 * 4 + 10 * kAlign;
     const size_t lists = j.algorithm == VF_FLOOD
                              ? 65536ull * relax_tasks(j.dims[0], j.dims[1], j.dims[2]) + 2ull * kFloodXcds * 4096 * 8
                              : 0;
@@ -217,9 +216,10 @@ void Engine::alloc(EJob& e)
         d.cs[q] = (j.aabb_max[q] - j.aabb_min[q]) / (float)j.dims[q];  // RegularGrid::setAABB
     }
     d.labels = reinterpret_cast<uint16_t*>(base + Lo.labels);
-    d.occ = base + Lo.occ;
     d.shell_bits = reinterpret_cast<uint32_t*>(base + Lo.bits);
     d.toggle_bits = d.shell_bits + Lo.words;
+    d.occ = d.shell_bits;
+    d.inv_ny = 1.0f / (float)j.dims[1];
     d.seeds = reinterpret_cast<uint4*>(base + Lo.seeds);
     d.S = j.num_seeds + (j.extra_seeds ? j.num_seeds + j.extra_seeds : 0);  // nearSeeds resets it on the device
     d.S_draw = j.seeds ? 0 : j.num_seeds;  // the caller's seeds are copied, not drawn
@@ -240,6 +240,7 @@ void Engine::alloc(EJob& e)
     d.seed_location = j.seed_location;
     d.seed_key = j.seed;
     d.stats = reinterpret_cast<unsigned long long*>(base + Lo.stats);
+    d.sums = reinterpret_cast<unsigned long long*>(base + Lo.sums);
     d.hist = reinterpret_cast<uint32_t*>(base + Lo.hist);
     d.fctl = reinterpret_cast<uint32_t*>(base + Lo.fctl);
     d.active = 1;
@@ -248,7 +249,6 @@ void Engine::alloc(EJob& e)
     if (j.algorithm == VF_FLOOD) {
         d.keys = reinterpret_cast<uint32_t*>(base + Lo.keys);
         d.bflags = base + Lo.bricks;
-        d.work = reinterpret_cast<unsigned long long*>(base + Lo.work);
         d.nbricks = relax_bricks(d.nx, d.ny, d.nz);
         d.sub = needs_sub(j) ? reinterpret_cast<uint32_t*>(base + Lo.sub) : nullptr;
     } else {
@@ -279,6 +279,7 @@ void Engine::alloc(EJob& e)
     }
     e.words = Lo.words;
     e.tiles = ceil_div(Lo.V, kTileCells);
+    e.wtiles = ceil_div(Lo.words, kTileWords);
     e.groups = ceil_div(Lo.words, 256);
 }
 
@@ -305,7 +306,8 @@ Table* Engine::make_table(const std::vector<EJob*>& js)
     t->jobs = js;
     const size_t o_jobs = 0;
     const size_t o_tile = align_up(o_jobs + n * sizeof(JobDev));
-    const size_t o_tri = align_up(o_tile + (n + 1) * 4);
+    const size_t o_wtile = align_up(o_tile + (n + 1) * 4);
+    const size_t o_tri = align_up(o_wtile + (n + 1) * 4);
     const size_t o_col = align_up(o_tri + (n + 1) * 4);
     const size_t o_bt = align_up(o_col + (n + 1) * 4);
     const size_t o_gather = align_up(o_bt + (n + 1) * 4);
@@ -321,16 +323,18 @@ Table* Engine::make_table(const std::vector<EJob*>& js)
     auto* lp = reinterpret_cast<uint32_t*>(img.data() + o_local);
     auto* jd = reinterpret_cast<JobDev*>(img.data() + o_jobs);
     auto* tp = reinterpret_cast<uint32_t*>(img.data() + o_tile);
+    auto* wt = reinterpret_cast<uint32_t*>(img.data() + o_wtile);
     auto* rp = reinterpret_cast<uint32_t*>(img.data() + o_tri);
     auto* cp = reinterpret_cast<uint32_t*>(img.data() + o_col);
     auto* bp = reinterpret_cast<uint32_t*>(img.data() + o_bt);
     auto* fp = reinterpret_cast<uint32_t*>(img.data() + o_done);
-    uint64_t tiles = 0, tris = 0, groups = 0, btiles = 0, fchunks = 0;
+    uint64_t tiles = 0, wtiles = 0, tris = 0, groups = 0, btiles = 0, fchunks = 0;
     uint32_t max_edge = 1;
     for (uint32_t i = 0; i < n; ++i) {
         EJob& e = *js[i];
         jd[i] = e.d;
         tp[i] = (uint32_t)tiles;
+        wt[i] = (uint32_t)wtiles;
         rp[i] = (uint32_t)tris;
         cp[i] = (uint32_t)groups;
         bp[i] = (uint32_t)btiles;
@@ -340,6 +344,7 @@ Table* Engine::make_table(const std::vector<EJob*>& js)
         max_edge = std::max(max_edge, std::max(e.d.nx, std::max(e.d.ny, e.d.nz)));
         t->any_wide |= e.d.bsize > 1;
         tiles += e.tiles;
+        wtiles += e.wtiles;
         tris += e.d.nt;
         groups += e.groups;
         t->any_flood |= e.d.algo == VF_FLOOD;
@@ -355,6 +360,7 @@ Table* Engine::make_table(const std::vector<EJob*>& js)
         xj[i].seeds = e.d.seeds + e.d.xoff;
         t->any_extra |= e.d.extra != 0;
         t->any_near |= e.d.impacts != 0;
+        t->any_located |= e.d.seed_location != VF_SEED_BOTH;
         t->any_sub |= e.d.sub != nullptr;
         ej[i] = e.d;
         ej[i].bsize = 1;
@@ -364,9 +370,10 @@ Table* Engine::make_table(const std::vector<EJob*>& js)
         lp[4 * i + 2] = 0;
         lp[4 * i + 3] = brick_count(e.d.nx, e.d.ny, e.d.nz);
     }
-    if (tiles > 0xFFFFFFFFull || tris > 0xFFFFFFFFull || groups > 0xFFFFFFFFull || fchunks > 0xFFFFFFFFull)
+    if (tiles > 0xFFFFFFFFull || wtiles > 0xFFFFFFFFull || btiles > 0xFFFFFFFFull || tris > 0xFFFFFFFFull || groups > 0xFFFFFFFFull || fchunks > 0xFFFFFFFFull)
         fail(VF_ERR_INVALID_ARG, "table too large for 32-bit prefixes");
     tp[n] = (uint32_t)tiles;
+    wt[n] = (uint32_t)wtiles;
     rp[n] = (uint32_t)tris;
     cp[n] = (uint32_t)groups;
     bp[n] = (uint32_t)btiles;
@@ -379,11 +386,13 @@ Table* Engine::make_table(const std::vector<EJob*>& js)
     t->L.njobs = n;
     t->L.tile_prefix = reinterpret_cast<const uint32_t*>(base + o_tile);
     t->L.total_tiles = (uint32_t)tiles;
+    t->L.wtile_prefix = reinterpret_cast<const uint32_t*>(base + o_wtile);
+    t->L.total_wtiles = (uint32_t)wtiles;
     t->L.s = s;
     t->tri_prefix = reinterpret_cast<const uint32_t*>(base + o_tri);
     t->col_prefix = reinterpret_cast<const uint32_t*>(base + o_col);
-    t->bt_prefix = reinterpret_cast<const uint32_t*>(base + o_bt);
-    t->total_btiles = (uint32_t)btiles;
+    t->L.bt_prefix = reinterpret_cast<const uint32_t*>(base + o_bt);
+    t->L.total_bricks = (uint32_t)btiles;
     t->total_tris = (uint32_t)tris;
     t->total_groups = (uint32_t)groups;
     t->gather = reinterpret_cast<uint32_t*>(base + o_gather);
@@ -420,9 +429,9 @@ void Engine::reserve_front(const Table& t)
     vox_setup_.ensure((size_t)std::max<uint32_t>(nt, 1) * sizeof(TriSetup), cache_);
     vox_counts_.ensure((size_t)std::max<uint32_t>(nt, 1) * 8, cache_);
     vox_shell_off_.ensure((2 * (size_t)nt + 1) * 8, cache_);
-    scan_tmp_.ensure(std::max(scan_tmp_bytes(2 * (uint64_t)nt), scan_tmp_bytes(t.L.total_tiles)) + 64, cache_);
-    seed_cnt_.ensure((size_t)t.L.total_tiles * 4 + 64, cache_);
-    seed_off_.ensure(((size_t)t.L.total_tiles + 1) * 8 + 64, cache_);
+    scan_tmp_.ensure(std::max(scan_tmp_bytes(2 * (uint64_t)nt), scan_tmp_bytes(t.L.total_wtiles)) + 64, cache_);
+    seed_cnt_.ensure((size_t)t.L.total_wtiles * 4 + 64, cache_);
+    seed_off_.ensure(((size_t)t.L.total_wtiles + 1) * 8 + 64, cache_);
 }
 
 void Engine::release_front()
@@ -447,6 +456,7 @@ void Engine::front(Table& t, bool split)
     for (EJob* e : t.jobs) e->fronted = true;
     const Launch& L = t.L;
     launch_job_init(L);
+    launch_clear_labels(L);
     VoxScratch X;
     const uint32_t nt = t.total_tris;
     X.setup = vox_setup_.as<TriSetup>();
@@ -457,13 +467,13 @@ void Engine::front(Table& t, bool split)
     X.scan_tmp = scan_tmp_.p;
     X.scan_tmp_bytes = scan_tmp_.bytes;
     launch_voxelize(L, X, t.col_prefix, t.total_groups, seed_cnt_.as<uint32_t>());  // counts tiles of VF_SEED_BOTH jobs
-    launch_seed_count(L, seed_cnt_.as<uint32_t>(), true);
-    scan_exclusive_u32_to_u64(seed_cnt_.as<uint32_t>(), seed_off_.as<unsigned long long>(), L.total_tiles, scan_tmp_.p, s);
+    if (t.any_located) launch_seed_count(L, seed_cnt_.as<uint32_t>(), true);
+    scan_exclusive_u32_to_u64(seed_cnt_.as<uint32_t>(), seed_off_.as<unsigned long long>(), L.total_wtiles, scan_tmp_.p, s);
     launch_seed_pick(L, seed_off_.as<unsigned long long>());
     if (t.any_near) launch_seed_near_jobs(L);  // nearSeeds after the fragment seeds
     if (t.any_extra) {  // mergeSeeds: the extra draw over all occupied cells, then the merge
         launch_seed_count(t.xL, seed_cnt_.as<uint32_t>(), false);
-        scan_exclusive_u32_to_u64(seed_cnt_.as<uint32_t>(), seed_off_.as<unsigned long long>(), L.total_tiles, scan_tmp_.p, s);
+        scan_exclusive_u32_to_u64(seed_cnt_.as<uint32_t>(), seed_off_.as<unsigned long long>(), L.total_wtiles, scan_tmp_.p, s);
         launch_seed_pick(t.xL, seed_off_.as<unsigned long long>());
         launch_seed_merge(L);
     }
@@ -517,7 +527,7 @@ void Engine::post(Table& t)
     const Launch& L = t.L;
     if (t.any_flood) launch_flood_finish(L);
     if (t.any_erode) erode(t);
-    launch_boundaries_tiled(L, t.bt_prefix, t.total_btiles, t.any_wide, true);  // + grid checksum
+    launch_boundaries_tiled(L, t.any_wide, true);  // + grid checksum
     launch_hist_summary(L);
     launch_gather(L, t.gather);
 }
@@ -535,9 +545,10 @@ void Engine::erode(Table& t)
         one.njobs = 1;
         one.tile_prefix = t.local_prefix + 4 * i;
         one.total_tiles = e.tiles;
-        const uint32_t bricks = brick_count(e.d.nx, e.d.ny, e.d.nz);
+        one.bt_prefix = t.local_prefix + 4 * i + 2;
+        one.total_bricks = brick_count(e.d.nx, e.d.ny, e.d.nz);
         for (uint32_t it = 0; it < e.spec.erosion_iterations; ++it) {
-            launch_boundaries_tiled(one, t.local_prefix + 4 * i + 2, bricks, false, false);
+            launch_boundaries_tiled(one, false, false);
             launch_erode_step(one, e.erode_out, e.erode_mask, e.erode_side, e.erode_limit, e.spec.erosion_probability,
                               e.spec.erosion_seed, e.d.V);
             VF_HIP(hipMemcpyAsync(e.d.labels, e.erode_out, e.d.V * 2, hipMemcpyDeviceToDevice, s));

@@ -28,7 +28,7 @@ struct EJob {
     void* mem = nullptr;             // one device block per job
     size_t bytes = 0;
     uint64_t words = 0;
-    uint32_t tiles = 0, groups = 0;
+    uint32_t tiles = 0, wtiles = 0, groups = 0;
     vf_result res{};
     uint64_t ticket = 0;
     double t_submit = 0, t_admit = 0;
@@ -59,8 +59,6 @@ struct Table {
     const uint32_t* tri_prefix = nullptr;
     const uint32_t* col_prefix = nullptr;
     uint32_t total_tris = 0, total_groups = 0;
-    const uint32_t* bt_prefix = nullptr;  // boundary bricks per job
-    uint32_t total_btiles = 0;
     bool any_wide = false;                // some job uses a boundary window wider than 1
     uint32_t* gather = nullptr;       // 16 words per job
     FloodRoundScratch flood{};      // chunk prefix + worklists of the flood rounds
@@ -68,6 +66,7 @@ struct Table {
     void* flood_lists = nullptr;    // separate allocation of flood.lists
     size_t dev_bytes = 0, list_bytes = 0;  // class sizes of the two blocks
     bool any_flood = false, any_naive32 = false, any_naive64 = false;
+    bool any_located = false;             // some job seeds on the surface or inside only
     bool any_extra = false, any_sub = false, any_erode = false, any_near = false;
     Launch xL{};                          // the jobs as their extra-seed draw sees them
     const JobDev* ejobs = nullptr;        // the jobs as their erosion passes see them (boundary size 1)

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256) void k_flood_seed(Launch L)
         const uint4 q = J->seeds[s];
         const size_t c = ((size_t)q.x * J->ny + q.y) * J->nz + q.z;
         if (J->keys[c] != seed_key(s, c)) continue;
-        J->occ[c] = 1;
+        atomicOr(J->occ + ((size_t)q.x * J->ny + q.y) * J->wp + (q.z >> 5), 1u << (q.z & 31u));
         // bricks of the 3x3x3 neighbourhood: at most two brick indices per axis
         const uint32_t bx0 = (q.x ? q.x - 1 : 0) / kRelaxBrick, bx1 = min(q.x + 1, J->nx - 1) / kRelaxBrick;
         const uint32_t by0 = (q.y ? q.y - 1 : 0) / kRelaxBrick, by1 = min(q.y + 1, J->ny - 1) / kRelaxBrick;
@@ -249,7 +249,7 @@ struct RelaxJob {
     uint32_t par;               // parity of the round
     VF_AS_GLOBAL uint32_t* keys;
     VF_AS_GLOBAL uint32_t* ctl;  // the job's control words
-    unsigned long long* work;   // its work counters
+    unsigned long long* sums;   // its spread statistics
     uint8_t* flags;             // brick flags of both parities, then the liveness words and neighbour masks
     VF_AS_GLOBAL uint8_t* nxt;  // brick flags for the next round
     const VF_AS_GLOBAL uint32_t* nmask;  // per brick: liveness of the brick and its 26 neighbours
@@ -486,12 +486,12 @@ __device__ inline uint32_t relax_brick(const RelaxJob& R, uint32_t brick, uint32
 
     // write back the rows with a dropped cell, whole: the other cells rewrite the values they hold
     // (a brick is visited at most once per round, so nothing else writes them meanwhile); two
-    // 16-byte stores where the row is aligned and complete, else cell by cell within the grid
+    // 16-byte stores where the row is complete, else cell by cell within the grid
     if (changed) {
         const uint32_t row = (((uint32_t)X0 + x) * ny + ((uint32_t)Y0 + y)) * nz + (uint32_t)Z0;
-        if ((uint32_t)Z0 + 8u <= nz && (nz & 3u) == 0) {
-            *(VF_AS_GLOBAL vf_u32x4*)(R.keys + row) = vf_u32x4{ k[0], k[1], k[2], k[3] };
-            *(VF_AS_GLOBAL vf_u32x4*)(R.keys + row + 4) = vf_u32x4{ k[4], k[5], k[6], k[7] };
+        if ((uint32_t)Z0 + 8u <= nz) {
+            gstore4_words(R.keys + row, make_uint4(k[0], k[1], k[2], k[3]));
+            gstore4_words(R.keys + row + 4, make_uint4(k[4], k[5], k[6], k[7]));
         } else {
 #pragma unroll
             for (int z = 0; z < 8; ++z)
@@ -546,7 +546,7 @@ __device__ inline void load_relax_fields(const JobDev* J, RelaxJob& R)
     R.keys = gcast<uint32_t>(uni_ptr(J->keys));
     R.ctl = gcast<uint32_t>(uni_ptr(J->fctl));
     R.flags = uni_ptr(J->bflags);
-    R.work = uni_ptr(J->work);
+    R.sums = uni_ptr(J->sums);
     R.nmask = gcast<const uint32_t>(reinterpret_cast<const uint32_t*>(live_base(R.flags, R.nb) + live_words(R.nbx, R.nby, R.nbz)));
     R.n26 = uni((uint32_t)J->neighbourhood) != 6u;
 }
@@ -728,7 +728,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
     auto flush = [&]() {
         if (!work) return;
         if (lane == 0) {
-            if (R.work) atomicAdd(R.work + (blockIdx.x % kFloodWorkSlots) * kFloodWorkStride, work);
+            if (R.sums) atomicAdd(R.sums + (blockIdx.x % kSumSlots) * kStatCount + kStatFloodWork, work);
             if (activated) R.ctl[2 + (R.par ^ 1u)] = 1u;
             if (error) atomicOr(reinterpret_cast<unsigned int*>(R.J->stats + kStatError), (unsigned int)kDevErrRelax);
         }
@@ -779,26 +779,19 @@ __global__ __launch_bounds__(1024) void k_flood_plan(Launch L)
 // its keys are written (EMPTY, or unreached with the cell's weight).  The keys of the other bricks
 // (most of a vessel's box) are never written and never read: the relaxation takes the cells of
 // bricks whose bit is clear as EMPTY, and the other kernels read a key only where the cell's
-// occupancy byte is set.
+// occupancy bit is set.
 //
-// One wave per bitmap word, i.e. per column chunk (bx, by, 64 bricks along z).  First lane l reads
-// brick bz = 64 * chunk + l over the column's 64 rows (x, y), each load of the wave 512 contiguous
-// bytes of one row, and packs its 512 occupancy bits into 16 words in LDS.  Then the live bricks are
+// One wave per bitmap word, i.e. per column chunk (bx, by, 64 bricks along z).  A brick's 8 cells of a row are
+// one byte of the row's occupancy, so lane l reads the 64 bytes of brick bz = 64 * chunk + l, each load of the
+// wave 64 contiguous bytes of one row, and keeps them packed in 16 words in LDS.  Then the live bricks are
 // written one after another, lane x * 8 + y writing row (x, y) of the brick from the packed bits.
 // Every word of the bitmap is written whole.  A job's words are dealt over the 64 slots of each of
-// its compaction tasks (a task is 64 flag groups).
+// its compaction tasks (a task is 64 flag groups).  Bound by HBM and the latency of a wave's loads: 512^3 98 -> 62 us,
+// 203x150x177 (whose rows of bytes were never aligned) 260 -> 29 us, reading bits instead of bytes.
 constexpr uint32_t kInitBitStride = 65;  // LDS words between a wave's packed-bit planes (odd: no bank conflicts)
-
-// one bit per byte of v: bit k set iff byte k is not zero
-__device__ inline uint32_t nonzero_bytes4(uint32_t v)
-{
-    const uint32_t h = ((((v & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | v) & 0x80808080u) >> 7;  // 0 or 1 per byte
-    return (h * 0x01020408u) >> 24;  // byte k lands on bit 24 + k; the other products fall on distinct lower bits
-}
 
 __global__ __launch_bounds__(256) void k_flood_init(Launch L, const uint32_t* task_prefix, uint32_t total_tasks)
 {
-    constexpr uint32_t kRows = 16;  // rows per step of the packing pass: their loads are issued together
     __shared__ uint32_t packed[4 * 16 * kInitBitStride];
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t* pw = packed + (threadIdx.x >> 6) * 16u * kInitBitStride;  // this wave's 16 planes
@@ -814,62 +807,33 @@ __global__ __launch_bounds__(256) void k_flood_init(Launch L, const uint32_t* ta
         const uint32_t nwords = bdim(nx) * nby * wpc;
         const uint64_t noise_seed = ((uint64_t)uni((uint32_t)(J->noise_seed >> 32)) << 32) | uni((uint32_t)J->noise_seed);
         const VF_AS_GLOBAL uint8_t* occ = gcast<const uint8_t>(uni_ptr(J->occ));
+        const uint32_t rowb = uni(J->wp) * 4u;  // occupancy bytes of a row
         VF_AS_GLOBAL uint32_t* keys = gcast<uint32_t>(uni_ptr(J->keys));
         VF_AS_GLOBAL unsigned long long* live =
             gcast<unsigned long long>(live_base(uni_ptr(J->bflags), uni(J->nbricks)));
-        const bool quads = (nz & 3u) == 0u;  // rows of full bricks start on 4-cell boundaries
         for (uint32_t w = g - t0 * 64u; w < nwords; w += nslots) {
             const uint32_t chunk = w % wpc, col = w / wpc, by = col % nby, bx = col / nby;
-            // packing: lane l holds brick bz = 64 * chunk + l, cells z0 .. z0 + 7 of each row.  With rows of
-            // a multiple of 4 cells every load is unconditional (no wait between rows): two 4-cell loads at
-            // addresses clamped into the row, masked where they leave the brick column or the grid.
-            const uint32_t bz = chunk * 64u + lane, z0 = bz * kRelaxBrick;
-            const bool inz = bz < nbz;
+            // packing: lane l holds brick bz = 64 * chunk + l, a byte of each row; addresses are clamped into the
+            // grid so that every load is unconditional and all are issued before the first is waited for
+            const uint32_t bz = chunk * 64u + lane, ob = min(bz, nbz - 1u);
+            uint32_t raw[64];
+#pragma unroll
+            for (uint32_t r = 0; r < 64u; ++r) {
+                const uint32_t x = min(bx * kRelaxBrick + (r >> 3), nx - 1u), y = min(by * kRelaxBrick + (r & 7u), ny - 1u);
+                raw[r] = occ[((uint64_t)x * ny + y) * rowb + ob];
+            }
+            __builtin_amdgcn_sched_barrier(0);
             uint32_t bits[16];
-            if (quads) {
-                const uint32_t zlo = min(z0, nz - 4u), zhi = min(z0 + 4u, nz - 4u);
-                const uint32_t mlo = inz ? ~0u : 0u, mhi = inz && z0 + 4u < nz ? ~0u : 0u;
 #pragma unroll
-                for (uint32_t r0 = 0; r0 < 64u; r0 += kRows) {
-                    uint32_t lo[kRows], hi[kRows];
+            for (uint32_t i = 0; i < 16u; ++i) {
+                uint32_t word = 0;
 #pragma unroll
-                    for (uint32_t r = 0; r < kRows; ++r) {
-                        const uint32_t x = bx * kRelaxBrick + ((r0 + r) >> 3), y = by * kRelaxBrick + ((r0 + r) & 7u);
-                        const uint64_t base = ((uint64_t)min(x, nx - 1u) * ny + min(y, ny - 1u)) * nz;
-                        lo[r] = *(const VF_AS_GLOBAL uint32_t*)(occ + base + zlo);
-                        hi[r] = *(const VF_AS_GLOBAL uint32_t*)(occ + base + zhi);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);  // every load of the step is issued before the first wait
-#pragma unroll
-                    for (uint32_t r = 0; r < kRows; ++r) {
-                        const uint32_t x = bx * kRelaxBrick + ((r0 + r) >> 3), y = by * kRelaxBrick + ((r0 + r) & 7u);
-                        const uint32_t rm = x < nx && y < ny ? ~0u : 0u;
-                        lo[r] &= mlo & rm;
-                        hi[r] &= mhi & rm;
-                    }
-#pragma unroll
-                    for (uint32_t r = 0; r < kRows; r += 4) {
-                        uint32_t word = 0;
-#pragma unroll
-                        for (uint32_t q = 0; q < 4u; ++q)
-                            word |= (nonzero_bytes4(lo[r + q]) | (nonzero_bytes4(hi[r + q]) << 4)) << (8u * q);
-                        bits[(r0 + r) >> 2] = word;
-                    }
+                for (uint32_t q = 0; q < 4u; ++q) {
+                    const uint32_t r = 4u * i + q;
+                    const bool in = bx * kRelaxBrick + (r >> 3) < nx && by * kRelaxBrick + (r & 7u) < ny;  // uniform
+                    word |= (in ? raw[r] : 0u) << (8u * q);
                 }
-            } else {
-                const uint32_t zn = inz ? min(kRelaxBrick, nz - z0) : 0u;
-#pragma unroll
-                for (uint32_t i = 0; i < 16u; ++i) bits[i] = 0u;
-                for (uint32_t r = 0; r < 64u; ++r) {
-                    const uint32_t x = bx * kRelaxBrick + (r >> 3), y = by * kRelaxBrick + (r & 7u);
-                    if (x >= nx || y >= ny) continue;
-                    const uint64_t c = ((uint64_t)x * ny + y) * nz + z0;
-                    uint32_t b8 = 0;
-                    for (uint32_t k = 0; k < zn; ++k) b8 |= (occ[c + k] ? 1u : 0u) << k;
-#pragma unroll
-                    for (uint32_t i = 0; i < 16u; ++i)
-                        if (i == (r >> 2)) bits[i] |= b8 << (8u * (r & 3u));
-                }
+                bits[i] = bz < nbz ? word : 0u;
             }
             uint32_t any = 0;
 #pragma unroll
@@ -901,9 +865,9 @@ __global__ __launch_bounds__(256) void k_flood_init(Launch L, const uint32_t* ta
                     for (uint32_t k = 0; k < 8u; ++k)
                         if ((b8 >> k) & 1u) key[k] = kUnreachedKey | flood_weight(noise_seed, (uint32_t)(c + k), amp);
                 }
-                if (zr == kRelaxBrick && quads) {
-                    *(VF_AS_GLOBAL vf_u32x4*)(keys + c) = vf_u32x4{ key[0], key[1], key[2], key[3] };
-                    *(VF_AS_GLOBAL vf_u32x4*)(keys + c + 4) = vf_u32x4{ key[4], key[5], key[6], key[7] };
+                if (zr == kRelaxBrick) {
+                    gstore4_words(keys + c, make_uint4(key[0], key[1], key[2], key[3]));
+                    gstore4_words(keys + c + 4, make_uint4(key[4], key[5], key[6], key[7]));
                 } else {
                     for (uint32_t k = 0; k < zr; ++k) keys[c + k] = key[k];
                 }
@@ -913,13 +877,16 @@ __global__ __launch_bounds__(256) void k_flood_init(Launch L, const uint32_t* ta
     }
 }
 
+// Labels of the occupied cells from their keys (launch_clear_labels has written the others).  Bound by HBM and the
+// latency of two dependent loads; 512^3: 86 us reading an occupancy byte and writing a label for every cell, 49 us and
+// 35 us of clearing by bricks, which batches share with the naive jobs.
 __global__ __launch_bounds__(kCellThreads) void k_flood_finish(Launch L)
 {
-    constexpr uint32_t kRun = 2;  // tiles per step: all key loads are issued before any label is written
+    constexpr uint32_t kRun = 4;  // bricks per step: all key loads are issued before any label is written
     __shared__ JobDev sJ;
     __shared__ uint16_t lab[kMaxDeviceSeeds];  // seed index -> 8-bit fragment label of the staged job
     uint32_t staged = 0xFFFFFFFFu;
-    walk_tile_runs<kRun>(L, L.tile_prefix, L.total_tiles, &sJ, [&](const JobDev& J, uint32_t j, uint32_t local, uint32_t n) {
+    walk_tile_runs<kRun>(L, L.bt_prefix, L.total_bricks, &sJ, [&](const JobDev& J, uint32_t j, uint32_t brick, uint32_t n) {
         if (!J.active || J.algo != VF_FLOOD) return;
         if (j != staged) {  // block-uniform
             for (uint32_t i = threadIdx.x; i < J.S && i < kMaxDeviceSeeds; i += blockDim.x)
@@ -927,45 +894,45 @@ __global__ __launch_bounds__(kCellThreads) void k_flood_finish(Launch L)
             __syncthreads();
             staged = j;
         }
-        const uint64_t V = J.V;
         const uint32_t mask = (1u << J.key_bits) - 1u;
-        // a cell's key is EMPTY exactly where its occupancy byte is 0 (the init writes EMPTY there, relax never
-        // lowers an EMPTY key, a seed cell gets its occupancy byte set): keys are read only for the 8-cell
-        // segments that hold an occupied cell, a small part of a vessel's box
-        uint64_t occ[kRun];
+        const auto* keys = gcast<const uint32_t>(J.keys);
+        // a cell's key is EMPTY exactly where its occupancy bit is 0 (the init writes EMPTY there, relax never
+        // lowers an EMPTY key, a seed cell gets its occupancy bit set): keys are read only for the 8-cell
+        // groups that hold an occupied cell, a small part of a vessel's box
+        CellGroup grp[kRun];
+        uint32_t occ[kRun];
 #pragma unroll
         for (uint32_t r = 0; r < kRun; ++r) {
-            const uint64_t c0 = (uint64_t)(local + r) * kTileCells + threadIdx.x * kCellsPerThread;
-            occ[r] = r < n && c0 < V ? load8b(J.occ, c0, V) : 0ull;
+            grp[r] = cell_group(J, brick + min(r, n - 1u));
+            occ[r] = r < n ? group_occ(J, grp[r]) : 0u;
         }
         uint32_t key[kRun][8];
 #pragma unroll
         for (uint32_t r = 0; r < kRun; ++r) {
-            const uint64_t c0 = (uint64_t)(local + r) * kTileCells + threadIdx.x * kCellsPerThread;
-            if (occ[r] == 0ull) {
 #pragma unroll
-                for (int k = 0; k < 8; ++k) key[r][k] = kEmptyKey;
-            } else if (c0 + 8 <= V) {
-                const uint4 a = gload4(J.keys + c0);
-                const uint4 b = gload4(J.keys + c0 + 4);
+            for (int k = 0; k < 8; ++k) key[r][k] = kEmptyKey;
+            if (occ[r] == 0u) continue;
+            if (grp[r].n == 8u) {
+                const uint4 a = gload4_words(keys + grp[r].c0), b = gload4_words(keys + grp[r].c0 + 4);
                 key[r][0] = a.x; key[r][1] = a.y; key[r][2] = a.z; key[r][3] = a.w;
                 key[r][4] = b.x; key[r][5] = b.y; key[r][6] = b.z; key[r][7] = b.w;
             } else {
-                for (int k = 0; k < 8; ++k)
-                    key[r][k] = r < n && c0 + k < V ? gcast<const uint32_t>(J.keys)[c0 + k] : kEmptyKey;
+#pragma unroll
+                for (uint32_t k = 0; k < 8u; ++k)
+                    if (k < grp[r].n) key[r][k] = keys[grp[r].c0 + k];
             }
         }
 #pragma unroll
         for (uint32_t r = 0; r < kRun; ++r) {
-            const uint64_t c0 = (uint64_t)(local + r) * kTileCells + threadIdx.x * kCellsPerThread;
-            if (r >= n || c0 >= V) break;
+            if (!occ[r]) continue;  // EMPTY already (launch_clear_labels)
             uint16_t out[8];
+#pragma unroll
             for (int k = 0; k < 8; ++k) {
-                if (((occ[r] >> (8 * k)) & 0xFFull) == 0ull || key[r][k] == kEmptyKey) out[k] = kEmpty;
+                if (((occ[r] >> k) & 1u) == 0u || key[r][k] == kEmptyKey) out[k] = kEmpty;
                 else if (key[r][k] >= kUnreachedKey) out[k] = kFree;
                 else out[k] = lab[(key[r][k] >> 2) & mask];
             }
-            store8(J.labels, c0, V, out);
+            store_group(J.labels, grp[r], pack_cells(out));
         }
     });
 }
@@ -1033,7 +1000,7 @@ __global__ __launch_bounds__(kCellThreads) void k_flood_sub_touch(Launch L)
     __shared__ JobDev sJ;
     __shared__ uint8_t frag[kMaxDeviceSeeds];
     uint32_t staged = 0xFFFFFFFFu;
-    walk_tiles(L, L.tile_prefix, L.total_tiles, &sJ, [&](const JobDev& J, uint32_t j, uint32_t local, uint32_t) {
+    walk_tiles(L, L.bt_prefix, L.total_bricks, &sJ, [&](const JobDev& J, uint32_t j, uint32_t brick, uint32_t) {
         if (!J.active || J.algo != VF_FLOOD || !J.sub) return;
         if (j != staged) {  // block-uniform
             for (uint32_t i = threadIdx.x; i < J.S && i < kMaxDeviceSeeds; i += blockDim.x)
@@ -1041,16 +1008,17 @@ __global__ __launch_bounds__(kCellThreads) void k_flood_sub_touch(Launch L)
             __syncthreads();
             staged = j;
         }
-        const uint64_t c0 = (uint64_t)local * kTileCells + threadIdx.x * kCellsPerThread;
-        if (c0 >= J.V) return;
+        const CellGroup grp = cell_group(J, brick);
+        const uint32_t occ = group_occ(J, grp);
+        if (!occ) return;
         const uint32_t mask = (1u << J.key_bits) - 1u;
         const bool n26 = J.neighbourhood != 6;
-        uint32_t x, y, z;
-        decompose(c0, J, x, y, z);
+        const uint32_t x = small_div(grp.col, J.ny, J.inv_ny), y = grp.col - x * J.ny;
         uint32_t last_s = 0xFFFFFFFFu, last_t = 0xFFFFFFFFu;
-        for (int k = 0; k < kCellsPerThread && c0 + k < J.V; ++k, advance(x, y, z, J)) {
-            if (!J.occ[c0 + k]) continue;  // keys exist only in bricks with an occupied cell
-            const uint32_t key = J.keys[c0 + k];
+        for (uint32_t k = 0; k < grp.n; ++k) {
+            if (!((occ >> k) & 1u)) continue;  // keys exist only in bricks with an occupied cell
+            const uint32_t z = grp.z0 + k;
+            const uint32_t key = J.keys[grp.c0 + k];
             if (!reached_key(key)) continue;
             const uint32_t s = (key >> 2) & mask;
             for (int i = 0; i < (n26 ? 13 : 3); ++i) {
@@ -1064,7 +1032,7 @@ __global__ __launch_bounds__(kCellThreads) void k_flood_sub_touch(Launch L)
                 const int xx = (int)x + dx, yy = (int)y + dy, zz = (int)z + dz;
                 if (xx >= (int)J.nx || yy < 0 || yy >= (int)J.ny || zz < 0 || zz >= (int)J.nz) continue;
                 const size_t cn = ((size_t)xx * J.ny + (uint32_t)yy) * J.nz + (uint32_t)zz;
-                if (!J.occ[cn]) continue;
+                if (!occ_bit(J, (uint32_t)xx, (uint32_t)yy, (uint32_t)zz)) continue;
                 const uint32_t kn = J.keys[cn];
                 if (!reached_key(kn)) continue;
                 const uint32_t t = (kn >> 2) & mask;
@@ -1131,7 +1099,7 @@ __global__ __launch_bounds__(kCellThreads) void k_flood_sub_reseed(Launch L)
     __shared__ JobDev sJ;
     __shared__ uint8_t keep[kMaxDeviceSeeds];
     uint32_t staged = 0xFFFFFFFFu;
-    walk_tiles(L, L.tile_prefix, L.total_tiles, &sJ, [&](const JobDev& J, uint32_t j, uint32_t local, uint32_t) {
+    walk_tiles(L, L.bt_prefix, L.total_bricks, &sJ, [&](const JobDev& J, uint32_t j, uint32_t brick, uint32_t) {
         if (!J.active || J.algo != VF_FLOOD || !J.sub || J.fctl[1] != 0u) return;
         if (j != staged) {  // block-uniform
             for (uint32_t i = threadIdx.x; i < J.S && i < kMaxDeviceSeeds; i += blockDim.x)
@@ -1139,22 +1107,25 @@ __global__ __launch_bounds__(kCellThreads) void k_flood_sub_reseed(Launch L)
             __syncthreads();
             staged = j;
         }
-        const uint64_t c0 = (uint64_t)local * kTileCells + threadIdx.x * kCellsPerThread;
-        if (c0 >= J.V) return;
+        const CellGroup grp = cell_group(J, brick);
+        const uint32_t occ = group_occ(J, grp);
+        if (!occ) return;
         const uint32_t b = J.key_bits, mask = (1u << b) - 1u;
         const uint32_t nby = bdim(J.ny), nbz = bdim(J.nz);
         uint8_t* flags1 = parity_flags(J.bflags, J.nbricks, 1u);  // round 1 consumes parity 1
-        uint32_t x, y, z, last = 0xFFFFFFFFu;
-        decompose(c0, J, x, y, z);
-        for (int k = 0; k < kCellsPerThread && c0 + k < J.V; ++k, advance(x, y, z, J)) {
-            if (!J.occ[c0 + k]) continue;  // keys exist only in bricks with an occupied cell
-            const uint32_t key = J.keys[c0 + k];
+        const uint32_t x = small_div(grp.col, J.ny, J.inv_ny), y = grp.col - x * J.ny;
+        uint32_t last = 0xFFFFFFFFu;
+        for (uint32_t k = 0; k < grp.n; ++k) {
+            if (!((occ >> k) & 1u)) continue;  // keys exist only in bricks with an occupied cell
+            const uint64_t c = grp.c0 + k;
+            const uint32_t z = grp.z0 + k;
+            const uint32_t key = J.keys[c];
             if (!reached_key(key)) continue;
             const uint32_t s = (key >> 2) & mask;
             if (keep[s]) {
-                J.keys[c0 + k] = (((1u << b) | s) << 2) | (key & 3u);
+                J.keys[c] = (((1u << b) | s) << 2) | (key & 3u);
             } else {
-                J.keys[c0 + k] = kUnreachedKey | (key & 3u);
+                J.keys[c] = kUnreachedKey | (key & 3u);
                 const uint32_t id = ((x / kRelaxBrick) * nby + y / kRelaxBrick) * nbz + z / kRelaxBrick;
                 if (id != last) {
                     flags1[id] = 1u;
@@ -1219,7 +1190,7 @@ void launch_flood_rounds(const Launch& L, const FloodRoundScratch& W, uint32_t r
 
 void launch_flood_sub(const Launch& L)
 {
-    const uint32_t blocks = std::max(1u, std::min(L.total_tiles, active_shape().cell_blocks));
+    const uint32_t blocks = std::max(1u, std::min(L.total_bricks, active_shape().cell_blocks));
     {
         TimedLaunch tl("flood_sub_init", L.s);
         k_flood_sub_init<<<L.njobs, 256, 0, L.s>>>(L);
@@ -1243,7 +1214,7 @@ void launch_flood_sub(const Launch& L)
 void launch_flood_finish(const Launch& L)
 {
     TimedLaunch tl("flood_finish", L.s);
-    const uint32_t blocks = std::max(1u, std::min(L.total_tiles, active_shape().cell_blocks));
+    const uint32_t blocks = std::max(1u, std::min(L.total_bricks, active_shape().cell_blocks));
     k_flood_finish<<<blocks, kCellThreads, 0, L.s>>>(L);
     VF_CHECK_LAUNCH();
 }

@@ -10,9 +10,9 @@ struct vf_grid {
     int device = 0;
     hipStream_t stream = nullptr;
 
-    vf::DevBuf labels, occ;          // uint16 cells, uint8 occupancy
+    vf::DevBuf labels, occ;          // uint16 cells, occupancy bits (JobDev::occ)
     vf::DevBuf jobdev, prefix, stats, hist, seeds;
-    vf::DevBuf bits;                 // shell + toggle bitmasks
+    vf::DevBuf bits;                 // toggle bitmask
     vf::DevBuf vox_setup, vox_counts, vox_shell_off, scan_tmp, occ_tmp;
     vf::DevBuf mesh_xyz, mesh_tri;
     vf::DevBuf seed_tile_cnt, seed_tile_off;

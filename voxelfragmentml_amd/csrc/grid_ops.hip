@@ -21,24 +21,68 @@ __device__ inline void for_each_tile(const Launch& L, F&& f)
     });
 }
 
+// the same over bricks: f(J, group) for every group of cells
+template <class F>
+__device__ inline void for_each_group(const Launch& L, F&& f)
+{
+    __shared__ JobDev sJ;
+    walk_tiles(L, L.bt_prefix, L.total_bricks, &sJ, [&](const JobDev& J, uint32_t, uint32_t brick, uint32_t) {
+        if (!J.active) return;
+        const CellGroup g = cell_group(J, brick);
+        if (g.n) f(J, g);
+    });
+}
+
 __global__ __launch_bounds__(kCellThreads) void k_occ_to_labels(Launch L)
 {
-    for_each_tile(L, [&](const JobDev& J, uint64_t c0) {
-        uint64_t o = load8b(J.occ, c0, J.V);
+    for_each_group(L, [&](const JobDev& J, const CellGroup& g) {
+        const uint32_t o = group_occ(J, g);
         uint16_t v[8];
-        for (int k = 0; k < 8; ++k) v[k] = (uint16_t)((o >> (8 * k)) & 1u);
-        store8(J.labels, c0, J.V, v);
+        for (int k = 0; k < 8; ++k) v[k] = (uint16_t)((o >> k) & 1u);
+        store_group(J.labels, g, pack_cells(v));
     });
 }
 
 __global__ __launch_bounds__(kCellThreads) void k_labels_to_occ(Launch L)
 {
-    for_each_tile(L, [&](const JobDev& J, uint64_t c0) {
-        uint16_t v[8];
-        load8(J.labels, c0, J.V, v);
-        uint64_t o = 0;
-        for (int k = 0; k < 8; ++k) o |= (uint64_t)(v[k] != 0) << (8 * k);
-        store8b(J.occ, c0, J.V, o);
+    for_each_group(L, [&](const JobDev& J, const CellGroup& g) {
+        const uint4 q = load_group(J.labels, g);
+        const uint32_t w[4] = { q.x, q.y, q.z, q.w };
+        uint32_t o = 0;
+        for (int k = 0; k < 8; ++k) o |= ((w[k >> 1] >> (16 * (k & 1))) & 0xFFFFu ? 1u : 0u) << k;
+        gcast<uint8_t>(J.occ)[group_byte(J, g)] = (uint8_t)o;
+    });
+}
+
+__global__ __launch_bounds__(kCellThreads) void k_occ_free(Launch L, const uint32_t* bits)
+{
+    for_each_group(L, [&](const JobDev& J, const CellGroup& g) {
+        const uint32_t o = gcast<const uint8_t>(bits)[group_byte(J, g)];
+        for (uint32_t k = 0; k < 8u; ++k)
+            if ((o >> k) & 1u) gcast<uint16_t>(J.labels)[g.c0 + k] = kFree;
+    });
+}
+
+__global__ __launch_bounds__(kCellThreads) void k_occ_bytes(Launch L, uint8_t* out)
+{
+    for_each_group(L, [&](const JobDev& J, const CellGroup& g) {
+        const uint32_t o = group_occ(J, g);
+        for (uint32_t k = 0; k < g.n; ++k) gcast<uint8_t>(out)[g.c0 + k] = (uint8_t)((o >> k) & 1u);
+    });
+}
+
+// All cells EMPTY, in the cells' linear order: whole lines written one after another run at the rate of a fill (512^3:
+// 268 MB in 35 us), where the fractures' bricks write rows of 64 bytes (the same bytes in 87 to 115 us).
+__global__ __launch_bounds__(kCellThreads) void k_clear_labels(Launch L)
+{
+    __shared__ JobDev sJ;
+    walk_tile_runs<8>(L, L.tile_prefix, L.total_tiles, &sJ, [&](const JobDev& J, uint32_t, uint32_t tile, uint32_t n) {
+        if (!J.active) return;
+        const uint16_t zero[8] = {};
+        for (uint32_t r = 0; r < n; ++r) {
+            const uint64_t c0 = (uint64_t)(tile + r) * kTileCells + threadIdx.x * kCellsPerThread;
+            if (c0 < J.V) store8(J.labels, c0, J.V, zero);
+        }
     });
 }
 
@@ -77,8 +121,10 @@ constexpr uint32_t kTiledBins = 1024;  // LDS histogram bins of the tiled bounda
 // Per-job sum of a per-thread value: wave sums, then one device atomic per block and job.
 struct BlockSum {
     unsigned long long part[kCellThreads / 64];
-    __device__ void flush(unsigned long long& acc, unsigned long long* dst)
+    // stat of job J, in the block's line of its sums where it has any
+    __device__ void flush(unsigned long long& acc, const JobDev& J, int stat)
     {
+        unsigned long long* dst = J.sums ? J.sums + (blockIdx.x % kSumSlots) * kStatCount + stat : J.stats + stat;
         const unsigned long long s = wave_sum_u64(acc);
         if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
         __syncthreads();
@@ -209,8 +255,9 @@ constexpr int kBHX = kBTX + 2, kBHY = kBTY + 2, kBHZ = kBTZ + 2;
 // fall on distinct bank groups
 constexpr int kAZ = kBTZ + 4;
 
-// CSUM: also accumulate the grid checksum of the final cells (jobs with a
-// window size <= 1; the others get theirs from k_checksum<true>).
+// CSUM: the jobs of a table, whose labels follow their occupancy; also accumulate
+// the grid checksum of the final cells (jobs with a window size <= 1; the others
+// get theirs from k_checksum<true>).
 //
 // Each thread owns an 8-cell z segment of one of the brick's 64 rows and loads
 // it with its two z neighbours (clamped coordinates = replicate padding), so
@@ -227,7 +274,7 @@ __device__ inline uint32_t pk_max_u16(uint32_t a, uint32_t b)
 __device__ inline uint32_t packed_self(uint32_t m) { return m | ((0xFFFFu - m) << 16); }
 
 template <bool HIST, bool CSUM, uint32_t RUN>
-__global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L, const uint32_t* bt_prefix, uint32_t total)
+__global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
 {
     // z-window max (low 16 bits) | 0xFFFF - min (high 16) over labelled cells (EMPTY / FREE contribute 0),
     // so one packed u16 max combines both halves; row = hx * kBHY + hy
@@ -240,7 +287,7 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L, const uint32
         for (uint32_t i = threadIdx.x; i < kTiledBins; i += blockDim.x) bins[i] = 0;
     }
     auto flush = [&](uint32_t j) {
-        if (CSUM) csum_part.flush(csum, L.jobs[j].stats + kStatChecksum);
+        if (CSUM) csum_part.flush(csum, L.jobs[j], kStatChecksum);
         if (!HIST) return;
         __syncthreads();
         uint32_t* h = L.jobs[j].hist;
@@ -278,7 +325,7 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L, const uint32
         for (int k = 0; k < 8; ++k) out[k] = pk_max_u16(pk_max_u16(p[k], p[k + 1]), p[k + 2]);
     };
     constexpr uint32_t kRun = RUN;  // bricks per step: their interior loads are issued together
-    walk_tile_runs<kRun>(L, bt_prefix, total, &sJ, [&](const JobDev& J, uint32_t, uint32_t first, uint32_t nrun) {
+    walk_tile_runs<kRun>(L, L.bt_prefix, L.total_bricks, &sJ, [&](const JobDev& J, uint32_t, uint32_t first, uint32_t nrun) {
         if (!J.active || J.bsize > 1) return;
         const int nx = (int)J.nx, ny = (int)J.ny, nz = (int)J.nz;
         const uint32_t tz = ceil_div_d(J.nz, kBTZ), tyn = ceil_div_d(J.ny, kBTY);
@@ -332,9 +379,23 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L, const uint32
             }
         };
 
-        // phase 1: the interior segments of the whole run, loaded together; bricks without a label end here
+        // phase 1: whether each brick of the run holds a label, all loads issued together; the others end here
         uint32_t live = 0;
-        {
+        if constexpr (CSUM) {
+            // a table's labels are not EMPTY only where the occupancy is set, and a brick's rows are one occupancy
+            // word each: 4 bytes a row instead of its 64 bytes of labels; bricks without a bit add nothing
+            uint32_t occ[kRun];
+#pragma unroll
+            for (uint32_t r = 0; r < kRun; ++r) {
+                int x0, y0, z0, gx, gy, gz, nval;
+                segment(first + r, x0, y0, z0, gx, gy, gz, nval);
+                occ[r] = r < nrun && gx < nx && gy < ny
+                             ? gcast<const uint32_t>(J.occ)[((size_t)gx * ny + gy) * J.wp + (uint32_t)z0 / 32u] : 0u;
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < kRun; ++r) live |= occ[r] ? 1u << r : 0u;
+            live = (uint32_t)__ockl_wgred_or_i32((int)live);  // block-uniform: bit r = brick r holds an occupied cell
+        } else {
             uint32_t pr[kRun][4];
 #pragma unroll
             for (uint32_t r = 0; r < kRun; ++r) {
@@ -350,18 +411,6 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L, const uint32
                 live |= mine ? 1u << r : 0u;
             }
             live = (uint32_t)__ockl_wgred_or_i32((int)live);  // block-uniform: bit r = brick r holds a label
-            if (CSUM) {
-#pragma unroll
-                for (uint32_t r = 0; r < kRun; ++r) {
-                    if (r >= nrun || ((live >> r) & 1u)) continue;
-                    int x0, y0, z0, gx, gy, gz, nval;
-                    segment(first + r, x0, y0, z0, gx, gy, gz, nval);
-                    uint16_t v[8];
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) v[k] = (uint16_t)(pr[r][k >> 1] >> (16 * (k & 1)));
-                    add_checksum(v, gx, gy, gz, nval);
-                }
-            }
         }
 
         // phase 2: bricks with a label
@@ -469,7 +518,7 @@ __global__ __launch_bounds__(kCellThreads) void k_checksum(Launch L)
         uint16_t v[8];
         load8(J.labels, c0, J.V, v);
         for (int k = 0; k < 8; ++k) acc += checksum_term(v[k], (uint32_t)(c0 + k));  // cells beyond V load as 0
-    }, [&](uint32_t j) { bs.flush(acc, L.jobs[j].stats + kStatChecksum); });
+    }, [&](uint32_t j) { bs.flush(acc, L.jobs[j], kStatChecksum); });
 }
 
 __global__ __launch_bounds__(kCellThreads) void k_count_occupied(Launch L)
@@ -477,13 +526,9 @@ __global__ __launch_bounds__(kCellThreads) void k_count_occupied(Launch L)
     __shared__ BlockSum bs;
     __shared__ JobDev sJ;
     unsigned long long acc = 0;
-    walk_tiles(L, L.tile_prefix, L.total_tiles, &sJ, [&](const JobDev& J, uint32_t, uint32_t local, uint32_t) {
-        if (!J.active) return;
-        const uint64_t c0 = (uint64_t)local * kTileCells + threadIdx.x * kCellsPerThread;
-        if (c0 >= J.V) return;
-        const uint64_t o = load8b(J.occ, c0, J.V);
-        acc += __popcll(o & 0x0101010101010101ull);
-    }, [&](uint32_t j) { bs.flush(acc, L.jobs[j].stats + kStatOccupied); });
+    walk_tiles(L, L.bt_prefix, L.total_bricks, &sJ, [&](const JobDev& J, uint32_t, uint32_t brick, uint32_t) {
+        if (J.active) acc += __popc(group_occ(J, cell_group(J, brick)));
+    }, [&](uint32_t j) { bs.flush(acc, L.jobs[j], kStatOccupied); });
 }
 
 // One block per job: number of labels >= 2 with a nonzero count.
@@ -528,7 +573,8 @@ __global__ __launch_bounds__(256) void k_job_init(Launch L)
         const size_t n = 2u * relax_parity_bytes(J->nbricks) / 16u;
         for (size_t i = threadIdx.x; i < n; i += blockDim.x) gstore4(J->bflags + 16u * i, make_uint4(0u, 0u, 0u, 0u));
     }
-    if (J->work && threadIdx.x < kFloodWorkSlots) J->work[threadIdx.x * kFloodWorkStride] = 0ull;
+    if (J->sums)
+        for (uint32_t i = threadIdx.x; i < kSumSlots * kStatCount; i += blockDim.x) J->sums[i] = 0ull;
 }
 
 // Block per job: stats and flood state into a compact table for one readback.
@@ -537,15 +583,19 @@ __global__ void k_gather(Launch L, uint32_t* out)
     const JobDev* J = L.jobs + blockIdx.x;
     uint32_t* o = out + 16 * (size_t)blockIdx.x;
     const uint32_t t = threadIdx.x;
-    static_assert(kFloodWorkSlots == 64, "one slot per lane");
-    const unsigned long long work = wave_sum_u64(J->active && J->work ? J->work[t * kFloodWorkStride] : 0ull);
+    static_assert(kSumSlots == 64 && kStatCount == 8, "8 lines a step, a sum per lane");
+    unsigned long long v = 0;
+    if (J->active && J->sums)
+        for (uint32_t i = t; i < kSumSlots * kStatCount; i += 64u) v += J->sums[i];
+    for (int o = 8; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);  // lanes with the same statistic
     if (t < kStatCount) {
-        const unsigned long long v = t == kStatFloodWork ? work : J->active ? J->stats[t] : 0ull;
+        if (J->active) v += J->stats[t];
         o[2 * t] = (uint32_t)v;
         o[2 * t + 1] = (uint32_t)(v >> 32);
     }
 }
 
+inline uint32_t bgrid_for(const Launch& L) { return std::max(1u, std::min(L.total_bricks, active_shape().cell_blocks)); }
 inline uint32_t grid_for(const Launch& L) { return std::max(1u, std::min(L.total_tiles, active_shape().cell_blocks)); }
 
 }  // namespace
@@ -553,14 +603,35 @@ inline uint32_t grid_for(const Launch& L) { return std::max(1u, std::min(L.total
 void launch_occ_to_labels(const Launch& L)
 {
     TimedLaunch tl("occ_to_labels", L.s);
-    k_occ_to_labels<<<grid_for(L), kCellThreads, 0, L.s>>>(L);
+    k_occ_to_labels<<<bgrid_for(L), kCellThreads, 0, L.s>>>(L);
     VF_CHECK_LAUNCH();
 }
 
 void launch_labels_to_occ(const Launch& L)
 {
     TimedLaunch tl("labels_to_occ", L.s);
-    k_labels_to_occ<<<grid_for(L), kCellThreads, 0, L.s>>>(L);
+    k_labels_to_occ<<<bgrid_for(L), kCellThreads, 0, L.s>>>(L);
+    VF_CHECK_LAUNCH();
+}
+
+void launch_occ_free(const Launch& L, const uint32_t* bits)
+{
+    TimedLaunch tl("occ_free", L.s);
+    k_occ_free<<<bgrid_for(L), kCellThreads, 0, L.s>>>(L, bits);
+    VF_CHECK_LAUNCH();
+}
+
+void launch_occ_bytes(const Launch& L, uint8_t* out)
+{
+    TimedLaunch tl("occ_bytes", L.s);
+    k_occ_bytes<<<bgrid_for(L), kCellThreads, 0, L.s>>>(L, out);
+    VF_CHECK_LAUNCH();
+}
+
+void launch_clear_labels(const Launch& L)
+{
+    TimedLaunch tl("clear_labels", L.s);
+    k_clear_labels<<<grid_for(L), kCellThreads, 0, L.s>>>(L);
     VF_CHECK_LAUNCH();
 }
 
@@ -604,17 +675,16 @@ void launch_boundaries(const Launch& L, int size, int with_hist)
     VF_CHECK_LAUNCH();
 }
 
-void launch_boundaries_tiled(const Launch& L, const uint32_t* bt_prefix, uint32_t total_btiles, bool any_wide,
-                             bool with_checksum)
+void launch_boundaries_tiled(const Launch& L, bool any_wide, bool with_checksum)
 {
     {
         TimedLaunch tl("boundaries_hist", L.s);
         const LaunchShape sh = active_shape();
-        const uint32_t blocks = std::max(1u, std::min(total_btiles, sh.brick_blocks));
+        const uint32_t blocks = std::max(1u, std::min(L.total_bricks, sh.brick_blocks));
         auto go = [&](auto run) {
             constexpr uint32_t R = decltype(run)::value;
-            if (with_checksum) k_boundaries_tiled<true, true, R><<<blocks, 256, 0, L.s>>>(L, bt_prefix, total_btiles);
-            else k_boundaries_tiled<true, false, R><<<blocks, 256, 0, L.s>>>(L, bt_prefix, total_btiles);
+            if (with_checksum) k_boundaries_tiled<true, true, R><<<blocks, 256, 0, L.s>>>(L);
+            else k_boundaries_tiled<true, false, R><<<blocks, 256, 0, L.s>>>(L);
         };
         if (sh.brick_run == 2) go(std::integral_constant<uint32_t, 2>{});
         else if (sh.brick_run == 8) go(std::integral_constant<uint32_t, 8>{});
@@ -663,7 +733,7 @@ void launch_hist_summary(const Launch& L)
 void launch_count_occupied(const Launch& L)
 {
     TimedLaunch tl("count_occupied", L.s);
-    k_count_occupied<<<grid_for(L), kCellThreads, 0, L.s>>>(L);
+    k_count_occupied<<<bgrid_for(L), kCellThreads, 0, L.s>>>(L);
     VF_CHECK_LAUNCH();
 }
 

@@ -17,14 +17,28 @@ namespace vf {
 constexpr uint32_t kMaxNoiseAmp = 2;  // flood cell weights are 1 + [0, amp]
 constexpr uint32_t kRelaxBrick = 8;   // flood relaxation brick edge (cells)
 constexpr uint32_t kTileCells = 2048; // cells per tile for cell-parallel stages (256 threads x 8 cells)
+constexpr uint32_t kTileWords = 64;   // occupancy words per word tile, in the cells' linear order (seed candidates)
+inline uint64_t occ_words(const uint32_t d[3]) { return (uint64_t)d[0] * d[1] * next_pow2(ceil_div(d[2], 32)); }
+inline uint32_t word_tiles(const uint32_t d[3]) { return ceil_div(occ_words(d), kTileWords); }
+// Bricks of 8 x 8 columns by one occupancy word of 32 cells: the tiles of the stages that go by occupancy (256
+// threads x 8 cells, a byte of a word each).  Numbered with z fastest.
+constexpr uint32_t kBrickX = 8, kBrickY = 8, kBrickZ = 32;
+__host__ __device__ inline uint32_t brick_count(uint32_t nx, uint32_t ny, uint32_t nz)
+{
+    return ((nx + kBrickX - 1) / kBrickX) * ((ny + kBrickY - 1) / kBrickY) * ((nz + kBrickZ - 1) / kBrickZ);
+}
 
+// Statistics many workgroups add to: workgroup g adds to line g % kSumSlots of JobDev::sums, a cache line each.  Same-address
+// atomics execute one after another, about 8 ns each: one counter for the 3000 visits of a flood round cost 30 us, one
+// for the 8192 workgroups of a 512^3 fill 60 us.
+constexpr uint32_t kSumSlots = 64;
 enum StatSlot : int {
     kStatOccupied = 0,   // non-EMPTY cells after voxelization
     kStatChecksum = 1,   // order-independent grid checksum
     kStatShellPairs = 2, // (triangle, cell) SAT candidates
     kStatColPairs = 3,   // (triangle, column) parity candidates
     kStatError = 4,      // first error flag raised on the device
-    kStatFloodWork = 5,  // flood work: (sweeps << 32) + brick visits (summed from JobDev::work when gathered)
+    kStatFloodWork = 5,  // flood work: (sweeps << 32) + brick visits (kept in JobDev::sums only)
     kStatFloodDone = 6,  // flood relaxation rounds run (0 while running)
     kStatLabels = 7,     // labels >= 2 with a nonzero count
     kStatCount = 8
@@ -40,6 +54,8 @@ enum DevError : uint32_t {
     kDevErrMerge = 16,      // mergeSeeds: a fragment would get more than 255 sub-seeds
 };
 
+constexpr size_t kSumBytes = (size_t)kSumSlots * kStatCount * 8;
+
 struct TriSetup {
     float P[3][3];             // FP32 vertices (SAT input)
     int32_t X[3], Y[3], Z[3];  // snapped fixed-point vertices (CCW in xy)
@@ -54,12 +70,13 @@ struct JobDev {
     uint64_t V;
     float mn[3], mx[3], cs[3];
     uint16_t* labels;
-    uint8_t* occ;
+    uint32_t* occ;          // occupancy, one bit per cell: nx*ny*wp words, cell (x, y, z) is bit z % 32 of word (x*ny + y)*wp + z / 32, bits past nz are 0
+    float inv_ny;           // 1 / ny (small_div)
     // voxelizer input / scratch
     const float* xyz;
     const uint32_t* tri;
     uint32_t nt, nv;
-    uint32_t* shell_bits;   // nx*ny*wp words
+    uint32_t* shell_bits;   // nx*ny*wp words; the fill leaves the occupancy here
     uint32_t* toggle_bits;  // nx*ny*wp words
     // seeds {x,y,z,label}
     uint4* seeds;
@@ -82,7 +99,7 @@ struct JobDev {
     uint32_t* sub;          // sub-seed pass (null when the seeds carry one id per fragment): S union-find parents, S keep flags
     uint8_t* bflags;        // brick flags for even / odd rounds (relax_parity_bytes each, one byte per brick), then the brick liveness words
     uint32_t nbricks;       // relaxation bricks (kRelaxBrick^3 cells each)
-    unsigned long long* work;  // kFloodWorkSlots sums of (sweeps << 32) + brick visits, each on a cache line of its own (null: not counted)
+    unsigned long long* sums;  // kSumSlots lines of kStatCount sums, added to stats when gathered (null: none)
     uint32_t* fctl;         // flood control: [0] round, [1] rounds run once drained (0 = running), [2..3] flags non-empty, [4..5] round started by the compaction of an even / odd round of a chunk
     unsigned long long* stats;  // kStatCount slots
     uint32_t* hist;         // 65536 counts
@@ -144,6 +161,10 @@ struct Launch {
     uint32_t njobs;
     const uint32_t* tile_prefix; // device, njobs+1 (kTileCells tiles)
     uint32_t total_tiles;
+    const uint32_t* wtile_prefix;  // device, njobs+1 (kTileWords tiles)
+    uint32_t total_wtiles;
+    const uint32_t* bt_prefix;   // device, njobs+1 (bricks of 8 x 8 x 32 cells)
+    uint32_t total_bricks;
     hipStream_t s;
 };
 
@@ -159,31 +180,28 @@ struct VoxScratch {
     void* scan_tmp;                    // scan scratch
     size_t scan_tmp_bytes;
 };
-// tile_cnt (or null): also count the occupied cells per tile (L.tile_prefix) of jobs that seed anywhere
+// tile_cnt (or null): also count the occupied cells per tile (L.wtile_prefix) of jobs that seed anywhere
 // (VF_SEED_BOTH), as launch_seed_count does; launch_seed_count(..., true) then skips those jobs
 void launch_voxelize(const Launch& L, const VoxScratch& X, const uint32_t* col_prefix, uint32_t total_col_groups,
                      uint32_t* tile_cnt);
-void launch_clear_bits(const Launch& L, const uint32_t* col_prefix, uint32_t total_col_groups, uint32_t* tile_cnt);
+void launch_clear_bits(const Launch& L, const uint32_t* col_prefix, uint32_t total_col_groups);
 
 // grid_ops.hip
 void launch_occ_to_labels(const Launch& L);
 void launch_labels_to_occ(const Launch& L);
+void launch_occ_free(const Launch& L, const uint32_t* bits);  // labels of the cells set in bits (laid out as occ) become FREE
+void launch_occ_bytes(const Launch& L, uint8_t* out);        // job 0's occupancy as one byte per cell
 void launch_homogenize(const Launch& L);
+// every cell of every job EMPTY: the fractures (launch_naive, launch_flood_finish) write only around occupied cells
+void launch_clear_labels(const Launch& L);
 void launch_undo_mask(const Launch& L, uint16_t keep_mask);
 void launch_clear_hist(const Launch& L);
 void launch_histogram(const Launch& L);
 void launch_boundaries(const Launch& L, int size /* < 0: per-job bsize */, int with_hist);
-// detectBoundaries(size <= 1 per job) fused with the histogram, 8x8x32 LDS
-// bricks; bt_prefix: njobs+1 prefix of bricks; jobs with size > 1 go through
-// the generic kernel when any_wide.
-constexpr uint32_t kBrickX = 8, kBrickY = 8, kBrickZ = 32;
-inline uint32_t brick_count(uint32_t nx, uint32_t ny, uint32_t nz)
-{
-    return ((nx + kBrickX - 1) / kBrickX) * ((ny + kBrickY - 1) / kBrickY) * ((nz + kBrickZ - 1) / kBrickZ);
-}
-// with_checksum: also sum every job's grid checksum into kStatChecksum
-void launch_boundaries_tiled(const Launch& L, const uint32_t* bt_prefix, uint32_t total_btiles, bool any_wide,
-                             bool with_checksum);
+// detectBoundaries(size <= 1 per job) fused with the histogram, brick by brick;
+// jobs with size > 1 go through the generic kernel when any_wide.
+// with_checksum: a table's jobs (cells outside the occupancy are EMPTY); also sum every job's grid checksum into kStatChecksum
+void launch_boundaries_tiled(const Launch& L, bool any_wide, bool with_checksum);
 void launch_job_init(const Launch& L);     // zero stats, histogram and flood control of every job
 void launch_gather(const Launch& L, uint32_t* out);  // 16 words per job: stats (low 32 bits) + flood state
 void launch_checksum(const Launch& L);
@@ -216,9 +234,6 @@ inline uint32_t relax_tasks(uint32_t nx, uint32_t ny, uint32_t nz)
 {
     return (relax_groups(relax_bricks(nx, ny, nz)) + 63u) / 64u;
 }
-// Work counters of a flood job: a workgroup adds to slot workgroup % kFloodWorkSlots (one address for all of
-// them cost a round of 3000 visits about 30 us: same-address atomics execute one after another).
-constexpr uint32_t kFloodWorkSlots = 64, kFloodWorkStride = 8;  // stride in 64-bit words
 // Brick liveness (bricks holding an occupied cell, whose keys the init writes), after the two flag
 // parities: a bitmap with one 64-bit word per 64 bricks of a brick column (bx, by), bit bz % 64 of word
 // (bx * nby + by) * wpc + bz / 64, then one 32-bit word per brick with the liveness of the brick and its
@@ -272,7 +287,7 @@ void launch_flood_sub(const Launch& L);
 // seed.hip
 constexpr uint32_t kMaxDeviceSeeds = 4096;
 void launch_seed_count(const Launch& L, uint32_t* tile_cnt, bool skip_both);
-// tile_off: exclusive prefix over the global tiles (total_tiles + 1 entries)
+// tile_off: exclusive prefix over the global word tiles (total_wtiles + 1 entries)
 void launch_seed_pick(const Launch& L, const unsigned long long* tile_off);
 // Seeder::mergeSeeds for every job with extra seeds (one block each): seeds[S0..2 S0) get copies of the
 // fragment seeds [0, S0), seeds[2 S0..2 S0 + extra) hold the extra draw; each of these S0 + extra seeds

@@ -198,15 +198,6 @@ __device__ inline UnitOrigin unit_origin(const McJob& J, uint32_t local)
     return UnitOrigin{ px | ((col - px * J.Ny) << 16), (local - col * J.cz) * kMcZ };
 }
 
-// x / d for x below 2^17: a float estimate off by at most one, corrected.
-__device__ inline uint32_t small_div(uint32_t x, uint32_t d, float inv)
-{
-    uint32_t q = (uint32_t)((float)x * inv);
-    const int r = (int)x - (int)(q * d);
-    if (r < 0) --q;
-    else if (r >= (int)d) ++q;
-    return q;
-}
 // The origin of the unit `lane` units after unit `local0` of grid J, from local0's column (col0 = local0 / cz,
 // split as px0 = col0 / Ny, py0 = col0 % Ny) and its remainder rz0 = local0 % cz: the divisions left are of
 // numbers below 2^17 (lane < 256, rz0 < cz, py0 < Ny, all below 2^16).

@@ -9,8 +9,11 @@
 // ranks by the float root itself.
 // The argmin is a single unsigned min over packed keys (distance << b | i),
 // so ties go to the lowest index exactly as the reference's strict '<' does.
-// Seeds are staged through LDS in chunks; each tile's occupied cells are
-// compacted and a thread applies every seed to its few cells in registers.
+// Work goes by bricks of 8 x 8 x 32 cells: a brick's occupied cells are
+// compacted, the seeds that cannot be nearest to any of its cells are dropped,
+// and a thread applies the rest to its few cells in registers.
+#include <type_traits>
+
 #include "cellops.hpp"
 
 namespace vf {
@@ -18,6 +21,7 @@ namespace vf {
 namespace {
 
 constexpr uint32_t kSeedChunk = 1024;
+constexpr uint32_t kNaiveSmall = 8192;  // bricks of a launch below which runs are of one
 
 // (d << b) | i.  32-bit keys: d < 2^24 (at most 3 * 2047^2) and b <= 17, so it is one 24-bit
 // multiply-add, d * 2^b + i.
@@ -32,102 +36,127 @@ __device__ inline K pack_key(uint32_t d, uint32_t i, uint32_t b)
 // coordinates are below 2^11 (grid edges of at most 2048 cells), so the halves never wrap.
 __device__ inline uint32_t sad16(uint32_t a, uint32_t b, uint32_t acc) { return __builtin_amdgcn_sad_u16(a, b, acc); }
 
-// Distance key of one cell to one seed; xy and sxy hold x | y << 16.  kDistEuclidF32 (64-bit keys
-// only) ranks by the bits of the correctly rounded float root of the squared distance, which is
-// below 2^24 and so converts exactly: the reference's float sqrt (NaiveFracturer.cpp:12-15).
+// The distance of offsets (ax, ay, az), each below 2^11.  kDistEuclidF32 (64-bit keys only) ranks by the bits of the
+// correctly rounded float root of the squared distance, which is below 2^24 and so converts exactly: the
+// reference's float sqrt (NaiveFracturer.cpp:12-15).
+template <int DIST>
+__device__ inline uint32_t offset_dist(uint32_t ax, uint32_t ay, uint32_t az)
+{
+    if (DIST == VF_MANHATTAN) return ax + ay + az;
+    if (DIST == VF_CHEBYSHEV) return max(ax, max(ay, az));
+    // offsets < 2^11: 16-bit operands select the full-rate 24-bit multiply
+    const uint32_t d = (ax & 0xFFFFu) * (ax & 0xFFFFu) + (ay & 0xFFFFu) * (ay & 0xFFFFu) + (az & 0xFFFFu) * (az & 0xFFFFu);
+    return DIST == kDistEuclidF32 ? sqrt_rn_bits(d) : d;
+}
+
+// Distance key of one cell (xy = x | y << 16, z) to one seed (sxy, sz).
 template <int DIST, typename K>
-__device__ inline K seed_key(uint32_t x, uint32_t y, uint32_t z, uint32_t xy, uint32_t sx, uint32_t sy, uint32_t sz,
-                             uint32_t sxy, uint32_t id, uint32_t b)
+__device__ inline K seed_key(uint32_t xy, uint32_t z, uint32_t sxy, uint32_t sz, uint32_t id, uint32_t b)
 {
     uint32_t d;
     if (DIST == VF_MANHATTAN) {
         d = sad16(xy, sxy, sad16(z, sz, 0u));
     } else {
-        const uint32_t ax = sad16(x, sx, 0u), ay = sad16(y, sy, 0u), az = sad16(z, sz, 0u);
-        if (DIST == VF_CHEBYSHEV) d = max(ax, max(ay, az));
-        else  // offsets < 2^11: 16-bit operands select the full-rate 24-bit multiply
-            d = (ax & 0xFFFFu) * (ax & 0xFFFFu) + (ay & 0xFFFFu) * (ay & 0xFFFFu) + (az & 0xFFFFu) * (az & 0xFFFFu);
-        if (DIST == kDistEuclidF32) d = sqrt_rn_bits(d);
+        const uint32_t ax = sad16(xy & 0xFFFFu, sxy & 0xFFFFu, 0u), ay = sad16(xy >> 16, sxy >> 16, 0u), az = sad16(z, sz, 0u);
+        d = offset_dist<DIST>(ax, ay, az);
     }
     return pack_key<DIST, K>(d, id, b);
 }
 
-// argmin over seeds [base, base + n) (staged in LDS) for Q compacted cells of
-// a thread: each seed is read once (an LDS broadcast) and applied to all Q
-// cells held in registers.
+// Seeds in LDS: x | y << 16, then z | (index in the chunk) << 16.
+static_assert(kSeedChunk <= 65536, "16-bit seed index");
+
+// argmin over the n seeds of `list` for Q compacted cells of a thread: each seed is read once (an LDS broadcast, its
+// parts split on the scalar unit) and applied to all Q cells held in registers.
 template <int DIST, typename K, int Q>
-__device__ inline void naive_cells_q(K best[4], const uint32_t cx[4], const uint32_t cy[4], const uint32_t cz[4],
-                                     const uint32_t* sx, const uint32_t* sy, const uint32_t* sz, uint32_t base, uint32_t n,
-                                     uint32_t b)
+__device__ inline void naive_cells_q(K best[4], const uint32_t cxy[4], const uint32_t cz[4], const uint2* list, uint32_t base,
+                                     uint32_t n, uint32_t b)
 {
     K m[Q];
-    uint32_t cxy[Q];
+    uint32_t xy[Q], z[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         m[q] = best[q];
-        cxy[q] = cx[q] | (cy[q] << 16);
+        xy[q] = cxy[q];
+        z[q] = cz[q];
     }
-    // four seeds per step, one 16-byte LDS read per coordinate array (the arrays are 16-byte aligned)
-    uint32_t i = 0;
-    for (; i + 4 <= n; i += 4) {
-        const uint4 X4 = *reinterpret_cast<const uint4*>(sx + i), Y4 = *reinterpret_cast<const uint4*>(sy + i),
-                    Z4 = *reinterpret_cast<const uint4*>(sz + i);
-        const uint32_t xs[4] = { X4.x, X4.y, X4.z, X4.w }, ys[4] = { Y4.x, Y4.y, Y4.z, Y4.w },
-                       zs[4] = { Z4.x, Z4.y, Z4.z, Z4.w };
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t xy = xs[k] | (ys[k] << 16), id = base + i + k;
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                const K key = seed_key<DIST, K>(cx[q], cy[q], cz[q], cxy[q], xs[k], ys[k], zs[k], xy, id, b);
-                m[q] = key < m[q] ? key : m[q];
-            }
-        }
-    }
-    for (; i < n; ++i) {
-        const uint32_t x = sx[i], y = sy[i], z = sz[i], xy = x | (y << 16), id = base + i;
+    auto apply = [&](uint32_t vxy, uint32_t vzi) {
+        const uint32_t sxy = (uint32_t)__builtin_amdgcn_readfirstlane((int)vxy), szi = (uint32_t)__builtin_amdgcn_readfirstlane((int)vzi);
+        const uint32_t sz = szi & 0xFFFFu, id = base + (szi >> 16);
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            const K key = seed_key<DIST, K>(cx[q], cy[q], cz[q], cxy[q], x, y, z, xy, id, b);
+            const K key = seed_key<DIST, K>(xy[q], z[q], sxy, sz, id, b);
             m[q] = key < m[q] ? key : m[q];
         }
+    };
+    // four seeds per step, two 16-byte LDS reads (the list is 16-byte aligned)
+    uint32_t i = 0;
+    for (; i + 4 <= n; i += 4) {
+        const uint4 a = *reinterpret_cast<const uint4*>(list + i), c = *reinterpret_cast<const uint4*>(list + i + 2);
+        apply(a.x, a.y);
+        apply(a.z, a.w);
+        apply(c.x, c.y);
+        apply(c.z, c.w);
+    }
+    for (; i < n; ++i) {
+        const uint2 a = list[i];
+        apply(a.x, a.y);
     }
 #pragma unroll
     for (int q = 0; q < Q; ++q) best[q] = m[q];
 }
 
 // qmax (1..4): cells per thread, the same for the whole wave (lanes past the
-// tile's last occupied cell compute on a dummy cell)
+// brick's last occupied cell compute on a dummy cell)
 template <int DIST, typename K>
-__device__ inline void naive_cells(K best[4], const uint32_t cx[4], const uint32_t cy[4], const uint32_t cz[4], uint32_t qmax,
-                                   const uint32_t* sx, const uint32_t* sy, const uint32_t* sz, uint32_t base, uint32_t n,
-                                   uint32_t b)
+__device__ inline void naive_cells(K best[4], const uint32_t cxy[4], const uint32_t cz[4], uint32_t qmax, const uint2* list,
+                                   uint32_t base, uint32_t n, uint32_t b)
 {
-    if (qmax <= 1) naive_cells_q<DIST, K, 1>(best, cx, cy, cz, sx, sy, sz, base, n, b);
-    else if (qmax == 2) naive_cells_q<DIST, K, 2>(best, cx, cy, cz, sx, sy, sz, base, n, b);
-    else if (qmax == 3) naive_cells_q<DIST, K, 3>(best, cx, cy, cz, sx, sy, sz, base, n, b);
-    else naive_cells_q<DIST, K, 4>(best, cx, cy, cz, sx, sy, sz, base, n, b);
+    if (qmax <= 1) naive_cells_q<DIST, K, 1>(best, cxy, cz, list, base, n, b);
+    else if (qmax == 2) naive_cells_q<DIST, K, 2>(best, cxy, cz, list, base, n, b);
+    else if (qmax == 3) naive_cells_q<DIST, K, 3>(best, cxy, cz, list, base, n, b);
+    else naive_cells_q<DIST, K, 4>(best, cxy, cz, list, base, n, b);
 }
 
+// The least and the greatest distance of a seed from the cells of a box.
+template <int DIST>
+__device__ inline void box_dist(uint32_t xy, uint32_t z, const uint32_t lo[3], const uint32_t hi[3], uint32_t& dmin, uint32_t& dmax)
+{
+    const uint32_t s[3] = { xy & 0xFFFFu, xy >> 16, z };
+    uint32_t a[3], f[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const int below = (int)lo[q] - (int)s[q], above = (int)s[q] - (int)hi[q];  // > 0 outside the box
+        a[q] = (uint32_t)max(max(below, above), 0);
+        f[q] = (uint32_t)max(-below, -above);
+    }
+    dmin = offset_dist<DIST>(a[0], a[1], a[2]);
+    dmax = offset_dist<DIST>(f[0], f[1], f[2]);
+}
 
-// One tile per step: the tile's occupied cells are compacted in LDS, so the
-// seed loop runs over occupied cells only (shells occupy a few percent of
-// their box); labels return through LDS and leave as one 16-byte store per
-// thread.  A tile costs several block barriers and dependent LDS steps, so
-// the register budget is set for more waves in flight: 5 per SIMD with
-// 32-bit keys (95 VGPRs instead of 127, 1.06 -> 0.94 ms on the mixed batch),
-// 4 with 64-bit keys, both without spills.  RUN tiles form a walker run whose
-// occupancy loads are issued together (a launch shape the tuner picks).
+// Seeds below which a brick applies all of them: dropping the far ones (a box distance per seed, a block minimum, a
+// compaction) costs about as much as applying this many.
+constexpr uint32_t kPruneSeeds = 16;
+
+// One brick per step.  Its occupied cells are compacted in LDS, so the seed loop runs over occupied cells only (shells
+// occupy a few percent of their box); of more than kPruneSeeds seeds, those farther from the whole brick than some
+// other seed's farthest cell are dropped first (strictly farther: ties stay, and a dropped seed is never nearest or
+// tied), which leaves a few of 128; labels return through LDS and leave as one 16-byte store per
+// occupied group (launch_clear_labels has written the rest).  Bound by the latency of the block's barriers, so the
+// register budget is set for more waves in flight: 5 per SIMD with 32-bit keys, 4 with 64-bit keys.  RUN bricks form a walker run
+// whose occupancy loads are issued together (a launch shape the tuner picks).
+// 512^3, 128 seeds, Chebyshev: 442 us applying every seed in linear tiles, 83 us and 34 us of clearing now.
 template <typename K, uint32_t RUN>
 __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(sizeof(K) == 4 ? 5 : 4))) void k_naive(Launch L)
 {
-    __shared__ __attribute__((aligned(16))) uint32_t sx[kSeedChunk], sy[kSeedChunk], sz[kSeedChunk];
+    __shared__ __attribute__((aligned(16))) uint2 seeds[kSeedChunk];
+    __shared__ __attribute__((aligned(16))) uint2 near[kSeedChunk];
     __shared__ uint16_t sw[kSeedChunk];
     __shared__ uint16_t cells[kTileCells];  // compacted offsets of the occupied cells
-    __shared__ uint4 lab4[kTileCells / 8];  // the tile's output labels, 8 per thread
+    __shared__ uint4 lab4[kTileCells / 8];  // the brick's output labels, 8 per thread
     typedef uint16_t __attribute__((may_alias)) label_alias;  // single labels of lab4
     label_alias* lab = reinterpret_cast<label_alias*>(lab4);
-    __shared__ uint32_t wsum[kCellThreads / 64];
+    __shared__ uint32_t wsum[kCellThreads / 64], wmin[kCellThreads / 64];
     __shared__ JobDev sJ;
     __shared__ uint32_t sp[kWalkMaxJobs + 1];
     constexpr int kWant = sizeof(K) == 8 ? 1 : 0;
@@ -137,13 +166,52 @@ __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(si
         __syncthreads();
         for (uint32_t i = tid; i < n; i += blockDim.x) {
             const uint4 q = J.seeds[base + i];
-            sx[i] = q.x; sy[i] = q.y; sz[i] = q.z; sw[i] = (uint16_t)q.w;
+            seeds[i] = make_uint2(q.x | q.y << 16, q.z | i << 16);
+            sw[i] = (uint16_t)q.w;
         }
         __syncthreads();
     };
+    // the seeds of the n staged ones that may be nearest to a cell of the box, into near; bound: the least of the seeds'
+    // greatest distances so far.  Block-wide.
+    auto prune = [&](auto dist, uint32_t n, const uint32_t lo[3], const uint32_t hi[3], uint32_t& bound) {
+        constexpr int DIST = decltype(dist)::value;
+        constexpr uint32_t kPer = kSeedChunk / kCellThreads;
+        uint32_t dmin[kPer], far = 0xFFFFFFFFu;
+#pragma unroll
+        for (uint32_t c = 0; c < kPer; ++c) {
+            dmin[c] = 0xFFFFFFFFu;
+            const uint32_t i = c * kCellThreads + tid;
+            if (c * kCellThreads < n && i < n) {
+                uint32_t dmax;
+                box_dist<DIST>(seeds[i].x, seeds[i].y & 0xFFFFu, lo, hi, dmin[c], dmax);
+                far = min(far, dmax);
+            }
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) far = min(far, (uint32_t)__shfl_xor((int)far, o, 64));
+        if (lane == 0) wmin[wave] = far;
+        __syncthreads();
+        for (uint32_t w = 0; w < kCellThreads / 64; ++w) bound = min(bound, wmin[w]);
+        uint32_t m = 0;
+#pragma unroll
+        for (uint32_t c = 0; c < kPer; ++c) {
+            if (c * kCellThreads >= n) break;
+            const uint64_t keep = __ballot(dmin[c] <= bound);
+            if (lane == 0) wsum[wave] = (uint32_t)__popcll(keep);
+            __syncthreads();
+            uint32_t pos = m;
+            for (uint32_t w = 0; w < kCellThreads / 64; ++w) {
+                if (w < wave) pos += wsum[w];
+                m += wsum[w];
+            }
+            if ((keep >> lane) & 1u) near[pos + (uint32_t)__popcll(keep & ((1ull << lane) - 1ull))] = seeds[c * kCellThreads + tid];
+            __syncthreads();
+        }
+        return m;
+    };
     constexpr uint32_t kRun = RUN;
-    walk_tile_runs_strided<kRun>(L, L.tile_prefix, L.total_tiles, &sJ, sp, [&](const JobDev& J, uint32_t j, uint32_t first,
-                                                                              uint32_t nrun) {
+    walk_tile_runs_strided<kRun>(L, L.bt_prefix, L.total_bricks, &sJ, sp, [&](const JobDev& J, uint32_t j, uint32_t first,
+                                                                             uint32_t nrun) {
         if (!J.active || J.algo != VF_NAIVE || J.naive_key64 != kWant || J.S == 0) return;
         const uint32_t S = J.S;
         const bool one_chunk = S <= kSeedChunk;
@@ -151,24 +219,15 @@ __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(si
             stage(J, 0, S);
             staged = j;
         }
-        uint64_t occs[kRun];
+        uint32_t occs[(kRun + 3) / 4] = {};  // a byte per brick of the run
 #pragma unroll
-        for (uint32_t r = 0; r < kRun; ++r) {
-            const uint64_t c0 = (uint64_t)(first + r) * kTileCells + tid * kCellsPerThread;
-            occs[r] = r < nrun && c0 < J.V ? load8b(J.occ, c0, J.V) : 0ull;
-        }
-        auto tile = [&](uint32_t local, uint64_t occ) {
-        const uint64_t t0 = (uint64_t)local * kTileCells;
-        const uint64_t c0 = t0 + tid * kCellsPerThread;
-        if (!__syncthreads_or(occ != 0ull)) {  // an EMPTY tile (most of a vessel's box): labels stay EMPTY
-            if (c0 < J.V) {
-                const uint16_t zero[8] = { 0, 0, 0, 0, 0, 0, 0, 0 };
-                store8(J.labels, c0, J.V, zero);
-            }
-            return;
-        }
+        for (uint32_t r = 0; r < kRun; ++r)
+            occs[r / 4] |= (r < nrun ? group_occ(J, cell_group(J, first + r)) : 0u) << (8 * (r % 4));
+        auto brick = [&](uint32_t id, uint32_t occ) {
+        const BrickAt at = brick_at(J, id);
+        const CellGroup grp = cell_group(J, at);
         // block-wide exclusive scan of the occupied counts -> compacted positions
-        const uint32_t n = (uint32_t)__popcll(occ & 0x0101010101010101ull);
+        const uint32_t n = (uint32_t)__popc(occ);
         uint32_t inc = n;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -184,68 +243,84 @@ __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(si
             total += wsum[w];
         }
         for (int k = 0; k < 8; ++k)
-            if ((occ >> (8 * k)) & 0xFFu) cells[pos++] = (uint16_t)(tid * 8 + k);
+            if ((occ >> k) & 1u) cells[pos++] = (uint16_t)(tid * 8 + k);  // row of the brick * 32 + z
         __syncthreads();
-        if (total) {
-            // thread t holds compacted cells t, t + 256, ...: a wave's first lane holds the most, so
-            // waves past the last cell skip the seed loop.  Cells are taken four per thread at a time
-            // (the second group only in tiles with more than 1024 occupied cells), so the registers
-            // hold four cells' coordinates and keys, not eight.
-            const uint32_t nq = tid < total ? (total - tid + kCellThreads - 1) / kCellThreads : 0u;
-            const uint32_t tid0 = wave * 64u;
-            const uint32_t qmax = tid0 < total ? (total - tid0 + kCellThreads - 1) / kCellThreads : 0u;  // wave-uniform
-            const uint32_t b = J.key_bits;
-            const int dist = J.dist;
-            const K mask = ((K)1 << b) - 1;
-            const uint32_t groups = total > 4u * kCellThreads ? 2u : 1u;  // block-uniform
-            for (uint32_t g = 0; g < groups; ++g) {
-                const uint32_t q0 = 4u * g;
-                const uint32_t gq = nq > q0 ? min(nq - q0, 4u) : 0u;
-                const uint32_t gqmax = qmax > q0 ? min(qmax - q0, 4u) : 0u;  // wave-uniform
-                uint32_t cx[4], cy[4], cz[4];
+        const uint32_t lo[3] = { at.x, at.y, at.z },
+                       hi[3] = { min(at.x + kBrickX, J.nx) - 1u, min(at.y + kBrickY, J.ny) - 1u, min(at.z + kBrickZ, J.nz) - 1u };
+        const int dist = J.dist;
+        const bool drop = S > kPruneSeeds;
+        uint32_t bound = 0xFFFFFFFFu;
+        auto prune_any = [&](uint32_t m) {
+            if (dist == VF_MANHATTAN) return prune(std::integral_constant<int, VF_MANHATTAN>{}, m, lo, hi, bound);
+            if (dist == VF_CHEBYSHEV) return prune(std::integral_constant<int, VF_CHEBYSHEV>{}, m, lo, hi, bound);
+            if constexpr (sizeof(K) == 8)
+                if (dist == kDistEuclidF32) return prune(std::integral_constant<int, kDistEuclidF32>{}, m, lo, hi, bound);
+            return prune(std::integral_constant<int, VF_EUCLIDEAN>{}, m, lo, hi, bound);
+        };
+        uint32_t nnear = S;
+        if (one_chunk && drop) nnear = prune_any(S);
+        const uint2* list = drop ? near : seeds;
+        // thread t holds compacted cells t, t + 256, ...: a wave's first lane holds the most, so
+        // waves past the last cell skip the seed loop.  Cells are taken four per thread at a time
+        // (the second group only in bricks with more than 1024 occupied cells), so the registers
+        // hold four cells' coordinates and keys, not eight.
+        const uint32_t nq = tid < total ? (total - tid + kCellThreads - 1) / kCellThreads : 0u;
+        const uint32_t tid0 = wave * 64u;
+        const uint32_t qmax = tid0 < total ? (total - tid0 + kCellThreads - 1) / kCellThreads : 0u;  // wave-uniform
+        const uint32_t b = J.key_bits;
+        const K mask = ((K)1 << b) - 1;
+        const uint32_t groups = total > 4u * kCellThreads ? 2u : 1u;  // block-uniform
+        for (uint32_t g = 0; g < groups; ++g) {
+            const uint32_t q0 = 4u * g;
+            const uint32_t gq = nq > q0 ? min(nq - q0, 4u) : 0u;
+            const uint32_t gqmax = qmax > q0 ? min(qmax - q0, 4u) : 0u;  // wave-uniform
+            uint32_t cxy[4], cz[4];
 #pragma unroll
-                for (uint32_t q = 0; q < 4; ++q) {
-                    cx[q] = cy[q] = cz[q] = 0;
-                    if (q < gq) decompose(t0 + cells[tid + (q0 + q) * kCellThreads], J, cx[q], cy[q], cz[q]);
-                }
-                K best[4];
+            for (uint32_t q = 0; q < 4; ++q) {
+                const uint32_t c = q < gq ? cells[tid + (q0 + q) * kCellThreads] : 0u, row = c >> 5;
+                cxy[q] = (at.x + row / kBrickY) | (at.y + row % kBrickY) << 16;
+                cz[q] = at.z + (c & 31u);
+            }
+            K best[4];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) best[q] = ~(K)0;
-                for (uint32_t base = 0; base < S; base += kSeedChunk) {
-                    const uint32_t m = min(kSeedChunk, S - base);
-                    if (!one_chunk) {
-                        stage(J, base, m);
-                        staged = 0xFFFFFFFFu;
-                    }
-                    if (gqmax == 0) continue;  // staging above stays block-wide
-                    if (dist == VF_MANHATTAN) naive_cells<VF_MANHATTAN, K>(best, cx, cy, cz, gqmax, sx, sy, sz, base, m, b);
-                    else if (dist == VF_CHEBYSHEV) naive_cells<VF_CHEBYSHEV, K>(best, cx, cy, cz, gqmax, sx, sy, sz, base, m, b);
-                    else if (dist == VF_EUCLIDEAN) naive_cells<VF_EUCLIDEAN, K>(best, cx, cy, cz, gqmax, sx, sy, sz, base, m, b);
-                    else if constexpr (sizeof(K) == 8) naive_cells<kDistEuclidF32, K>(best, cx, cy, cz, gqmax, sx, sy, sz, base, m, b);
+            for (int q = 0; q < 4; ++q) best[q] = ~(K)0;
+            for (uint32_t base = 0; base < S; base += kSeedChunk) {
+                uint32_t m = one_chunk ? nnear : min(kSeedChunk, S - base);
+                if (!one_chunk) {
+                    stage(J, base, m);
+                    staged = 0xFFFFFFFFu;
+                    m = prune_any(m);
                 }
+                if (gqmax == 0) continue;  // staging above stays block-wide
+                if (dist == VF_MANHATTAN) naive_cells<VF_MANHATTAN, K>(best, cxy, cz, gqmax, list, base, m, b);
+                else if (dist == VF_CHEBYSHEV) naive_cells<VF_CHEBYSHEV, K>(best, cxy, cz, gqmax, list, base, m, b);
+                else if (dist == VF_EUCLIDEAN) naive_cells<VF_EUCLIDEAN, K>(best, cxy, cz, gqmax, list, base, m, b);
+                else if constexpr (sizeof(K) == 8) naive_cells<kDistEuclidF32, K>(best, cxy, cz, gqmax, list, base, m, b);
+            }
 #pragma unroll
-                for (uint32_t q = 0; q < 4; ++q) {
-                    if (q >= gq) break;
-                    const uint32_t id = (uint32_t)(best[q] & mask);
-                    lab[cells[tid + (q0 + q) * kCellThreads]] = one_chunk ? sw[id] : (uint16_t)J.seeds[id].w;
-                }
+            for (uint32_t q = 0; q < 4; ++q) {
+                if (q >= gq) break;
+                const uint32_t id = (uint32_t)(best[q] & mask);
+                lab[cells[tid + (q0 + q) * kCellThreads]] = one_chunk ? sw[id] : (uint16_t)J.seeds[id].w;
             }
         }
         __syncthreads();
-        if (c0 < J.V) {
-            const uint4 v = lab4[tid];
-            const uint16_t out[8] = { (uint16_t)v.x, (uint16_t)(v.x >> 16), (uint16_t)v.y, (uint16_t)(v.y >> 16),
-                                      (uint16_t)v.z, (uint16_t)(v.z >> 16), (uint16_t)v.w, (uint16_t)(v.w >> 16) };
-            store8(J.labels, c0, J.V, out);
-        }
-        __syncthreads();  // lab and cells are reused by the next tile
+        if (occ) store_group(J.labels, grp, lab4[tid]);
+        __syncthreads();  // lab and cells are reused by the next brick
         };
+        // the bricks of the run with an occupied cell; the others (most of a vessel's box) stay EMPTY
+        uint32_t any = 0;
+#pragma unroll
+        for (uint32_t r = 0; r < kRun; ++r) any |= ((occs[r / 4] >> (8 * (r % 4))) & 0xFFu) ? 1u << r : 0u;
+        any = (uint32_t)__ockl_wgred_or_i32((int)any);
 #pragma unroll 1
         for (uint32_t r = 0; r < nrun; ++r) {
-            uint64_t occ = occs[0];  // occs[r] by selects (a dynamic index would put occs in scratch)
+            if (!((any >> r) & 1u)) continue;
+            uint32_t occ = occs[0];  // the run's byte r, its word by selects (a dynamic index would put occs in scratch)
 #pragma unroll
-            for (uint32_t i = 1; i < kRun; ++i) occ = r == i ? occs[i] : occ;
-            tile(first + r, occ);
+            for (uint32_t i = 1; i < (kRun + 3) / 4; ++i) occ = r / 4 == i ? occs[i] : occ;
+            occ = (occ >> (8 * (r % 4))) & 0xFFu;
+            brick(first + r, occ);
         }
     });
 }
@@ -312,18 +387,20 @@ __global__ void k_ri_reset(uint32_t* counters, uint32_t idx) { counters[idx] = 0
 void launch_naive(const Launch& L, bool key64)
 {
     if (L.njobs > kWalkMaxJobs) fail(VF_ERR_INVALID_ARG, "naive launch with %u jobs (max %u)", L.njobs, kWalkMaxJobs);
-    const uint32_t blocks = std::max(1u, std::min(L.total_tiles, active_shape().cell_blocks));
+    const uint32_t blocks = std::max(1u, std::min(L.total_bricks, active_shape().cell_blocks));
     TimedLaunch tl(key64 ? "naive64" : "naive", L.s);
-    const uint32_t run = active_shape().naive_run;
-    if (key64) {
-        if (run == 4) k_naive<unsigned long long, 4><<<blocks, kCellThreads, 0, L.s>>>(L);
-        else if (run == 16) k_naive<unsigned long long, 16><<<blocks, kCellThreads, 0, L.s>>>(L);
-        else k_naive<unsigned long long, 8><<<blocks, kCellThreads, 0, L.s>>>(L);
-    } else {
-        if (run == 4) k_naive<uint32_t, 4><<<blocks, kCellThreads, 0, L.s>>>(L);
-        else if (run == 16) k_naive<uint32_t, 16><<<blocks, kCellThreads, 0, L.s>>>(L);
-        else k_naive<uint32_t, 8><<<blocks, kCellThreads, 0, L.s>>>(L);
-    }
+    // grids of few bricks: one brick per run, so that they spread over the device (in runs of 8 a 64^3 grid's 128
+    // bricks kept 16 workgroups busy)
+    const uint32_t run = L.total_bricks < kNaiveSmall ? 1u : active_shape().naive_run;
+    auto go = [&](auto r) {
+        constexpr uint32_t R = decltype(r)::value;
+        if (key64) k_naive<unsigned long long, R><<<blocks, kCellThreads, 0, L.s>>>(L);
+        else k_naive<uint32_t, R><<<blocks, kCellThreads, 0, L.s>>>(L);
+    };
+    if (run == 1) go(std::integral_constant<uint32_t, 1>{});
+    else if (run == 4) go(std::integral_constant<uint32_t, 4>{});
+    else if (run == 16) go(std::integral_constant<uint32_t, 16>{});
+    else go(std::integral_constant<uint32_t, 8>{});
     VF_CHECK_LAUNCH();
 }
 

@@ -1,10 +1,10 @@
 // Naive fracture of a caller-owned device grid without any device allocation.
 //
-// vf_fracture_naive works on a grid handle whose occupancy bytes, launch
+// vf_fracture_naive works on a grid handle whose occupancy bits, launch
 // descriptor and seed copy live in buffers the library allocated.  This
 // variant takes the cells as a plain device pointer and keeps everything else
 // in one file-scope device array, `scratch`, of a fixed size: the descriptor,
-// the one-job tile prefix, the seeds and the occupancy bytes of at most
+// the one-job prefixes, the seeds and the occupancy bits of at most
 // kNoAllocMaxCells cells.  The kernels are the ones vf_fracture_naive runs
 // (labels -> occupancy, then the naive labelling), given the array's device
 // address, which hipGetSymbolAddress returns once per device.  Every call on a
@@ -20,7 +20,8 @@ namespace vf {
 namespace {
 
 constexpr uint64_t kNoAllocMaxCells = VF_NOALLOC_MAX_CELLS;
-// layout of the array: descriptor, tile prefix and statistics, seeds, occupancy bytes
+// layout of the array: descriptor, tile and brick prefixes and statistics, seeds, occupancy bits (32-bit words of a column:
+// at most kNoAllocMaxCells bytes, the most being 4 bytes for each of 2048 x 2048 columns of up to 4 cells)
 constexpr size_t kOffJob = 0;
 constexpr size_t kOffPrefix = 512;
 constexpr size_t kOffStats = 576;
@@ -29,7 +30,7 @@ constexpr size_t kOffOcc = kOffSeeds + (size_t)kMaxDeviceSeeds * 16;
 constexpr size_t kScratchBytes = kOffOcc + kNoAllocMaxCells;
 static_assert(sizeof(JobDev) <= kOffPrefix - kOffJob, "descriptor slot");
 static_assert(kOffStats + kStatCount * 8 <= kOffSeeds, "statistics slot");
-static_assert(kOffOcc % 256 == 0, "occupancy bytes are 256-byte aligned");
+static_assert(kOffOcc % 256 == 0, "the occupancy is 256-byte aligned");
 static_assert(kScratchBytes == VF_NOALLOC_SCRATCH_BYTES, "the header states the array's size");
 
 // The array itself.  Host code never uses this name as an address: its device address
@@ -93,7 +94,7 @@ extern "C" int vf_fracture_naive_noalloc(uint16_t* d_cells, const uint32_t dims[
         uint8_t* base = scratch_ptr(device);
         hipStream_t s = static_cast<hipStream_t>(stream);
 
-        // descriptor, one-job tile prefix, zeroed statistics and seeds, staged on the host and copied once
+        // descriptor, one-job prefixes, zeroed statistics and seeds, staged on the host and copied once
         const NaiveKeyForm kf = naive_key_form(dims, distance, S);
         JobDev J{};
         J.nx = dims[0];
@@ -102,7 +103,8 @@ extern "C" int vf_fracture_naive_noalloc(uint16_t* d_cells, const uint32_t dims[
         J.wp = next_pow2(ceil_div(dims[2], 32));
         J.V = V;
         J.labels = d_cells;
-        J.occ = base + kOffOcc;
+        J.occ = reinterpret_cast<uint32_t*>(base + kOffOcc);
+        J.inv_ny = 1.0f / (float)dims[1];
         J.seeds = reinterpret_cast<uint4*>(base + kOffSeeds);
         J.S = S;
         J.S_draw = S;
@@ -112,11 +114,12 @@ extern "C" int vf_fracture_naive_noalloc(uint16_t* d_cells, const uint32_t dims[
         J.stats = reinterpret_cast<unsigned long long*>(base + kOffStats);
         J.active = 1;
         J.algo = VF_NAIVE;
-        const uint32_t tiles = ceil_div(V, kTileCells);
+        const uint32_t bricks = brick_count(dims[0], dims[1], dims[2]);
+        if (occ_words(dims) * 4 > kNoAllocMaxCells) fail(VF_ERR_OVERFLOW, "occupancy exceeds the no-allocation scratch");
         uint8_t* st = t_stage.bytes;
         std::memset(st, 0, kOffSeeds);
         std::memcpy(st + kOffJob, &J, sizeof J);
-        const uint32_t prefix[2] = { 0, tiles };
+        const uint32_t tiles = ceil_div(V, kTileCells), prefix[4] = { 0, tiles, 0, bricks };
         std::memcpy(st + kOffPrefix, prefix, sizeof prefix);
         std::memcpy(st + kOffSeeds, seeds, (size_t)S * sizeof(vf_seed));
         VF_HIP(hipMemcpyAsync(base, st, kOffSeeds + (size_t)S * sizeof(vf_seed), hipMemcpyHostToDevice, s));
@@ -128,8 +131,13 @@ extern "C" int vf_fracture_naive_noalloc(uint16_t* d_cells, const uint32_t dims[
         L.njobs = 1;
         L.tile_prefix = reinterpret_cast<const uint32_t*>(base + kOffPrefix);
         L.total_tiles = tiles;
+        L.wtile_prefix = nullptr;  // no seeding here
+        L.total_wtiles = 0;
+        L.bt_prefix = L.tile_prefix + 2;
+        L.total_bricks = bricks;
         L.s = s;
         launch_labels_to_occ(L);
+        launch_clear_labels(L);
         launch_naive(L, kf.key64 != 0);
         VF_HIP(hipStreamSynchronize(s));  // the staging is reused by the thread's next call
     });

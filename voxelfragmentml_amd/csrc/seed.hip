@@ -15,74 +15,111 @@ namespace {
 constexpr uint32_t kSeedThreads = 256;
 constexpr uint32_t kMaxDraws = 1000000u;
 
-__device__ inline bool surface_cell(const JobDev* J, uint32_t x, uint32_t y, uint32_t z)
+// Occupancy words of a 32-cell run and its two z neighbours: the word itself, and the words whose bit k is the
+// cell below (above) cell k, cells beyond the grid counting as occupied.
+struct ColumnRun {
+    uint32_t own, dn, up;
+};
+__device__ inline ColumnRun column_run(const JobDev& J, uint32_t x, uint32_t y, uint32_t wz)
 {
-    const int nx = (int)J->nx, ny = (int)J->ny, nz = (int)J->nz;
-    const int x0 = max((int)x - 1, 0), x1 = min((int)x + 1, nx - 1);
-    const int y0 = max((int)y - 1, 0), y1 = min((int)y + 1, ny - 1);
-    const int z0 = max((int)z - 1, 0), z1 = min((int)z + 1, nz - 1);
-    for (int a = x0; a <= x1; ++a)
-        for (int b = y0; b <= y1; ++b)
-            for (int c = z0; c <= z1; ++c)
-                if (J->occ[((size_t)a * ny + b) * nz + c] == 0) return true;
+    const auto* p = gcast<const uint32_t>(J.occ) + ((size_t)x * J.ny + y) * J.wp;
+    const uint32_t z0 = wz * 32u;
+    const uint32_t w = p[wz];
+    const uint32_t below = wz ? p[wz - 1u] >> 31 : 1u;
+    const uint32_t above = z0 + 32u < J.nz ? p[wz + 1u] & 1u : 1u;
+    ColumnRun r{ w, (w << 1) | below, (w >> 1) | (above << 31) };
+    if (J.nz - z0 < 32u) r.up |= 1u << (J.nz - z0 - 1u);  // the last cell has no upper neighbour
+    return r;
+}
+
+// Seed candidates among the cells of word wz of column (x, y): occupied cells, of jobs that seed on the surface or
+// inside only those whose clamped 3x3x3 window holds an EMPTY cell (RegularGrid::isBoundary) or none.
+__device__ inline uint32_t candidates(const JobDev& J, uint32_t x, uint32_t y, uint32_t wz)
+{
+    if (wz * 32u >= J.nz) return 0u;
+    const uint32_t own = gcast<const uint32_t>(J.occ)[((size_t)x * J.ny + y) * J.wp + wz];
+    if (J.seed_location == VF_SEED_BOTH || own == 0u) return own;
+    uint32_t inner = ~0u;
+    for (uint32_t a = x ? x - 1u : 0u; a <= min(x + 1u, J.nx - 1u); ++a)
+        for (uint32_t b = y ? y - 1u : 0u; b <= min(y + 1u, J.ny - 1u); ++b) {
+            const ColumnRun r = column_run(J, a, b, wz);
+            inner &= r.own & r.dn & r.up;
+        }
+    return J.seed_location == VF_SEED_OUTER ? own & ~inner : own & inner;
+}
+
+__device__ inline bool surface_cell(const JobDev& J, uint32_t x, uint32_t y, uint32_t z)
+{
+    for (uint32_t a = x ? x - 1u : 0u; a <= min(x + 1u, J.nx - 1u); ++a)
+        for (uint32_t b = y ? y - 1u : 0u; b <= min(y + 1u, J.ny - 1u); ++b) {
+            const ColumnRun r = column_run(J, a, b, z >> 5);
+            if (!(((r.own & r.dn & r.up) >> (z & 31u)) & 1u)) return true;
+        }
     return false;
 }
 
-__device__ inline bool candidate(const JobDev* J, uint64_t c, uint32_t x, uint32_t y, uint32_t z)
+// the candidates of word w of job J (0 past its last word)
+__device__ inline uint32_t word_candidates(const JobDev& J, uint32_t w)
 {
-    if (J->occ[c] == 0) return false;
-    if (J->seed_location == VF_SEED_BOTH) return true;
-    const bool s = surface_cell(J, x, y, z);
-    return (J->seed_location == VF_SEED_OUTER) == s;
+    const uint32_t lg = (uint32_t)__builtin_ctz(J.wp), col = w >> lg;
+    if (col >= J.nx * J.ny) return 0u;
+    const uint32_t x = col / J.ny;
+    return candidates(J, x, col - x * J.ny, w & (J.wp - 1u));
 }
 
-// skip_both: jobs that seed anywhere were counted by the voxelizer's fill
+// Candidates per word tile, one wave per tile and one lane per word: surface and interior cells are found 32 at a
+// time from the words of nine columns (cell by cell, 27 byte loads each, eight grids of 64^3 to 160^3 took
+// 310 us).  skip_both: jobs that seed anywhere were counted by the voxelizer's fill.
 __global__ __launch_bounds__(kCellThreads) void k_seed_count(Launch L, uint32_t* tile_cnt, bool skip_both)
 {
-    constexpr uint32_t kRun = 4;  // tiles per step: loads first, one block reduction for all of them
-    __shared__ uint32_t wsum[kRun][kCellThreads / 64];
-    __shared__ JobDev sJ;
-    walk_tile_runs<kRun>(L, L.tile_prefix, L.total_tiles, &sJ, [&](const JobDev& J, uint32_t j, uint32_t local, uint32_t nrun) {
-        if (skip_both && J.seed_location == VF_SEED_BOTH) return;  // block-uniform
-        uint32_t n[kRun];
-        uint64_t o[kRun];
+    const uint32_t lane = threadIdx.x & 63u, waves = gridDim.x * (kCellThreads / 64u);
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kCellThreads / 64u) + (threadIdx.x >> 6)));
+    for (uint32_t t = first; t < L.total_wtiles; t += waves) {
+        const uint32_t j = find_job(L.wtile_prefix, L.njobs, t);
+        const JobDev& J = L.jobs[j];
+        if (skip_both && J.seed_location == VF_SEED_BOTH) continue;  // wave-uniform
+        uint32_t n = J.active ? (uint32_t)__popc(word_candidates(J, (t - L.wtile_prefix[j]) * kTileWords + lane)) : 0u;
 #pragma unroll
-        for (uint32_t r = 0; r < kRun; ++r) {
-            const uint64_t c0 = (uint64_t)(local + r) * kTileCells + threadIdx.x * kCellsPerThread;
-            o[r] = J.active && r < nrun && c0 < J.V ? load8b(J.occ, c0, J.V) : 0ull;
-        }
-#pragma unroll
-        for (uint32_t r = 0; r < kRun; ++r) {
-            n[r] = 0;
-            if (J.seed_location == VF_SEED_BOTH) {
-                n[r] = __popcll(o[r] & 0x0101010101010101ull);
-            } else if (o[r]) {
-                const JobDev* Jg = L.jobs + j;
-                const uint64_t c0 = (uint64_t)(local + r) * kTileCells + threadIdx.x * kCellsPerThread;
-                uint32_t x, y, z;
-                decompose(c0, J, x, y, z);
-                for (int k = 0; k < 8 && c0 + k < J.V; ++k) {
-                    if ((o[r] >> (8 * k)) & 0xFFu) n[r] += candidate(Jg, c0 + k, x, y, z) ? 1u : 0u;
-                    advance(x, y, z, J);
-                }
-            }
-            for (int ofs = 32; ofs > 0; ofs >>= 1) n[r] += __shfl_xor(n[r], ofs, 64);
-        }
-        if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-            for (uint32_t r = 0; r < kRun; ++r) wsum[r][threadIdx.x >> 6] = n[r];
-        }
-        __syncthreads();
-        if (threadIdx.x < nrun) {
-            uint32_t tot = 0;
-            for (uint32_t w = 0; w < kCellThreads / 64; ++w) tot += wsum[threadIdx.x][w];
-            tile_cnt[L.tile_prefix[j] + local + threadIdx.x] = tot;
-        }
-        __syncthreads();
-    });
+        for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+        if (lane == 0) tile_cnt[t] = n;
+    }
 }
 
-// One block per job.
+// The largest t in [lo, hi) with off[t] <= want, off ascending and off[lo] <= want, searched by a wave with 64
+// probes a step.
+__device__ inline uint32_t wave_last_below(const unsigned long long* off, uint32_t lo, uint32_t hi, unsigned long long want)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    while (hi - lo > 1u) {
+        const uint32_t step = (hi - lo + 63u) / 64u, idx = lo + lane * step;
+        const uint64_t m = __ballot(idx < hi && off[idx] <= want);
+        lo += (63u - (uint32_t)__clzll((long long)m)) * step;
+        hi = min(lo + step, hi);
+    }
+    return lo;
+}
+
+// The index of the n-th set bit of v (n below its bit count).
+__device__ inline uint32_t nth_bit(uint32_t v, uint32_t n)
+{
+    uint32_t pos = 0;
+#pragma unroll
+    for (uint32_t half = 16u; half; half >>= 1) {
+        const uint32_t c = (uint32_t)__popc(v & ((1u << half) - 1u));
+        if (n >= c) {
+            n -= c;
+            v >>= half;
+            pos += half;
+        }
+    }
+    return pos;
+}
+
+// kPickParts blocks per job: each draws and sorts the job's ranks by itself (in LDS, a few microseconds) and then
+// finds the cells of its share of them, a wave per seed.  Bound by latency: three dependent probes of the tile
+// offsets, the tile's words, a bit select.  One block per job, a binary search per seed and a walk over the tile's
+// cells took 180 us for the 128 seeds of a 512^3 grid.
+constexpr uint32_t kPickParts = 8;
 __global__ __launch_bounds__(kSeedThreads) void k_seed_pick(Launch L, const unsigned long long* tile_off)
 {
     __shared__ uint32_t chosen[kMaxDeviceSeeds];
@@ -90,16 +127,18 @@ __global__ __launch_bounds__(kSeedThreads) void k_seed_pick(Launch L, const unsi
     __shared__ uint32_t cand[kSeedThreads];
     __shared__ uint32_t wsum[kSeedThreads / 64];
     __shared__ uint32_t s_got;
-    const uint32_t j = blockIdx.x;
+    const uint32_t j = blockIdx.x / kPickParts, part = blockIdx.x % kPickParts;
     const JobDev* J = L.jobs + j;
     if (!J->active) return;
     const uint32_t S = J->S_draw;
-    const uint32_t t0 = L.tile_prefix[j], t1 = L.tile_prefix[j + 1];
+    constexpr uint32_t kWaves = kSeedThreads / 64u;
+    if (part * kWaves >= S) return;  // no seed of this part
+    const uint32_t t0 = L.wtile_prefix[j], t1 = L.wtile_prefix[j + 1];
     const unsigned long long base = tile_off[t0];
     const unsigned long long O = tile_off[t1] - base;
-    if (S == 0) return;
     // on failure every seed is parked on cell (0,0,0) so later stages stay in bounds
     auto park = [&]() {
+        if (part) return;
         if (threadIdx.x == 0) atomicOr(reinterpret_cast<unsigned int*>(J->stats + kStatError), (unsigned int)kDevErrSeeding);
         for (uint32_t i = threadIdx.x; i < S; i += blockDim.x) J->seeds[i] = make_uint4(0u, 0u, 0u, 2u + (i & 0xFFu));
     };
@@ -151,47 +190,16 @@ __global__ __launch_bounds__(kSeedThreads) void k_seed_pick(Launch L, const unsi
         sorted[p] = r;
     }
     __syncthreads();
-    // rank -> tile: one binary search over the tile prefix per seed (the ranks are sorted, so
-    // chosen[] is free to hold the tile index)
-    for (uint32_t i = threadIdx.x; i < S; i += blockDim.x) {
-        const unsigned long long want = base + sorted[i];
-        uint32_t lo = t0, hi = t1;  // largest t with tile_off[t] <= want
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (tile_off[mid] <= want) lo = mid; else hi = mid;
-        }
-        chosen[i] = lo;
-    }
-    __syncthreads();
-    // tile -> cell: one wave per seed; lane l counts the candidates among the tile's cells
-    // [32 l, 32 l + 32), a wave scan finds the lane holding the wanted one, and that lane walks
-    // its 32 cells.  Cells outside the grid are no candidates.
+    // rank -> tile -> cell: lane l holds the candidates of the tile's word l, a wave scan finds the lane with the
+    // wanted one
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    for (uint32_t i = wave; i < S; i += kSeedThreads / 64u) {
-        const uint32_t t = chosen[i];
-        const uint32_t need = (uint32_t)(base + sorted[i] - tile_off[t]);
-        const uint64_t c0 = (uint64_t)(t - t0) * kTileCells + (uint64_t)lane * 32u;
-        uint32_t cnt = 0;
-        if (c0 < J->V) {
-            if (J->seed_location == VF_SEED_BOTH) {
-                if (c0 + 32u <= J->V) {
-                    const uint4 a = gload4(J->occ + c0);
-                    const uint4 b = gload4(J->occ + c0 + 16u);
-                    const uint64_t m = 0x0101010101010101ull;
-                    cnt = __popcll((((uint64_t)a.y << 32) | a.x) & m) + __popcll((((uint64_t)a.w << 32) | a.z) & m) +
-                          __popcll((((uint64_t)b.y << 32) | b.x) & m) + __popcll((((uint64_t)b.w << 32) | b.z) & m);
-                } else {
-                    for (uint64_t c = c0; c < J->V; ++c) cnt += J->occ[c] != 0;
-                }
-            } else {
-                uint32_t x, y, z;
-                decompose(c0, J, x, y, z);
-                for (uint64_t c = c0; c < c0 + 32u && c < J->V; ++c) {
-                    cnt += candidate(J, c, x, y, z) ? 1u : 0u;
-                    advance(x, y, z, J);
-                }
-            }
-        }
+    for (uint32_t i = part * kWaves + wave; i < S; i += kPickParts * kWaves) {
+        const unsigned long long want = base + sorted[i];
+        const uint32_t t = wave_last_below(tile_off, t0, t1, want);
+        const uint32_t need = (uint32_t)(want - tile_off[t]);
+        const uint32_t w = (t - t0) * kTileWords + lane;
+        const uint32_t bits = word_candidates(*J, w);
+        const uint32_t cnt = (uint32_t)__popc(bits);
         uint32_t inc = cnt;  // wave inclusive scan
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -200,19 +208,8 @@ __global__ __launch_bounds__(kSeedThreads) void k_seed_pick(Launch L, const unsi
         }
         const bool holder = inc > need && inc - cnt <= need;
         if (holder) {
-            uint32_t left = need - (inc - cnt);
-            uint32_t x, y, z;
-            decompose(c0, J, x, y, z);
-            for (uint64_t c = c0; c < c0 + 32u && c < J->V; ++c) {
-                if (candidate(J, c, x, y, z)) {
-                    if (left == 0) {
-                        J->seeds[i] = make_uint4(x, y, z, 2u + i);
-                        break;
-                    }
-                    --left;
-                }
-                advance(x, y, z, J);
-            }
+            const uint32_t col = w >> (uint32_t)__builtin_ctz(J->wp), x = col / J->ny;
+            J->seeds[i] = make_uint4(x, col - x * J->ny, (w & (J->wp - 1u)) * 32u + nth_bit(bits, need - (inc - cnt)), 2u + i);
         }
         if (__ballot(holder) == 0ull && lane == 0) {  // the counts disagree with the tile prefix
             J->seeds[i] = make_uint4(0u, 0u, 0u, 2u + i);
@@ -333,7 +330,7 @@ __device__ __forceinline__ uint32_t near_draw(const JobDev* J, const uint4* frag
             uint32_t id = 0xFFFFFFFFu;
             if (t < kMaxDraws && d2 <= (int64_t)mind * mind) {
                 const size_t cell = ((size_t)c[0] * n[1] + c[1]) * n[2] + c[2];
-                if (J->occ[cell] && surface_cell(J, c[0], c[1], c[2])) {
+                if (occ_bit(*J, c[0], c[1], c[2]) && surface_cell(*J, c[0], c[1], c[2])) {
                     id = (uint32_t)cell;
                     for (uint32_t q = 0; q < s_n && id != 0xFFFFFFFFu; ++q)
                         if (chosen[q] == id) id = 0xFFFFFFFFu;
@@ -457,7 +454,7 @@ void launch_seed_counts(const Launch& L)
 void launch_seed_count(const Launch& L, uint32_t* tile_cnt, bool skip_both)
 {
     TimedLaunch tl("seed_count", L.s);
-    const uint32_t blocks = std::max(1u, std::min(L.total_tiles, active_shape().cell_blocks));
+    const uint32_t blocks = std::max(1u, std::min(ceil_div(L.total_wtiles, kCellThreads / 64u), active_shape().cell_blocks));
     k_seed_count<<<blocks, kCellThreads, 0, L.s>>>(L, tile_cnt, skip_both);
     VF_CHECK_LAUNCH();
 }
@@ -465,7 +462,7 @@ void launch_seed_count(const Launch& L, uint32_t* tile_cnt, bool skip_both)
 void launch_seed_pick(const Launch& L, const unsigned long long* tile_off)
 {
     TimedLaunch tl("seed_pick", L.s);
-    k_seed_pick<<<L.njobs, kSeedThreads, 0, L.s>>>(L, tile_off);
+    k_seed_pick<<<L.njobs * kPickParts, kSeedThreads, 0, L.s>>>(L, tile_off);
     VF_CHECK_LAUNCH();
 }
 

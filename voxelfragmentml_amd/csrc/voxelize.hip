@@ -13,7 +13,7 @@
 //                    column centres toggle the first cell centre above the
 //                    crossing (exact int64 edge functions), atomicXor
 //   5. k_vox_fill    one lane per 32-cell column word: prefix-XOR in the word,
-//                    carry across the column by wave ballot, occupancy bytes
+//                    carry across the column by wave ballot, occupancy bits
 //                    = shell | parity, occupied count
 // Compiled with -ffp-contract=off: FP32 results equal the CPU oracle's.
 #include "cellops.hpp"
@@ -503,21 +503,16 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_parity(const JobDev* jobs, 
     });
 }
 
-// 4 bits -> 4 bytes of 0/1 (bit i -> byte i)
-__device__ inline uint32_t spread4(uint32_t b) { return ((b & 0xFu) * 0x00204081u) & 0x01010101u; }
-
-// tile_cnt (or null): per 2048-cell tile (indexed by L.tile_prefix) occupied-cell counts for jobs that seed
-// anywhere, added here from the occupancy bits (zeroed by k_vox_clear); a wave's 64 words are whole
-// columns, at most 2048 consecutive cells, so they touch at most two tiles
+// Occupancy bits = shell | parity interior, left in place of the shell bits.  Bound by HBM: 8 bytes read and 4
+// written per 32 cells (as one byte per cell, 32 written, the 512^3 fill took 80 us, and every later stage
+// read those bytes).  tile_cnt (or null): a wave's 64 words are one word tile, whose occupied cells it counts
+// for jobs that seed anywhere.
 __global__ __launch_bounds__(kVoxThreads) void k_vox_fill(Launch L, const uint32_t* col_prefix, uint32_t total_groups,
                                                           uint32_t* tile_cnt)
 {
     __shared__ JobDev sJ;
     __shared__ unsigned long long part[kVoxThreads / 64];
-    // a wave's 64 words are whole columns (wp divides 64): at most 2048 consecutive occupancy bytes, staged
-    // here and stored as dwords with consecutive lanes on consecutive dwords (a lane's own 32 bytes would
-    // put a wave's 16-byte stores 32 bytes apart)
-    __shared__ uint32_t stage[kVoxThreads / 64][512];
+    static_assert(kTileWords == 64, "a wave's words are one tile");
     unsigned long long acc = 0;
     constexpr uint32_t kRun = 4;  // column groups per step: all their bit loads are issued first
     walk_tile_runs<kRun>(L, col_prefix, total_groups, &sJ, [&](const JobDev& J, uint32_t jidx, uint32_t first, uint32_t nrun) {
@@ -531,79 +526,33 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_fill(Launch L, const uint32
             tgs[r] = valid ? gcast<const uint32_t>(J.toggle_bits)[w] : 0u;
             shs[r] = valid ? gcast<const uint32_t>(J.shell_bits)[w] : 0u;
         }
+        const uint32_t lane = threadIdx.x & 63u;
+        const uint32_t seg = lane & ~(J.wp - 1u);
+        const uint64_t below = (lane ? (~0ull >> (64u - lane)) : 0ull) & ~(seg ? (~0ull >> (64u - seg)) : 0ull);
 #pragma unroll
         for (uint32_t r = 0; r < kRun; ++r) {
             if (r >= nrun) break;
             const uint64_t w = (uint64_t)(first + r) * kVoxThreads + threadIdx.x;
-            const bool valid = w < nwords;
             const uint32_t tg = tgs[r];
-            const uint32_t sh = shs[r];
             uint32_t p = tg;
             p ^= p << 1; p ^= p << 2; p ^= p << 4; p ^= p << 8; p ^= p << 16;
             const uint64_t par = __ballot(__popc(tg) & 1);
-            const uint32_t lane = threadIdx.x & 63;
-            const uint32_t seg = lane & ~(J.wp - 1);
-            const uint64_t below = (lane ? (~0ull >> (64 - lane)) : 0ull) & ~(seg ? (~0ull >> (64 - seg)) : 0ull);
             if (__popcll(par & below) & 1) p = ~p;
             uint32_t bits = 0;
-            uint32_t nb = 0;
-            uint64_t base = 0;
-            if (valid) {
-                const uint32_t lgwp = (uint32_t)__builtin_ctz(J.wp);  // wp is a power of two
-                const uint64_t col = w >> lgwp;
+            if (w < nwords) {
                 const uint32_t z0 = (uint32_t)(w & (J.wp - 1u)) * 32u;
                 if (z0 < J.nz) {
-                    nb = min(32u, J.nz - z0);
-                    bits = (sh | p) & (nb == 32 ? 0xFFFFFFFFu : ((1u << nb) - 1u));
-                    base = col * J.nz + z0;
+                    const uint32_t nb = min(32u, J.nz - z0);
+                    bits = (shs[r] | p) & (nb == 32 ? 0xFFFFFFFFu : ((1u << nb) - 1u));
                 }
+                gcast<uint32_t>(J.shell_bits)[w] = bits;
             }
-            if ((J.nz & 3u) == 0) {
-                // the wave's region starts at lane 0's cell (a column start when lane 0's word is valid;
-                // when it is not, no lane's is) and spans its valid columns
-                const uint32_t lgwp = (uint32_t)__builtin_ctz(J.wp);
-                const uint64_t w0 = w - lane;
-                const uint64_t col0 = w0 >> lgwp, cols = (uint64_t)J.nx * J.ny;
-                const uint32_t ncols = col0 < cols ? (uint32_t)min<uint64_t>(64u >> lgwp, cols - col0) : 0u;
-                const uint32_t ndw = ncols * (J.nz / 4);  // dwords of the region, <= 512
-                uint32_t* st = stage[threadIdx.x >> 6];
-                if (nb) {
-                    const uint32_t off = (uint32_t)((w & (64u - 1u)) >> lgwp) * (J.nz / 4) + (uint32_t)(w & (J.wp - 1u)) * 8u;
+            uint32_t cnt = (uint32_t)__popc(bits);
+            acc += cnt;
+            if (tile_cnt && J.seed_location == VF_SEED_BOTH) {  // block-uniform
 #pragma unroll
-                    for (uint32_t q = 0; q < 8; ++q)
-                        if (4 * q < nb) st[off + q] = spread4(bits >> (4 * q));
-                }
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                auto* dst = gcast<uint32_t>(J.occ + (col0 * J.nz));
-                for (uint32_t i = lane; i < ndw; i += 64) dst[i] = st[i];
-                __builtin_amdgcn_wave_barrier();  // the stage is rewritten by the next group
-            } else if (nb) {
-                uint8_t* o = J.occ + base;
-                for (uint32_t q = 0; q < nb; ++q) o[q] = (uint8_t)((bits >> q) & 1u);
-            }
-            acc += (unsigned long long)__popc(bits);
-            if (tile_cnt && J.seed_location == VF_SEED_BOTH) {
-                const uint64_t b0 = __builtin_amdgcn_readfirstlane((uint32_t)base) |
-                                    ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) << 32);
-                const uint64_t ta = b0 >> 11;  // the wave's first tile (lane 0 holds a column start)
-                const uint64_t split = (ta + 1) << 11;  // first cell of the next tile
-                uint32_t na = 0;
-                if (nb) {
-                    const uint32_t below = base >= split ? 0u : (uint32_t)min<uint64_t>(split - base, 32);
-                    na = __popc(bits & (below == 32 ? 0xFFFFFFFFu : ((1u << below) - 1u)));
-                }
-                // both counts (<= 32 per lane, <= 2048 per wave) packed in one 32-bit wave sum
-                uint32_t both = na | ((uint32_t)__popc(bits) - na) << 16;
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) both += __shfl_xor(both, o, 64);
-                const uint32_t sa = both & 0xFFFFu, sb = both >> 16;
-                if ((threadIdx.x & 63u) == 0) {
-                    const uint32_t t0 = L.tile_prefix[jidx];
-                    if (sa) atomicAdd(tile_cnt + t0 + (uint32_t)ta, sa);
-                    if (sb) atomicAdd(tile_cnt + t0 + (uint32_t)ta + 1u, sb);
-                }
+                for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
+                if (lane == 0 && w < nwords) tile_cnt[L.wtile_prefix[jidx] + (uint32_t)(w / kTileWords)] = cnt;
             }
         }
     }, [&](uint32_t j) {
@@ -613,18 +562,16 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_fill(Launch L, const uint32
         if (threadIdx.x == 0) {
             unsigned long long tot = 0;
             for (uint32_t w = 0; w < kVoxThreads / 64; ++w) tot += part[w];
-            if (tot) atomicAdd(L.jobs[j].stats + kStatOccupied, tot);
+            const JobDev& J = L.jobs[j];
+            if (tot && J.sums) atomicAdd(J.sums + (blockIdx.x % kSumSlots) * kStatCount + kStatOccupied, tot);
         }
         __syncthreads();
         acc = 0;
     });
 }
 
-__global__ __launch_bounds__(kVoxThreads) void k_vox_clear(Launch L, const uint32_t* col_prefix, uint32_t total_groups,
-                                                           uint32_t* tile_cnt)
+__global__ __launch_bounds__(kVoxThreads) void k_vox_clear(Launch L, const uint32_t* col_prefix, uint32_t total_groups)
 {
-    if (tile_cnt)
-        for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < L.total_tiles; i += gridDim.x * blockDim.x) tile_cnt[i] = 0u;
     __shared__ JobDev sJ;
     walk_tiles(L, col_prefix, total_groups, &sJ, [&](const JobDev& J, uint32_t, uint32_t group, uint32_t) {
         if (!J.active) return;
@@ -634,18 +581,17 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_clear(Launch L, const uint3
             gcast<uint32_t>(J.toggle_bits)[w] = 0u;
             gcast<uint32_t>(J.shell_bits)[w] = 0u;
         }
-        if (w == 0) J.stats[kStatOccupied] = 0;
     });
 }
 
 }  // namespace
 
 
-void launch_clear_bits(const Launch& L, const uint32_t* col_prefix, uint32_t total_groups, uint32_t* tile_cnt)
+void launch_clear_bits(const Launch& L, const uint32_t* col_prefix, uint32_t total_groups)
 {
     TimedLaunch tl("vox_clear", L.s);
     const uint32_t blocks = std::max(1u, std::min(total_groups, active_shape().cell_blocks));
-    k_vox_clear<<<blocks, kVoxThreads, 0, L.s>>>(L, col_prefix, total_groups, tile_cnt);
+    k_vox_clear<<<blocks, kVoxThreads, 0, L.s>>>(L, col_prefix, total_groups);
     VF_CHECK_LAUNCH();
 }
 
@@ -654,7 +600,7 @@ void launch_voxelize(const Launch& L, const VoxScratch& X, const uint32_t* col_p
                      uint32_t* tile_cnt)
 {
     if (L.njobs > kWalkMaxJobs) fail(VF_ERR_INVALID_ARG, "voxelize launch with %u jobs (max %u)", L.njobs, kWalkMaxJobs);
-    launch_clear_bits(L, col_prefix, total_groups, tile_cnt);
+    launch_clear_bits(L, col_prefix, total_groups);
     if (X.total_tris) {
         uint32_t* cnt_shell = X.counts;
         uint32_t* cnt_col = cnt_shell + X.total_tris;
