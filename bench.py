@@ -108,7 +108,7 @@ def build_jobs(vf, specs, mc=False):
 # histogram 2 B per cell (labels read); marching cubes 2 B per cell + 12 B per
 # vertex and per triangle.  A kernel that fuses stages counts each stage's bytes.
 STAGES = {
-    "voxelize": ["job_init", "vox_clear", "vox_setup", "scan", "vox_shell", "vox_parity", "vox_fill"],
+    "voxelize": ["job_init", "vox_clear", "vox_setup", "scan", "vox_pairs", "vox_fill"],
     "seed": ["seed_count", "seed_pick"],
     "naive": ["naive", "naive64"],
     "flood": ["flood_init", "flood_seed", "flood_compact", "flood_relax", "flood_plan", "flood_finish"],
@@ -226,7 +226,7 @@ def roofline(prof, specs, res, traffic_ok):
         out["limiter"] = ("latency of each visit's dependent chain (halo loads, then sweeps of LDS round trips) over "
                           "dependent rounds: 13 of 18 waves per CU resident (4 x SQ_WAVE_CYCLES / SQ_BUSY_CYCLES per "
                           "CU), waiting on results 42 % and on issue 30 % of their time (SQ_WAIT_ANY, SQ_WAIT_INST_ANY), "
-                          "VALU at 40 % of the rate k_vox_shell sustains (SQ_INSTS_VALU); not HBM")
+                          "VALU at 40 % of the rate the voxelizer sustains (SQ_INSTS_VALU); not HBM")
         out["unit_work"] = {"brick_visits_per_step": visits, "visit_bytes_per_step": 4096 * visits,
                             "sweeps_per_step": sum(r["flood_sweeps"] for r in res),
                             "visit_gbs": round(4096 * visits / launches / (prof[dom]["avg_ms"] * 1e-3) / 1e9, 1)}

@@ -6,13 +6,13 @@
 //   1. k_vox_setup   per triangle: SAT candidate cell box, snapped fixed-point
 //                    vertices, parity column range, pair counts
 //   2. scans         exclusive prefix of the pair counts (load balancing)
-//   3. k_vox_shell   one thread per (triangle, column, 32-cell z word): SAT
+//   3. k_vox_pairs   shell: one thread per (triangle, column, 32-cell z word): SAT
 //                    (Intersections3D.h:204-420 arithmetic) per cell with the
-//                    z-free terms once per column, one atomicOr per word
-//   4. k_vox_parity  one thread per (triangle, column) pair: top-left covered
+//                    z-free terms once per column, one atomicOr per word;
+//                    parity: one thread per (triangle, column) pair: top-left covered
 //                    column centres toggle the first cell centre above the
 //                    crossing (exact int64 edge functions), atomicXor
-//   5. k_vox_fill    one lane per 32-cell column word: prefix-XOR in the word,
+//   4. k_vox_fill    one lane per 32-cell column word: prefix-XOR in the word,
 //                    carry across the column by wave ballot, occupancy bits
 //                    = shell | parity, occupied count
 // Compiled with -ffp-contract=off: FP32 results equal the CPU oracle's.
@@ -28,15 +28,70 @@ constexpr uint32_t kVoxThreads = 256;
 constexpr float kRangeMargin = 0.015625f;   // 1/64 cell
 constexpr uint32_t kInlineShell = 8;        // SAT candidates a setup thread tests itself
 constexpr uint32_t kInlineCols = 8;         // parity columns a setup thread toggles itself
+constexpr uint32_t kWildTriangle = 1u << 31;  // TriSetup::job flag: coordinates of kTameLimit or more
 constexpr uint32_t kColBits = 4;            // column index bits in the setup kernel's owner tables
 static_assert(kInlineShell <= (1u << kColBits) && kInlineCols <= (1u << kColBits), "owner table encoding");
 
-__device__ inline bool axis_sep(float pa, float pb, float rad)
+// A separating-axis test in two forms with the same outcome.  Exact: comparisons as the reference makes them.  Tame (no
+// operand is infinite or NaN): each axis yields a value above 0 where it separates, and a cell's values are combined by
+// one running maximum, which takes fewer instructions than a comparison each: x > y exactly where x - y > 0.
+template <bool TAME>
+struct Separation {
+    float most = -1.0f;
+    bool sep = false;
+    // projections pa, pb both beyond rad on one side: min(pa, pb) > rad || max(pa, pb) < -rad (the median of pa, pb and
+    // 0 is the one nearer to 0 when both lie on one side of it, else 0)
+    __device__ inline void axis(float pa, float pb, float rad)
+    {
+        if (TAME) {
+            most = __builtin_fmaxf(most, fabsf(__builtin_amdgcn_fmed3f(pa, pb, 0.0f)) - rad);
+        } else {
+            float mn = pa < pb ? pa : pb;
+            float mx = pa < pb ? pb : pa;
+            sep |= mn > rad || mx < -rad;
+        }
+    }
+    // a box face: all three of a, b, c beyond h on one side
+    __device__ inline void face(float a, float b, float c, float h)
+    {
+        if (TAME) {
+            const float mn = __builtin_fminf(__builtin_fminf(a, b), c), mx = __builtin_fmaxf(__builtin_fmaxf(a, b), c);
+            most = __builtin_fmaxf(most, __builtin_fmaxf(mn, -mx) - h);
+        } else {
+            float mn = a, mx = a;
+            if (b < mn) mn = b;
+            if (b > mx) mx = b;
+            if (c < mn) mn = c;
+            if (c > mx) mx = c;
+            sep |= mn > h || mx < -h;
+        }
+    }
+    // the triangle's plane: the box's least and greatest distance along the normal
+    __device__ inline void plane(float dmin, float dmax)
+    {
+        if (TAME) most = __builtin_fmaxf(__builtin_fmaxf(most, dmin), -dmax);
+        else sep |= dmin > 0.0f || !(dmax >= 0.0f);
+    }
+    __device__ inline bool any() const { return TAME ? most > 0.0f : sep; }
+};
+
+// n times the end of [lo, hi] that makes it least, and greatest.
+template <bool TAME>
+__device__ inline void span(float n, float lo, float hi, float& least, float& greatest)
 {
-    float mn = pa < pb ? pa : pb;
-    float mx = pa < pb ? pb : pa;
-    return mn > rad || mx < -rad;
+    if (TAME) {
+        const float a = n * lo, b = n * hi;
+        least = __builtin_fminf(a, b);
+        greatest = __builtin_fmaxf(a, b);
+    } else {
+        least = n * (n > 0.0f ? lo : hi);
+        greatest = n * (n > 0.0f ? hi : lo);
+    }
 }
+
+// Coordinates below this keep every product and sum of the SAT finite (three factors of at most 4e12 and sums of
+// three of them stay below 3e38), so no operand of a comparison is NaN.
+constexpr float kTameLimit = 1e12f;
 
 __device__ inline void cell_box(int i, float mn, float cs, float* center, float* half)
 {
@@ -47,69 +102,111 @@ __device__ inline void cell_box(int i, float mn, float cs, float* center, float*
 }
 
 // The triangle/box SAT of Intersections3D::intersect(Triangle3D&, AABB&) (Intersections3D.h:204-420:
-// nine edge-cross axes, the three box faces, the triangle plane) for the cells (x, y, z0..z1) of one
-// grid column, z0..z1 inside one 32-cell word: bit (z & 31) is set when cell (x, y, z) passes.  For
+// nine edge-cross axes, the three box faces, the triangle plane) for the cells of one grid column.  For
 // each cell every FP32 operation is the reference's (same operands, same order, no contraction), so
-// a cell passes exactly when the per-cell test passes; the operations that do not depend on z (x and
-// y offsets and edge components, the third axis of each edge, the x and y box faces, the normal's z
-// component) are evaluated once per column, and a cell's tests are combined without branches (which
-// axis separates first does not change the outcome).
-__device__ uint32_t sat_column(const float* a, const float* b, const float* c, float cx, float hx, float cy, float hy,
-                               int z0, int z1, float mnz, float csz)
+// a cell passes exactly when the per-cell test passes; which axis separates first does not change the outcome.
+// Column: what a column of cells shares, the vertices' x and y offsets from its centre, its half extents and the
+// vertices' z.
+struct Column {
+    float v0x, v1x, v2x, v0y, v1y, v2y, hx, hy, az, bz, cz;
+};
+__device__ inline Column make_column(const float* a, const float* b, const float* c, float cx, float hx, float cy, float hy)
 {
-    const float v0x = a[0] - cx, v1x = b[0] - cx, v2x = c[0] - cx;
-    const float v0y = a[1] - cy, v1y = b[1] - cy, v2y = c[1] - cy;
-    const float e0x = v1x - v0x, e1x = v2x - v1x, e2x = v0x - v2x;
-    const float e0y = v1y - v0y, e1y = v2y - v1y, e2y = v0y - v2y;
+    return Column{ a[0] - cx, b[0] - cx, c[0] - cx, a[1] - cy, b[1] - cy, c[1] - cy, hx, hy, a[2], b[2], c[2] };
+}
+
+// The tests that do not depend on z (the third axis of each edge, the x and y faces): false when no cell passes.
+template <bool TAME>
+__device__ __forceinline__ bool column_open(const Column& q)
+{
+    const float e0x = q.v1x - q.v0x, e1x = q.v2x - q.v1x, e2x = q.v0x - q.v2x;
+    const float e0y = q.v1y - q.v0y, e1y = q.v2y - q.v1y, e2y = q.v0y - q.v2y;
+    Separation<TAME> s;
+    s.axis(e0y * q.v1x - e0x * q.v1y, e0y * q.v2x - e0x * q.v2y, fabsf(e0y) * q.hx + fabsf(e0x) * q.hy);
+    s.axis(e1y * q.v0x - e1x * q.v0y, e1y * q.v1x - e1x * q.v1y, fabsf(e1y) * q.hx + fabsf(e1x) * q.hy);
+    s.axis(e2y * q.v1x - e2x * q.v1y, e2y * q.v2x - e2x * q.v2y, fabsf(e2y) * q.hx + fabsf(e2x) * q.hy);
+    s.face(q.v0x, q.v1x, q.v2x, q.hx);
+    s.face(q.v0y, q.v1y, q.v2y, q.hy);
+    return !s.any();
+}
+
+// The tests that do, for the cell between z planes lo and hi of an open column.
+template <bool TAME>
+__device__ __forceinline__ bool cell_passes(const Column& q, float lo, float hi)
+{
+    const float e0x = q.v1x - q.v0x, e1x = q.v2x - q.v1x, e2x = q.v0x - q.v2x;
+    const float e0y = q.v1y - q.v0y, e1y = q.v2y - q.v1y, e2y = q.v0y - q.v2y;
     const float f0x = fabsf(e0x), f0y = fabsf(e0y), f1x = fabsf(e1x), f1y = fabsf(e1y), f2x = fabsf(e2x), f2y = fabsf(e2y);
-    bool sep = axis_sep(e0y * v1x - e0x * v1y, e0y * v2x - e0x * v2y, f0y * hx + f0x * hy);
-    sep |= axis_sep(e1y * v0x - e1x * v0y, e1y * v1x - e1x * v1y, f1y * hx + f1x * hy);
-    sep |= axis_sep(e2y * v1x - e2x * v1y, e2y * v2x - e2x * v2y, f2y * hx + f2x * hy);
-    {
-        float mn = v0x, mx = v0x;
-        if (v1x < mn) mn = v1x;
-        if (v1x > mx) mx = v1x;
-        if (v2x < mn) mn = v2x;
-        if (v2x > mx) mx = v2x;
-        sep |= mn > hx || mx < -hx;
-        mn = v0y; mx = v0y;
-        if (v1y < mn) mn = v1y;
-        if (v1y > mx) mx = v1y;
-        if (v2y < mn) mn = v2y;
-        if (v2y > mx) mx = v2y;
-        sep |= mn > hy || mx < -hy;
-    }
-    if (sep) return 0u;
+    const float cz = (hi + lo) / 2.0f, hz = hi - cz;
+    const float v0z = q.az - cz, v1z = q.bz - cz, v2z = q.cz - cz;
+    const float e0z = v1z - v0z, e1z = v2z - v1z, e2z = v0z - v2z;
+    const float f0z = fabsf(e0z), f1z = fabsf(e1z), f2z = fabsf(e2z);
+    Separation<TAME> s;
+    s.axis(e0z * q.v0y - e0y * v0z, e0z * q.v2y - e0y * v2z, f0z * q.hy + f0y * hz);
+    s.axis(-e0z * q.v0x + e0x * v0z, -e0z * q.v2x + e0x * v2z, f0z * q.hx + f0x * hz);
+    s.axis(e1z * q.v0y - e1y * v0z, e1z * q.v2y - e1y * v2z, f1z * q.hy + f1y * hz);
+    s.axis(-e1z * q.v0x + e1x * v0z, -e1z * q.v2x + e1x * v2z, f1z * q.hx + f1x * hz);
+    s.axis(e2z * q.v0y - e2y * v0z, e2z * q.v1y - e2y * v1z, f2z * q.hy + f2y * hz);
+    s.axis(-e2z * q.v0x + e2x * v0z, -e2z * q.v1x + e2x * v1z, f2z * q.hx + f2x * hz);
+    s.face(v0z, v1z, v2z, hz);
+    const float n0 = e0y * e1z - e1y * e0z;
+    const float n1 = e0z * e1x - e1z * e0x;
     const float n2 = e0x * e1y - e1x * e0y;
-    const float xlo = -hx - v0x, xhi = hx - v0x, ylo = -hy - v0y, yhi = hy - v0y;
+    float min0, max0, min1, max1, min2, max2;
+    span<TAME>(n0, -q.hx - q.v0x, q.hx - q.v0x, min0, max0);
+    span<TAME>(n1, -q.hy - q.v0y, q.hy - q.v0y, min1, max1);
+    span<TAME>(n2, -hz - v0z, hz - v0z, min2, max2);
+    s.plane(min0 + min1 + min2, max0 + max1 + max2);
+    return !s.any();
+}
+
+// Narrows the cells z0..z1 of a column to those near the triangle's plane; every other cell fails the SAT's plane test.
+// Along the column the distance of a cell's centre from the plane, times the normal, is f(cz) = f0 + n2 (cz - a2) with
+// f0 = n0 (cx - ax) + n1 (cy - ay), and the plane test separates where |f| exceeds r = |n0| hx + |n1| hy + |n2| hz.  The test's
+// rounding, and this function's, stay below err: with m the triangle's extent plus a cell (no offset v or edge e of
+// the test is larger than a few m) and A the largest coordinate, an edge component is off by a few 2^-24 m, the
+// normal by a few 2^-24 m^2, the distances by a few 2^-24 m^3, and a cell's centre by a few 2^-24 A, which moves f by
+// m^2 times that; err takes 2^-18 of both, and the range a sixteenth of a cell more at each end.
+__device__ __forceinline__ void plane_range(const Column& q, float mnz, float csz, int& z0, int& z1)
+{
+    const float e0x = q.v1x - q.v0x, e1x = q.v2x - q.v1x, e0y = q.v1y - q.v0y, e1y = q.v2y - q.v1y;
+    const float e0z = q.bz - q.az, e1z = q.cz - q.bz;
+    const float n0 = e0y * e1z - e1y * e0z, n1 = e0z * e1x - e1z * e0x, n2 = e0x * e1y - e1x * e0y;
+    const float v0x = q.v0x, v0y = q.v0y, hx = q.hx, hy = q.hy, az = q.az;
+    const float f0 = -(n0 * v0x + n1 * v0y);
+    // |v0x|, |v0y| are at most the extent plus a cell where the column lies in the candidate box
+    const float ex = __builtin_fmaxf(fabsf(e0x), __builtin_fmaxf(fabsf(e1x), fabsf(e0x + e1x)));
+    const float ey = __builtin_fmaxf(fabsf(e0y), __builtin_fmaxf(fabsf(e1y), fabsf(e0y + e1y)));
+    const float ez = __builtin_fmaxf(fabsf(e0z), __builtin_fmaxf(fabsf(e1z), fabsf(e0z + e1z)));
+    const float m = __builtin_fmaxf(ex, __builtin_fmaxf(ey, ez)) + 2.0f * (hx + hy + csz) + __builtin_fmaxf(fabsf(v0x), fabsf(v0y));
+    const float A = __builtin_fmaxf(fabsf(az), fabsf(mnz)) + m;
+    const float err = m * m * (m + A) * 0x1p-18f;
+    const float an2 = fabsf(n2);
+    const float w = fabsf(n0) * hx + fabsf(n1) * hy + an2 * csz * 0.5f + err;
+    // cells with |f0 + n2 ((z + 1/2) csz + mnz - az)| <= w, in cells from az
+    const float inv = __builtin_amdgcn_rcpf(an2 * csz);
+    const float at = (n2 > 0.0f ? -f0 : f0) * inv, half = w * inv + fabsf(at) * 0x1p-18f + 0.0625f;
+    const float base = (az - mnz) * __builtin_amdgcn_rcpf(csz) - 0.5f;
+    const float lo = __builtin_ceilf(base + at - half), hi = __builtin_floorf(base + at + half);
+    // NaN or infinity (a plane along z) leaves the range as it is
+    if (lo > (float)z0) z0 = lo > (float)z1 ? z1 + 1 : (int)lo;
+    if (hi < (float)z1) z1 = hi < (float)z0 ? z0 - 1 : (int)hi;
+}
+
+// z plane k of a grid (the lower face of cell k, the upper of cell k - 1), as cell_box has it
+__device__ inline float z_plane(int k, float mnz, float csz) { return mnz + (float)k * csz; }
+
+// The cells z0..z1 (inside one 32-cell word) of a column: bit (z & 31) is set when cell z passes.
+template <bool TAME>
+__device__ __forceinline__ uint32_t sat_column(const Column& q, int z0, int z1, float mnz, float csz)
+{
+    if (!column_open<TAME>(q)) return 0u;
     uint32_t bits = 0;
+    float lo = z_plane(z0, mnz, csz);
     for (int z = z0; z <= z1; ++z) {
-        float cz, hz;
-        cell_box(z, mnz, csz, &cz, &hz);
-        const float v0z = a[2] - cz, v1z = b[2] - cz, v2z = c[2] - cz;
-        const float e0z = v1z - v0z, e1z = v2z - v1z, e2z = v0z - v2z;
-        const float f0z = fabsf(e0z), f1z = fabsf(e1z), f2z = fabsf(e2z);
-        bool s = axis_sep(e0z * v0y - e0y * v0z, e0z * v2y - e0y * v2z, f0z * hy + f0y * hz);
-        s |= axis_sep(-e0z * v0x + e0x * v0z, -e0z * v2x + e0x * v2z, f0z * hx + f0x * hz);
-        s |= axis_sep(e1z * v0y - e1y * v0z, e1z * v2y - e1y * v2z, f1z * hy + f1y * hz);
-        s |= axis_sep(-e1z * v0x + e1x * v0z, -e1z * v2x + e1x * v2z, f1z * hx + f1x * hz);
-        s |= axis_sep(e2z * v0y - e2y * v0z, e2z * v1y - e2y * v1z, f2z * hy + f2y * hz);
-        s |= axis_sep(-e2z * v0x + e2x * v0z, -e2z * v1x + e2x * v1z, f2z * hx + f2x * hz);
-        float mn = v0z, mx = v0z;
-        if (v1z < mn) mn = v1z;
-        if (v1z > mx) mx = v1z;
-        if (v2z < mn) mn = v2z;
-        if (v2z > mx) mx = v2z;
-        s |= mn > hz || mx < -hz;
-        const float n0 = e0y * e1z - e1y * e0z;
-        const float n1 = e0z * e1x - e1z * e0x;
-        const float vmin0 = n0 > 0.0f ? xlo : xhi, vmax0 = n0 > 0.0f ? xhi : xlo;
-        const float vmin1 = n1 > 0.0f ? ylo : yhi, vmax1 = n1 > 0.0f ? yhi : ylo;
-        const float vmin2 = n2 > 0.0f ? -hz - v0z : hz - v0z, vmax2 = n2 > 0.0f ? hz - v0z : -hz - v0z;
-        const float dmin = n0 * vmin0 + n1 * vmin1 + n2 * vmin2;
-        const float dmax = n0 * vmax0 + n1 * vmax1 + n2 * vmax2;
-        s |= dmin > 0.0f || !(dmax >= 0.0f);
-        bits |= s ? 0u : 1u << (z & 31);
+        const float hi = z_plane(z + 1, mnz, csz);
+        bits |= cell_passes<TAME>(q, lo, hi) ? 1u << (z & 31) : 0u;
+        lo = hi;
     }
     return bits;
 }
@@ -173,9 +270,9 @@ __device__ inline int64_t floordiv64(int64_t a, int64_t b)
 }
 
 // Column (i, j): if its centre is covered by the triangle's xy projection
-// (top-left rule on exact int64 edge functions), toggle the parity bit of the
-// first cell whose centre lies above the crossing.
-__device__ inline void parity_column(const JobDev* J, const TriSetup& S, int i, int jj)
+// (top-left rule on exact int64 edge functions), the parity bit of the
+// first cell whose centre lies above the crossing, to be toggled.
+__device__ inline void parity_column(const JobDev* J, const TriSetup& S, int i, int jj, uint32_t& word, uint32_t& bit)
 {
     const int64_t X0 = S.X[0], X1 = S.X[1], X2 = S.X[2];
     const int64_t Y0 = S.Y[0], Y1 = S.Y[1], Y2 = S.Y[2];
@@ -189,8 +286,8 @@ __device__ inline void parity_column(const JobDev* J, const TriSetup& S, int i, 
     int64_t k = floordiv64(num - (int64_t)(kSub / 2) * S.area, (int64_t)kSub * S.area) + 1;
     if (k < 0) k = 0;
     if (k >= (int64_t)J->nz) return;
-    const size_t word = ((size_t)i * J->ny + (size_t)jj) * J->wp + (size_t)(k >> 5);
-    atomicXor(J->toggle_bits + word, 1u << (k & 31));
+    word = (uint32_t)(((size_t)i * J->ny + (size_t)jj) * J->wp + (size_t)(k >> 5));
+    bit = 1u << (k & 31);
 }
 
 __global__ __launch_bounds__(kVoxThreads) void k_vox_setup(const JobDev* jobs, uint32_t njobs, const uint32_t* tri_prefix,
@@ -224,7 +321,7 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_setup(const JobDev* jobs, u
         uint32_t nshell = 0, ncol = 0;
         const uint32_t t = g - sp[j];
         uint32_t vi[3] = { 0, 0, 0 };
-        bool in_range = true;
+        bool in_range = true, wild = false;
         if (valid && J->active) {
             for (int k = 0; k < 3; ++k) {
                 vi[k] = J->tri[3 * (size_t)t + k];
@@ -242,7 +339,9 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_setup(const JobDev* jobs, u
                     P[k][q] = p[k][q];
                     S.P[k][q] = P[k][q];
                     finite &= __builtin_isfinite(P[k][q]);
+                    wild |= !(fabsf(P[k][q]) < kTameLimit);
                 }
+            for (int q = 0; q < 3; ++q) wild |= !(fabsf(J->mn[q]) < kTameLimit) || !(fabsf(J->mx[q]) < kTameLimit);
             const uint32_t dims[3] = { J->nx, J->ny, J->nz };
             if (finite) {
                 // vertex coordinates in cells; (v - mn) / cs is monotone in v, so the extremes
@@ -307,7 +406,8 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_setup(const JobDev* jobs, u
         // small triangles are tested here; the others go to the pair kernels, the shell as segments of
         // a column (x, y) that lie in one 32-cell word of z
         uint32_t nis = 0, nip = 0;  // this lane's inline shell columns and parity columns
-        if (nshell && nshell <= kInlineShell) {
+        S.job |= wild ? kWildTriangle : 0u;
+        if (nshell && nshell <= kInlineShell && !wild) {
             nis = (uint32_t)(S.hi[0] - S.lo[0] + 1) * (uint32_t)(S.hi[1] - S.lo[1] + 1);
             nshell = 0;
         } else if (nshell) {
@@ -374,8 +474,8 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_setup(const JobDev* jobs, u
             cell_box(x, Jo->mn[0], Jo->cs[0], &cx, &hx);
             cell_box(y, Jo->mn[1], Jo->cs[1], &cy, &hy);
             for (int w = lo2 >> 5; w <= hi2 >> 5; ++w) {
-                const uint32_t bits = sat_column(pa, pb, pc, cx, hx, cy, hy, max(lo2, 32 * w), min(hi2, 32 * w + 31),
-                                                 Jo->mn[2], Jo->cs[2]);
+                const uint32_t bits = sat_column<true>(make_column(pa, pb, pc, cx, hx, cy, hy), max(lo2, 32 * w),
+                                                       min(hi2, 32 * w + 31), Jo->mn[2], Jo->cs[2]);
                 if (bits) atomicOr(Jo->shell_bits + ((size_t)x * Jo->ny + (size_t)y) * Jo->wp + (size_t)w, bits);
             }
         }
@@ -390,7 +490,10 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_setup(const JobDev* jobs, u
             }
             Q.area = (int64_t)(((uint64_t)(uint32_t)sF[wave][kAreaHi][o] << 32) | (uint32_t)sF[wave][kAreaLo][o]);
             const int nj = sF[wave][kEyNj][o] >> 16, ij = sF[wave][kI0J0][o];
-            parity_column(jobs + sF[wave][kJob][o], Q, (ij & 0xFFFF) + (int)c / nj, (ij >> 16) + (int)c % nj);
+            const JobDev* Jo = jobs + sF[wave][kJob][o];
+            uint32_t word = 0, bit = 0;
+            parity_column(Jo, Q, (ij & 0xFFFF) + (int)c / nj, (ij >> 16) + (int)c % nj, word, bit);
+            if (bit) atomicXor(Jo->toggle_bits + word, bit);
         }
         __syncthreads();  // the slots and owner tables are reused by the next 256 triangles
     }
@@ -417,90 +520,215 @@ __device__ inline uint32_t wave_search(const unsigned long long* off, uint32_t n
     return lo + (63u - (uint32_t)__clzll((long long)m));
 }
 
-// Pair kernels: a block takes chunks of kPairChunk consecutive pairs.  Two
-// waves locate the chunk's first and last triangle, the block caches their
-// offsets in LDS and each thread finds its triangle there.
+// A block takes chunks of kPairChunk consecutive pairs.  Two waves locate the chunk's first and last triangle, the
+// block caches their offsets in LDS and each thread finds its triangle there.
 constexpr uint32_t kPairChunk = 4 * kVoxThreads;
 constexpr uint32_t kOffCache = 1024;
 
+// The pairs p0 .. p1 - 1 (at most kPairChunk) of the ntris triangles whose offsets are off: f(g, local, valid) for pair
+// `local` of triangle g, called by whole waves (valid: the lane has a pair).
 template <class F>
-__device__ inline void for_each_pair(const unsigned long long* off, uint32_t ntris, F&& f)
+__device__ inline void pair_chunk(const unsigned long long* off, uint32_t ntris, unsigned long long p0, unsigned long long p1,
+                                  uint32_t* soff, uint32_t* sg, F&& f)
 {
-    __shared__ unsigned long long soff[kOffCache + 1];
-    __shared__ uint32_t sg[2];
-    const unsigned long long start = off[0], total = off[ntris];  // pairs start..total - 1
     const uint32_t wave = threadIdx.x >> 6;
-    for (unsigned long long p0 = start + (unsigned long long)blockIdx.x * kPairChunk; p0 < total;
-         p0 += (unsigned long long)gridDim.x * kPairChunk) {
-        const unsigned long long p1 = min(p0 + kPairChunk, total);
-        if (wave < 2) {
-            const uint32_t g = wave_search(off, ntris + 1, wave == 0 ? p0 : p1 - 1);
-            if ((threadIdx.x & 63u) == 0) sg[wave] = g;
-        }
-        __syncthreads();
-        const uint32_t g0 = sg[0], n = sg[1] - g0 + 1;  // triangles g0 .. g0 + n - 1 hold the chunk
-        const bool cached = n <= kOffCache;
-        if (cached)
-            for (uint32_t i = threadIdx.x; i <= n; i += blockDim.x) soff[i] = off[g0 + i];
-        __syncthreads();
-        // every lane of a wave calls f in each step (valid == false past the chunk),
-        // so f may combine its result across the wave
-        for (unsigned long long base = p0; base < p1; base += blockDim.x) {
-            const unsigned long long p = base + threadIdx.x;
-            const bool valid = p < p1;
-            uint32_t lo = 0, hi = n;  // largest i with off[g0 + i] <= p
-            while (valid && hi - lo > 1) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if ((cached ? soff[mid] : off[g0 + mid]) <= p) lo = mid; else hi = mid;
-            }
-            const uint32_t g = g0 + lo;
-            f(g, valid ? p - (cached ? soff[lo] : off[g]) : 0ull, valid);
-        }
-        __syncthreads();
+    if (wave < 2) {
+        const uint32_t g = wave_search(off, ntris + 1, wave == 0 ? p0 : p1 - 1);
+        if ((threadIdx.x & 63u) == 0) sg[wave] = g;
     }
+    __syncthreads();
+    const uint32_t g0 = sg[0], n = sg[1] - g0 + 1;  // triangles g0 .. g0 + n - 1 hold the chunk
+    const unsigned long long base = off[g0];
+    const bool cached = n <= kOffCache;
+    if (cached)  // from the first triangle's offset on: below it by less than 2^32 pairs of a triangle
+        for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) soff[i] = (uint32_t)(off[g0 + i] - base);
+    __syncthreads();
+    for (unsigned long long pw = p0 + wave * 64u; pw < p1; pw += blockDim.x) {  // wave-uniform
+        const unsigned long long p = min(pw + (threadIdx.x & 63u), p1 - 1);
+        const uint32_t at = (uint32_t)(p - base);
+        uint32_t lo = 0, hi = n;  // largest i with off[g0 + i] <= p
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if ((cached ? soff[mid] : (uint32_t)(off[g0 + mid] - base)) <= at) lo = mid; else hi = mid;
+        }
+        const uint32_t g = g0 + lo;
+        f(g, at - (cached ? soff[lo] : (uint32_t)(off[g] - base)), pw + (threadIdx.x & 63u) < p1);
+    }
+    __syncthreads();
 }
 
-// One thread per column segment of a triangle's candidate box: the cells (x, y, z) with z in one
-// 32-cell word, tested by sat_column and merged into the shell word with one atomicOr.  Held to 64
-// VGPRs (8 waves per SIMD instead of 6, no spills: 1.97 -> 1.94 ms on the mixed batch).
-__global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_vox_shell(const JobDev* jobs, const TriSetup* setup,
+// The words that a wave's lanes are to change, combined in LDS first: neighbouring triangles meet the same words, and
+// each change is an atomic at the memory side, of which the chip executes about 24 a nanosecond.
+struct WordTable {
+    uint32_t key[128], bits[128];  // open addressing; a key is 0xFFFFFFFF and its bits 0 while free
+};
+__device__ inline void wave_lds_fence()
+{
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ inline void clear_table(WordTable& T)
+{
+    for (uint32_t e = threadIdx.x & 63u; e < 128u; e += 64u) {
+        T.key[e] = 0xFFFFFFFFu;
+        T.bits[e] = 0u;
+    }
+    wave_lds_fence();
+}
+// XOR (parity) or OR of bits into words[word], by all lanes of a wave; words: the lane's job's array (bits 0: nothing)
+template <bool XOR>
+__device__ inline void combine_words(WordTable& T, uint32_t* words, uint32_t word, uint32_t bits)
+{
+    auto change = [](uint32_t* p, uint32_t b) {
+        if (XOR) atomicXor(p, b);
+        else atomicOr(p, b);
+    };
+    const uint64_t with = __ballot(bits != 0u);
+    if (with == 0ull) return;
+    // lanes of one job share the table; a wave across two jobs changes its words one by one
+    const uint32_t first = (uint32_t)__builtin_ctzll(with);
+    const uint64_t w0 = (uint64_t)words;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)w0, (int)first),
+                   hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(w0 >> 32), (int)first);
+    uint32_t* const base = (uint32_t*)(((uint64_t)hi << 32) | lo);
+    if (__ballot(bits != 0u && words != base)) {
+        if (bits) change(words + word, bits);
+        return;
+    }
+    bool pending = bits != 0u;
+    uint32_t h = (word * 0x9E3779B1u) >> 25;
+    while (__ballot(pending)) {  // at most 64 distinct words in 128 entries: every lane finds its own or a free one
+        if (pending) {
+            const uint32_t old = atomicCAS(&T.key[h], 0xFFFFFFFFu, word);
+            if (old == 0xFFFFFFFFu || old == word) {
+                if (XOR) atomicXor(&T.bits[h], bits);
+                else atomicOr(&T.bits[h], bits);
+                pending = false;
+            } else {
+                h = (h + 1u) & 127u;
+            }
+        }
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (uint32_t e = threadIdx.x & 63u; e < 128u; e += 64u) {
+        const uint32_t k = T.key[e], b = T.bits[e];
+        if (k != 0xFFFFFFFFu) {
+            if (b) change(base + k, b);
+            T.key[e] = 0xFFFFFFFFu;
+            T.bits[e] = 0u;
+        }
+    }
+    wave_lds_fence();
+}
+
+// A wave's column segments and the cells left of them.
+struct ShellWave {
+    float col[13][64];     // Column, then the grid's first z plane and cell size
+    uint32_t first[64];    // a segment's first cell in the wave's list | its z << 12
+    uint32_t word[64];     // its cells that pass
+    uint8_t owner[64 * 32];  // the segment of every cell of the list
+    WordTable table;
+};
+
+// The pairs left by the setup kernel, shell and parity in one launch (one after the other, each paid a launch of
+// thousands of workgroups and a tail).
+// Shell: one lane per column segment of a triangle's candidate box, the cells (x, y, z) with z in one 32-cell word: the
+// tests that do not depend on z, and the range of z near the triangle's plane.  The cells left, of very uneven
+// number, are listed over the wave and tested one per lane; the words found are combined and then merged by atomicOr.
+// Bound by FP32 instruction issue (81 % of the rate; about 140 of them a cell).  A lane that looped over its own cells
+// ran as long as the wave's longest column and merged every segment's word by itself, 50.3 M atomics on 64 mixed grids
+// instead of 33.7 M: 2.14 -> 1.82 ms there, 181 -> 136 us at 512^3 with a million triangles.
+// Parity: one lane per column of a triangle's column range.
+__global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_vox_pairs(const JobDev* jobs, const TriSetup* setup,
                                                            const unsigned long long* off, uint32_t ntris)
 {
-    for_each_pair(off, ntris, [&](uint32_t g, unsigned long long local, bool valid) {
-        if (!valid) return;
-        const TriSetup Sg = load_setup(setup, ntris, g);
-        const TriSetup* S = &Sg;
-        const JobDev* J = jobs + S->job;
-        const int lo2 = S->lo[2], hi2 = S->hi[2];
-        const uint32_t w0 = (uint32_t)lo2 >> 5, nseg = ((uint32_t)hi2 >> 5) - w0 + 1;
-        const uint32_t ey = (uint32_t)(S->hi[1] - S->lo[1] + 1);
-        uint32_t col = (uint32_t)local, seg = 0;  // < 2^32: columns x segments of one triangle
-        if (nseg > 1) {
-            seg = col % nseg;
-            col /= nseg;
+    __shared__ uint32_t soff[kOffCache];
+    __shared__ uint32_t sg[2];
+    __shared__ ShellWave sw[kVoxThreads / 64];
+    ShellWave& W = sw[threadIdx.x >> 6];
+    const uint32_t lane = threadIdx.x & 63u;
+    clear_table(W.table);
+    // pairs [0, off[ntris]) are the shell's, [off[ntris], off[2 ntris]) the parity's
+    const unsigned long long shell = off[ntris], total = off[2 * (size_t)ntris];
+    const unsigned long long ns = (shell + kPairChunk - 1) / kPairChunk, np = (total - shell + kPairChunk - 1) / kPairChunk;
+    for (unsigned long long c = blockIdx.x; c < ns + np; c += gridDim.x) {
+        if (c < ns) {
+            const unsigned long long p0 = c * kPairChunk;
+            pair_chunk(off, ntris, p0, min(p0 + kPairChunk, shell), soff, sg, [&](uint32_t g, uint32_t col, bool valid) {
+                const TriSetup Sg = load_setup(setup, ntris, g);
+                const TriSetup* S = &Sg;
+                const JobDev* J = jobs + (S->job & ~kWildTriangle);
+                const int lo2 = S->lo[2], hi2 = S->hi[2];
+                const uint32_t w0 = (uint32_t)lo2 >> 5, nseg = ((uint32_t)hi2 >> 5) - w0 + 1;
+                const uint32_t ey = (uint32_t)(S->hi[1] - S->lo[1] + 1);
+                uint32_t seg = 0;
+                if (nseg > 1) {
+                    seg = col % nseg;
+                    col /= nseg;
+                }
+                const int y = S->lo[1] + (int)(col % ey), x = S->lo[0] + (int)(col / ey);
+                const uint32_t w = w0 + seg;
+                const float mnz = J->mn[2], csz = J->cs[2];
+                float cx, hx, cy, hy;
+                cell_box(x, J->mn[0], J->cs[0], &cx, &hx);
+                cell_box(y, J->mn[1], J->cs[1], &cy, &hy);
+                int z0 = max(lo2, (int)(32 * w)), z1 = min(hi2, (int)(32 * w + 31));
+                const Column q = make_column(S->P[0], S->P[1], S->P[2], cx, hx, cy, hy);
+                uint32_t bits = 0, n = 0;
+                if (valid) {
+                    if (S->job & kWildTriangle) {
+                        bits = sat_column<false>(q, z0, z1, mnz, csz);
+                    } else if (column_open<true>(q)) {
+                        plane_range(q, mnz, csz, z0, z1);
+                        n = (uint32_t)max(z1 - z0 + 1, 0);
+                    }
+                }
+                uint32_t inc = n;  // wave inclusive scan
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const uint32_t t = __shfl_up(inc, o, 64);
+                    if (lane >= (uint32_t)o) inc += t;
+                }
+                const uint32_t cells = __shfl(inc, 63, 64), start = inc - n;
+                if (n) {
+                    const float f[13] = { q.v0x, q.v1x, q.v2x, q.v0y, q.v1y, q.v2y, q.hx, q.hy, q.az, q.bz, q.cz, mnz, csz };
+#pragma unroll
+                    for (int k = 0; k < 13; ++k) W.col[k][lane] = f[k];
+                    W.first[lane] = start | (uint32_t)z0 << 12;
+                    W.word[lane] = 0u;
+                    for (uint32_t k = 0; k < n; ++k) W.owner[start + k] = (uint8_t)lane;
+                }
+                wave_lds_fence();
+                for (uint32_t i0 = 0; i0 < cells; i0 += 64u) {
+                    const uint32_t i = i0 + lane;
+                    if (i < cells) {
+                        const uint32_t o = W.owner[i], first = W.first[o];
+                        const int z = (int)(first >> 12) + (int)(i - (first & 0xFFFu));
+                        const Column r{ W.col[0][o], W.col[1][o], W.col[2][o], W.col[3][o], W.col[4][o], W.col[5][o],
+                                        W.col[6][o], W.col[7][o], W.col[8][o], W.col[9][o], W.col[10][o] };
+                        const float rmn = W.col[11][o], rcs = W.col[12][o];
+                        if (cell_passes<true>(r, z_plane(z, rmn, rcs), z_plane(z + 1, rmn, rcs)))
+                            atomicOr(&W.word[o], 1u << (z & 31));
+                    }
+                }
+                wave_lds_fence();
+                if (n) bits = W.word[lane];
+                combine_words<false>(W.table, J->shell_bits, (uint32_t)(((size_t)x * J->ny + (size_t)y) * J->wp + w), bits);
+            });
+        } else {
+            const unsigned long long p0 = shell + (c - ns) * kPairChunk;
+            pair_chunk(off + ntris, ntris, p0, min(p0 + kPairChunk, total), soff, sg, [&](uint32_t g, uint32_t local, bool valid) {
+                const TriSetup Sg = load_setup(setup, ntris, g);
+                const uint32_t nj = (uint32_t)(Sg.j1 - Sg.j0 + 1);
+                const JobDev* J = jobs + (Sg.job & ~kWildTriangle);
+                uint32_t word = 0, bit = 0;
+                if (valid) parity_column(J, Sg, Sg.i0 + (int)(local / nj), Sg.j0 + (int)(local % nj), word, bit);
+                combine_words<true>(W.table, J->toggle_bits, word, bit);
+            });
         }
-        const int y = S->lo[1] + (int)(col % ey), x = S->lo[0] + (int)(col / ey);
-        const uint32_t w = w0 + seg;
-        float cx, hx, cy, hy;
-        cell_box(x, J->mn[0], J->cs[0], &cx, &hx);
-        cell_box(y, J->mn[1], J->cs[1], &cy, &hy);
-        const uint32_t bits = sat_column(S->P[0], S->P[1], S->P[2], cx, hx, cy, hy, max(lo2, (int)(32 * w)),
-                                         min(hi2, (int)(32 * w + 31)), J->mn[2], J->cs[2]);
-        if (bits) atomicOr(J->shell_bits + ((size_t)x * J->ny + (size_t)y) * J->wp + w, bits);
-    });
-}
-
-__global__ __launch_bounds__(kVoxThreads) void k_vox_parity(const JobDev* jobs, const TriSetup* setup,
-                                                            const unsigned long long* off, uint32_t ntris)
-{
-    for_each_pair(off, ntris, [&](uint32_t g, unsigned long long local, bool valid) {
-        if (!valid) return;
-        const TriSetup Sg = load_setup(setup, ntris, g);
-        const TriSetup* S = &Sg;
-        const JobDev* J = jobs + S->job;
-        const uint32_t nj = (uint32_t)(S->j1 - S->j0 + 1);
-        parity_column(J, *S, S->i0 + (int)(local / nj), S->j0 + (int)(local % nj));
-    });
+    }
 }
 
 // Occupancy bits = shell | parity interior, left in place of the shell bits.  Bound by HBM: 8 bytes read and 4
@@ -612,18 +840,13 @@ void launch_voxelize(const Launch& L, const VoxScratch& X, const uint32_t* col_p
         }
         // one scan over both count arrays (contiguous): the parity offsets continue from the shell total
         scan_exclusive_u32_to_u64(cnt_shell, X.shell_off, 2ull * X.total_tris, X.scan_tmp, L.s);
-        const unsigned long long* col_off = X.shell_off + X.total_tris;
-        {
-            TimedLaunch tl("vox_shell", L.s);
-            k_vox_shell<<<active_shape().pair_blocks, kVoxThreads, 0, L.s>>>(L.jobs, X.setup, X.shell_off, X.total_tris);
-            VF_CHECK_LAUNCH();
-        }
-        {
-            TimedLaunch tl("vox_parity", L.s);
-            k_vox_parity<<<std::max(64u, active_shape().pair_blocks / 2), kVoxThreads, 0, L.s>>>(L.jobs, X.setup, col_off,
-                                                                                                X.total_tris);
-            VF_CHECK_LAUNCH();
-        }
+        // workgroups for as many pairs as a mesh of this size commonly leaves (a few surfaces across every column, a few
+        // columns per triangle); more pairs take more steps
+        const uint32_t likely = ceil_div((uint64_t)total_groups * 256u * 4u + 8ull * X.total_tris, kPairChunk);
+        TimedLaunch tl("vox_pairs", L.s);
+        k_vox_pairs<<<std::min(active_shape().pair_blocks, std::max(256u, likely)), kVoxThreads, 0, L.s>>>(L.jobs, X.setup,
+                                                                                                        X.shell_off, X.total_tris);
+        VF_CHECK_LAUNCH();
     }
     TimedLaunch tl("vox_fill", L.s);
     const uint32_t blocks = std::max(1u, std::min(total_groups, active_shape().cell_blocks));
