@@ -4,7 +4,9 @@
 // support), launches the multi-job kernels with a one-job table, and reports
 // failures through vf_last_error().
 #include <algorithm>
+#include <atomic>
 #include <cfloat>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -73,8 +75,9 @@ static void grid_setup_shape(vf_grid* g, const uint32_t dims[3], const float mn[
     g->labels.ensure(g->V * 2 + 64);
     const uint64_t words = occ_words(dims);
     g->occ.ensure(words * 4 + 64);
-    VF_HIP(hipMemsetAsync(g->occ.p, 0, words * 4, g->stream));
-    g->labels_from_occ = true;  // every cell EMPTY, written when something reads the cells
+    // every cell EMPTY: written when something reads the cells or their occupancy
+    g->occ_unset = true;
+    g->labels_from_occ = true;
     g->clean = true;
     g->mc.valid = false;
     JobDev& J = g->job;
@@ -96,29 +99,36 @@ static void grid_setup_shape(vf_grid* g, const uint32_t dims[3], const float mn[
     J.hist = g->hist.as<uint32_t>();
     J.active = 1;
     g->job_dirty = true;
-    const uint32_t pre[6] = { 0, grid_tiles(g), 0, brick_count(dims[0], dims[1], dims[2]), 0, word_tiles(dims) };
-    VF_HIP(hipMemcpyAsync(g->prefix.p, pre, sizeof pre, hipMemcpyHostToDevice, g->stream));
-    VF_HIP(hipStreamSynchronize(g->stream));
+    g->words[kHeadTiles + 1] = grid_tiles(g);
+    g->words[kHeadBricks + 1] = brick_count(dims[0], dims[1], dims[2]);
+    g->words[kHeadWordTiles + 1] = word_tiles(dims);
+    g->words[kHeadTasks + 1] = relax_tasks(dims[0], dims[1], dims[2]);
 }
 
 Launch grid_launch(vf_grid* g)
 {
     if (g->job_dirty) {
-        std::memcpy(g->pinned + 256, &g->job, sizeof(JobDev));
-        VF_HIP(hipMemcpyAsync(g->jobdev.p, g->pinned + 256, sizeof(JobDev), hipMemcpyHostToDevice, g->stream));
-        VF_HIP(hipStreamSynchronize(g->stream));
+        GridHead h;
+        h.job = g->job;
+        std::memcpy(h.words, g->words, sizeof h.words);
+        launch_put_head(g->head.as<GridHead>(), h, g->stream);
         g->job_dirty = false;
+    }
+    if (g->occ_unset) {
+        VF_HIP(hipMemsetAsync(g->occ.p, 0, occ_words(g->dims) * 4, g->stream));
+        g->occ_unset = false;
     }
     set_active_bucket(tune_bucket(std::max(g->dims[0], std::max(g->dims[1], g->dims[2]))));
     Launch L;
-    L.jobs = g->jobdev.as<JobDev>();
+    const uint32_t* pre = g->head.as<GridHead>()->words;
+    L.jobs = &g->head.as<GridHead>()->job;
     L.njobs = 1;
-    L.tile_prefix = g->prefix.as<uint32_t>();
-    L.total_tiles = grid_tiles(g);
-    L.wtile_prefix = g->prefix.as<uint32_t>() + 4;
-    L.total_wtiles = word_tiles(g->dims);
-    L.bt_prefix = g->prefix.as<uint32_t>() + 2;
-    L.total_bricks = brick_count(g->dims[0], g->dims[1], g->dims[2]);
+    L.tile_prefix = pre + kHeadTiles;
+    L.total_tiles = g->words[kHeadTiles + 1];
+    L.wtile_prefix = pre + kHeadWordTiles;
+    L.total_wtiles = g->words[kHeadWordTiles + 1];
+    L.bt_prefix = pre + kHeadBricks;
+    L.total_bricks = g->words[kHeadBricks + 1];
     L.s = g->stream;
     return L;
 }
@@ -130,18 +140,21 @@ void grid_materialize(vf_grid* g)
     g->labels_from_occ = false;
 }
 
-uint64_t read_stat(vf_grid* g, int slot)
+void grid_report(vf_grid* g, uint32_t S)
 {
-    VF_HIP(hipMemcpyAsync(g->pinned, g->stats.as<unsigned long long>() + slot, 8, hipMemcpyDeviceToHost, g->stream));
+    launch_report(g->stats.as<unsigned long long>(), g->seeds.as<uint4>(), S, g->pinned, g->stream);
     VF_HIP(hipStreamSynchronize(g->stream));
+}
+
+uint64_t reported_stat(const vf_grid* g, int slot)
+{
     uint64_t v;
-    std::memcpy(&v, g->pinned, 8);
+    std::memcpy(&v, g->pinned + kPinStats + 2 * slot, 8);
     return v;
 }
 
-void check_device_error(vf_grid* g, const char* stage)
+void check_device_error(vf_grid* g, const char* stage, uint64_t e)
 {
-    uint64_t e = read_stat(g, kStatError);
     if (!e) return;
     VF_HIP(hipMemsetAsync(g->stats.as<unsigned long long>() + kStatError, 0, 8, g->stream));
     if (e & kDevErrSeeding) fail(VF_ERR_SEEDING, "%s: fewer candidate cells than seeds", stage);
@@ -163,14 +176,14 @@ static void validate_seeds(const vf_grid* g, const vf_seed* seeds, uint32_t S)
 static void upload_seeds(vf_grid* g, const vf_seed* seeds, uint32_t S)
 {
     g->seeds.ensure((size_t)std::max<uint32_t>(S, 1) * sizeof(uint4));
-    if (S) VF_HIP(hipMemcpyAsync(g->seeds.p, seeds, (size_t)S * sizeof(uint4), hipMemcpyHostToDevice, g->stream));
-    if (g->job.seeds != g->seeds.as<uint4>() || g->job.S != S) {
+    if (S <= kMaxDeviceSeeds) launch_put_seeds(g->seeds.as<uint4>(), seeds, S, g->stream);
+    else VF_HIP(hipMemcpyAsync(g->seeds.p, seeds, (size_t)S * sizeof(uint4), hipMemcpyHostToDevice, g->stream));
+    if (g->job.seeds != g->seeds.as<uint4>() || g->job.S != S || g->job.S_draw != S) {
         g->job.seeds = g->seeds.as<uint4>();
-        g->job.S = S;
+        g->job.S = g->job.S_draw = S;
         g->job_dirty = true;
     }
-    g->job.S_draw = S;
-    VF_HIP(hipStreamSynchronize(g->stream));
+    if (S > kMaxDeviceSeeds) VF_HIP(hipStreamSynchronize(g->stream));  // the caller's list may go
 }
 
 static vf_grid* checked(vf_grid* g)
@@ -202,12 +215,10 @@ int vf_grid_create(const uint32_t dims[3], const float aabb_min[3], const float 
         try {
             VF_HIP(hipGetDevice(&g->device));
             VF_HIP(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
-            VF_HIP(hipHostMalloc(reinterpret_cast<void**>(&g->pinned), 4096));
-            g->jobdev.ensure(sizeof(JobDev));
-            g->prefix.ensure(64);
+            VF_HIP(hipHostMalloc(reinterpret_cast<void**>(&g->pinned), kPinWords * 4, hipHostMallocMapped | hipHostMallocCoherent));
+            g->head.ensure(sizeof(GridHead));
             g->stats.ensure(kStatCount * 8);
-            g->hist.ensure(65536 * 4);
-            g->ctl.ensure(256);
+            g->hist.ensure(65536 * 4 + kHistPartBytes);
             VF_HIP(hipMemsetAsync(g->stats.p, 0, kStatCount * 8, g->stream));
             grid_setup_shape(g, dims, aabb_min, aabb_max);
         } catch (...) {
@@ -292,7 +303,8 @@ int vf_grid_count_occupied(vf_grid* g, uint64_t* out)
         if (!out) fail(VF_ERR_INVALID_ARG, "out is NULL");
         VF_HIP(hipMemsetAsync(g->stats.as<unsigned long long>() + kStatOccupied, 0, 8, g->stream));
         launch_count_occupied(grid_launch(g));
-        *out = read_stat(g, kStatOccupied);
+        grid_report(g);
+        *out = reported_stat(g, kStatOccupied);
     });
 }
 
@@ -338,25 +350,26 @@ int vf_voxelize_device(vf_grid* g, const float* d_xyz, uint32_t nv, const uint32
         }
         g->job_dirty = true;
         const uint32_t groups = ceil_div(words, 256);
-        uint32_t pre[4] = { 0, nt, 0, groups };
         g->vox_setup.ensure((size_t)std::max<uint32_t>(nt, 1) * sizeof(TriSetup));
         g->vox_counts.ensure((size_t)std::max<uint32_t>(nt, 1) * 8);
         g->vox_shell_off.ensure((2 * (size_t)nt + 1) * 8);
         g->scan_tmp.ensure(scan_tmp_bytes(2 * (uint64_t)nt) + 64);
-        g->ctl.ensure(256);
-        std::memcpy(g->pinned + 512, pre, sizeof pre);
-        VF_HIP(hipMemcpyAsync(g->ctl.p, g->pinned + 512, sizeof pre, hipMemcpyHostToDevice, g->stream));
+        g->words[kHeadTris + 1] = nt;
+        g->words[kHeadGroups + 1] = groups;
+        if (!merge) g->occ_unset = false;  // written whole below
         Launch L = grid_launch(g);
+        const uint32_t* pre = g->head.as<GridHead>()->words;
         VoxScratch X;
         X.setup = g->vox_setup.as<TriSetup>();
         X.counts = g->vox_counts.as<uint32_t>();
         X.shell_off = g->vox_shell_off.as<unsigned long long>();
-        X.tri_prefix = g->ctl.as<uint32_t>();
+        X.tri_prefix = pre + kHeadTris;
         X.total_tris = nt;
         X.scan_tmp = g->scan_tmp.p;
         X.scan_tmp_bytes = g->scan_tmp.bytes;
-        launch_voxelize(L, X, g->ctl.as<uint32_t>() + 2, groups, nullptr);
-        check_device_error(g, "voxelize");
+        launch_voxelize(L, X, pre + kHeadGroups, groups, nullptr);
+        grid_report(g);
+        check_device_error(g, "voxelize", reported_stat(g, kStatError));
         if (merge) {
             // labels = new ? FREE : old, occupancy as the labels then say
             grid_materialize(g);
@@ -364,12 +377,12 @@ int vf_voxelize_device(vf_grid* g, const float* d_xyz, uint32_t nv, const uint32
             launch_occ_free(M, J.shell_bits);
             launch_labels_to_occ(M);
             g->labels_from_occ = false;
+            VF_HIP(hipStreamSynchronize(g->stream));
         } else {
             g->labels_from_occ = true;
         }
         g->clean = false;
         g->mc.valid = false;
-        VF_HIP(hipStreamSynchronize(g->stream));
     });
 }
 
@@ -378,8 +391,11 @@ int vf_voxelize(vf_grid* g, const float* xyz, uint32_t nv, const uint32_t* tri, 
     return guard([&] {
         checked(g);
         if (nt && (!xyz || !tri)) fail(VF_ERR_INVALID_ARG, "mesh pointer is NULL");
-        for (uint64_t i = 0; i < 3ull * nt; ++i)
-            if (tri[i] >= nv) fail(VF_ERR_INVALID_ARG, "triangle %llu references vertex %u of %u", (unsigned long long)(i / 3), tri[i], nv);
+        uint32_t top = 0;  // one vectorised pass; a search only on failure
+        for (uint64_t i = 0; i < 3ull * nt; ++i) top = std::max(top, tri[i]);
+        if (nt && top >= nv)
+            for (uint64_t i = 0; i < 3ull * nt; ++i)
+                if (tri[i] >= nv) fail(VF_ERR_INVALID_ARG, "triangle %llu references vertex %u of %u", (unsigned long long)(i / 3), tri[i], nv);
         g->mesh_xyz.ensure((size_t)std::max<uint32_t>(nv, 1) * 12);
         g->mesh_tri.ensure((size_t)std::max<uint32_t>(nt, 1) * 12);
         if (nv) VF_HIP(hipMemcpyAsync(g->mesh_xyz.p, xyz, (size_t)nv * 12, hipMemcpyHostToDevice, g->stream));
@@ -414,9 +430,9 @@ int vf_seed_uniform(vf_grid* g, uint32_t S, uint64_t seed, int location, vf_seed
         scan_exclusive_u32_to_u64(g->seed_tile_cnt.as<uint32_t>(), g->seed_tile_off.as<unsigned long long>(), tiles,
                                   g->scan_tmp.p, g->stream);
         launch_seed_pick(L, g->seed_tile_off.as<unsigned long long>());
-        check_device_error(g, "seed_uniform");
-        VF_HIP(hipMemcpyAsync(out, g->seeds.p, (size_t)S * sizeof(uint4), hipMemcpyDeviceToHost, g->stream));
-        VF_HIP(hipStreamSynchronize(g->stream));
+        grid_report(g, S);
+        check_device_error(g, "seed_uniform", reported_stat(g, kStatError));
+        std::memcpy(out, g->pinned + kPinSeeds, (size_t)S * sizeof(uint4));
     });
 }
 
@@ -553,7 +569,9 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
         if (S > kMaxDeviceSeeds) fail(VF_ERR_TOO_MANY_SEEDS, "%u flood seeds (max %u)", S, kMaxDeviceSeeds);
         // the sub-seed pass matters only when some fragment's live seeds carry different ids
         bool sub = false;
-        {
+        bool one_id = true;
+        for (uint32_t s = 1; s < S; ++s) one_id &= seeds[s].w >> 8 == seeds[0].w >> 8;
+        if (!one_id) {
             std::map<uint64_t, uint32_t> last;  // cell -> last seed on it
             for (uint32_t s = 0; s < S; ++s)
                 last[((uint64_t)seeds[s].x * g->dims[1] + seeds[s].y) * g->dims[2] + seeds[s].z] = s;
@@ -580,45 +598,61 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
         J.algo = VF_FLOOD;
         g->job_dirty = true;
         Launch L = grid_launch(g);
-        // fctl words 32..33: task prefix of the one job; 48..63: worklist counters (two list sets)
-        const uint32_t tasks = relax_tasks(g->dims[0], g->dims[1], g->dims[2]);
+        // fctl words 48..63: worklist counters (two list sets)
+        const uint32_t tasks = g->words[kHeadTasks + 1];
         FloodRoundScratch W{};
-        W.task_prefix = g->fctl.as<uint32_t>() + 32;
+        W.task_prefix = g->head.as<GridHead>()->words + kHeadTasks;
         W.total_tasks = tasks;
         W.list_cap = flood_list_cap(tasks);
         g->flood_lists.ensure(2ull * kFloodXcds * W.list_cap * 8);
         W.lists = g->flood_lists.as<unsigned long long>();
         W.counts = g->fctl.as<uint32_t>() + 48;
-        std::memset(g->pinned, 0, 128);
-        g->pinned[1] = tasks;
-        VF_HIP(hipMemcpyAsync(g->fctl.as<uint32_t>() + 32, g->pinned, 128, hipMemcpyHostToDevice, g->stream));
-        VF_HIP(hipMemsetAsync(J.bflags, 0, 2ull * relax_parity_bytes(nbricks), g->stream));  // both flag parities
-        VF_HIP(hipStreamSynchronize(g->stream));  // the pinned words are reused below
+        launch_clear_labels(L);
         launch_flood_init(L, W);
         launch_flood_seed(L, W);
-        auto drain = [&]() {
-            uint32_t chunk = 4, rounds = 0;
-            for (;;) {
-                launch_flood_rounds(L, W, chunk, active_shape().flood_blocks);
-                rounds += chunk;
-                VF_HIP(hipMemcpyAsync(g->pinned, g->fctl.p, 8, hipMemcpyDeviceToHost, g->stream));
-                VF_HIP(hipStreamSynchronize(g->stream));
-                if (g->pinned[1] != 0) return g->pinned[1];
-                chunk = std::min<uint32_t>(chunk * 2, 32);
-                // every round lowers a cell's key at least one step along a shortest path, so the
-                // worklist drains within (cells + 1) rounds
-                if ((uint64_t)rounds > g->V + S + 16) fail(VF_ERR_OVERFLOW, "flood did not drain");
+        // Rounds are queued kAhead ahead of the one running, whose number the device stores to pinned memory, so the
+        // device never waits for the host between rounds; those queued past the drain find nothing to do.  (In chunks
+        // of 4, 8, 16 ... rounds with a wait after each, a flood of 22 rounds ran 28 and waited three times.)
+        constexpr uint32_t kAhead = 6;
+        volatile uint32_t* pr = g->pinned + kPinProgress;
+        W.progress = g->pinned + kPinProgress;
+        auto drain = [&]() -> uint32_t {
+            pr[0] = pr[1] = pr[2] = 0;
+            std::atomic_thread_fence(std::memory_order_seq_cst);
+            // every round lowers a cell's key at least one step along a shortest path, so the
+            // worklist drains within (cells + 1) rounds
+            const uint64_t limit = g->V + S + 16;
+            uint64_t queued = 0;
+            uint32_t seen = 0;
+            auto moved = std::chrono::steady_clock::now();
+            while (pr[1] == 0) {
+                const uint32_t at = pr[0];
+                if (queued < (uint64_t)at + kAhead) {
+                    if (queued > limit) fail(VF_ERR_OVERFLOW, "flood did not drain");
+                    launch_flood_rounds(L, W, 2, active_shape().flood_blocks);
+                    queued += 2;
+                    seen = at;
+                    moved = std::chrono::steady_clock::now();
+                } else if (at != seen) {
+                    seen = at;
+                    moved = std::chrono::steady_clock::now();
+                } else if (std::chrono::steady_clock::now() - moved > std::chrono::milliseconds(20)) {
+                    // a long round, or no word will come: wait for what is queued, then there is progress or an error
+                    VF_HIP(hipStreamSynchronize(g->stream));
+                    if (pr[1] == 0 && pr[0] == at) fail(VF_ERR_DEVICE, "flood rounds stopped");
+                }
             }
+            check_device_error(g, "flood", pr[2]);
+            return pr[1];
         };
         g->last_flood_levels = drain();
         if (sub) {
             launch_flood_sub(L);
-            VF_HIP(hipMemcpyAsync(g->pinned, g->fctl.p, 8, hipMemcpyDeviceToHost, g->stream));
+            uint32_t ctl[2];
+            VF_HIP(hipMemcpyAsync(ctl, g->fctl.p, 8, hipMemcpyDeviceToHost, g->stream));
             VF_HIP(hipStreamSynchronize(g->stream));
-            if (g->pinned[1] == 0) g->last_flood_levels += drain();  // regions were freed: second growth
+            if (ctl[1] == 0) g->last_flood_levels += drain();  // regions were freed: second growth
         }
-        check_device_error(g, "flood");
-        launch_clear_labels(L);
         launch_flood_finish(L);
         g->labels_from_occ = false;
         g->mc.valid = false;
@@ -638,7 +672,7 @@ int vf_detect_boundaries(vf_grid* g, int size)
         }
         Launch L = grid_launch(g);
         if (size <= 1) launch_boundaries_tiled(L, false, false);
-        else launch_boundaries(L, size, 0);
+        else launch_boundaries(L, size);
         g->mc.valid = false;
         VF_HIP(hipStreamSynchronize(g->stream));
     });
@@ -722,12 +756,16 @@ int vf_histogram(vf_grid* g, uint32_t* counts, uint32_t ncounts)
         if (ncounts && !counts) fail(VF_ERR_INVALID_ARG, "counts is NULL");
         grid_materialize(g);
         Launch L = grid_launch(g);
-        launch_clear_hist(L);
-        launch_histogram(L);
-        const uint32_t n = std::min<uint32_t>(ncounts, 65536);
-        if (n) VF_HIP(hipMemcpyAsync(counts, g->hist.p, (size_t)n * 4, hipMemcpyDeviceToHost, g->stream));
+        launch_histogram(L, g->hist.as<uint32_t>(), g->hist.as<uint32_t>() + 65536, g->pinned + kPinHist);
+        // most grids have labels below kHistBins only: the other counts are cleared while the device counts
+        const uint32_t n = std::min<uint32_t>(ncounts, 65536), head = std::min(n, kHistBins);
+        if (ncounts > head) std::memset(counts + head, 0, (size_t)(ncounts - head) * 4);
         VF_HIP(hipStreamSynchronize(g->stream));
-        for (uint32_t i = n; i < ncounts; ++i) counts[i] = 0;
+        std::memcpy(counts, g->pinned + kPinHist, (size_t)head * 4);
+        if (n > head && g->pinned[kPinHist + kHistBins]) {
+            VF_HIP(hipMemcpyAsync(counts, g->hist.p, (size_t)n * 4, hipMemcpyDeviceToHost, g->stream));
+            VF_HIP(hipStreamSynchronize(g->stream));
+        }
     });
 }
 

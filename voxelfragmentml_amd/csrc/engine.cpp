@@ -84,12 +84,12 @@ size_t job_footprint(const vf_job& j)
     // work counts and their 64-bit scans, the seed-candidate counts per tile and their scan (each buffer
     // at least 256 bytes plus 64 bytes of slack), the launch table's descriptor and prefix entries (with
     // the alignment of its nine arrays), and the flood worklists (2 sets x 8 XCD lists of
-    // ceil(tasks / 8) x 4096 eight-byte entries: 64 KiB per task, plus one rounding step)
+    // ceil(tasks / 8) x 4096 + 64 per task eight-byte entries: 72 KiB per task, plus one rounding step)
     const size_t front = (size_t)j.nt * (sizeof(TriSetup) + 8 + 16) + scan_tmp_bytes(2ull * j.nt) +
                          (size_t)tiles * 12 + scan_tmp_bytes(tiles) + 6 * (256 + 64);
     const size_t table = 3 * sizeof(JobDev) + 16 * 4 + 11 * 4 + 10 * kAlign;
     const size_t lists = j.algorithm == VF_FLOOD
-                             ? 65536ull * relax_tasks(j.dims[0], j.dims[1], j.dims[2]) + 2ull * kFloodXcds * 4096 * 8
+                             ? 73728ull * relax_tasks(j.dims[0], j.dims[1], j.dims[2]) + 2ull * kFloodXcds * 4096 * 8
                              : 0;
     // blocks come from the engine's size classes: at most an eighth more than asked, and 256 bytes at least
     const size_t shared = front + table + lists;
@@ -533,8 +533,7 @@ void Engine::post(Table& t)
 }
 
 // RegularGrid::erode (RegularGrid.cpp:82-159) for each job that asks for it, in place of boundary detection:
-// iterations x (detectBoundaries(1), one erosion step), then the isolated-cell pass; its histogram is
-// cleared afterwards (the boundary passes count into it) and recounted by the post stage.  Launch-only.
+// iterations x (detectBoundaries(1), one erosion step), then the isolated-cell pass.  Launch-only.
 void Engine::erode(Table& t)
 {
     for (uint32_t i = 0; i < t.L.njobs; ++i) {
@@ -555,7 +554,6 @@ void Engine::erode(Table& t)
         }
         launch_isolated_cells(one, e.erode_out, e.d.V);
         VF_HIP(hipMemcpyAsync(e.d.labels, e.erode_out, e.d.V * 2, hipMemcpyDeviceToDevice, s));
-        launch_clear_hist(one);
     }
 }
 

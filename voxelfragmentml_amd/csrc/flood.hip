@@ -82,6 +82,7 @@ constexpr uint32_t kRelaxLdsWords = kTileWords + kZtWords;
 constexpr uint32_t kRelaxRun = 3;
 // A worklist entry: job << 32 | parity of its round << 31 | brick (a grid has fewer than 2^31 cells, 2^22 bricks).
 constexpr uint32_t kEntryParity = 1u << 31;
+constexpr uint32_t kSplitTasks = 64;               // tables of fewer compaction tasks cut each job's bricks into a share per XCD
 constexpr uint32_t kMaxSweeps = 2048;              // a brick of 512 cells is stable after at most 513 sweeps
 constexpr uint32_t kXcds = kFloodXcds;             // XCDs of the device; workgroups are dealt round-robin
 
@@ -110,15 +111,21 @@ __device__ inline T* uni_ptr(T* p)
 // One block per job: stamp the seeds (a later seed on the same cell wins, as
 // FloodFracturer.cpp:99-105 writes them in list order), mark seed cells
 // occupied and flag, for round 1, every brick that holds a seed cell or one of
-// its neighbours.  Both flag arrays were zeroed by an earlier launch.  A seed
+// its neighbours.  Both flag arrays were zeroed by the key init.  A seed
 // on an EMPTY cell can sit in a brick the key init left without keys: such a
 // brick gets EMPTY keys and its liveness bit first.
-__global__ __launch_bounds__(256) void k_flood_seed(Launch L)
+__global__ __launch_bounds__(256) void k_flood_seed(Launch L, uint32_t* counts)
 {
     __shared__ uint32_t todo[256];
     __shared__ uint32_t ntodo;
     const JobDev* J = L.jobs + blockIdx.x;
+    if (blockIdx.x == 0 && threadIdx.x < 2u * kXcds) counts[threadIdx.x] = 0u;
     if (!J->active || J->algo != VF_FLOOD) return;
+    // both parities' flags: the init cleared the bricks', the rest of the last group here
+    for (uint32_t i = threadIdx.x; i < 2u * (relax_parity_bytes(J->nbricks) - J->nbricks); i += blockDim.x) {
+        const uint32_t pad = (uint32_t)relax_parity_bytes(J->nbricks) - J->nbricks;
+        parity_flags(J->bflags, J->nbricks, i / pad)[J->nbricks + i % pad] = 0u;
+    }
     const uint32_t S = J->S, b = J->key_bits;
     const uint32_t nby = bdim(J->ny), nbz = bdim(J->nz);
     unsigned long long* live = live_base(J->bflags, J->nbricks);
@@ -596,7 +603,8 @@ __device__ inline uint32_t flood_job_active(const JobDev* J)
 // values from words no workgroup writes in this launch, and writes them: no ordering is needed.
 // The loads come in two dependent batches: the job's fields, then its control words together with
 // both parities' flag group w (lane w of the task), of which *m receives the new round's bits.
-__device__ inline bool start_round(const Launch& L, uint32_t j, uint32_t i, uint32_t w, RelaxJob& R, uint64_t& m)
+// progress (or null): host words told of it (FloodRoundScratch::progress).
+__device__ inline bool start_round(const Launch& L, uint32_t j, uint32_t i, uint32_t w, RelaxJob& R, uint64_t& m, uint32_t* progress)
 {
     const JobDev* J = L.jobs + j;
     const uint32_t act = flood_job_active(J);
@@ -606,18 +614,28 @@ __device__ inline bool start_round(const Launch& L, uint32_t j, uint32_t i, uint
     const uint32_t done = uni(ctl[1]), s0 = uni(ctl[4]), s1 = uni(ctl[5]), f0 = uni(ctl[2]), f1 = uni(ctl[3]);
     const uint32_t ng = relax_groups(R.nb), wc = min(w, ng - 1u);
     const FlagGroup g0 = load_group(parity_flags(R.flags, R.nb, 0u), wc), g1 = load_group(parity_flags(R.flags, R.nb, 1u), wc);
-    if (done) return false;
-    const uint32_t rp = ((i + 1u) & 1u) ? s1 : s0;
     const bool lead = threadIdx.x == 0;
+    auto tell_done = [&](uint32_t rounds) {
+        if (!lead || !progress || blockIdx.x != 0) return;
+        __hip_atomic_store(progress + 2, (uint32_t)J->stats[kStatError], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(progress + 1, rounds, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    };
+    if (done) {  // drained by an earlier round, or just now by another workgroup of this launch
+        tell_done(done);
+        return false;
+    }
+    const uint32_t rp = ((i + 1u) & 1u) ? s1 : s0;
     if ((((rp + 1u) & 1u) ? f1 : f0) == 0u) {
         if (lead) {
             ctl[1] = rp;
             J->stats[kStatFloodDone] = rp;
         }
+        tell_done(rp);
         return false;
     }
     const uint32_t r = rp + 1u;
     if (lead) {
+        if (progress && blockIdx.x == 0) __hip_atomic_store(progress, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         ctl[4 + (i & 1u)] = r;
         ctl[0] = r;
         ctl[2 + (rp & 1u)] = 0u;
@@ -631,7 +649,7 @@ __device__ inline bool start_round(const Launch& L, uint32_t j, uint32_t i, uint
 // turn its flags into worklists.
 // A task is 64 flag groups (4096 bricks, one group per lane) of one job; each
 // lane clears its group and appends its flagged bricks (with the job and the round's parity)
-// to the worklist of the task's XCD, with one list reservation per wave.
+// to the worklist of the task's XCD (or of its share of the job's groups), with one list reservation per wave and list.
 // Tasks are dealt to the XCDs round-robin like workgroups, so the relax step,
 // which serves list x from the workgroups of XCD x, finds the halos of
 // neighbouring bricks (mostly in the same task) in the same L2.
@@ -641,7 +659,7 @@ __device__ inline bool start_round(const Launch& L, uint32_t j, uint32_t i, uint
 // i: the round's index in its chunk.
 __global__ __launch_bounds__(64) void k_flood_compact(Launch L, const uint32_t* prefix, uint32_t total_tasks,
                                                       unsigned long long* lists, uint32_t list_cap, uint32_t* counts,
-                                                      uint32_t* stale, uint32_t i)
+                                                      uint32_t* stale, uint32_t i, uint32_t* progress)
 {
     __shared__ uint32_t sp[kFloodMaxJobs + 1];
     const uint32_t lane = threadIdx.x;
@@ -666,29 +684,45 @@ __global__ __launch_bounds__(64) void k_flood_compact(Launch L, const uint32_t* 
         uint64_t m = 0ull;
         if (j != cur_job) {
             cur_job = j;
-            running = start_round(L, j, i, w, R, m);
+            running = start_round(L, j, i, w, R, m, progress);
         } else if (running) {
             m = w < relax_groups(R.nb) ? group_bits(load_group(parity_flags(R.flags, R.nb, R.par), w)) : 0ull;
         }
         if (!running) continue;
-        const uint32_t n = (uint32_t)__popcll(m);
-        uint32_t inc = n;  // wave inclusive scan of the per-lane counts
+        if (__ballot(m != 0ull) == 0ull) continue;
+        // the list of the lane's group: the task's, or, in a table of few tasks, the one whose share of the job's
+        // groups it lies in (whole tasks would leave XCDs without work: a grid of up to 128^3 is one task)
+        const uint32_t n = (uint32_t)__popcll(m), ng = relax_groups(R.nb);
+        uint32_t mine = xcd, x0 = xcd, x1 = xcd;
+        if (total_tasks < kSplitTasks) {
+            mine = 0;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t t = __shfl_up(inc, o, 64);
-            if (lane >= (uint32_t)o) inc += t;
+            for (uint32_t x = 1; x < kXcds; ++x) mine += w * kXcds >= x * ng ? 1u : 0u;
+            x0 = uni(mine);
+            x1 = (uint32_t)__builtin_amdgcn_readlane((int)mine, 63);
         }
-        const uint32_t total = __shfl(inc, 63, 64);
-        if (total == 0) continue;
         uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(counts + xcd, total);
-        base = __shfl(base, 0, 64) + inc - n;
+        for (uint32_t x = x0; x <= x1; ++x) {
+            const uint32_t nx = mine == x ? n : 0u;
+            uint32_t inc = nx;  // wave inclusive scan of the per-lane counts
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t t = __shfl_up(inc, o, 64);
+                if (lane >= (uint32_t)o) inc += t;
+            }
+            const uint32_t total = __shfl(inc, 63, 64);
+            if (total == 0) continue;
+            uint32_t first = 0;
+            if (lane == 0) first = atomicAdd(counts + x, total);
+            first = __shfl(first, 0, 64);
+            if (mine == x) base = first + inc - nx;
+        }
         if (m) {
             uint8_t* cur = parity_flags(R.flags, R.nb, R.par) + (size_t)w * 64u;  // consumed
 #pragma unroll
             for (int i = 0; i < 4; ++i) gstore4(cur + 16 * i, make_uint4(0u, 0u, 0u, 0u));
             uint64_t bits = m;
-            unsigned long long* dst = lists + (size_t)xcd * list_cap;
+            unsigned long long* dst = lists + (size_t)mine * list_cap;
             while (bits) {
                 const uint32_t bit = (uint32_t)__ffsll((long long)bits) - 1u;
                 bits &= bits - 1ull;
@@ -809,8 +843,9 @@ __global__ __launch_bounds__(256) void k_flood_init(Launch L, const uint32_t* ta
         const VF_AS_GLOBAL uint8_t* occ = gcast<const uint8_t>(uni_ptr(J->occ));
         const uint32_t rowb = uni(J->wp) * 4u;  // occupancy bytes of a row
         VF_AS_GLOBAL uint32_t* keys = gcast<uint32_t>(uni_ptr(J->keys));
-        VF_AS_GLOBAL unsigned long long* live =
-            gcast<unsigned long long>(live_base(uni_ptr(J->bflags), uni(J->nbricks)));
+        uint8_t* flags = uni_ptr(J->bflags);
+        const uint32_t nb = uni(J->nbricks);
+        VF_AS_GLOBAL unsigned long long* live = gcast<unsigned long long>(live_base(flags, nb));
         for (uint32_t w = g - t0 * 64u; w < nwords; w += nslots) {
             const uint32_t chunk = w % wpc, col = w / wpc, by = col % nby, bx = col / nby;
             // packing: lane l holds brick bz = 64 * chunk + l, a byte of each row; addresses are clamped into the
@@ -843,6 +878,8 @@ __global__ __launch_bounds__(256) void k_flood_init(Launch L, const uint32_t* ta
             }
             const uint64_t m0 = __ballot(any != 0u);
             if (lane == 0u) live[(size_t)col * wpc + chunk] = m0;
+            if (bz < nbz)  // the bricks' flags of both parities
+                for (uint32_t par = 0; par < 2u; ++par) parity_flags(flags, nb, par)[(size_t)col * nbz + bz] = 0u;
             if (m0 == 0ull) continue;
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1150,7 +1187,7 @@ void launch_flood_init(const Launch& L, const FloodRoundScratch& W)
 void launch_flood_seed(const Launch& L, const FloodRoundScratch& W)
 {
     TimedLaunch tl("flood_seed", L.s);
-    k_flood_seed<<<L.njobs, 256, 0, L.s>>>(L);
+    k_flood_seed<<<L.njobs, 256, 0, L.s>>>(L, W.counts);
     VF_CHECK_LAUNCH();
     if (W.total_tasks == 0) return;
     const uint32_t blocks = std::max(1u, std::min(W.total_tasks * 16u, active_shape().cell_blocks));  // 4096 bricks a task
@@ -1158,7 +1195,8 @@ void launch_flood_seed(const Launch& L, const FloodRoundScratch& W)
     VF_CHECK_LAUNCH();
 }
 
-uint32_t flood_list_cap(uint32_t total_tasks) { return (total_tasks + kXcds - 1) / kXcds * 4096u; }
+// whole tasks dealt to the lists, or every job's groups cut into 8 shares (up to 64 bricks more per job and list)
+uint32_t flood_list_cap(uint32_t total_tasks) { return (total_tasks + kXcds - 1) / kXcds * 4096u + 64u * std::min(total_tasks, kSplitTasks); }
 
 void launch_flood_rounds(const Launch& L, const FloodRoundScratch& W, uint32_t rounds, uint32_t blocks)
 {
@@ -1176,13 +1214,14 @@ void launch_flood_rounds(const Launch& L, const FloodRoundScratch& W, uint32_t r
         {
             TimedLaunch tl("flood_compact", L.s);
             k_flood_compact<<<cblocks, 64, 0, L.s>>>(L, W.task_prefix, W.total_tasks, lists[p], W.list_cap, counts[p],
-                                                     counts[p ^ 1u], i);
+                                                     counts[p ^ 1u], i, W.progress);
             VF_CHECK_LAUNCH();
         }
         TimedLaunch tl("flood_relax", L.s);
         k_flood_relax<<<blocks, 64, 0, L.s>>>(L, lists[p], W.list_cap, counts[p]);
         VF_CHECK_LAUNCH();
     }
+    if (W.progress) return;  // a compaction finds the drain and tells the host itself
     TimedLaunch tl("flood_plan", L.s);
     k_flood_plan<<<1, 1024, 0, L.s>>>(L);
     VF_CHECK_LAUNCH();

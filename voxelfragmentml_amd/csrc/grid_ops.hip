@@ -106,13 +106,116 @@ __global__ __launch_bounds__(kCellThreads) void k_undo_mask(Launch L, uint16_t k
     });
 }
 
-__global__ void k_clear_hist(Launch L)
+__global__ void k_put_head(GridHead* dst, GridHead h)
 {
-    for (uint32_t j = 0; j < L.njobs; ++j) {
-        const JobDev* J = L.jobs + j;
-        if (!J->active) continue;
-        for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 65536; i += gridDim.x * blockDim.x) J->hist[i] = 0;
+    static_assert(sizeof(GridHead) % 4 == 0, "copied as words");
+    const uint32_t* s = reinterpret_cast<const uint32_t*>(&h);
+    for (uint32_t i = threadIdx.x; i < sizeof(GridHead) / 4; i += blockDim.x) reinterpret_cast<uint32_t*>(dst)[i] = s[i];
+}
+
+constexpr uint32_t kPutSeeds = 128;  // seeds per launch: 2 KiB of arguments
+struct SeedArgs {
+    uint4 s[kPutSeeds];
+};
+__global__ void k_put_seeds(uint4* dst, SeedArgs a, uint32_t n)
+{
+    if (threadIdx.x < n) dst[threadIdx.x] = a.s[threadIdx.x];
+}
+
+__global__ void k_report(const unsigned long long* stats, const uint4* seeds, uint32_t n, uint32_t* host)
+{
+    if (threadIdx.x < kStatCount) reinterpret_cast<unsigned long long*>(host + kPinStats)[threadIdx.x] = stats[threadIdx.x];
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) reinterpret_cast<uint4*>(host + kPinSeeds)[i] = seeds[i];
+}
+
+// The histogram of a single grid.  Labels below kHistBins are counted in LDS by kHistBlocks workgroups of 16 waves,
+// which then store their counts (1 MiB) for k_hist_sum; larger ones go to the counts in HBM.  Bound by HBM: 2 bytes
+// per cell.  A lane adds the cells of one label among its 8 with one LDS atomic; lanes of a wave that hold the same label
+// follow each other at one a cycle, which costs less than counting them over the wave first (110 us for a 512^3 grid).
+// 8192 workgroups that added their counts to the same few addresses in HBM took 98 us for a 512^3 grid and 57 us for a
+// 256^3 one; now 75 and 20 us, of which clearing and summing take 10.  The word after the partial counts is set when a
+// larger label occurs.
+constexpr uint32_t kHistThreads = 1024;
+__global__ __launch_bounds__(kHistThreads) void k_histogram(Launch L, uint32_t* part)
+{
+    __shared__ uint32_t bins[kHistBins];
+    const JobDev& J = L.jobs[0];
+    const uint16_t* labels = J.labels;
+    const uint64_t V = J.V;
+    for (uint32_t i = threadIdx.x; i < kHistBins; i += kHistThreads) bins[i] = 0;
+    __syncthreads();
+    constexpr uint64_t kStep = (uint64_t)kHistThreads * kCellsPerThread;
+    constexpr uint32_t kRun = 4;  // steps whose loads are issued together
+    const uint64_t steps = (V + kStep - 1) / kStep;
+    const uint32_t lane = threadIdx.x & 63u;
+    // steps are dealt round-robin: a vessel's cells lie in some slabs of the box and not in others
+    for (uint64_t s = blockIdx.x; s < steps; s += (uint64_t)kRun * gridDim.x) {
+        uint4 q[kRun];
+#pragma unroll
+        for (uint32_t r = 0; r < kRun; ++r) {
+            const uint64_t c0 = (s + (uint64_t)r * gridDim.x) * kStep + threadIdx.x * kCellsPerThread;
+            q[r] = make_uint4(0u, 0u, 0u, 0u);
+            if (c0 < V) {
+                uint16_t v[8];
+                load8(labels, c0, V, v);
+                q[r] = pack_cells(v);
+            }
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < kRun; ++r) {
+            const uint32_t w[4] = { q[r].x, q[r].y, q[r].z, q[r].w };
+            if ((w[0] | w[1] | w[2] | w[3]) == 0u) continue;
+            uint32_t m[8], rest = 0;  // masked labels; the cells still to count
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k) {
+                const uint32_t raw = (w[k >> 1] >> (16u * (k & 1u))) & 0xFFFFu;
+                m[k] = raw & kMask15;
+                rest |= raw > kFree ? 1u << k : 0u;
+            }
+            while (rest) {
+                uint32_t l = 0, eq = 0;  // the first cell still to count; the cells of its label
+#pragma unroll
+                for (int k = 7; k >= 0; --k) l = (rest >> k) & 1u ? m[k] : l;
+#pragma unroll
+                for (uint32_t k = 0; k < 8u; ++k) eq |= m[k] == l ? 1u << k : 0u;
+                eq &= rest;
+                rest &= ~eq;
+                if (l < kHistBins) {
+                    atomicAdd(&bins[l], (uint32_t)__popc(eq));
+                } else {
+                    atomicAdd(J.hist + l, (uint32_t)__popc(eq));
+                    part[kHistBlocks * kHistBins] = 1u;
+                }
+            }
+        }
     }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < kHistBins; i += kHistThreads) part[blockIdx.x * kHistBins + i] = bins[i];
+}
+
+// Sums nparts partial counts of 64 bins per workgroup into hist and, where given, host memory.
+__global__ __launch_bounds__(256) void k_hist_sum(const uint32_t* part, uint32_t nparts, uint32_t* hist, uint32_t* host)
+{
+    __shared__ uint32_t sum[4][64];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, bin = blockIdx.x * 64u + lane;
+    uint32_t n = 0;
+#pragma unroll 8
+    for (uint32_t p = wave; p < nparts; p += 4u) n += part[p * kHistBins + bin];
+    sum[wave][lane] = n;
+    __syncthreads();
+    if (wave == 0) {
+        n = sum[0][lane] + sum[1][lane] + sum[2][lane] + sum[3][lane];
+        hist[bin] = n;
+        if (host) host[bin] = n;
+    }
+    if (host && blockIdx.x == 0 && threadIdx.x == 0) host[kHistBins] = part[kHistBlocks * kHistBins];
+}
+
+__global__ void k_hist_clear(uint32_t* hist, uint32_t* flag)
+{
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 65536 / 4; i += gridDim.x * blockDim.x)
+        gstore4(hist + 4 * i, make_uint4(0u, 0u, 0u, 0u));
+    if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0u;
 }
 
 constexpr uint32_t kLdsBins = 4096;
@@ -169,10 +272,10 @@ __device__ inline bool is_boundary_cell(const JobDev* J, uint32_t x, uint32_t y,
     return false;
 }
 
-// HIST: accumulate the per-fragment histogram; BOUND: set the boundary bit.
-// Generic path (any window size; used for jobs with size > 1).  ONLY_WIDE
-// restricts it to those jobs when the tiled kernel handles the rest.
-template <bool HIST, bool BOUND, bool ONLY_WIDE = false>
+// Sets the boundary bits; HIST: and accumulates the per-fragment histogram.
+// Generic path (any window size; used for jobs with size > 1).  In a table (HIST)
+// it is restricted to those jobs, the tiled kernel handles the rest.
+template <bool HIST>
 __global__ __launch_bounds__(kCellThreads) void k_cells_post(Launch L, int bsize)
 {
     __shared__ uint32_t bins[HIST ? kLdsBins : 1];
@@ -204,7 +307,7 @@ __global__ __launch_bounds__(kCellThreads) void k_cells_post(Launch L, int bsize
             cur_job = j;
         }
         const JobDev* J = L.jobs + j;
-        if (!J->active || (ONLY_WIDE && J->bsize <= 1)) continue;
+        if (!J->active || (HIST && J->bsize <= 1)) continue;
         uint64_t c0 = (uint64_t)(t - L.tile_prefix[j]) * kTileCells + threadIdx.x * kCellsPerThread;
         if (c0 >= J->V) continue;
         uint16_t v[8];
@@ -213,7 +316,7 @@ __global__ __launch_bounds__(kCellThreads) void k_cells_post(Launch L, int bsize
         for (int k = 0; k < 8; ++k) any |= v[k] > kFree;
         if (!any) continue;
         bool changed = false;
-        if (BOUND) {
+        {
             const int bs = bsize >= 0 ? bsize : J->bsize;
             uint32_t x, y, z;
             decompose(c0, J, x, y, z);
@@ -255,8 +358,8 @@ constexpr int kBHX = kBTX + 2, kBHY = kBTY + 2, kBHZ = kBTZ + 2;
 // fall on distinct bank groups
 constexpr int kAZ = kBTZ + 4;
 
-// CSUM: the jobs of a table, whose labels follow their occupancy; also accumulate
-// the grid checksum of the final cells (jobs with a window size <= 1; the others
+// TABLE: the jobs of a table, whose labels follow their occupancy; also accumulate
+// the histogram and the grid checksum of the final cells (jobs with a window size <= 1; the others
 // get theirs from k_checksum<true>).
 //
 // Each thread owns an 8-cell z segment of one of the brick's 64 rows and loads
@@ -273,22 +376,22 @@ __device__ inline uint32_t pk_max_u16(uint32_t a, uint32_t b)
 // a label as the packed pair (label | 0xFFFF - label)
 __device__ inline uint32_t packed_self(uint32_t m) { return m | ((0xFFFFu - m) << 16); }
 
-template <bool HIST, bool CSUM, uint32_t RUN>
+template <bool TABLE, uint32_t RUN>
 __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
 {
     // z-window max (low 16 bits) | 0xFFFF - min (high 16) over labelled cells (EMPTY / FREE contribute 0),
     // so one packed u16 max combines both halves; row = hx * kBHY + hy
     __shared__ __attribute__((aligned(16))) uint32_t zmm[kBHX * kBHY * kAZ];
-    __shared__ uint32_t bins[HIST ? kTiledBins : 1];
+    __shared__ uint32_t bins[TABLE ? kTiledBins : 1];
     __shared__ JobDev sJ;
     __shared__ BlockSum csum_part;
     unsigned long long csum = 0;
-    if (HIST) {
+    if (TABLE) {
         for (uint32_t i = threadIdx.x; i < kTiledBins; i += blockDim.x) bins[i] = 0;
     }
     auto flush = [&](uint32_t j) {
-        if (CSUM) csum_part.flush(csum, L.jobs[j], kStatChecksum);
-        if (!HIST) return;
+        if (TABLE) csum_part.flush(csum, L.jobs[j], kStatChecksum);
+        if (!TABLE) return;
         __syncthreads();
         uint32_t* h = L.jobs[j].hist;
         for (uint32_t i = threadIdx.x; i < kTiledBins; i += blockDim.x) {
@@ -359,7 +462,7 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
             nval = gx < nx && gy < ny ? max(0, min(8, nz - gz)) : 0;
         };
         auto add_checksum = [&](const uint16_t v[8], int gx, int gy, int gz, int nval) {
-            if (CSUM)
+            if (TABLE)
                 if (nval && (v[0] | v[1] | v[2] | v[3] | v[4] | v[5] | v[6] | v[7])) {  // EMPTY cells add nothing
                     const uint32_t c0 = (uint32_t)(((size_t)gx * ny + gy) * nz + gz);
                     for (int k = 0; k < nval; ++k) csum += checksum_term(v[k], c0 + k);
@@ -381,7 +484,7 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
 
         // phase 1: whether each brick of the run holds a label, all loads issued together; the others end here
         uint32_t live = 0;
-        if constexpr (CSUM) {
+        if constexpr (TABLE) {
             // a table's labels are not EMPTY only where the occupancy is set, and a brick's rows are one occupancy
             // word each: 4 bytes a row instead of its 64 bytes of labels; bricks without a bit add nothing
             uint32_t occ[kRun];
@@ -423,7 +526,7 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
             uint16_t v[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) v[k] = k < nval ? w[k + 1] : (uint16_t)0;
-            if (HIST) {
+            if (TABLE) {
                 // run-length over the 8 cells: one LDS atomic per run of equal labels
                 uint32_t cur = 0, run = 0;
                 for (int k = 0; k < 8; ++k) {
@@ -566,13 +669,9 @@ __global__ __launch_bounds__(256) void k_job_init(Launch L)
 {
     const JobDev* J = L.jobs + blockIdx.x;
     if (!J->active) return;
-    for (uint32_t i = threadIdx.x; i < 65536; i += blockDim.x) J->hist[i] = 0;
+    for (uint32_t i = threadIdx.x; i < 65536 / 4; i += blockDim.x) gstore4(J->hist + 4 * i, make_uint4(0u, 0u, 0u, 0u));
     if (threadIdx.x < kStatCount) J->stats[threadIdx.x] = 0;
     if (J->fctl && threadIdx.x < 64) J->fctl[threadIdx.x] = 0;
-    if (J->algo == VF_FLOOD && J->bflags) {  // both brick flag parities of the flood rounds
-        const size_t n = 2u * relax_parity_bytes(J->nbricks) / 16u;
-        for (size_t i = threadIdx.x; i < n; i += blockDim.x) gstore4(J->bflags + 16u * i, make_uint4(0u, 0u, 0u, 0u));
-    }
     if (J->sums)
         for (uint32_t i = threadIdx.x; i < kSumSlots * kStatCount; i += blockDim.x) J->sums[i] = 0ull;
 }
@@ -599,6 +698,34 @@ inline uint32_t bgrid_for(const Launch& L) { return std::max(1u, std::min(L.tota
 inline uint32_t grid_for(const Launch& L) { return std::max(1u, std::min(L.total_tiles, active_shape().cell_blocks)); }
 
 }  // namespace
+
+void launch_put_head(GridHead* dst, const GridHead& h, hipStream_t s)
+{
+    TimedLaunch tl("put_head", s);
+    k_put_head<<<1, 128, 0, s>>>(dst, h);
+    VF_CHECK_LAUNCH();
+}
+
+void launch_put_seeds(uint4* dst, const vf_seed* seeds, uint32_t n, hipStream_t s)
+{
+    static_assert(sizeof(vf_seed) == sizeof(uint4), "copied as they are");
+    for (uint32_t i = 0; i < n; i += kPutSeeds) {
+        SeedArgs a;
+        const uint32_t m = std::min(kPutSeeds, n - i);
+        __builtin_memcpy(a.s, seeds + i, (size_t)m * sizeof(uint4));
+        TimedLaunch tl("put_seeds", s);
+        k_put_seeds<<<1, kPutSeeds, 0, s>>>(dst + i, a, m);
+        VF_CHECK_LAUNCH();
+    }
+}
+
+void launch_report(const unsigned long long* stats, const uint4* seeds, uint32_t n, uint32_t* host, hipStream_t s)
+{
+    if (n > kMaxDeviceSeeds) fail(VF_ERR_INVALID_ARG, "report of %u seeds", n);
+    TimedLaunch tl("report", s);
+    k_report<<<1, 256, 0, s>>>(stats, seeds, n, host);
+    VF_CHECK_LAUNCH();
+}
 
 void launch_occ_to_labels(const Launch& L)
 {
@@ -649,33 +776,26 @@ void launch_undo_mask(const Launch& L, uint16_t keep)
     VF_CHECK_LAUNCH();
 }
 
-void launch_clear_hist(const Launch& L)
-{
-    TimedLaunch tl("clear_hist", L.s);
-    k_clear_hist<<<64, 256, 0, L.s>>>(L);
-    VF_CHECK_LAUNCH();
-}
-
-void launch_histogram(const Launch& L)
+void launch_histogram(const Launch& L, uint32_t* hist, uint32_t* part, uint32_t* host)
 {
     TimedLaunch tl("histogram", L.s);
-    k_cells_post<true, false><<<grid_for(L), kCellThreads, 0, L.s>>>(L, 0);
+    const uint32_t blocks = std::max(1u, std::min(kHistBlocks, ceil_div((uint64_t)L.total_tiles * kTileCells, kHistThreads * kCellsPerThread)));
+    k_hist_clear<<<16, 256, 0, L.s>>>(hist, part + kHistBlocks * kHistBins);
+    VF_CHECK_LAUNCH();
+    k_histogram<<<blocks, kHistThreads, 0, L.s>>>(L, part);
+    VF_CHECK_LAUNCH();
+    k_hist_sum<<<kHistBins / 64, 256, 0, L.s>>>(part, blocks, hist, host);
     VF_CHECK_LAUNCH();
 }
 
-void launch_boundaries(const Launch& L, int size, int with_hist)
+void launch_boundaries(const Launch& L, int size)
 {
-    if (with_hist) {
-        TimedLaunch tl("boundaries_hist", L.s);
-        k_cells_post<true, true><<<grid_for(L), kCellThreads, 0, L.s>>>(L, size);
-    } else {
-        TimedLaunch tl("boundaries", L.s);
-        k_cells_post<false, true><<<grid_for(L), kCellThreads, 0, L.s>>>(L, size);
-    }
+    TimedLaunch tl("boundaries", L.s);
+    k_cells_post<false><<<grid_for(L), kCellThreads, 0, L.s>>>(L, size);
     VF_CHECK_LAUNCH();
 }
 
-void launch_boundaries_tiled(const Launch& L, bool any_wide, bool with_checksum)
+void launch_boundaries_tiled(const Launch& L, bool any_wide, bool table)
 {
     {
         TimedLaunch tl("boundaries_hist", L.s);
@@ -683,8 +803,8 @@ void launch_boundaries_tiled(const Launch& L, bool any_wide, bool with_checksum)
         const uint32_t blocks = std::max(1u, std::min(L.total_bricks, sh.brick_blocks));
         auto go = [&](auto run) {
             constexpr uint32_t R = decltype(run)::value;
-            if (with_checksum) k_boundaries_tiled<true, true, R><<<blocks, 256, 0, L.s>>>(L);
-            else k_boundaries_tiled<true, false, R><<<blocks, 256, 0, L.s>>>(L);
+            if (table) k_boundaries_tiled<true, R><<<blocks, 256, 0, L.s>>>(L);
+            else k_boundaries_tiled<false, R><<<blocks, 256, 0, L.s>>>(L);
         };
         if (sh.brick_run == 2) go(std::integral_constant<uint32_t, 2>{});
         else if (sh.brick_run == 8) go(std::integral_constant<uint32_t, 8>{});
@@ -693,9 +813,9 @@ void launch_boundaries_tiled(const Launch& L, bool any_wide, bool with_checksum)
     }
     if (any_wide) {
         TimedLaunch tl("boundaries_wide", L.s);
-        k_cells_post<true, true, true><<<grid_for(L), kCellThreads, 0, L.s>>>(L, -1);
+        k_cells_post<true><<<grid_for(L), kCellThreads, 0, L.s>>>(L, -1);
         VF_CHECK_LAUNCH();
-        if (with_checksum) {
+        if (table) {
             TimedLaunch tc("checksum", L.s);
             k_checksum<true><<<grid_for(L), kCellThreads, 0, L.s>>>(L);
             VF_CHECK_LAUNCH();

@@ -187,6 +187,19 @@ void launch_voxelize(const Launch& L, const VoxScratch& X, const uint32_t* col_p
 void launch_clear_bits(const Launch& L, const uint32_t* col_prefix, uint32_t total_col_groups);
 
 // grid_ops.hip
+// A single grid's launch table: its descriptor and one-job prefixes, {0, count} pairs from kHeadTiles on.
+constexpr uint32_t kHeadTiles = 0, kHeadBricks = 2, kHeadWordTiles = 4, kHeadTris = 6, kHeadGroups = 8, kHeadTasks = 10,
+                   kHeadWords = 12;
+struct GridHead {
+    JobDev job;
+    uint32_t words[kHeadWords];
+};
+// Small uploads ride in a launch's arguments and small results are stored to pinned host memory by a kernel: a copy
+// each way costs a transfer launch, and a wait before its staging can be used again.
+void launch_put_head(GridHead* dst, const GridHead& h, hipStream_t s);
+void launch_put_seeds(uint4* dst, const vf_seed* seeds, uint32_t n, hipStream_t s);
+// stats (kStatCount 64-bit words) and n seeds (at most kMaxDeviceSeeds) to their places in a grid's pinned words
+void launch_report(const unsigned long long* stats, const uint4* seeds, uint32_t n, uint32_t* host, hipStream_t s);
 void launch_occ_to_labels(const Launch& L);
 void launch_labels_to_occ(const Launch& L);
 void launch_occ_free(const Launch& L, const uint32_t* bits);  // labels of the cells set in bits (laid out as occ) become FREE
@@ -195,13 +208,20 @@ void launch_homogenize(const Launch& L);
 // every cell of every job EMPTY: the fractures (launch_naive, launch_flood_finish) write only around occupied cells
 void launch_clear_labels(const Launch& L);
 void launch_undo_mask(const Launch& L, uint16_t keep_mask);
-void launch_clear_hist(const Launch& L);
-void launch_histogram(const Launch& L);
-void launch_boundaries(const Launch& L, int size /* < 0: per-job bsize */, int with_hist);
-// detectBoundaries(size <= 1 per job) fused with the histogram, brick by brick;
+// job 0's histogram of labels above FREE into its hist (given again; cleared first); part: kHistPartBytes of scratch; host (or
+// null): pinned memory for the first kHistBins counts and a flag, not 0 when a larger label occurs
+constexpr uint32_t kHistBins = 1024, kHistBlocks = 256;
+// pinned words of a grid that kernels report to: statistics, flood progress (three words), a histogram's first counts
+// and its flag, seeds
+constexpr uint32_t kPinStats = 0, kPinProgress = 2 * kStatCount, kPinHist = 64, kPinSeeds = kPinHist + kHistBins + 64,
+                   kPinWords = kPinSeeds + 4 * 4096;
+constexpr size_t kHistPartBytes = ((size_t)kHistBlocks * kHistBins + 64) * 4;
+void launch_histogram(const Launch& L, uint32_t* hist, uint32_t* part, uint32_t* host);
+void launch_boundaries(const Launch& L, int size /* < 0: per-job bsize */);
+// detectBoundaries(size <= 1 per job), brick by brick, for a table fused with the histogram;
 // jobs with size > 1 go through the generic kernel when any_wide.
-// with_checksum: a table's jobs (cells outside the occupancy are EMPTY); also sum every job's grid checksum into kStatChecksum
-void launch_boundaries_tiled(const Launch& L, bool any_wide, bool with_checksum);
+// table: a table's jobs (cells outside the occupancy are EMPTY); also their histograms and grid checksums (kStatChecksum)
+void launch_boundaries_tiled(const Launch& L, bool any_wide, bool table);
 void launch_job_init(const Launch& L);     // zero stats, histogram and flood control of every job
 void launch_gather(const Launch& L, uint32_t* out);  // 16 words per job: stats (low 32 bits) + flood state
 void launch_checksum(const Launch& L);
@@ -255,7 +275,9 @@ struct FloodRoundScratch {
     uint32_t total_tasks;
     unsigned long long* lists;     // 2 x kFloodXcds brick worklists (even and odd rounds of a chunk), list_cap entries each
     uint32_t list_cap;             // >= flood_list_cap(total_tasks)
-    uint32_t* counts;              // 2 x kFloodXcds list lengths; zero before the first round (a chunk leaves them zero)
+    uint32_t* counts;              // 2 x kFloodXcds list lengths, zeroed with the seeds (a chunk leaves them zero)
+    uint32_t* progress = nullptr;  // one job, or null: pinned host words that receive the last round started, the rounds
+                                   // run once drained, and then the job's error flags
 };
 constexpr uint32_t kFloodXcds = 8;
 uint32_t flood_list_cap(uint32_t total_tasks);  // entries per XCD list
@@ -286,6 +308,7 @@ void launch_flood_sub(const Launch& L);
 
 // seed.hip
 constexpr uint32_t kMaxDeviceSeeds = 4096;
+static_assert(kPinWords == kPinSeeds + 4 * kMaxDeviceSeeds, "room for the reported seeds");
 void launch_seed_count(const Launch& L, uint32_t* tile_cnt, bool skip_both);
 // tile_off: exclusive prefix over the global word tiles (total_wtiles + 1 entries)
 void launch_seed_pick(const Launch& L, const unsigned long long* tile_off);

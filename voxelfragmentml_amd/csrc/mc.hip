@@ -1385,8 +1385,7 @@ void mc_smooth(McScratch& W, hipStream_t s, uint32_t nb_iters, float nb_weight, 
 void grid_marching_cubes(vf_grid* g, uint32_t want, vf_mesh_info* info)
 {
     Launch L = grid_launch(g);
-    launch_clear_hist(L);
-    launch_histogram(L);
+    launch_histogram(L, g->hist.as<uint32_t>(), g->hist.as<uint32_t>() + 65536, nullptr);
     g->mc.valid = false;
     mc_run(g->mc, g->stream, g->labels.as<uint16_t>(), g->dims, g->mn, g->cs, g->hist.as<uint32_t>(), want, info);
 }

@@ -1,5 +1,5 @@
 // Exclusive prefix sum, uint32 in -> uint64 out (n+1 entries, out[n] = total).
-// Three launches (block reduce, scan of block sums, block rescan), no host
+// Three launches (block reduce, scan of block sums, block rescan; one for few items), no host
 // synchronisation and no memset, so it can sit inside a captured HIP graph.
 #include "jobs.hpp"
 
@@ -120,6 +120,37 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_down(const uint32_t* in, 
     if (blockIdx.x == nb - 1 && threadIdx.x == 0) out[n] = sums[nb];
 }
 
+// Up to kScanSmall items in one workgroup of 16 waves: three launches of a few blocks cost three launches' latency.
+constexpr uint32_t kSmallThreads = 1024, kScanSmall = kSmallThreads * kScanItems;
+__global__ __launch_bounds__(kSmallThreads) void k_scan_small(const uint32_t* in, uint32_t n, unsigned long long* out)
+{
+    __shared__ unsigned long long smem[kSmallThreads / 64];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, base = threadIdx.x * kScanItems;
+    uint32_t v[kScanItems];
+    load_items(in, base, n, vec_ok(in, in, base, n), v);
+    unsigned long long s = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kScanItems; ++k) s += v[k];
+    unsigned long long x = s;
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned long long y = __shfl_up(x, o, 64);
+        if (lane >= (uint32_t)o) x += y;
+    }
+    if (lane == 63u) smem[wave] = x;
+    __syncthreads();
+    unsigned long long e = x - s, total = 0;
+    for (uint32_t w = 0; w < kSmallThreads / 64; ++w) {
+        if (w < wave) e += smem[w];
+        total += smem[w];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kScanItems; ++k) {
+        if (base + k < n) out[base + k] = e;
+        e += v[k];
+    }
+    if (threadIdx.x == 0) out[n] = total;
+}
+
 __global__ void k_scan_empty(unsigned long long* out) { out[0] = 0; }
 }  // namespace
 
@@ -134,6 +165,12 @@ void scan_exclusive_u32_to_u64(const uint32_t* in, unsigned long long* out, uint
     if (n == 0) {
         TimedLaunch tl("scan", s);
         k_scan_empty<<<1, 1, 0, s>>>(out);
+        VF_CHECK_LAUNCH();
+        return;
+    }
+    if (n <= kScanSmall) {
+        TimedLaunch tl("scan", s);
+        k_scan_small<<<1, kSmallThreads, 0, s>>>(in, (uint32_t)n, out);
         VF_CHECK_LAUNCH();
         return;
     }

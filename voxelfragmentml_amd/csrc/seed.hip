@@ -122,9 +122,9 @@ __device__ inline uint32_t nth_bit(uint32_t v, uint32_t n)
 constexpr uint32_t kPickParts = 8;
 __global__ __launch_bounds__(kSeedThreads) void k_seed_pick(Launch L, const unsigned long long* tile_off)
 {
-    __shared__ uint32_t chosen[kMaxDeviceSeeds];
+    __shared__ __attribute__((aligned(16))) uint32_t chosen[kMaxDeviceSeeds];
     __shared__ uint32_t sorted[kMaxDeviceSeeds];
-    __shared__ uint32_t cand[kSeedThreads];
+    __shared__ __attribute__((aligned(16))) uint32_t cand[kSeedThreads];
     __shared__ uint32_t wsum[kSeedThreads / 64];
     __shared__ uint32_t s_got;
     const uint32_t j = blockIdx.x / kPickParts, part = blockIdx.x % kPickParts;
@@ -148,16 +148,32 @@ __global__ __launch_bounds__(kSeedThreads) void k_seed_pick(Launch L, const unsi
     }
     if (threadIdx.x == 0) s_got = 0;
     __syncthreads();
-    for (uint32_t j0 = 0; j0 < kMaxDraws; j0 += kSeedThreads) {
+    // how many of the first n entries of a list equal r (n may differ by lane): 16-byte reads, no early way out, so that
+    // the reads of a wave's lanes stream
+    auto count_if = [](const uint32_t* list, uint32_t n, auto&& test) {
+        uint32_t c = 0;
+        for (uint32_t k = 0; k < n; k += 4u) {
+            const uint4 q = *reinterpret_cast<const uint4*>(list + k);
+            c += (test(q.x) ? 1u : 0u) + (k + 1u < n && test(q.y) ? 1u : 0u) + (k + 2u < n && test(q.z) ? 1u : 0u) +
+                 (k + 3u < n && test(q.w) ? 1u : 0u);
+        }
+        return c;
+    };
+    // as many draws a step as seeds are missing: a draw is accepted or not by those before it alone
+    for (uint32_t j0 = 0; j0 < kMaxDraws;) {
         const uint32_t got = s_got;
         if (got >= S) break;
+        const uint32_t step = min(S - got, kSeedThreads);
         const uint32_t draw = j0 + threadIdx.x;
+        j0 += step;
         const uint32_t r = (uint32_t)(((unsigned long long)hash32(J->seed_key, draw) * O) >> 32);
         cand[threadIdx.x] = r;
         __syncthreads();
-        bool dup = draw >= kMaxDraws;
-        for (uint32_t k = 0; k < got && !dup; ++k) dup = chosen[k] == r;
-        for (uint32_t k = 0; k < threadIdx.x && !dup; ++k) dup = cand[k] == r;
+        bool dup = draw >= kMaxDraws || threadIdx.x >= step;
+        if (!dup) {
+            auto same = [&](uint32_t v) { return v == r; };
+            dup = count_if(chosen, got, same) + count_if(cand, threadIdx.x, same) != 0u;
+        }
         // block exclusive scan of the accept flags
         uint32_t a = dup ? 0u : 1u, x = a;
         const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -185,9 +201,7 @@ __global__ __launch_bounds__(kSeedThreads) void k_seed_pick(Launch L, const unsi
     // sort the distinct ranks: position = number of smaller ranks
     for (uint32_t i = threadIdx.x; i < S; i += blockDim.x) {
         const uint32_t r = chosen[i];
-        uint32_t p = 0;
-        for (uint32_t k = 0; k < S; ++k) p += chosen[k] < r ? 1u : 0u;
-        sorted[p] = r;
+        sorted[count_if(chosen, S, [&](uint32_t v) { return v < r; })] = r;
     }
     __syncthreads();
     // rank -> tile -> cell: lane l holds the candidates of the tile's word l, a wave scan finds the lane with the
