@@ -265,8 +265,8 @@ int vf_grid_read(vf_grid* g, uint16_t* out)
         checked(g);
         if (!out) fail(VF_ERR_INVALID_ARG, "out is NULL");
         grid_materialize(g);
-        VF_HIP(hipMemcpyAsync(out, g->labels.p, g->V * 2, hipMemcpyDeviceToHost, g->stream));
-        VF_HIP(hipStreamSynchronize(g->stream));
+        g->to_host.add(out, g->labels.p, g->V * 2);
+        g->to_host.run(g->stream);
     });
 }
 
@@ -291,8 +291,8 @@ int vf_occupancy_read(vf_grid* g, uint8_t* out)
         if (!out) fail(VF_ERR_INVALID_ARG, "out is NULL");
         g->occ_tmp.ensure(g->V + 64);
         launch_occ_bytes(grid_launch(g), g->occ_tmp.as<uint8_t>());
-        VF_HIP(hipMemcpyAsync(out, g->occ_tmp.p, g->V, hipMemcpyDeviceToHost, g->stream));
-        VF_HIP(hipStreamSynchronize(g->stream));
+        g->to_host.add(out, g->occ_tmp.p, g->V);
+        g->to_host.run(g->stream);
     });
 }
 

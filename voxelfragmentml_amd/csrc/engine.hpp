@@ -110,8 +110,10 @@ public:
     void erode(Table& t);      // per-job erosion (post calls it)
     void flood_sub(Table& t);  // the flood's sub-seed pass for the jobs with merged seeds
     void gather(Table& t, uint32_t* host16);  // async copy of the gathered stats
-    // fill j.res from 16 gathered words and make the optional grid and histogram copies
-    void finish(EJob& j, const uint32_t* w16);
+    // after post(t): waits for it, fills the jobs' results and makes their optional grid and histogram copies.
+    // later: copies that the device makes by itself may be left in flight on the stream `copies`; true if they are.
+    bool collect(Table& t, bool later = false);
+    hipStream_t copies = nullptr;
     // marching cubes (and smoothing) of every listed job with marching_cubes set and no error, in one
     // launch set: counts into the results, meshes into the jobs' mesh_out.  reserve: see mc_run_jobs.
     void extract(const std::vector<EJob*>& js, const std::function<bool(size_t)>& reserve = nullptr);
@@ -125,6 +127,10 @@ private:
     BlockCache cache_;       // job blocks, tables, worklists and front scratch
     CacheBuf vox_setup_, vox_counts_, vox_shell_off_, scan_tmp_, seed_cnt_, seed_off_;
     McScratch mc_;
+    HostCopies to_host_;
+    uint32_t* hist_pinned_ = nullptr;  // the first counts of a table's jobs, kHistBins each
+    uint32_t hist_jobs_ = 0;           // jobs it has room for
+    void finish(EJob& j, const uint32_t* w16, const uint32_t* hist);
 };
 
 double now_ms();

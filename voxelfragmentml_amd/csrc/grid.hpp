@@ -11,6 +11,7 @@ struct vf_grid {
     hipStream_t stream = nullptr;
 
     vf::DevBuf labels, occ;          // uint16 cells, occupancy bits (JobDev::occ)
+    vf::HostCopies to_host;
     vf::DevBuf head, stats, seeds;
     vf::DevBuf hist;                 // 65536 counts, then kHistPartBytes of partial counts
     vf::DevBuf bits;                 // toggle bitmask

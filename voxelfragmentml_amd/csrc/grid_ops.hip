@@ -211,6 +211,12 @@ __global__ __launch_bounds__(256) void k_hist_sum(const uint32_t* part, uint32_t
     if (host && blockIdx.x == 0 && threadIdx.x == 0) host[kHistBins] = part[kHistBlocks * kHistBins];
 }
 
+// The first kHistBins counts of every job to host memory.
+__global__ __launch_bounds__(kHistBins / 4) void k_hist_heads(const JobDev* jobs, uint32_t* host)
+{
+    reinterpret_cast<uint4*>(host)[blockIdx.x * (kHistBins / 4) + threadIdx.x] = reinterpret_cast<const uint4*>(jobs[blockIdx.x].hist)[threadIdx.x];
+}
+
 __global__ void k_hist_clear(uint32_t* hist, uint32_t* flag)
 {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 65536 / 4; i += gridDim.x * blockDim.x)
@@ -773,6 +779,13 @@ void launch_undo_mask(const Launch& L, uint16_t keep)
 {
     TimedLaunch tl("undo_mask", L.s);
     k_undo_mask<<<grid_for(L), kCellThreads, 0, L.s>>>(L, keep);
+    VF_CHECK_LAUNCH();
+}
+
+void launch_hist_heads(const Launch& L, uint32_t* host)
+{
+    TimedLaunch tl("hist_heads", L.s);
+    k_hist_heads<<<L.njobs, kHistBins / 4, 0, L.s>>>(L.jobs, host);
     VF_CHECK_LAUNCH();
 }
 

@@ -1,0 +1,34 @@
+// Copies of device memory to a caller's host memory.
+#pragma once
+#include <memory>
+#include <vector>
+
+#include "common.hpp"
+
+namespace vf {
+
+class CopyPool;
+
+// A list of copies, made by run() after the work queued on the stream; run returns when the last byte is in place.
+// Held by the object whose stream it uses, so that the pool behind it lives as long as one of them does.
+class HostCopies {
+public:
+    void add(void* dst, const void* src, size_t bytes)
+    {
+        if (bytes) list_.push_back(Part{ static_cast<uint8_t*>(dst), static_cast<const uint8_t*>(src), bytes });
+    }
+    void run(hipStream_t s);
+    // as run, but copies that the device makes by itself (to pinned memory) may be left in flight: true if they are
+    bool start(hipStream_t s);
+    struct Part {
+        uint8_t* dst;
+        const uint8_t* src;
+        size_t bytes;
+    };
+
+private:
+    std::vector<Part> list_;
+    std::shared_ptr<CopyPool> pool_;
+};
+
+}  // namespace vf

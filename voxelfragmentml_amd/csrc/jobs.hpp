@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "hostcopy.hpp"
 
 namespace vf {
 
@@ -216,6 +217,7 @@ constexpr uint32_t kHistBins = 1024, kHistBlocks = 256;
 constexpr uint32_t kPinStats = 0, kPinProgress = 2 * kStatCount, kPinHist = 64, kPinSeeds = kPinHist + kHistBins + 64,
                    kPinWords = kPinSeeds + 4 * 4096;
 constexpr size_t kHistPartBytes = ((size_t)kHistBlocks * kHistBins + 64) * 4;
+void launch_hist_heads(const Launch& L, uint32_t* host);  // every job's first kHistBins counts to pinned host memory
 void launch_histogram(const Launch& L, uint32_t* hist, uint32_t* part, uint32_t* host);
 void launch_boundaries(const Launch& L, int size /* < 0: per-job bsize */);
 // detectBoundaries(size <= 1 per job), brick by brick, for a table fused with the histogram;
@@ -337,6 +339,7 @@ struct McScratch {
     BlockCache* cache = &own;
     uint32_t nv = 0, nt = 0, nl = 0;  // totals of the last run; nl counts (grid, label) segments
     bool valid = false;
+    HostCopies to_host;
     std::vector<uint32_t> label_base;  // first segment of each grid of the last run, and the total
     void ensure(int slot, size_t n);
     void release_all();               // every buffer back to the cache (the result is dropped)

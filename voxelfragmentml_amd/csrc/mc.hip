@@ -1256,11 +1256,11 @@ void mc_read_range(McScratch& W, hipStream_t s, uint32_t seg0, uint32_t nseg, fl
     VF_HIP(hipMemcpyAsync(to.data(), seg + (W.nl + 1) + seg0, (nseg + 1) * 8, hipMemcpyDeviceToHost, s));
     VF_HIP(hipStreamSynchronize(s));
     const unsigned long long v0 = vo[0], nv = vo[nseg] - v0, t0 = to[0], nt = to[nseg] - t0;
-    if (xyz && nv) VF_HIP(hipMemcpyAsync(xyz, B[kBXyz].as<float>() + 3 * v0, nv * 12, hipMemcpyDeviceToHost, s));
-    if (tri && nt) VF_HIP(hipMemcpyAsync(tri, B[kBTri].as<uint32_t>() + 3 * t0, nt * 12, hipMemcpyDeviceToHost, s));
-    if (tri_flag && nt) VF_HIP(hipMemcpyAsync(tri_flag, B[kBFlag].as<uint8_t>() + t0, nt, hipMemcpyDeviceToHost, s));
-    if (labels && nseg) VF_HIP(hipMemcpyAsync(labels, B[kBLabels].as<uint16_t>() + seg0, (size_t)nseg * 2, hipMemcpyDeviceToHost, s));
-    VF_HIP(hipStreamSynchronize(s));
+    if (xyz) W.to_host.add(xyz, B[kBXyz].as<float>() + 3 * v0, nv * 12);
+    if (tri) W.to_host.add(tri, B[kBTri].as<uint32_t>() + 3 * t0, nt * 12);
+    if (tri_flag) W.to_host.add(tri_flag, B[kBFlag].as<uint8_t>() + t0, nt);
+    if (labels) W.to_host.add(labels, B[kBLabels].as<uint16_t>() + seg0, (size_t)nseg * 2);
+    W.to_host.run(s);
     for (uint32_t l = 0; l <= nseg; ++l) {
         if (voff) voff[l] = (uint32_t)(vo[l] - v0);
         if (toff) toff[l] = (uint32_t)(to[l] - t0);
@@ -1287,18 +1287,17 @@ void mc_read_jobs(McScratch& W, hipStream_t s, const McJobResult* res, vf_mesh_o
         if (r.status != VF_OK || r.nv > o->cap_vertices || r.nt > o->cap_triangles || r.nl > o->cap_labels) continue;
         if ((r.nv && !o->xyz) || (r.nt && !o->tri)) continue;
         const unsigned long long v0 = vo[r.seg0], t0 = to[r.seg0];
-        if (r.nv) VF_HIP(hipMemcpyAsync(o->xyz, B[kBXyz].as<float>() + 3 * v0, (size_t)r.nv * 12, hipMemcpyDeviceToHost, s));
-        if (r.nt) VF_HIP(hipMemcpyAsync(o->tri, B[kBTri].as<uint32_t>() + 3 * t0, (size_t)r.nt * 12, hipMemcpyDeviceToHost, s));
-        if (r.nt && o->tri_flag) VF_HIP(hipMemcpyAsync(o->tri_flag, B[kBFlag].as<uint8_t>() + t0, r.nt, hipMemcpyDeviceToHost, s));
-        if (r.nl && o->labels)
-            VF_HIP(hipMemcpyAsync(o->labels, B[kBLabels].as<uint16_t>() + r.seg0, (size_t)r.nl * 2, hipMemcpyDeviceToHost, s));
+        W.to_host.add(o->xyz, B[kBXyz].as<float>() + 3 * v0, (size_t)r.nv * 12);
+        W.to_host.add(o->tri, B[kBTri].as<uint32_t>() + 3 * t0, (size_t)r.nt * 12);
+        if (o->tri_flag) W.to_host.add(o->tri_flag, B[kBFlag].as<uint8_t>() + t0, r.nt);
+        if (o->labels) W.to_host.add(o->labels, B[kBLabels].as<uint16_t>() + r.seg0, (size_t)r.nl * 2);
         for (uint32_t l = 0; l <= r.nl; ++l) {
             if (o->vert_offsets) o->vert_offsets[l] = (uint32_t)(vo[r.seg0 + l] - v0);
             if (o->tri_offsets) o->tri_offsets[l] = (uint32_t)(to[r.seg0 + l] - t0);
         }
         o->copied = 1;
     }
-    VF_HIP(hipStreamSynchronize(s));
+    W.to_host.run(s);
 }
 
 void mc_read(McScratch& W, hipStream_t s, float* xyz, uint32_t* tri, uint8_t* tri_flag, uint16_t* labels, uint32_t* voff,
@@ -1400,9 +1399,9 @@ void grid_mesh_slice(vf_grid* g, uint32_t v0, uint32_t nv, uint32_t t0, uint32_t
 {
     auto& B = g->mc.buf;
     if ((uint64_t)v0 + nv > g->mc.nv || (uint64_t)t0 + nt > g->mc.nt) fail(VF_ERR_INVALID_ARG, "mesh slice out of range");
-    if (nv) VF_HIP(hipMemcpyAsync(xyz, B[kBXyz].as<float>() + 3ull * v0, (size_t)nv * 12, hipMemcpyDeviceToHost, g->stream));
-    if (nt) VF_HIP(hipMemcpyAsync(tri, B[kBTri].as<uint32_t>() + 3ull * t0, (size_t)nt * 12, hipMemcpyDeviceToHost, g->stream));
-    VF_HIP(hipStreamSynchronize(g->stream));
+    g->to_host.add(xyz, B[kBXyz].as<float>() + 3ull * v0, (size_t)nv * 12);
+    g->to_host.add(tri, B[kBTri].as<uint32_t>() + 3ull * t0, (size_t)nt * 12);
+    g->to_host.run(g->stream);
 }
 
 }  // namespace vf
