@@ -701,7 +701,7 @@ int vf_erode(vf_grid* g, int convolution, uint32_t size, uint32_t iterations, fl
         if (side < 0) fail(VF_ERR_INVALID_ARG, "unknown erosion convolution %d", convolution);
         const float limit = act * threshold;
         grid_materialize(g);
-        g->erode_tmp.ensure(g->V * 2 + 64);
+        g->erode_bits.ensure(erode_bytes(g->dims));
         g->erode_mask.ensure(mask.size() + 64);
         VF_HIP(hipMemcpyAsync(g->erode_mask.p, mask.data(), mask.size(), hipMemcpyHostToDevice, g->stream));
         if (g->job.bsize != 1) {
@@ -711,12 +711,10 @@ int vf_erode(vf_grid* g, int convolution, uint32_t size, uint32_t iterations, fl
         Launch L = grid_launch(g);
         for (uint32_t it = 0; it < iterations; ++it) {
             launch_boundaries_tiled(L, false, false);
-            launch_erode_step(L, g->erode_tmp.as<uint16_t>(), g->erode_mask.as<uint8_t>(), (uint32_t)side, limit,
-                              probability, noise_seed, g->V);
-            VF_HIP(hipMemcpyAsync(g->labels.p, g->erode_tmp.p, g->V * 2, hipMemcpyDeviceToDevice, g->stream));
+            launch_erode_step(L, g->erode_bits.as<uint8_t>(), g->erode_mask.as<uint8_t>(), (uint32_t)side, limit,
+                              probability, noise_seed);
         }
-        launch_isolated_cells(L, g->erode_tmp.as<uint16_t>(), g->V);
-        VF_HIP(hipMemcpyAsync(g->labels.p, g->erode_tmp.p, g->V * 2, hipMemcpyDeviceToDevice, g->stream));
+        launch_isolated_cells(L, g->erode_bits.as<uint8_t>());
         launch_labels_to_occ(L);
         g->mc.valid = false;
         VF_HIP(hipStreamSynchronize(g->stream));
@@ -728,10 +726,9 @@ int vf_remove_isolated_cells(vf_grid* g)
     return guard([&] {
         checked(g);
         grid_materialize(g);
-        g->erode_tmp.ensure(g->V * 2 + 64);
+        g->erode_bits.ensure(erode_bytes(g->dims));
         Launch L = grid_launch(g);
-        launch_isolated_cells(L, g->erode_tmp.as<uint16_t>(), g->V);
-        VF_HIP(hipMemcpyAsync(g->labels.p, g->erode_tmp.p, g->V * 2, hipMemcpyDeviceToDevice, g->stream));
+        launch_isolated_cells(L, g->erode_bits.as<uint8_t>());
         launch_labels_to_occ(L);
         g->mc.valid = false;
         VF_HIP(hipStreamSynchronize(g->stream));

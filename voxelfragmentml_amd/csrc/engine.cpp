@@ -66,7 +66,7 @@ Layout layout_of(const vf_job& j)
     L.bricks = o; if (flood) o = align_up(o + relax_flag_bytes(j.dims[0], j.dims[1], j.dims[2]));
     L.sums = o; o = align_up(o + kSumBytes);
     L.sub = o; if (needs_sub(j)) o = align_up(o + 8ull * seed_total(j));  // union-find parents + keep flags
-    L.erode = o; if (j.erode) o = align_up(o + L.V * 2);                          // erosion output grid
+    L.erode = o; if (j.erode) o = align_up(o + erode_bytes(j.dims));              // cells an erosion step empties
     L.mask = o; if (j.erode) o = align_up(o + (size_t)kMaxErosionSide * kMaxErosionSide * kMaxErosionSide);
     L.mesh_xyz = o; if (!j.mesh_on_device) o = align_up(o + (size_t)j.nv * 12);
     L.mesh_tri = o; if (!j.mesh_on_device) o = align_up(o + (size_t)j.nt * 12);
@@ -270,13 +270,13 @@ void Engine::alloc(EJob& e)
     upload_inputs(e);
     d.nt = j.nt;
     d.nv = j.nv;
-    e.erode_out = nullptr;
+    e.erode_bits = nullptr;
     if (j.erode) {  // RegularGrid::erode's window and output grid
         std::vector<uint8_t> mask;
         float act = 0;
         e.erode_side = (uint32_t)erosion_mask(j.erosion_convolution, j.erosion_size, mask, act);
         e.erode_limit = act * j.erosion_threshold;
-        e.erode_out = reinterpret_cast<uint16_t*>(base + Lo.erode);
+        e.erode_bits = base + Lo.erode;
         e.erode_mask = base + Lo.mask;
         VF_HIP(hipMemcpyAsync(e.erode_mask, mask.data(), mask.size(), hipMemcpyHostToDevice, s));
         VF_HIP(hipStreamSynchronize(s));  // the pageable mask goes out of scope
@@ -552,12 +552,10 @@ void Engine::erode(Table& t)
         one.total_bricks = brick_count(e.d.nx, e.d.ny, e.d.nz);
         for (uint32_t it = 0; it < e.spec.erosion_iterations; ++it) {
             launch_boundaries_tiled(one, false, false);
-            launch_erode_step(one, e.erode_out, e.erode_mask, e.erode_side, e.erode_limit, e.spec.erosion_probability,
-                              e.spec.erosion_seed, e.d.V);
-            VF_HIP(hipMemcpyAsync(e.d.labels, e.erode_out, e.d.V * 2, hipMemcpyDeviceToDevice, s));
+            launch_erode_step(one, e.erode_bits, e.erode_mask, e.erode_side, e.erode_limit, e.spec.erosion_probability,
+                              e.spec.erosion_seed);
         }
-        launch_isolated_cells(one, e.erode_out, e.d.V);
-        VF_HIP(hipMemcpyAsync(e.d.labels, e.erode_out, e.d.V * 2, hipMemcpyDeviceToDevice, s));
+        launch_isolated_cells(one, e.erode_bits);
     }
 }
 

@@ -36,7 +36,7 @@ struct EJob {
     int vstatus = 0;                 // job_validate's status when the job was prepared
     bool sub_done = false;           // the flood's sub-seed pass has run (served form)
     bool fronted = false;            // the front stage is queued: nearSeeds' counts are in fctl
-    uint16_t* erode_out = nullptr;   // erosion output grid and window (jobs with erode set)
+    uint8_t* erode_bits = nullptr;   // cells an erosion step empties, and its window (jobs with erode set)
     uint8_t* erode_mask = nullptr;
     uint32_t erode_side = 0;
     float erode_limit = 0;

@@ -18,7 +18,7 @@ struct vf_grid {
     vf::DevBuf vox_setup, vox_counts, vox_shell_off, scan_tmp, occ_tmp;
     vf::DevBuf mesh_xyz, mesh_tri;
     vf::DevBuf seed_tile_cnt, seed_tile_off;
-    vf::DevBuf keys, buckets, fctl, flood_lists, flood_sub, near_in, near_out, erode_tmp, erode_mask;
+    vf::DevBuf keys, buckets, fctl, flood_lists, flood_sub, near_in, near_out, erode_bits, erode_mask;
     vf::DevBuf ri_a, ri_b, ri_cnt, ri_vis, ri_out;
     vf::McScratch mc;              // marching-cubes workspace and last result
 

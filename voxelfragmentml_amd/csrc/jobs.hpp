@@ -296,12 +296,13 @@ void launch_flood_seed(const Launch& L, const FloodRoundScratch& W);
 void launch_flood_rounds(const Launch& L, const FloodRoundScratch& W, uint32_t rounds, uint32_t blocks);
 void launch_flood_finish(const Launch& L);
 // erode.hip: RegularGrid::erode.  erosion_mask returns the odd window side (or -1) and fills
-// side^3 mask bytes and the active fraction; the stencils read L.jobs[0]'s labels.
+// side^3 mask bytes and the active fraction; the stencils change L.jobs[0]'s labels by way of erode_bytes() of bits.
 constexpr uint32_t kMaxErosionSide = 15;
 int erosion_mask(int type, uint32_t size, std::vector<uint8_t>& mask, float& activations);
-void launch_erode_step(const Launch& L, uint16_t* out, const uint8_t* mask, uint32_t side, float limit,
-                       float probability, uint64_t noise_seed, uint64_t V);
-void launch_isolated_cells(const Launch& L, uint16_t* out, uint64_t V);
+size_t erode_bytes(const uint32_t dims[3]);
+void launch_erode_step(const Launch& L, uint8_t* kill, const uint8_t* mask, uint32_t side, float limit, float probability,
+                       uint64_t noise_seed);
+void launch_isolated_cells(const Launch& L, uint8_t* kill);
 
 // Sub-seed pass after the first drain (jobs with a non-null sub): merge touching
 // same-fragment seed regions, keep each fragment's smallest-id component, and,
