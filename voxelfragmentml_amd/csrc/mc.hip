@@ -892,93 +892,136 @@ bool g_table_loaded = false;
 // finishLaplacianSmoothing-comp.glsl:18-30): a face adds each of its vertices,
 // scaled by 10^4 and truncated to int, to its other two vertices; a target
 // vertex then moves to mix(p, sum / count / 10^4, weight).  The sums are
-// gathered per vertex over a vertex -> triangle adjacency, in integers, so the
-// result does not depend on order.  A vertex is a boundary vertex when any of
-// its triangles is flagged.
+// gathered per vertex, in integers, so the result does not depend on order.  A
+// vertex is a boundary vertex when any of its triangles is flagged.
+//
+// Each corner of a triangle is an entry of its vertex: the triangle's two other vertices, by index.  A step reads, for a
+// vertex, its entries and the truncated positions of 16 bytes that they name; it changes its own float position in
+// place and writes the truncated one to the other of two buffers, which hold the same values for vertices that no
+// longer move.  Bound by the gathers (about 12 of 16 bytes a vertex, from L2).  Going from the vertex to its triangles,
+// to their vertices' indices, flags and float positions took 77 us a step for 8 grids with 1.1 M vertices in all; now 38, and 180 instead of 285 us to prepare.
 struct SmoothDev {
     uint32_t nv, nt, nl;
     const uint32_t* tri;                 // local indices
     const uint8_t* tri_flag;
     const unsigned long long* voff;      // per label
     const unsigned long long* toff;
-    uint32_t* tri_g;                     // 3 * nt global vertex indices
-    uint32_t* vflag;                     // nv
-    uint32_t* deg;                       // nv incidence counts, then fill cursors
+    uint32_t* corner;                    // 4 * nt: global vertex indices, the corners' places among their vertices' entries
+    uint32_t* info;                      // nv: boundary flag, then with the grid of the vertex << 1
+    uint32_t* deg;                       // nv entry counts
     const unsigned long long* adj_off;   // nv + 1
-    uint32_t* adj;                       // 3 * nt triangle ids
+    uint2* adj;                          // 3 * nt entries
     const uint32_t* label_base;          // njobs + 1: first segment of each grid
     uint32_t njobs;
     uint32_t* vjob;                      // nv: grid of each vertex
     const uint4* params;                 // per grid: non-boundary steps, boundary steps, their weights (float bits)
+    float* xyz;
 };
+constexpr uint32_t kNoVertex = 0x7FFFFFFFu;       // an entry's vertex that is the entry's own (a degenerate triangle)
+constexpr uint32_t kMixedTriangle = 0x80000000u;  // flag of an entry's first vertex: some vertex of the triangle is a boundary one
 
 __global__ void k_smooth_prep(SmoothDev D)
 {
-    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < D.nt; t += gridDim.x * blockDim.x) {
-        uint32_t lo = 0, hi = D.nl;  // label of triangle t: largest l with toff[l] <= t
+    for (uint32_t t0 = blockIdx.x * blockDim.x; t0 < D.nt; t0 += gridDim.x * blockDim.x) {
+        // label of triangle t: the largest l with toff[l] <= t, from the wave's first triangle's on
+        const uint32_t tw = (uint32_t)__builtin_amdgcn_readfirstlane((int)(t0 + threadIdx.x)), t = t0 + threadIdx.x;
+        if (t >= D.nt) break;
+        uint32_t lo = 0, hi = D.nl;
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
-            if (D.toff[mid] <= t) lo = mid; else hi = mid;
+            if (D.toff[mid] <= tw) lo = mid; else hi = mid;
         }
+        while (lo + 1 < D.nl && D.toff[lo + 1] <= t) ++lo;
         const uint32_t base = (uint32_t)D.voff[lo];
         const uint32_t job = find_seg_job(D.label_base, D.njobs, lo);
+        const bool flag = D.tri_flag[t] != 0;
+        uint32_t g[3], slots = 0;
+#pragma unroll
         for (int i = 0; i < 3; ++i) {
-            const uint32_t g = base + D.tri[3 * (size_t)t + i];
-            D.tri_g[3 * (size_t)t + i] = g;
-            D.vjob[g] = job;  // every triangle of a vertex belongs to the same grid
-            atomicAdd(D.deg + g, 1u);
-            if (D.tri_flag[t]) atomicOr(D.vflag + g, 1u);
+            g[i] = base + D.tri[3 * (size_t)t + i];
+            D.vjob[g[i]] = job;  // every triangle of a vertex belongs to the same grid
+            if (flag) D.info[g[i]] = 1u;
+            // at most 4 cubes of 5 triangles meet at a vertex
+            slots |= atomicAdd(D.deg + g[i], 1u) << (8 * i);
+        }
+        reinterpret_cast<uint4*>(D.corner)[t] = make_uint4(g[0], g[1], g[2], slots);
+    }
+}
+__global__ void k_smooth_fill(SmoothDev D)
+{
+    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < D.nt; t += gridDim.x * blockDim.x) {
+        const uint4 c = reinterpret_cast<const uint4*>(D.corner)[t];
+        const uint32_t g[3] = { c.x, c.y, c.z };
+        const uint32_t mixed = D.info[g[0]] | D.info[g[1]] | D.info[g[2]] ? kMixedTriangle : 0u;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const uint32_t a = g[(i + 1) % 3], b = g[(i + 2) % 3];
+            D.adj[D.adj_off[g[i]] + ((c.w >> (8 * i)) & 0xFFu)] =
+                make_uint2((a == g[i] ? kNoVertex : a) | mixed, b == g[i] ? kNoVertex : b);
         }
     }
 }
-
-__global__ void k_smooth_fill(SmoothDev D)
+// truncated positions into both buffers
+__device__ inline int4 truncated(float x, float y, float z)
 {
-    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < D.nt; t += gridDim.x * blockDim.x)
-        for (int i = 0; i < 3; ++i) {
-            const uint32_t g = D.tri_g[3 * (size_t)t + i];
-            const uint32_t slot = atomicAdd(D.deg + g, 1u);  // deg was reset to 0 after the scan
-            D.adj[D.adj_off[g] + slot] = t;
-        }
+    return make_int4((int32_t)(x * 10000.0f), (int32_t)(y * 10000.0f), (int32_t)(z * 10000.0f), 0);
 }
-
-// Step `it` of a pass: a vertex of the pass's class moves when its grid runs more than `it` steps of
-// that pass (pass 0: non-boundary vertices over faces of non-boundary vertices, pass 1: boundary
-// vertices over all faces), with its grid's weight; every other vertex keeps its position.
-__global__ void k_smooth_step(SmoothDev D, const float* src, float* dst, uint32_t target, int check, uint32_t it)
+__global__ void k_smooth_init(SmoothDev D, int4* a, int4* b)
 {
     for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < D.nv; v += gridDim.x * blockDim.x) {
-        const float* p = src + 3 * (size_t)v;
-        float* o = dst + 3 * (size_t)v;
-        float px = p[0], py = p[1], pz = p[2];
-        const uint4 prm = D.params[D.vjob[v]];
+        const float* p = D.xyz + 3 * (size_t)v;
+        const int4 q = truncated(p[0], p[1], p[2]);
+        a[v] = q;
+        b[v] = q;
+        D.info[v] |= D.vjob[v] << 1;
+    }
+}
+// Step `it` of the vertices whose boundary flag is `target`; inner: by triangles without boundary vertices only.
+__global__ __launch_bounds__(256) void k_smooth_step(SmoothDev D, const int4* src, int4* dst, uint32_t target, bool inner, uint32_t it)
+{
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < D.nv; v += gridDim.x * blockDim.x) {
+        const uint32_t info = D.info[v];
+        const uint4 prm = D.params[info >> 1];
         const uint32_t steps = target == 0 ? prm.x : prm.y;
         const float weight = __uint_as_float(target == 0 ? prm.z : prm.w);
-        if (D.vflag[v] == target && it < steps) {
-            int32_t sx = 0, sy = 0, sz = 0, cnt = 0;
-            for (unsigned long long e = D.adj_off[v]; e < D.adj_off[v + 1]; ++e) {
-                const uint32_t* f = D.tri_g + 3 * (size_t)D.adj[e];
-                if (check && !(D.vflag[f[0]] == target && D.vflag[f[1]] == target && D.vflag[f[2]] == target)) continue;
-                for (int i = 0; i < 3; ++i) {
-                    if (f[i] == v) continue;
-                    const float* q = src + 3 * (size_t)f[i];
-                    sx += (int32_t)(q[0] * 10000.0f);
-                    sy += (int32_t)(q[1] * 10000.0f);
-                    sz += (int32_t)(q[2] * 10000.0f);
-                    ++cnt;
-                }
-            }
-            if (cnt > 0) {
-                const float ax = (float)sx / (float)cnt / 10000.0f, ay = (float)sy / (float)cnt / 10000.0f,
-                            az = (float)sz / (float)cnt / 10000.0f;
-                px = px * (1.0f - weight) + ax * weight;
-                py = py * (1.0f - weight) + ay * weight;
-                pz = pz * (1.0f - weight) + az * weight;
-            }
+        if ((info & 1u) != target || it >= steps) {
+            // the last step that moved it left its place in src only
+            if (it == ((info & 1u) != target ? 0u : steps)) dst[v] = src[v];
+            continue;
         }
-        o[0] = px;
-        o[1] = py;
-        o[2] = pz;
+        int32_t sx = 0, sy = 0, sz = 0, cnt = 0;
+        auto add = [&](uint32_t id) {
+            if (id == kNoVertex) return;
+            const int4 q = src[id];
+            sx += q.x;
+            sy += q.y;
+            sz += q.z;
+            ++cnt;
+        };
+        const unsigned long long e0 = D.adj_off[v];
+        const uint32_t n = (uint32_t)(D.adj_off[v + 1] - e0);
+        const uint2* adj = D.adj + e0;
+#pragma unroll 4
+        for (uint32_t e = 0; e < n; ++e) {
+            const uint2 c = adj[e];
+            if (inner && (c.x & kMixedTriangle)) continue;
+            add(c.x & ~kMixedTriangle);
+            add(c.y);
+        }
+        if (cnt == 0) {
+            dst[v] = src[v];
+            continue;
+        }
+        float* p = D.xyz + 3 * (size_t)v;
+        const float ax = (float)sx / (float)cnt / 10000.0f, ay = (float)sy / (float)cnt / 10000.0f,
+                    az = (float)sz / (float)cnt / 10000.0f;
+        const float px = p[0] * (1.0f - weight) + ax * weight;
+        const float py = p[1] * (1.0f - weight) + ay * weight;
+        const float pz = p[2] * (1.0f - weight) + az * weight;
+        p[0] = px;
+        p[1] = py;
+        p[2] = pz;
+        dst[v] = truncated(px, py, pz);
     }
 }
 
@@ -991,7 +1034,7 @@ enum : int {
     kBJobs, kBLidx, kBUnitPre, kBBase, kBLabels, kBTot, kBUnit, kBTile, kBTileOff, kBScan, kBKeys0, kBKeys1, kBVals0,
     kBVals1, kBSort, kBCntT, kBCntV, kBTpre, kBVpre, kBSeg, kBFlag, kBXyz, kBTri, kBSegJob,
     // smoothing
-    kBSmTriG, kBSmFlag, kBSmAdjOff, kBSmTmp, kBSmAdj, kBSmScan, kBSmPrm, kBCount
+    kBSmFlag, kBSmAdjOff, kBSmTmp, kBSmAdj, kBSmScan, kBSmPrm, kBCount
 };
 static_assert(kBCount <= McScratch::kBuffers, "scratch slots");
 
@@ -1336,42 +1379,47 @@ void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32
     D.toff = D.voff + (W.nl + 1);
     D.label_base = B[kBBase].as<uint32_t>();
     D.njobs = njobs;
-    W.ensure(kBSmTriG, (size_t)W.nt * 12 + 64);
-    W.ensure(kBSmFlag, (size_t)W.nv * 12 + 64);  // vflag, deg, vjob
+    // (such a mesh, its pairs and these buffers would not fit 288 GB)
+    if (W.nv >= kNoVertex) fail(VF_ERR_OVERFLOW, "smoothing of 2^31 vertices or more");
+    W.ensure(kBSmTmp, std::max((size_t)W.nt * 16, (size_t)W.nv * 32) + 64);  // corners, then truncated positions, twice
+    W.ensure(kBSmFlag, (size_t)W.nv * 12 + 64);  // info, deg, vjob
     W.ensure(kBSmScan, scan_tmp_bytes(W.nv) + 64);
-    W.ensure(kBSmAdj, (size_t)W.nt * 12 + 64);
+    W.ensure(kBSmAdj, (size_t)W.nt * 24 + 64);
     W.ensure(kBSmAdjOff, ((size_t)W.nv + 1) * 8 + 64);
-    W.ensure(kBSmTmp, (size_t)W.nv * 12 + 64);  // ping-pong positions
     W.ensure(kBSmPrm, (size_t)njobs * sizeof(uint4) + 64);
     VF_HIP(hipMemcpyAsync(B[kBSmPrm].p, prm.data(), (size_t)njobs * sizeof(uint4), hipMemcpyHostToDevice, s));
     D.params = B[kBSmPrm].as<uint4>();
-    D.tri_g = B[kBSmTriG].as<uint32_t>();
-    D.vflag = B[kBSmFlag].as<uint32_t>();
-    D.deg = D.vflag + W.nv;
+    D.corner = B[kBSmTmp].as<uint32_t>();
+    D.info = B[kBSmFlag].as<uint32_t>();
+    D.deg = D.info + W.nv;
     D.vjob = D.deg + W.nv;
-    VF_HIP(hipMemsetAsync(D.vflag, 0, (size_t)W.nv * 8, s));
+    D.xyz = B[kBXyz].as<float>();
+    VF_HIP(hipMemsetAsync(D.info, 0, (size_t)W.nv * 12, s));
     const uint32_t gt = stride_blocks(W.nt, 256, 8192), gv = stride_blocks(W.nv, 256, 8192);
-    k_smooth_prep<<<gt, 256, 0, s>>>(D);
-    VF_CHECK_LAUNCH();
-    scan_exclusive_u32_to_u64(D.deg, B[kBSmAdjOff].as<unsigned long long>(), W.nv, B[kBSmScan].p, s);
-    VF_HIP(hipMemsetAsync(D.deg, 0, (size_t)W.nv * 4, s));
-    D.adj_off = B[kBSmAdjOff].as<unsigned long long>();
-    D.adj = B[kBSmAdj].as<uint32_t>();
-    k_smooth_fill<<<gt, 256, 0, s>>>(D);
-    VF_CHECK_LAUNCH();
-    float* a = B[kBXyz].as<float>();
-    float* b = B[kBSmTmp].as<float>();
-    auto pass = [&](uint32_t iters, uint32_t target, int check) {
+    int4* a = B[kBSmTmp].as<int4>();
+    int4* b = a + W.nv;
+    {
+        TimedLaunch tl("mc_smooth_prep", s);
+        k_smooth_prep<<<gt, 256, 0, s>>>(D);
+        VF_CHECK_LAUNCH();
+        scan_exclusive_u32_to_u64(D.deg, B[kBSmAdjOff].as<unsigned long long>(), W.nv, B[kBSmScan].p, s);
+        D.adj_off = B[kBSmAdjOff].as<unsigned long long>();
+        D.adj = B[kBSmAdj].as<uint2>();
+        k_smooth_fill<<<gt, 256, 0, s>>>(D);
+        VF_CHECK_LAUNCH();
+        k_smooth_init<<<gv, 256, 0, s>>>(D, a, b);
+        VF_CHECK_LAUNCH();
+    }
+    auto pass = [&](uint32_t iters, uint32_t target, bool inner) {
         for (uint32_t i = 0; i < iters; ++i) {
             TimedLaunch tl("mc_smooth", s);
-            k_smooth_step<<<gv, 256, 0, s>>>(D, a, b, target, check, i);
+            k_smooth_step<<<gv, 256, 0, s>>>(D, a, b, target, inner, i);
             VF_CHECK_LAUNCH();
             std::swap(a, b);
         }
     };
-    pass(max_nb, 0, 1);
-    pass(max_b, 1, 0);
-    if (a != B[kBXyz].as<float>()) VF_HIP(hipMemcpyAsync(B[kBXyz].p, a, (size_t)W.nv * 12, hipMemcpyDeviceToDevice, s));
+    pass(max_nb, 0, true);
+    pass(max_b, 1, false);
     VF_HIP(hipStreamSynchronize(s));
 }
 
