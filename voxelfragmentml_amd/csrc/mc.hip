@@ -418,35 +418,86 @@ __device__ inline uint32_t block_excl_scan_u32(uint32_t v, uint32_t* wsum, uint3
 // One block per grid: dense indices of its target labels, the values countValues reports (a nonzero
 // count; raw values above FREE are counted unmasked, so a flagged EMPTY or FREE cell makes 0 or 1 a
 // label too, as in the reference), or the one wanted.
-__global__ __launch_bounds__(kMcThreads) void k_mc_labels(McRun R)
+// One workgroup per grid; a wave takes 4096 consecutive labels in 16 steps of 64 x 4 and
+// places them by ballots.  Bound by the latency of the loads and of the steps (a thread that walked 256 labels by
+// itself, twice, took 117 us): 12 us for one grid as for eight.
+constexpr uint32_t kLabelThreads = 1024;
+__global__ __launch_bounds__(kLabelThreads) void k_mc_labels(McRun R)
 {
-    __shared__ uint32_t wsum[kMcThreads / 64];
-    __shared__ uint32_t first;
+    constexpr uint32_t kWaves = kLabelThreads / 64, kSteps = 65536 / kLabelThreads / 4;
+    __shared__ uint32_t wsum[kWaves], wmin[kWaves];
     McJob& J = R.jobs[blockIdx.x];
-    constexpr uint32_t kPer = 65536 / kMcThreads;
-    const uint32_t l0 = threadIdx.x * kPer;
-    if (threadIdx.x == 0) first = 65536u;
-    auto target = [&](uint32_t l) { return J.hist[l] != 0 && (J.want == VF_ALL_LABELS || J.want == l); };
-    uint32_t c = 0;
-    for (uint32_t i = 0; i < kPer; ++i) c += target(l0 + i) ? 1u : 0u;
-    uint32_t total;
-    uint32_t idx = block_excl_scan_u32(c, wsum, &total);
-    const bool ok = total <= kMcMaxLabels;
-    for (uint32_t i = 0; i < kPer; ++i) {
-        const uint32_t l = l0 + i;
-        uint16_t li = kMcNoLabel;
-        if (ok && target(l)) {
-            J.lindex[65536 + idx] = (uint16_t)l;
-            li = (uint16_t)idx++;
-            atomicMin(&first, l);
-        }
-        J.lindex[l] = li;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, l0 = wave * (65536 / kWaves) + lane * 4u;
+    const uint4* hist = reinterpret_cast<const uint4*>(J.hist);
+    const uint32_t want = J.want;
+    constexpr uint32_t kRun = 8;  // steps whose loads are issued together
+    uint64_t bits = 0;  // the lane's target labels, four a step
+#pragma unroll 1
+    for (uint32_t s0 = 0; s0 < kSteps; s0 += kRun) {
+        uint4 q[kRun];
+#pragma unroll
+        for (uint32_t r = 0; r < kRun; ++r) q[r] = hist[(l0 + (s0 + r) * 256u) / 4u];
+        uint32_t some = 0;
+#pragma unroll
+        for (uint32_t r = 0; r < kRun; ++r)
+            some |= (q[r].x ? 1u << (4u * r) : 0u) | (q[r].y ? 2u << (4u * r) : 0u) | (q[r].z ? 4u << (4u * r) : 0u) |
+                    (q[r].w ? 8u << (4u * r) : 0u);
+        bits |= (uint64_t)some << (4u * s0);
+    }
+    if (want != VF_ALL_LABELS) {
+        const uint32_t s = (want - l0) / 256u, k = (want - l0) % 256u;  // of no step of this lane: s or k too large
+        bits &= want >= l0 && s < kSteps && k < 4u ? 1ull << (4u * s + k) : 0ull;
+    }
+    uint32_t n = (uint32_t)__builtin_popcountll(bits), first = 65536u;
+    if (bits) {
+        const uint32_t b = (uint32_t)__builtin_ctzll(bits);
+        first = l0 + (b >> 2) * 256u + (b & 3u);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        first = min(first, (uint32_t)__shfl_xor((int)first, o, 64));
+        n += (uint32_t)__shfl_xor((int)n, o, 64);
+    }
+    if (lane == 0) {
+        wsum[wave] = n;
+        wmin[wave] = first;
     }
     __syncthreads();
+    uint32_t idx = 0, total = 0;
+    first = 65536u;
+#pragma unroll
+    for (uint32_t w = 0; w < kWaves; ++w) {
+        idx += w < wave ? wsum[w] : 0u;
+        total += wsum[w];
+        first = min(first, wmin[w]);
+    }
+    const bool ok = total <= kMcMaxLabels;
+#pragma unroll 1
+    for (uint32_t s = 0; s < kSteps; ++s) {
+        const uint32_t own = ok ? (uint32_t)(bits >> (4u * s)) & 15u : 0u;
+        uint32_t at = idx, step = 0;  // the lane's first place: after the targets of the lanes before it
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            const uint64_t b = __ballot((own >> k) & 1u);
+            at += (uint32_t)__builtin_popcountll(b & ((1ull << lane) - 1ull));
+            step += (uint32_t)__builtin_popcountll(b);
+        }
+        uint16_t li[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            li[k] = kMcNoLabel;
+            if ((own >> k) & 1u) {
+                J.lindex[65536 + at] = (uint16_t)(l0 + s * 256u + k);
+                li[k] = (uint16_t)at++;
+            }
+        }
+        reinterpret_cast<uint2*>(J.lindex)[(l0 + s * 256u) / 4u] =
+            make_uint2((uint32_t)li[0] | (uint32_t)li[1] << 16, (uint32_t)li[2] | (uint32_t)li[3] << 16);
+        idx += step;
+    }
     if (threadIdx.x == 0) {
         R.job_nl[blockIdx.x] = ok ? total : 0u;
         R.job_err[blockIdx.x] = ok ? 0u : 1u;
-        J.min_target = first;
+        J.min_target = ok ? first : 65536u;
     }
 }
 
@@ -1134,7 +1185,7 @@ void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n,
     R.unit_pairs = W.buf[kBUnit].as<uint8_t>();
     R.tile_pairs = W.buf[kBTile].as<uint32_t>();
     R.tile_off = W.buf[kBTileOff].as<unsigned long long>();
-    k_mc_labels<<<n, kMcThreads, 0, s>>>(R);
+    k_mc_labels<<<n, kLabelThreads, 0, s>>>(R);
     VF_CHECK_LAUNCH();
     k_mc_base<<<1, 1024, 0, s>>>(R);
     VF_CHECK_LAUNCH();
