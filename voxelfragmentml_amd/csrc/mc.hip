@@ -1305,7 +1305,8 @@ void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n,
         VF_CHECK_LAUNCH();
         {
             TimedLaunch tl("mc_emit", s);
-            k_mc_emit<<<stride_blocks(np, kEmitPairs, 16384), kEmitPairs, 0, s>>>(R);
+            // a workgroup on every XCD: xcd_tiles gives each its share
+            k_mc_emit<<<std::max(kMcXcds, stride_blocks(np, kEmitPairs, 16384)), kEmitPairs, 0, s>>>(R);
             VF_CHECK_LAUNCH();
         }
     }
