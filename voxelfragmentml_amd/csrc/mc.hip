@@ -20,10 +20,10 @@
 //                 counts above FREE) -> dense index, and one global segment
 //                 per (grid, label)
 //   k_mc_count   one thread per unit (8 consecutive points of a z column)
-//                 loads its columns; units that can have output are queued
-//                 in LDS and worked one lane per point: the (segment, point)
-//                 pairs with output, and their triangle and vertex counts;
-//                 uniform units cost five column loads
+//                 looks at its columns two cells at a time; units that can
+//                 have output are queued in LDS, loaded a unit per lane and
+//                 worked a point per lane: the (segment, point) pairs with
+//                 output, and their triangle and vertex counts
 //   scan         pair offsets per tile of units
 //   (one host synchronisation: totals size the outputs)
 //   k_mc_pairs   the pairs, in (grid, point) order, as (segment, point |
@@ -39,7 +39,7 @@
 #include <functional>
 #include <vector>
 
-#include <hipcub/hipcub.hpp>
+#include <rocprim/rocprim.hpp>
 
 #include "cellops.hpp"
 #include "grid.hpp"
@@ -73,7 +73,6 @@ struct McJob {
     uint32_t cz;               // units per z column
     uint32_t want;             // VF_ALL_LABELS or one label
     uint32_t min_target;       // smallest target label (65536 when none): units below it emit nothing
-    uint32_t vec;              // grid rows 16-byte aligned (2), 8-byte aligned (1) or neither (0)
     float inv_cz, inv_Ny;      // 1 / cz and 1 / Ny (small_div)
     float mn[3], cs[3];
 };
@@ -89,7 +88,7 @@ struct McRun {
     uint32_t* job_err;                      // njobs: more than kMcMaxLabels labels
     uint16_t* labels_all;                   // one label per segment
     unsigned long long* job_tot;            // njobs x 4: pairs, triangles, vertices
-    uint8_t* unit_pairs;                    // total_units
+    uint32_t* unit_pairs;                   // total_units: pairs of each of the unit's points, four bits a point
     uint32_t* tile_pairs;                   // tiles
     const unsigned long long* tile_off;     // tiles + 1
     uint32_t* keys;                         // pairs: segment
@@ -211,13 +210,52 @@ __device__ inline UnitOrigin unit_origin_after(const McJob& J, uint32_t px0, uin
 // Zeros that lanes off the fast path of load_unit read in place of a grid row (16-byte aligned at +8).
 __device__ __align__(16) const uint16_t c_mc_zero[32] = {};
 
-// Loads unit `local`'s columns into v; false when no point of the unit can have output: the unit is uniform
-// (outside the vessel, inside one fragment) or holds no target label.  Every lane issues all of its loads
-// before waiting on any (interior columns are contiguous grid rows, lattice z0 + k being grid z0 - 1 + k;
-// z0 is a multiple of 8, so with 16-byte aligned rows lattice z0 + 1 .. z0 + 8 are one 16-byte load, with
-// 8-byte aligned rows two); lanes whose columns touch the padding or the lattice end read zeros and then
-// take those columns value by value.
-__device__ inline bool load_unit(const McJob& J, UnitOrigin uo, uint16_t v[kMcCols])
+// Two cells of a 32-bit word.
+typedef uint16_t cells2 __attribute__((ext_vector_type(2)));
+__device__ inline uint32_t max2(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(cells2, a), __builtin_bit_cast(cells2, b)));
+}
+
+// Whether a unit can have output, from its cells two at a time: not when none of them is a target label or above, nor
+// when all are equal (outside the vessel, inside one fragment).  Units that touch the padding or a column's end
+// take cells near theirs in place of those beyond, and count as mixed: true may be wrong, false never is.
+__device__ inline bool unit_live(const McJob& J, UnitOrigin uo)
+{
+    const int px = (int)(uo.pxy & 0xFFFFu), py = (int)(uo.pxy >> 16), z0 = (int)uo.z0, nz = (int)J.nz;
+    if (J.min_target <= kFree || nz < 8) return true;
+    const int cx[5] = { px, px - 1, px, px - 1, px + 1 }, cy[5] = { py, py, py + 1, py + 1, py };
+    const int zb = min(z0, nz - 8), zh = min(max(z0 - 1, 0), nz - 1);  // lattice z0 + 1 .. z0 + 8 and z0
+    bool inner = z0 >= 1 && z0 + 8 <= nz;
+    uint4 q[5];
+    uint32_t h[5];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+        const bool in = cx[c] >= 1 && cy[c] >= 1 && cx[c] <= (int)J.Nx - 2 && cy[c] <= (int)J.Ny - 2;
+        inner &= in;
+        const uint16_t* row = J.grid + ((size_t)(cx[c] - 1) * J.ny + (size_t)(cy[c] - 1)) * J.nz;
+        q[c] = gload4_cells(in ? row + zb : c_mc_zero);
+        h[c] = gcast<const uint16_t>(in ? row + zh : c_mc_zero)[0];
+    }
+    uint32_t most = 0, mixed = 0;
+    const uint32_t first = h[0] | h[0] << 16;
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+        const uint32_t w[5] = { q[c].x, q[c].y, q[c].z, q[c].w, h[c] | h[c] << 16 };
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            most = max2(most, w[k] & 0x7FFF7FFFu);
+            mixed |= w[k] ^ first;
+        }
+    }
+    if (max(most & 0xFFFFu, most >> 16) < J.min_target) return false;
+    return !inner || (mixed & 0x7FFF7FFFu) != 0;
+}
+
+// Loads a unit's columns into v.  Every lane issues all of its loads before waiting on any (interior columns are
+// contiguous grid rows, lattice z0 + k being grid z0 - 1 + k); lanes whose columns touch the padding or the
+// lattice end read zeros and then take those columns value by value.
+__device__ inline void load_unit(const McJob& J, UnitOrigin uo, uint16_t v[kMcCols])
 {
     const int px = (int)(uo.pxy & 0xFFFFu), py = (int)(uo.pxy >> 16), z0 = (int)uo.z0;
     constexpr int K = kMcZ + 1;
@@ -231,50 +269,23 @@ __device__ inline bool load_unit(const McJob& J, UnitOrigin uo, uint16_t v[kMcCo
         row[c] = fast[c] ? J.grid + (((size_t)(cx[c] - 1) * J.ny + (size_t)(cy[c] - 1)) * J.nz + (size_t)(z0 - 1))
                          : c_mc_zero + 7;
     }
-    auto put = [&](int c, const uint32_t w[4]) {  // lattice z0 + 1 .. from four packed words
+    uint4 q[5];
+    uint16_t h[5];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+        h[c] = gcast<const uint16_t>(row[c])[0];
+        q[c] = gload4_cells(row[c] + 1);
+    }
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+        v[c * K] = h[c];
+        const uint32_t w[4] = { q[c].x, q[c].y, q[c].z, q[c].w };
         const int n = c < 4 ? K : (int)kMcZ;
 #pragma unroll
         for (int k = 1; k < n; ++k) v[c * K + k] = (uint16_t)(w[(k - 1) >> 1] >> (16 * ((k - 1) & 1)));
-    };
-    if (J.vec == 2) {
-        uint4 q[5];
-        uint16_t h[5];
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            h[c] = gcast<const uint16_t>(row[c])[0];
-            q[c] = gload4(row[c] + 1);
-        }
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            v[c * K] = h[c];
-            const uint32_t w[4] = { q[c].x, q[c].y, q[c].z, q[c].w };
-            put(c, w);
-        }
-    } else if (J.vec == 1) {
-        uint2 qa[5], qb[5];
-        uint16_t h[5];
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            h[c] = gcast<const uint16_t>(row[c])[0];
-            qa[c] = gload2(row[c] + 1);
-            qb[c] = gload2(row[c] + 5);
-        }
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            v[c * K] = h[c];
-            const uint32_t w[4] = { qa[c].x, qa[c].y, qb[c].x, qb[c].y };
-            put(c, w);
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            const VF_AS_GLOBAL uint16_t* r = gcast<const uint16_t>(row[c]);
-#pragma unroll
-            for (int k = 0; k < (c < 4 ? K : (int)kMcZ); ++k) v[c * K + k] = r[k];
-        }
     }
-    // the units at a column's ends and the columns at or beyond the padding (a few lanes of most tiles): the
-    // column's state once, then each value from its lattice z alone
+    // the units at a column's ends and the columns at or beyond the padding: the column's state once, then each value
+    // from its lattice z alone
 #pragma unroll
     for (int c = 0; c < 5; ++c)
         if (!fast[c]) {
@@ -291,16 +302,6 @@ __device__ inline bool load_unit(const McJob& J, UnitOrigin uo, uint16_t v[kMcCo
                 v[c * K + k] = x;
             }
         }
-    uint32_t lo = 0xFFFFu, hi = 0;
-#pragma unroll
-    for (uint32_t m = 0; m < kMcCols; ++m) {
-        const uint16_t x = mask15(v[m]);
-        if (x != kMcNoLabel) {
-            lo = min(lo, (uint32_t)x);
-            hi = max(hi, (uint32_t)x);
-        }
-    }
-    return !(hi < J.min_target || lo == hi);
 }
 
 // Point k of unit `local` from the unit's columns v: f(point index, masked corners, masked +x neighbour,
@@ -321,7 +322,7 @@ __device__ inline void unit_point(const McJob& J, UnitOrigin uo, const uint16_t*
     f(p, c, nbx, cube, A[k]);
 }
 
-// The 8 lanes of a point group (lanes 8g .. 8g + 7, one per point of a unit): sum, and exclusive prefix.
+// The 8 lanes of a point group (lanes 8g .. 8g + 7, one per point of a unit): sum; and the sum of eight four-bit counts.
 __device__ inline uint32_t group8_sum(uint32_t x)
 {
     x += __shfl_xor(x, 1, 8);
@@ -329,15 +330,9 @@ __device__ inline uint32_t group8_sum(uint32_t x)
     x += __shfl_xor(x, 4, 8);
     return x;
 }
-__device__ inline uint32_t group8_excl(uint32_t x, uint32_t k)
+__device__ inline uint32_t nibble_sum(uint32_t n)
 {
-    uint32_t inc = x;
-#pragma unroll
-    for (uint32_t o = 1; o < 8; o <<= 1) {
-        const uint32_t y = __shfl_up(inc, o, 8);
-        if (k >= o) inc += y;
-    }
-    return inc - x;
+    return (((n & 0x0F0F0F0Fu) + ((n >> 4) & 0x0F0F0F0Fu)) * 0x01010101u) >> 24;
 }
 
 __device__ inline uint32_t find_job_u64(const unsigned long long* prefix, uint32_t n, unsigned long long u)
@@ -536,11 +531,27 @@ __global__ __launch_bounds__(1024) void k_mc_base(McRun R)
 // per point, so a surface unit costs one pass of its 8 points in parallel and a uniform unit its loads only.
 struct McQueue {
     uint16_t v[kMcThreads * kMcCols];  // columns of the queued units
+    uint32_t pxy[kMcThreads];          // their lattice origins (z below 2^16: grids have at most 2048 cells a side)
+    uint16_t z0[kMcThreads];
     uint16_t unit[kMcThreads];         // their unit index within the tile
-    UnitOrigin org[kMcThreads];        // their lattice origins
-    uint32_t off[kMcThreads];          // k_mc_pairs: their first pair's offset within the tile
+    __device__ void put(uint32_t q, uint32_t u, UnitOrigin uo)
+    {
+        pxy[q] = uo.pxy;
+        z0[q] = (uint16_t)uo.z0;
+        unit[q] = (uint16_t)u;
+    }
+    __device__ UnitOrigin org(uint32_t q) const { return UnitOrigin{ pxy[q], z0[q] }; }
+};
+// k_mc_pairs (its workgroup fits a fifth of a CU's LDS)
+struct McPairQueue : McQueue {
+    uint16_t off[kMcThreads];          // a unit's first pair's offset within the tile
+    uint32_t pairs[kMcThreads];        // its points' pairs (McRun::unit_pairs)
+    uint16_t point[kMcThreads * kMcZ]; // points with output: queued unit * kMcZ + point of the unit
 };
 
+// Bound by instructions: of the units' tests and, for the live units' points, of point_labels.  Unpacking every unit's 44
+// cells to test them took 142 us for a 256^3 grid with 1.3 M triangles, now 100; k_mc_pairs, which found each point's
+// pairs a second time to place them and visited every point of a live unit, 100, now 74.
 // Pairs with output, their triangle and vertex counts, per unit.  A tile's sums go to its first unit's grid
 // through the block's running sums (a few tiles straddle two grids: their other grid's points add their own).
 // The grid of a tile's first unit, staged in LDS with the first kMcLdsLabels entries of its label index
@@ -570,6 +581,20 @@ __device__ inline void xcd_tiles(uint32_t tiles, uint32_t& t0, uint32_t& t1, uin
     t0 = (uint32_t)((unsigned long long)tiles * x / kMcXcds) + blockIdx.x / kMcXcds;
     t1 = (uint32_t)((unsigned long long)tiles * (x + 1) / kMcXcds);
     step = (gridDim.x - x + kMcXcds - 1) / kMcXcds;  // blocks of this XCD
+}
+
+// The columns of the queued units, a unit per lane of full waves (the units of a tile that can have output are few and
+// scattered; loading them where they were found kept whole waves busy with the values of a few lanes).
+template <class F>
+__device__ inline void load_queue(McQueue& Q, uint32_t nq, F&& job)
+{
+    if (threadIdx.x < nq) {
+        uint16_t v[kMcCols];
+        load_unit(job(threadIdx.x), Q.org(threadIdx.x), v);
+#pragma unroll
+        for (uint32_t m = 0; m < kMcCols; ++m) Q.v[threadIdx.x * kMcCols + m] = v[m];
+    }
+    __syncthreads();
 }
 
 // Grid j's descriptor: from LDS when the whole tile lies in the staged grid (one, block-uniform).
@@ -612,7 +637,6 @@ __global__ __launch_bounds__(kMcThreads) __attribute__((amdgpu_waves_per_eu(5)))
         const bool one = sp[j0 + 1] >= ubase + kMcThreads;
         stage_grid(G, R, j0, staged);
         bool live = false;
-        uint16_t v[kMcCols];
         UnitOrigin uo{};
         // a tile in one grid: its first unit's column once (scalar), each lane's origin from it
         uint32_t px0 = 0, py0 = 0, rz0 = 0;
@@ -629,7 +653,7 @@ __global__ __launch_bounds__(kMcThreads) __attribute__((amdgpu_waves_per_eu(5)))
             const uint32_t j = one ? j0 : find_job_u64(sp, R.njobs, u);
             const McJob J = job_of(G, R, one, j);
             uo = one ? unit_origin_after(J, px0, py0, rz0, threadIdx.x) : unit_origin(J, (uint32_t)(u - sp[j]));
-            live = load_unit(J, uo, v);
+            live = unit_live(J, uo);
         }
         uint32_t nq = 0;
         const uint32_t pos = block_excl_scan_u32(live ? 1u : 0u, wsum, &nq);
@@ -639,12 +663,13 @@ __global__ __launch_bounds__(kMcThreads) __attribute__((amdgpu_waves_per_eu(5)))
         }
         if (!live && u < R.total_units) R.unit_pairs[u] = 0;
         if (live) {
-#pragma unroll
-            for (uint32_t m = 0; m < kMcCols; ++m) Q.v[pos * kMcCols + m] = v[m];
-            Q.unit[pos] = (uint16_t)threadIdx.x;
-            Q.org[pos] = uo;
+            Q.put(pos, threadIdx.x, uo);
         }
         __syncthreads();
+        load_queue(Q, nq, [&](uint32_t q) {
+            const unsigned long long uq = ubase + Q.unit[q];
+            return job_of(G, R, one, one ? j0 : find_job_u64(sp, R.njobs, uq));
+        });
         uint32_t tp = 0, p0 = 0, t0 = 0, v0 = 0;
         for (uint32_t i = threadIdx.x; i < nq * kMcZ; i += kMcThreads) {  // whole 8-lane groups
             const uint32_t q = i / kMcZ, k = i % kMcZ;
@@ -653,15 +678,15 @@ __global__ __launch_bounds__(kMcThreads) __attribute__((amdgpu_waves_per_eu(5)))
             const bool mine = j == j0;
             const McJob J = job_of(G, R, one, j);
             uint32_t pc = 0, tc = 0, vc = 0;
-            unit_point(J, Q.org[q], Q.v + q * kMcCols, (int)k, [&](uint32_t, const uint16_t* c, uint16_t nbx, bool cube, uint16_t) {
+            unit_point(J, Q.org(q), Q.v + q * kMcCols, (int)k, [&](uint32_t, const uint16_t* c, uint16_t nbx, bool cube, uint16_t) {
                 point_labels(J, ntri, G.lx, mine, c, nbx, cube, [&](uint16_t, uint16_t, uint32_t nt, uint32_t nv, uint32_t, uint32_t) {
                     ++pc;
                     tc += nt;
                     vc += nv;
                 });
             });
-            const uint32_t up = group8_sum(pc);
-            if (k == 0) R.unit_pairs[uq] = (uint8_t)up;
+            const uint32_t up = group8_sum(pc << (4u * k));  // at most 9 a point
+            if (k == 0) R.unit_pairs[uq] = up;
             tp += pc;
             if (mine) {
                 p0 += pc;
@@ -690,12 +715,12 @@ __global__ __launch_bounds__(kMcThreads) __attribute__((amdgpu_waves_per_eu(5)))
 
 // The pairs of every unit, in unit order (points in z order, a point's labels in candidate order), from the
 // tile offsets and the per-unit counts.
-__global__ __launch_bounds__(kMcThreads) void k_mc_pairs(McRun R)
+__global__ __launch_bounds__(kMcThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_mc_pairs(McRun R)
 {
     extern __shared__ unsigned long long sp[];  // njobs + 1 unit prefixes
     __shared__ uint32_t wsum[kMcThreads / 64];
     __shared__ uint8_t ntri[256];
-    __shared__ McQueue Q;
+    __shared__ McPairQueue Q;
     __shared__ McStage G;
     for (uint32_t i = threadIdx.x; i <= R.njobs; i += blockDim.x) sp[i] = R.unit_prefix[i];
     ntri[threadIdx.x] = (uint8_t)(c_mc_tri[threadIdx.x] >> 60);
@@ -711,40 +736,34 @@ __global__ __launch_bounds__(kMcThreads) void k_mc_pairs(McRun R)
         stage_grid(G, R, j0, staged);
         const uint32_t n = u < R.total_units ? R.unit_pairs[u] : 0u;
         // one scan of both counts: pairs in the low 16 bits (at most 256 x 72), queued units in the high 16
-        uint32_t both = 0;
-        const uint32_t exb = block_excl_scan_u32(n | (n ? 0x10000u : 0u), wsum, &both);
+        uint32_t both = 0, npoints = 0;
+        const uint32_t exb = block_excl_scan_u32(nibble_sum(n) | (n ? 0x10000u : 0u), wsum, &both);
+        const uint32_t some = (n | n >> 1 | n >> 2 | n >> 3) & 0x11111111u;  // points with pairs
+        uint32_t at = block_excl_scan_u32((uint32_t)__popc(some), wsum, &npoints);
         const uint32_t ex = exb & 0xFFFFu, pos = exb >> 16, nq = both >> 16;
         if (n) {
             const uint32_t j = one ? j0 : find_job_u64(sp, R.njobs, u);
             const McJob J = job_of(G, R, one, j);
-            uint16_t v[kMcCols];
-            const UnitOrigin uo = unit_origin(J, (uint32_t)(u - sp[j]));
-            load_unit(J, uo, v);
-#pragma unroll
-            for (uint32_t m = 0; m < kMcCols; ++m) Q.v[pos * kMcCols + m] = v[m];
-            Q.unit[pos] = (uint16_t)threadIdx.x;
-            Q.org[pos] = uo;
-            Q.off[pos] = ex;
+            Q.put(pos, threadIdx.x, unit_origin(J, (uint32_t)(u - sp[j])));
+            Q.off[pos] = (uint16_t)ex;
+            Q.pairs[pos] = n;
+            for (uint32_t b = some; b; b &= b - 1u) Q.point[at++] = (uint16_t)(pos * kMcZ + ((uint32_t)__builtin_ctz(b) >> 2));
         }
         __syncthreads();
+        load_queue(Q, nq, [&](uint32_t q) {
+            const unsigned long long uq = ubase + Q.unit[q];
+            return job_of(G, R, one, one ? j0 : find_job_u64(sp, R.njobs, uq));
+        });
         const unsigned long long tile_off = R.tile_off[t];
-        for (uint32_t i = threadIdx.x; i < nq * kMcZ; i += kMcThreads) {  // whole 8-lane groups
-            const uint32_t q = i / kMcZ, k = i % kMcZ;
+        for (uint32_t i = threadIdx.x; i < npoints; i += kMcThreads) {
+            const uint32_t q = Q.point[i] / kMcZ, k = Q.point[i] % kMcZ;
             const unsigned long long uq = ubase + Q.unit[q];
             const uint32_t j = one ? j0 : find_job_u64(sp, R.njobs, uq);
             const bool mine = j == j0;
             const McJob J = job_of(G, R, one, j);
             const uint32_t base = R.label_base[j];
-            const UnitOrigin local = Q.org[q];
-            const uint16_t* v = Q.v + q * kMcCols;
-            uint32_t pc = 0;
-            unit_point(J, local, v, (int)k, [&](uint32_t, const uint16_t* c, uint16_t nbx, bool cube, uint16_t) {
-                point_labels(J, ntri, G.lx, mine, c, nbx, cube,
-                             [&](uint16_t, uint16_t, uint32_t, uint32_t, uint32_t, uint32_t) { ++pc; });
-            });
-            unsigned long long o = tile_off + Q.off[q] + group8_excl(pc, k);
-            if (pc == 0) continue;
-            unit_point(J, local, v, (int)k, [&](uint32_t p, const uint16_t* c, uint16_t nbx, bool cube, uint16_t raw) {
+            unsigned long long o = tile_off + Q.off[q] + nibble_sum(Q.pairs[q] & ((1u << (4u * k)) - 1u));
+            unit_point(J, Q.org(q), Q.v + q * kMcCols, (int)k, [&](uint32_t p, const uint16_t* c, uint16_t nbx, bool cube, uint16_t raw) {
                 const unsigned long long flag = (unsigned long long)((raw >> 15) & 1u) << 51;
                 point_labels(J, ntri, G.lx, mine, c, nbx, cube,
                              [&](uint16_t li, uint16_t, uint32_t nt, uint32_t nv, uint32_t conf, uint32_t vax) {
@@ -1113,6 +1132,17 @@ McScratch::~McScratch()
     for (auto& b : buf) b.release(*cache);
 }
 
+// Stable sort of the pairs by the low bits of their segment.  The library takes merges of log2(n) passes over the pairs
+// below 2^20 of them by itself, one or two digit passes from there on: the digit passes are faster from kMergeBelow on
+// (128^3 grid, 300 k triangles: 58 -> 31 us; 256^3, 1.3 M: 148 -> 37).
+constexpr size_t kMergeBelow = 1u << 14;
+hipError_t sort_pairs(void* tmp, size_t& bytes, const uint32_t* keys, uint32_t* skeys, const unsigned long long* vals,
+                      unsigned long long* svals, size_t n, int bits, hipStream_t s)
+{
+    using Config = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config, rocprim::default_config, kMergeBelow>;
+    return rocprim::radix_sort_pairs<Config>(tmp, bytes, keys, skeys, vals, svals, n, 0u, (unsigned)bits, s);
+}
+
 void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n, McJobResult* out,
                  const std::function<bool(size_t)>& reserve)
 {
@@ -1140,8 +1170,6 @@ void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n,
         if (P > 0xFFFFFFFFull) fail(VF_ERR_INVALID_ARG, "grid too large for marching cubes");
         if (J.Nx > 0xFFFFu || J.Ny > 0xFFFFu) fail(VF_ERR_INVALID_ARG, "marching cubes: x and y dims must stay below 65534");
         J.cz = (J.Nz + kMcZ - 1) / kMcZ;
-        const uintptr_t a = reinterpret_cast<uintptr_t>(q.grid);
-        J.vec = (a % 16 == 0 && J.nz % 8 == 0) ? 2u : (a % 8 == 0 && J.nz % 4 == 0) ? 1u : 0u;
         J.inv_cz = 1.0f / (float)J.cz;
         J.inv_Ny = 1.0f / (float)J.Ny;
         J.want = q.want;
@@ -1156,7 +1184,7 @@ void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n,
     if (tiles64 > 0xFFFFFFFFull) fail(VF_ERR_INVALID_ARG, "marching-cubes lattice too large");
     // the first phase's buffers: label indices, per-unit pair counts, per-tile offsets and their scan
     const size_t phase1 = (size_t)n * kLindexWords * 2 + n * sizeof(McJob) + (size_t)n * (8 + 12 + 32 + 2 * kMcMaxLabels) +
-                          units + tiles64 * 12 + scan_tmp_bytes(tiles64) + 10 * 320;
+                          units * 4 + tiles64 * 12 + scan_tmp_bytes(tiles64) + 10 * 320;
     if (reserve && !reserve(BlockCache::class_size(phase1) + phase1 / 8)) {
         refuse();
         return;
@@ -1170,7 +1198,7 @@ void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n,
     W.ensure(kBBase, (3 * (size_t)n + 1) * 4);
     W.ensure(kBTot, (size_t)n * 32);
     W.ensure(kBLabels, (size_t)n * kMcMaxLabels * 2);
-    W.ensure(kBUnit, units + 64);
+    W.ensure(kBUnit, units * 4 + 64);
     W.ensure(kBTile, (size_t)R.tiles * 4 + 64);
     W.ensure(kBTileOff, ((size_t)R.tiles + 1) * 8 + 64);
     VF_HIP(hipMemcpyAsync(W.buf[kBJobs].p, jobs.data(), n * sizeof(McJob), hipMemcpyHostToDevice, s));
@@ -1182,7 +1210,7 @@ void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n,
     R.job_err = R.job_nl + n;
     R.labels_all = W.buf[kBLabels].as<uint16_t>();
     R.job_tot = W.buf[kBTot].as<unsigned long long>();
-    R.unit_pairs = W.buf[kBUnit].as<uint8_t>();
+    R.unit_pairs = W.buf[kBUnit].as<uint32_t>();
     R.tile_pairs = W.buf[kBTile].as<uint32_t>();
     R.tile_off = W.buf[kBTileOff].as<unsigned long long>();
     k_mc_labels<<<n, kLabelThreads, 0, s>>>(R);
@@ -1225,10 +1253,7 @@ void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n,
         for (uint32_t g = base[j]; g < base[j + 1]; ++g) sjob[g] = j;
     if (reserve) {  // the second phase's buffers: pairs (double-buffered, counts, prefixes) and the meshes
         size_t sort_bytes = 0;
-        if (npairs)
-            VF_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, (uint32_t*)nullptr, (uint32_t*)nullptr,
-                                                      (unsigned long long*)nullptr, (unsigned long long*)nullptr,
-                                                      (int)npairs, 0, 32, s));
+        if (npairs) VF_HIP(sort_pairs(nullptr, sort_bytes, nullptr, nullptr, nullptr, nullptr, (size_t)npairs, 32, s));
         const size_t phase2 = (size_t)npairs * (4 + 4 + 8 + 8 + 4 + 4 + 8 + 8) + sort_bytes + scan_tmp_bytes(npairs) +
                               (size_t)NT * (12 + 1) + (size_t)NV * 12 + 3 * ((size_t)S + 1) * 8 + ((size_t)S + 1) * 4 +
                               13 * 320;
@@ -1276,14 +1301,13 @@ void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n,
         int bits = 1;
         while (bits < 32 && (1ull << bits) < (unsigned long long)S) ++bits;
         size_t sort_bytes = 0;
-        VF_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, R.keys, W.buf[kBKeys1].as<uint32_t>(), R.vals,
-                                                  W.buf[kBVals1].as<unsigned long long>(), (int)np, 0, bits, s));
+        VF_HIP(sort_pairs(nullptr, sort_bytes, R.keys, W.buf[kBKeys1].as<uint32_t>(), R.vals,
+                          W.buf[kBVals1].as<unsigned long long>(), np, bits, s));
         W.ensure(kBSort, sort_bytes + 64);
         {
             TimedLaunch tl("mc_sort", s);
-            VF_HIP(hipcub::DeviceRadixSort::SortPairs(W.buf[kBSort].p, sort_bytes, R.keys, W.buf[kBKeys1].as<uint32_t>(),
-                                                      R.vals, W.buf[kBVals1].as<unsigned long long>(), (int)np, 0, bits,
-                                                      s));
+            VF_HIP(sort_pairs(W.buf[kBSort].p, sort_bytes, R.keys, W.buf[kBKeys1].as<uint32_t>(), R.vals,
+                              W.buf[kBVals1].as<unsigned long long>(), np, bits, s));
         }
         R.skeys = W.buf[kBKeys1].as<uint32_t>();
         R.svals = W.buf[kBVals1].as<unsigned long long>();
