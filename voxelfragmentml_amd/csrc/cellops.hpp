@@ -211,8 +211,8 @@ __device__ inline void walk_tiles(const Launch& L, const uint32_t* prefix, uint3
 // f(J, j, first_local_tile, n) handles tiles first .. first + n - 1 (n <= N),
 // so a streaming stage can issue all its loads before using any of them.
 // leave(j) runs when the block is done with job j (as in walk_tiles).
-template <uint32_t N, class F, class G>
-__device__ inline void walk_tile_runs(const Launch& L, const uint32_t* prefix, uint32_t total, JobDev* sJ, F&& f, G&& leave)
+template <uint32_t N, class F>
+__device__ inline void walk_tile_runs(const Launch& L, const uint32_t* prefix, uint32_t total, JobDev* sJ, F&& f)
 {
     uint32_t tb, te;
     block_tile_range(total, tb, te);
@@ -222,7 +222,6 @@ __device__ inline void walk_tile_runs(const Launch& L, const uint32_t* prefix, u
     stage_job(sJ, L.jobs + j);
     for (uint32_t t = tb; t < te;) {
         if (t >= je) {
-            leave(j);
             do {
                 ++j;
                 jb = je;
@@ -234,13 +233,25 @@ __device__ inline void walk_tile_runs(const Launch& L, const uint32_t* prefix, u
         f(*sJ, j, t - jb, n);
         t += n;
     }
-    leave(j);
 }
 
-template <uint32_t N, class F>
-__device__ inline void walk_tile_runs(const Launch& L, const uint32_t* prefix, uint32_t total, JobDev* sJ, F&& f)
+// Runs of N consecutive tiles by workgroups that keep to one job (their per-job sums are flushed once, by leave(j)):
+// job j has prefix[j + 1] / per - prefix[j] / per + 1 workgroups (total / per + njobs in all), which take its runs in
+// turn, so each sees the job's full and empty regions alike.
+template <uint32_t N, class F, class G>
+__device__ inline void walk_job_runs(const Launch& L, const uint32_t* prefix, uint32_t total, uint32_t per, JobDev* sJ, F&& f,
+                                     G&& leave)
 {
-    walk_tile_runs<N>(L, prefix, total, sJ, f, [](uint32_t) {});
+    uint32_t lo = 0, hi = L.njobs;  // largest j whose first workgroup, prefix[j] / per + j, is not after this one
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (prefix[mid] / per + mid <= blockIdx.x) lo = mid; else hi = mid;
+    }
+    const uint32_t jb = prefix[lo], n = prefix[lo + 1] - jb, b0 = jb / per + lo, nb = (jb + n) / per + lo + 1 - b0;
+    if ((uint64_t)(blockIdx.x - b0) * N >= n) return;
+    stage_job(sJ, L.jobs + lo);
+    for (uint64_t t = (uint64_t)(blockIdx.x - b0) * N; t < n; t += (uint64_t)nb * N) f(*sJ, (uint32_t)t, min(N, n - (uint32_t)t));
+    leave(lo);
 }
 
 // Job prefixes kept in LDS by the stages that search them per tile (njobs <= 1024).

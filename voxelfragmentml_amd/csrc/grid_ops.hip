@@ -373,6 +373,12 @@ constexpr int kAZ = kBTZ + 4;
 // the z window is done in registers; 144 of the threads also do one segment
 // of the 36 halo rows.  Only the z-window max/min of the 100 rows goes
 // through LDS, for the 3x3 x/y window of each labelled cell.
+//
+// Bound by instructions: 20 to 30 % of the cells of the bricks with labels are labelled, in 30 to 40 % of the
+// segments, but those lie in most of the waves.  The windows, counts and checksum are therefore worked for the
+// segments that are not EMPTY, listed in LDS, by the first waves: 64 mixed grids 1.36 -> 0.94 ms, of which
+// the runs dealt over a whole job (full and empty regions of a grid made some workgroups several times slower than
+// others) and the look at a run's bricks by 4-byte occupancy words together made 1.28 -> 0.94.
 // lane-wise max of two packed u16 pairs
 __device__ inline uint32_t pk_max_u16(uint32_t a, uint32_t b)
 {
@@ -383,7 +389,7 @@ __device__ inline uint32_t pk_max_u16(uint32_t a, uint32_t b)
 __device__ inline uint32_t packed_self(uint32_t m) { return m | ((0xFFFFu - m) << 16); }
 
 template <bool TABLE, uint32_t RUN>
-__global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
+__global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L, uint32_t per)
 {
     // z-window max (low 16 bits) | 0xFFFF - min (high 16) over labelled cells (EMPTY / FREE contribute 0),
     // so one packed u16 max combines both halves; row = hx * kBHY + hy
@@ -391,6 +397,9 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
     __shared__ uint32_t bins[TABLE ? kTiledBins : 1];
     __shared__ JobDev sJ;
     __shared__ BlockSum csum_part;
+    __shared__ uint4 cells[256];  // a brick's segments that are not EMPTY, by wave
+    __shared__ uint8_t listed[256];
+    __shared__ uint32_t count[4];
     unsigned long long csum = 0;
     if (TABLE) {
         for (uint32_t i = threadIdx.x; i < kTiledBins; i += blockDim.x) bins[i] = 0;
@@ -434,7 +443,7 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
         for (int k = 0; k < 8; ++k) out[k] = pk_max_u16(pk_max_u16(p[k], p[k + 1]), p[k + 2]);
     };
     constexpr uint32_t kRun = RUN;  // bricks per step: their interior loads are issued together
-    walk_tile_runs<kRun>(L, L.bt_prefix, L.total_bricks, &sJ, [&](const JobDev& J, uint32_t, uint32_t first, uint32_t nrun) {
+    walk_job_runs<kRun>(L, L.bt_prefix, L.total_bricks, per, &sJ, [&](const JobDev& J, uint32_t first, uint32_t nrun) {
         if (!J.active || J.bsize > 1) return;
         const int nx = (int)J.nx, ny = (int)J.ny, nz = (int)J.nz;
         const uint32_t tz = ceil_div_d(J.nz, kBTZ), tyn = ceil_div_d(J.ny, kBTY);
@@ -444,12 +453,10 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
         auto load_row = [&](int gx, int gy, int zs, uint16_t w[10]) {
             const int cx = min(max(gx, 0), nx - 1), cy = min(max(gy, 0), ny - 1);
             const uint16_t* r = lab + ((size_t)cx * ny + cy) * nz;
-            // zs is a multiple of 8, so with nz a multiple of 4 the 8 cells start 8-byte aligned
-            if (zs + 8 <= nz && (nz & 3) == 0) {
-                const uint2 a = gload2(r + zs);
-                const uint2 q = gload2(r + zs + 4);
-                w[1] = (uint16_t)a.x; w[2] = (uint16_t)(a.x >> 16); w[3] = (uint16_t)a.y; w[4] = (uint16_t)(a.y >> 16);
-                w[5] = (uint16_t)q.x; w[6] = (uint16_t)(q.x >> 16); w[7] = (uint16_t)q.y; w[8] = (uint16_t)(q.y >> 16);
+            if (zs + 8 <= nz) {
+                const uint4 q = gload4_cells(r + zs);
+                w[1] = (uint16_t)q.x; w[2] = (uint16_t)(q.x >> 16); w[3] = (uint16_t)q.y; w[4] = (uint16_t)(q.y >> 16);
+                w[5] = (uint16_t)q.z; w[6] = (uint16_t)(q.z >> 16); w[7] = (uint16_t)q.w; w[8] = (uint16_t)(q.w >> 16);
                 w[0] = gcast<const uint16_t>(r)[max(zs - 1, 0)];  // clamped window: z = -1 reads z = 0
                 w[9] = gcast<const uint16_t>(r)[min(zs + 8, nz - 1)];
             } else {
@@ -467,20 +474,13 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
             gz = z0 + seg;
             nval = gx < nx && gy < ny ? max(0, min(8, nz - gz)) : 0;
         };
-        auto add_checksum = [&](const uint16_t v[8], int gx, int gy, int gz, int nval) {
-            if (TABLE)
-                if (nval && (v[0] | v[1] | v[2] | v[3] | v[4] | v[5] | v[6] | v[7])) {  // EMPTY cells add nothing
-                    const uint32_t c0 = (uint32_t)(((size_t)gx * ny + gy) * nz + gz);
-                    for (int k = 0; k < nval; ++k) csum += checksum_term(v[k], c0 + k);
-                }
-        };
         // the 8 in-grid cells of a segment as packed pairs (cells beyond the grid read 0)
         auto load_seg = [&](int gx, int gy, int gz, int nval, uint32_t p[4]) {
             p[0] = p[1] = p[2] = p[3] = 0u;
             const uint16_t* r = lab + ((size_t)(nval ? gx : 0) * ny + (nval ? gy : 0)) * nz + gz;
-            if (nval == 8 && (nz & 3) == 0) {
-                const uint2 a = gload2(r), q = gload2(r + 4);
-                p[0] = a.x; p[1] = a.y; p[2] = q.x; p[3] = q.y;
+            if (nval == 8) {
+                const uint4 q = gload4_cells(r);
+                p[0] = q.x; p[1] = q.y; p[2] = q.z; p[3] = q.w;
             } else {
 #pragma unroll
                 for (int k = 0; k < 8; ++k)
@@ -493,16 +493,23 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
         if constexpr (TABLE) {
             // a table's labels are not EMPTY only where the occupancy is set, and a brick's rows are one occupancy
             // word each: 4 bytes a row instead of its 64 bytes of labels; bricks without a bit add nothing
-            uint32_t occ[kRun];
+            // (lane l of a wave looks at brick l % kRun)
+            constexpr uint32_t kRows = kRun < 4 ? 1 : kRun / 4;
+            const uint32_t r = threadIdx.x % kRun, row0 = threadIdx.x / kRun * kRows;
+            uint32_t occ = 0;
+            if (r < nrun && row0 < kBTX * kBTY) {
+                const uint32_t id = first + r, xy = id / tz, bx = xy / tyn, z = id - xy * tz;
+                const uint32_t gx0 = bx * kBTX, gy0 = (xy - bx * tyn) * kBTY;
 #pragma unroll
-            for (uint32_t r = 0; r < kRun; ++r) {
-                int x0, y0, z0, gx, gy, gz, nval;
-                segment(first + r, x0, y0, z0, gx, gy, gz, nval);
-                occ[r] = r < nrun && gx < nx && gy < ny
-                             ? gcast<const uint32_t>(J.occ)[((size_t)gx * ny + gy) * J.wp + (uint32_t)z0 / 32u] : 0u;
+                for (uint32_t k = 0; k < kRows; ++k) {
+                    const uint32_t gx = gx0 + (row0 + k) / kBTY, gy = gy0 + (row0 + k) % kBTY;
+                    if (gx < J.nx && gy < J.ny) occ |= gcast<const uint32_t>(J.occ)[((size_t)gx * J.ny + gy) * J.wp + z];
+                }
             }
+            uint64_t m = __ballot(occ != 0u);
 #pragma unroll
-            for (uint32_t r = 0; r < kRun; ++r) live |= occ[r] ? 1u << r : 0u;
+            for (uint32_t o = 32; o >= kRun; o >>= 1) m |= m >> o;
+            live = (uint32_t)m & ((1u << kRun) - 1u);
             live = (uint32_t)__ockl_wgred_or_i32((int)live);  // block-uniform: bit r = brick r holds an occupied cell
         } else {
             uint32_t pr[kRun][4];
@@ -529,81 +536,99 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L)
             segment(first + r, x0, y0, z0, gx, gy, gz, nval);
             uint16_t w[10];
             load_row(gx, gy, gz, w);  // the segment again (a cache hit) with its z neighbours
-            uint16_t v[8];
+            uint32_t own[4];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = k < nval ? w[k + 1] : (uint16_t)0;
-            if (TABLE) {
-                // run-length over the 8 cells: one LDS atomic per run of equal labels
-                uint32_t cur = 0, run = 0;
-                for (int k = 0; k < 8; ++k) {
-                    const uint32_t m = v[k] > kFree ? (uint32_t)(v[k] & kMask15) : 0xFFFFFFFFu;
-                    if (m != cur && run) {
-                        if (cur < kTiledBins) atomicAdd(&bins[cur], run);
-                        else atomicAdd(J.hist + cur, run);
-                        run = 0;
-                    }
-                    if (m != 0xFFFFFFFFu) {
-                        cur = m;
-                        ++run;
-                    }
-                }
-                if (run) {
-                    if (cur < kTiledBins) atomicAdd(&bins[cur], run);
-                    else atomicAdd(J.hist + cur, run);
-                }
+            for (int k = 0; k < 4; ++k)
+                own[k] = (2 * k < nval ? (uint32_t)w[2 * k + 1] : 0u) | (2 * k + 1 < nval ? (uint32_t)w[2 * k + 2] << 16 : 0u);
+            // list the segments with cells that are not EMPTY, a wave's after one another
+            const bool some = (own[0] | own[1] | own[2] | own[3]) != 0u;
+            const uint64_t mask = __ballot(some);
+            if (some) {
+                const uint32_t at = (threadIdx.x & ~63u) + (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+                listed[at] = (uint8_t)threadIdx.x;
+                cells[at] = make_uint4(own[0], own[1], own[2], own[3]);
             }
-            if (!bound) {
-                add_checksum(v, gx, gy, gz, nval);
-                continue;
-            }
-            {
+            if ((threadIdx.x & 63u) == 0) count[threadIdx.x >> 6] = (uint32_t)__builtin_popcountll(mask);
+            if (bound) {
                 uint32_t zw[8];
                 zwin(w, zw);
                 uint4* dst = reinterpret_cast<uint4*>(zmm + ((tx + 1) * kBHY + ty + 1) * kAZ + seg);
                 dst[0] = make_uint4(zw[0], zw[1], zw[2], zw[3]);
                 dst[1] = make_uint4(zw[4], zw[5], zw[6], zw[7]);
-            }
-            if (halo_task) {
-                uint16_t hw[10];
-                load_row(x0 + hhx - 1, y0 + hhy - 1, z0 + seg, hw);
-                uint32_t zw[8];
-                zwin(hw, zw);
-                uint4* dst = reinterpret_cast<uint4*>(zmm + (hhx * kBHY + hhy) * kAZ + seg);
-                dst[0] = make_uint4(zw[0], zw[1], zw[2], zw[3]);
-                dst[1] = make_uint4(zw[4], zw[5], zw[6], zw[7]);
+                if (halo_task) {
+                    uint16_t hw[10];
+                    load_row(x0 + hhx - 1, y0 + hhy - 1, z0 + seg, hw);
+                    zwin(hw, zw);
+                    dst = reinterpret_cast<uint4*>(zmm + (hhx * kBHY + hhy) * kAZ + seg);
+                    dst[0] = make_uint4(zw[0], zw[1], zw[2], zw[3]);
+                    dst[1] = make_uint4(zw[4], zw[5], zw[6], zw[7]);
+                }
             }
             __syncthreads();
-            // x and y windows together: a labelled cell without the bit is interior iff the packed
-            // window (max | 0xFFFF - min) equals its own packed value; cells beyond the grid are 0
-            uint32_t accs[8] = { 0, 0, 0, 0, 0, 0, 0, 0 };
+            uint32_t at = threadIdx.x, wv = 0;  // the at-th listed segment: place `at` of wave wv's
+            while (wv < 4u && at >= count[wv]) at -= count[wv++];
+            if (wv < 4u) {
+                const uint32_t id = listed[64u * wv + at];
+                const uint4 q = cells[64u * wv + at];
+                const int r2 = (int)(id >> 2), zs = (int)(id & 3u) * 8, sx = r2 / kBTY, sy = r2 % kBTY;
+                const uint32_t qw[4] = { q.x, q.y, q.z, q.w };
+                uint16_t v[8];
 #pragma unroll
-            for (int dx = 0; dx < 3; ++dx)
+                for (int k = 0; k < 8; ++k) v[k] = (uint16_t)(qw[k >> 1] >> (16 * (k & 1)));
+                if (TABLE) {
+                    // one LDS atomic per label of the segment
+                    uint32_t rest = 0;
 #pragma unroll
-                for (int dy = 0; dy < 3; ++dy) {
-                    const uint4* row = reinterpret_cast<const uint4*>(zmm + ((tx + dx) * kBHY + ty + dy) * kAZ + seg);
-                    const uint4 a = row[0], b = row[1];
-                    accs[0] = pk_max_u16(accs[0], a.x); accs[1] = pk_max_u16(accs[1], a.y);
-                    accs[2] = pk_max_u16(accs[2], a.z); accs[3] = pk_max_u16(accs[3], a.w);
-                    accs[4] = pk_max_u16(accs[4], b.x); accs[5] = pk_max_u16(accs[5], b.y);
-                    accs[6] = pk_max_u16(accs[6], b.z); accs[7] = pk_max_u16(accs[7], b.w);
+                    for (int k = 0; k < 8; ++k) rest |= v[k] > kFree ? 1u << k : 0u;
+                    while (rest) {
+                        uint32_t l = 0, eq = 0;  // the first cell still to count; the cells of its label
+#pragma unroll
+                        for (int k = 7; k >= 0; --k) l = (rest >> k) & 1u ? (uint32_t)(v[k] & kMask15) : l;
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) eq |= (v[k] & kMask15) == l ? 1u << k : 0u;
+                        eq &= rest;
+                        rest &= ~eq;
+                        if (l < kTiledBins) atomicAdd(&bins[l], (uint32_t)__popc(eq));
+                        else atomicAdd(J.hist + l, (uint32_t)__popc(eq));
+                    }
                 }
-            bool changed = false;
+                const int ax = x0 + sx, ay = y0 + sy, az = z0 + zs, n = min(8, nz - az);
+                bool changed = false;
+                if (bound) {
+                    // x and y windows together: a labelled cell without the bit is interior iff the packed
+                    // window (max | 0xFFFF - min) equals its own packed value; cells beyond the grid are 0
+                    uint32_t accs[8] = { 0, 0, 0, 0, 0, 0, 0, 0 };
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const uint32_t acc = accs[k];
-                const uint32_t c = v[k];
-                const bool bnd = c > kFree && (c & 0x8000u) == 0 && acc != packed_self(c);
-                v[k] = bnd ? (uint16_t)(c | 0x8000u) : (uint16_t)c;
-                changed |= bnd;
-            }
-            add_checksum(v, gx, gy, gz, nval);
-            if (changed) {
-                uint16_t* dst = J.labels + ((size_t)gx * ny + gy) * nz + gz;
-                if (nval == 8 && (nz & 3) == 0) {
-                    gstore2(dst, make_uint2((uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16)));
-                    gstore2(dst + 4, make_uint2((uint32_t)v[4] | ((uint32_t)v[5] << 16), (uint32_t)v[6] | ((uint32_t)v[7] << 16)));
-                } else {
-                    for (int k = 0; k < nval; ++k) dst[k] = v[k];
+                    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                        for (int dy = 0; dy < 3; ++dy) {
+                            const uint4* row = reinterpret_cast<const uint4*>(zmm + ((sx + dx) * kBHY + sy + dy) * kAZ + zs);
+                            const uint4 a = row[0], b = row[1];
+                            accs[0] = pk_max_u16(accs[0], a.x); accs[1] = pk_max_u16(accs[1], a.y);
+                            accs[2] = pk_max_u16(accs[2], a.z); accs[3] = pk_max_u16(accs[3], a.w);
+                            accs[4] = pk_max_u16(accs[4], b.x); accs[5] = pk_max_u16(accs[5], b.y);
+                            accs[6] = pk_max_u16(accs[6], b.z); accs[7] = pk_max_u16(accs[7], b.w);
+                        }
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const uint32_t c = v[k];
+                        const bool bnd = c > kFree && (c & 0x8000u) == 0 && accs[k] != packed_self(c);
+                        v[k] = bnd ? (uint16_t)(c | 0x8000u) : (uint16_t)c;
+                        changed |= bnd;
+                    }
+                }
+                if (TABLE) {
+                    const uint32_t c0 = (uint32_t)(((size_t)ax * ny + ay) * nz + az);
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) csum += checksum_term(v[k], c0 + k);  // EMPTY cells add nothing
+                }
+                if (changed) {
+                    uint16_t* dst = J.labels + ((size_t)ax * ny + ay) * nz + az;
+                    if (n == 8) {
+                        gstore4_cells(dst, pack_cells(v));
+                    } else {
+                        for (int k = 0; k < n; ++k) dst[k] = v[k];
+                    }
                 }
             }
             __syncthreads();
@@ -813,14 +838,18 @@ void launch_boundaries_tiled(const Launch& L, bool any_wide, bool table)
     {
         TimedLaunch tl("boundaries_hist", L.s);
         const LaunchShape sh = active_shape();
-        const uint32_t blocks = std::max(1u, std::min(L.total_bricks, sh.brick_blocks));
+        const uint32_t per = std::max(1u, L.total_bricks / std::max(1u, sh.brick_blocks));
+        const uint32_t blocks = L.total_bricks / per + L.njobs;
         auto go = [&](auto run) {
             constexpr uint32_t R = decltype(run)::value;
-            if (table) k_boundaries_tiled<true, R><<<blocks, 256, 0, L.s>>>(L);
-            else k_boundaries_tiled<false, R><<<blocks, 256, 0, L.s>>>(L);
+            if (table) k_boundaries_tiled<true, R><<<blocks, 256, 0, L.s>>>(L, per);
+            else k_boundaries_tiled<false, R><<<blocks, 256, 0, L.s>>>(L, per);
         };
-        if (sh.brick_run == 2) go(std::integral_constant<uint32_t, 2>{});
-        else if (sh.brick_run == 8) go(std::integral_constant<uint32_t, 8>{});
+        // long runs look at many bricks at once, but leave workgroups idle where there are few bricks: a 256^3 grid (8192)
+        // takes 26 us with runs of 4 and 30 with 8, a 512^3 grid (65536) 99 and 81, 64 mixed grids 1010 and 945
+        const uint32_t run = L.total_bricks < 32768u ? std::min(sh.brick_run, 4u) : sh.brick_run;
+        if (run == 2) go(std::integral_constant<uint32_t, 2>{});
+        else if (run == 8) go(std::integral_constant<uint32_t, 8>{});
         else go(std::integral_constant<uint32_t, 4>{});
         VF_CHECK_LAUNCH();
     }

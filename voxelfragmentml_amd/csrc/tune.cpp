@@ -27,10 +27,10 @@ std::mutex g_mu;
 // 10.95-10.98 at 4608, 11.02 at 3584, 11.30 at 5120).
 // Walker runs: 8 naive tiles, 4 boundary bricks.  Flood: chunks of 8 rounds, the first drain check after 3.
 LaunchShape g_shapes[kTuneBuckets] = {
-    { 8192, 4096, 8192, 16384, 8, 4, 8, 3, 2048 },
-    { 8192, 4096, 8192, 16384, 8, 4, 8, 3, 2048 },
-    { 8192, 4096, 8192, 16384, 8, 4, 8, 3, 2048 },
-    { 8192, 4096, 8192, 16384, 8, 4, 8, 3, 2048 },
+    { 8192, 4096, 8192, 16384, 8, 8, 8, 3, 2048 },
+    { 8192, 4096, 8192, 16384, 8, 8, 8, 3, 2048 },
+    { 8192, 4096, 8192, 16384, 8, 8, 8, 3, 2048 },
+    { 8192, 4096, 8192, 16384, 8, 8, 8, 3, 2048 },
 };
 uint64_t g_generation = 1;
 thread_local int t_bucket = kTuneBuckets - 1;
