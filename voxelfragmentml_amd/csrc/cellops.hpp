@@ -211,8 +211,8 @@ __device__ inline void walk_tiles(const Launch& L, const uint32_t* prefix, uint3
 // f(J, j, first_local_tile, n) handles tiles first .. first + n - 1 (n <= N),
 // so a streaming stage can issue all its loads before using any of them.
 // leave(j) runs when the block is done with job j (as in walk_tiles).
-template <uint32_t N, class F>
-__device__ inline void walk_tile_runs(const Launch& L, const uint32_t* prefix, uint32_t total, JobDev* sJ, F&& f)
+template <uint32_t N, class F, class G>
+__device__ inline void walk_tile_runs(const Launch& L, const uint32_t* prefix, uint32_t total, JobDev* sJ, F&& f, G&& leave)
 {
     uint32_t tb, te;
     block_tile_range(total, tb, te);
@@ -222,6 +222,7 @@ __device__ inline void walk_tile_runs(const Launch& L, const uint32_t* prefix, u
     stage_job(sJ, L.jobs + j);
     for (uint32_t t = tb; t < te;) {
         if (t >= je) {
+            leave(j);
             do {
                 ++j;
                 jb = je;
@@ -233,6 +234,13 @@ __device__ inline void walk_tile_runs(const Launch& L, const uint32_t* prefix, u
         f(*sJ, j, t - jb, n);
         t += n;
     }
+    leave(j);
+}
+
+template <uint32_t N, class F>
+__device__ inline void walk_tile_runs(const Launch& L, const uint32_t* prefix, uint32_t total, JobDev* sJ, F&& f)
+{
+    walk_tile_runs<N>(L, prefix, total, sJ, f, [](uint32_t) {});
 }
 
 // Runs of N consecutive tiles by workgroups that keep to one job (their per-job sums are flushed once, by leave(j)):
