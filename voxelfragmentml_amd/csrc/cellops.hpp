@@ -113,6 +113,30 @@ __device__ inline CellGroup cell_group(const JobDev& J, const BrickAt& b)
     return g;
 }
 __device__ inline CellGroup cell_group(const JobDev& J, uint32_t brick) { return cell_group(J, brick_at(J, brick)); }
+// Which of the n <= N bricks from brick `first` of job J on hold an occupied cell, as bits, the same for the whole workgroup
+// (of kCellThreads threads, all of which call this): a brick's rows are one occupancy word each, and lane l looks at rows of
+// brick first + l % N, so a run costs about as much as one brick by itself (which divides its index in every lane).
+template <uint32_t N>
+__device__ inline uint32_t live_bricks(const JobDev& J, uint32_t first, uint32_t n)
+{
+    static_assert((N & (N - 1)) == 0 && N <= 32, "lanes of a wave repeat the run");
+    constexpr uint32_t kRows = N < 4 ? 1 : N / 4, kColumns = kBrickX * kBrickY;
+    const uint32_t r = threadIdx.x % N, row0 = threadIdx.x / N * kRows;
+    uint32_t occ = 0;
+    if (r < n && row0 < kColumns) {
+        const BrickAt b = brick_at(J, first + r);
+#pragma unroll
+        for (uint32_t k = 0; k < kRows; ++k) {
+            const uint32_t x = b.x + (row0 + k) / kBrickY, y = b.y + (row0 + k) % kBrickY;
+            if (x < J.nx && y < J.ny) occ |= gcast<const uint32_t>(J.occ)[((size_t)x * J.ny + y) * J.wp + b.z / 32u];
+        }
+    }
+    uint64_t m = __ballot(occ != 0u);
+#pragma unroll
+    for (uint32_t o = 32; o >= N; o >>= 1) m |= m >> o;
+    const uint32_t mine = N < 32 ? (uint32_t)m & ((1u << (N & 31u)) - 1u) : (uint32_t)m;
+    return (uint32_t)__ockl_wgred_or_i32((int)mine);
+}
 // the group's byte of an array of occupancy words
 __device__ inline size_t group_byte(const JobDev& J, const CellGroup& g) { return (size_t)g.col * J.wp * 4u + (g.z0 >> 3); }
 // the group's occupancy bits (0 for a group without cells)

@@ -493,24 +493,7 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L, uint32_t per
         if constexpr (TABLE) {
             // a table's labels are not EMPTY only where the occupancy is set, and a brick's rows are one occupancy
             // word each: 4 bytes a row instead of its 64 bytes of labels; bricks without a bit add nothing
-            // (lane l of a wave looks at brick l % kRun)
-            constexpr uint32_t kRows = kRun < 4 ? 1 : kRun / 4;
-            const uint32_t r = threadIdx.x % kRun, row0 = threadIdx.x / kRun * kRows;
-            uint32_t occ = 0;
-            if (r < nrun && row0 < kBTX * kBTY) {
-                const uint32_t id = first + r, xy = id / tz, bx = xy / tyn, z = id - xy * tz;
-                const uint32_t gx0 = bx * kBTX, gy0 = (xy - bx * tyn) * kBTY;
-#pragma unroll
-                for (uint32_t k = 0; k < kRows; ++k) {
-                    const uint32_t gx = gx0 + (row0 + k) / kBTY, gy = gy0 + (row0 + k) % kBTY;
-                    if (gx < J.nx && gy < J.ny) occ |= gcast<const uint32_t>(J.occ)[((size_t)gx * J.ny + gy) * J.wp + z];
-                }
-            }
-            uint64_t m = __ballot(occ != 0u);
-#pragma unroll
-            for (uint32_t o = 32; o >= kRun; o >>= 1) m |= m >> o;
-            live = (uint32_t)m & ((1u << kRun) - 1u);
-            live = (uint32_t)__ockl_wgred_or_i32((int)live);  // block-uniform: bit r = brick r holds an occupied cell
+            live = live_bricks<kRun>(J, first, nrun);
         } else {
             uint32_t pr[kRun][4];
 #pragma unroll

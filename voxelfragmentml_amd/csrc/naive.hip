@@ -145,7 +145,8 @@ constexpr uint32_t kPruneSeeds = 16;
 // occupied group (launch_clear_labels has written the rest).  Bound by the latency of the block's barriers, so the
 // register budget is set for more waves in flight: 5 per SIMD with 32-bit keys, 4 with 64-bit keys.  RUN bricks form a walker run
 // whose occupancy loads are issued together (a launch shape the tuner picks).
-// 512^3, 128 seeds, Chebyshev: 442 us applying every seed in linear tiles, 83 us and 34 us of clearing now.
+// 512^3, 128 seeds, Chebyshev: 442 us applying every seed in linear tiles, 84 us by bricks and 34 us of clearing, 68 us
+// since a run's bricks are looked at by occupancy words together (live_bricks) instead of a byte a thread.
 template <typename K, uint32_t RUN>
 __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(sizeof(K) == 4 ? 5 : 4))) void k_naive(Launch L)
 {
@@ -219,13 +220,10 @@ __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(si
             stage(J, 0, S);
             staged = j;
         }
-        uint32_t occs[(kRun + 3) / 4] = {};  // a byte per brick of the run
-#pragma unroll
-        for (uint32_t r = 0; r < kRun; ++r)
-            occs[r / 4] |= (r < nrun ? group_occ(J, cell_group(J, first + r)) : 0u) << (8 * (r % 4));
-        auto brick = [&](uint32_t id, uint32_t occ) {
+        auto brick = [&](uint32_t id) {
         const BrickAt at = brick_at(J, id);
         const CellGroup grp = cell_group(J, at);
+        const uint32_t occ = group_occ(J, grp);
         // block-wide exclusive scan of the occupied counts -> compacted positions
         const uint32_t n = (uint32_t)__popc(occ);
         uint32_t inc = n;
@@ -309,19 +307,8 @@ __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(si
         __syncthreads();  // lab and cells are reused by the next brick
         };
         // the bricks of the run with an occupied cell; the others (most of a vessel's box) stay EMPTY
-        uint32_t any = 0;
-#pragma unroll
-        for (uint32_t r = 0; r < kRun; ++r) any |= ((occs[r / 4] >> (8 * (r % 4))) & 0xFFu) ? 1u << r : 0u;
-        any = (uint32_t)__ockl_wgred_or_i32((int)any);
 #pragma unroll 1
-        for (uint32_t r = 0; r < nrun; ++r) {
-            if (!((any >> r) & 1u)) continue;
-            uint32_t occ = occs[0];  // the run's byte r, its word by selects (a dynamic index would put occs in scratch)
-#pragma unroll
-            for (uint32_t i = 1; i < (kRun + 3) / 4; ++i) occ = r / 4 == i ? occs[i] : occ;
-            occ = (occ >> (8 * (r % 4))) & 0xFFu;
-            brick(first + r, occ);
-        }
+        for (uint32_t any = live_bricks<kRun>(J, first, nrun); any; any &= any - 1u) brick(first + (uint32_t)__builtin_ctz(any));
     });
 }
 
