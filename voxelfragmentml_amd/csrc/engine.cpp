@@ -661,8 +661,9 @@ void Engine::extract(const std::vector<EJob*>& js, const std::function<bool(size
         outs[i] = e.spec.mesh_out;
     }
     mc_run_jobs(mc_, s, spec.data(), n, res.data(), reserve);
-    if (mc_.valid && smooth) mc_smooth_jobs(mc_, s, sm.data(), n);
-    mc_read_jobs(mc_, s, res.data(), outs.data(), n);
+    // smoothing moves vertices only: triangles, flags and labels leave beside it
+    if (mc_.valid && smooth) mc_smooth_jobs(mc_, s, sm.data(), n, false);
+    mc_read_jobs(mc_, s, smooth ? side : s, res.data(), outs.data(), n);
     for (uint32_t i = 0; i < n; ++i) {
         vf_result& r = mj[i]->res;
         r.mc_vertices = res[i].nv;

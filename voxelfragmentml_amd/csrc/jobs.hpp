@@ -341,6 +341,7 @@ struct McScratch {
     uint32_t nv = 0, nt = 0, nl = 0;  // totals of the last run; nl counts (grid, label) segments
     bool valid = false;
     HostCopies to_host;
+    std::vector<uint4> smooth_params;  // of the last smoothing, until its copy is done
     std::vector<uint32_t> label_base;  // first segment of each grid of the last run, and the total
     void ensure(int slot, size_t n);
     void release_all();               // every buffer back to the cache (the result is dropped)
@@ -367,7 +368,8 @@ struct McJobResult {
 void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* jobs, uint32_t n, McJobResult* out,
                  const std::function<bool(size_t)>& reserve);
 // copies each grid's mesh of the last run to its vf_mesh_out (NULL entries skipped) when it fits
-void mc_read_jobs(McScratch& W, hipStream_t s, const McJobResult* res, vf_mesh_out* const* outs, uint32_t n);
+// fixed: a stream that does not wait for a smoothing still running on s (or s): all but the positions is copied on it
+void mc_read_jobs(McScratch& W, hipStream_t s, hipStream_t fixed, const McJobResult* res, vf_mesh_out* const* outs, uint32_t n);
 void mc_run(McScratch& W, hipStream_t s, const uint16_t* grid, const uint32_t dims[3], const float mn[3], const float cs[3],
             const uint32_t* hist_dev, uint32_t want, vf_mesh_info* info);
 void mc_read(McScratch& W, hipStream_t s, float* xyz, uint32_t* tri, uint8_t* tri_flag, uint16_t* labels, uint32_t* voff,
@@ -384,7 +386,8 @@ struct McSmooth {
     float b_weight;
 };
 void mc_smooth(McScratch& W, hipStream_t s, uint32_t nb_iters, float nb_weight, uint32_t b_iters, float b_weight);
-void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32_t njobs);
+// wait: until the positions are final
+void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32_t njobs, bool wait = true);
 
 // scan (scan.hip): exclusive prefix sums, graph-capturable, no host sync
 size_t scan_tmp_bytes(uint64_t n);

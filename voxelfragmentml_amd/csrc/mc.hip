@@ -1386,15 +1386,21 @@ void mc_read_range(McScratch& W, hipStream_t s, uint32_t seg0, uint32_t nseg, fl
     }
 }
 
-void mc_read_jobs(McScratch& W, hipStream_t s, const McJobResult* res, vf_mesh_out* const* outs, uint32_t n)
+void mc_read_jobs(McScratch& W, hipStream_t s, hipStream_t fixed, const McJobResult* res, vf_mesh_out* const* outs, uint32_t n)
 {
     if (!W.valid) return;
     auto& B = W.buf;
     std::vector<unsigned long long> seg(2 * ((size_t)W.nl + 1));
-    VF_HIP(hipMemcpyAsync(seg.data(), B[kBSeg].p, seg.size() * 8, hipMemcpyDeviceToHost, s));
-    VF_HIP(hipStreamSynchronize(s));
+    VF_HIP(hipMemcpyAsync(seg.data(), B[kBSeg].p, seg.size() * 8, hipMemcpyDeviceToHost, fixed));
+    VF_HIP(hipStreamSynchronize(fixed));
     const unsigned long long* vo = seg.data();
     const unsigned long long* to = seg.data() + W.nl + 1;
+    struct Positions {
+        float* to;
+        const float* from;
+        size_t bytes;
+    };
+    std::vector<Positions> moved;
     for (uint32_t j = 0; j < n; ++j) {
         vf_mesh_out* o = outs[j];
         if (!o) continue;
@@ -1406,7 +1412,7 @@ void mc_read_jobs(McScratch& W, hipStream_t s, const McJobResult* res, vf_mesh_o
         if (r.status != VF_OK || r.nv > o->cap_vertices || r.nt > o->cap_triangles || r.nl > o->cap_labels) continue;
         if ((r.nv && !o->xyz) || (r.nt && !o->tri)) continue;
         const unsigned long long v0 = vo[r.seg0], t0 = to[r.seg0];
-        W.to_host.add(o->xyz, B[kBXyz].as<float>() + 3 * v0, (size_t)r.nv * 12);
+        moved.push_back({ o->xyz, B[kBXyz].as<float>() + 3 * v0, (size_t)r.nv * 12 });
         W.to_host.add(o->tri, B[kBTri].as<uint32_t>() + 3 * t0, (size_t)r.nt * 12);
         if (o->tri_flag) W.to_host.add(o->tri_flag, B[kBFlag].as<uint8_t>() + t0, r.nt);
         if (o->labels) W.to_host.add(o->labels, B[kBLabels].as<uint16_t>() + r.seg0, (size_t)r.nl * 2);
@@ -1416,6 +1422,8 @@ void mc_read_jobs(McScratch& W, hipStream_t s, const McJobResult* res, vf_mesh_o
         }
         o->copied = 1;
     }
+    if (fixed != s) W.to_host.run(fixed);
+    for (const Positions& p : moved) W.to_host.add(p.to, p.from, p.bytes);
     W.to_host.run(s);
 }
 
@@ -1425,13 +1433,14 @@ void mc_read(McScratch& W, hipStream_t s, float* xyz, uint32_t* tri, uint8_t* tr
     mc_read_range(W, s, 0, W.nl, xyz, tri, tri_flag, labels, voff, toff);
 }
 
-void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32_t njobs)
+void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32_t njobs, bool wait)
 {
     if (!W.valid) fail(VF_ERR_INVALID_ARG, "no marching-cubes mesh to smooth");
     if (njobs + 1 != W.label_base.size()) fail(VF_ERR_INVALID_ARG, "smoothing parameters for %u grids, mesh of %zu", njobs,
                                                 W.label_base.size() - 1);
     uint32_t max_nb = 0, max_b = 0;
-    std::vector<uint4> prm(njobs);
+    std::vector<uint4>& prm = W.smooth_params;
+    prm.resize(njobs);
     for (uint32_t j = 0; j < njobs; ++j) {
         const McSmooth& q = per_job[j];
         if (!(q.nb_weight >= 0.0f && q.nb_weight <= 1.0f && q.b_weight >= 0.0f && q.b_weight <= 1.0f))
@@ -1496,7 +1505,7 @@ void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32
     };
     pass(max_nb, 0, true);
     pass(max_b, 1, false);
-    VF_HIP(hipStreamSynchronize(s));
+    if (wait) VF_HIP(hipStreamSynchronize(s));
 }
 
 void mc_smooth(McScratch& W, hipStream_t s, uint32_t nb_iters, float nb_weight, uint32_t b_iters, float b_weight)
