@@ -60,18 +60,26 @@ constexpr uint64_t halo_lanes(uint32_t c, uint32_t off, uint32_t n)
         if (halo_class(l + off) == c) m |= 1ull << l;
     return m;
 }
-constexpr uint64_t kHaloLanes1[9] = { halo_lanes(0, 0, 64), halo_lanes(1, 0, 64), halo_lanes(2, 0, 64),
-                                      halo_lanes(3, 0, 64), halo_lanes(4, 0, 64), halo_lanes(5, 0, 64),
-                                      halo_lanes(6, 0, 64), halo_lanes(7, 0, 64), halo_lanes(8, 0, 64) };
-constexpr uint64_t kHaloLanes2[9] = { halo_lanes(0, 64, 36), halo_lanes(1, 64, 36), halo_lanes(2, 64, 36),
-                                      halo_lanes(3, 64, 36), halo_lanes(4, 64, 36), halo_lanes(5, 64, 36),
-                                      halo_lanes(6, 64, 36), halo_lanes(7, 64, 36), halo_lanes(8, 64, 36) };
+// Positions off .. off + n - 1 of the halo plane whose row (y) or column (z) is of class 0 (below), 1 or 2 (above).
+constexpr uint64_t halo_rows(uint32_t c, uint32_t off, uint32_t n)
+{
+    return halo_lanes(3 * c, off, n) | halo_lanes(3 * c + 1, off, n) | halo_lanes(3 * c + 2, off, n);
+}
+constexpr uint64_t halo_columns(uint32_t c, uint32_t off, uint32_t n)
+{
+    return halo_lanes(c, off, n) | halo_lanes(3 + c, off, n) | halo_lanes(6 + c, off, n);
+}
+constexpr uint64_t kHaloRows1[3] = { halo_rows(0, 0, 64), halo_rows(1, 0, 64), halo_rows(2, 0, 64) },
+                   kHaloRows2[3] = { halo_rows(0, 64, 36), halo_rows(1, 64, 36), halo_rows(2, 64, 36) },
+                   kHaloColumns1[3] = { halo_columns(0, 0, 64), halo_columns(1, 0, 64), halo_columns(2, 0, 64) },
+                   kHaloColumns2[3] = { halo_columns(0, 64, 36), halo_columns(1, 64, 36), halo_columns(2, 64, 36) };
+__device__ inline uint64_t pick3(const uint64_t b[3], uint32_t i) { return i == 0u ? b[0] : i == 1u ? b[1] : b[2]; }
 constexpr uint32_t kTileWords = 10 * 10 * kRowWords;
-// 26-neighbour minima, separably: zt = z-window minima of the 100 halo-plane rows (8 per row),
-// yt = y-window minima of the 10 x-slabs' 8 rows; rows at an odd stride of 9 words.  yt reuses
-// the tile's words (the tile is read only while a visit starts).
+// 26-neighbour minima, separably: zt = z-window minima of the 36 halo rows (8 per row; rows 0..9 of x slab 0, of x slab 9,
+// then slabs 1..8 at y = 0 and at y = 9), yt = y-window minima of the 10 x-slabs' 8 rows; rows at an odd stride of 9
+// words.  yt reuses the tile's words (the tile is read only while a visit starts).
 constexpr uint32_t kSepStride = 9;
-constexpr uint32_t kZtWords = 100 * kSepStride;
+constexpr uint32_t kZtWords = 36 * kSepStride;
 constexpr uint32_t kYtWords = 80 * kSepStride;
 static_assert(kYtWords <= kTileWords, "yt reuses the tile");
 constexpr uint32_t kRelaxLdsWords = kTileWords + kZtWords;
@@ -274,7 +282,7 @@ __device__ inline uint32_t relax_brick(const RelaxJob& R, uint32_t brick, uint32
     const uint32_t bz = brick % R.nbz, t1 = brick / R.nbz, by = t1 % R.nby, bx = t1 / R.nby;
     const int X0 = (int)(bx * kRelaxBrick), Y0 = (int)(by * kRelaxBrick), Z0 = (int)(bz * kRelaxBrick);
 
-    uint32_t halo_live;  // 27 bits: halo classes holding a cell that is not EMPTY
+    uint64_t b1[3], b2[3];  // positions 0..63 and 64..99 of the halo plane that hold a cell that is not EMPTY, by x class
     // liveness of the brick and its 26 neighbours, bit ix * 9 + iy * 3 + iz (each 0: below, 1: the
     // brick's own range, 2: above), loaded with the halo.  Cells of a brick whose bit is clear (or
     // outside the grid) hold no keys and count as EMPTY.
@@ -315,13 +323,9 @@ __device__ inline uint32_t relax_brick(const RelaxJob& R, uint32_t brick, uint32
             bad1[ix] = in1 && ((nlive >> (ix * 9u + c1)) & 1u) ? 0u : kTileEmpty;
             bad2[ix] = in2 && ((nlive >> (ix * 9u + c2)) & 1u) ? 0u : kTileEmpty;
         }
-        // halo_live bit ix * 9 + iy * 3 + iz: a cell of that halo class (x, y, z each below the brick, beside
-        // it, above it) is not EMPTY; a neighbour brick in direction (ix, iy, iz) can only take a drop from
-        // this brick through those cells (EMPTY keys never change).  Per position and x class a ballot of
-        // "not all EMPTY" (across x slices 1..8 the AND of the keys is all ones iff all are EMPTY), then the
-        // lanes of each (y, z) class picked by constant masks.
+        // per position and x class a ballot of "not all EMPTY" (across x slices 1..8 the AND of the keys is all ones
+        // iff all are EMPTY)
         uint32_t m1 = ~0u, m2 = ~0u;
-        uint64_t b1[3], b2[3];
 #pragma unroll
         for (uint32_t hx = 0; hx < 10u; ++hx) {
             const uint32_t xbad = (uint32_t)(X0 + (int)hx - 1) < nx ? 0u : kTileEmpty;
@@ -339,13 +343,6 @@ __device__ inline uint32_t relax_brick(const RelaxJob& R, uint32_t brick, uint32
         }
         b1[1] = __ballot(m1 != ~0u);
         b2[1] = __ballot(m2 != ~0u);
-        uint32_t live = 0;
-#pragma unroll
-        for (uint32_t ix = 0; ix < 3u; ++ix)
-#pragma unroll
-            for (uint32_t c = 0; c < 9u; ++c)
-                if ((b1[ix] & kHaloLanes1[c]) | (b2[ix] & kHaloLanes2[c])) live |= 1u << (ix * 9u + c);
-        halo_live = live;
     }
     __syncthreads();
 
@@ -379,7 +376,7 @@ __device__ inline uint32_t relax_brick(const RelaxJob& R, uint32_t brick, uint32
     uint32_t hzlo = 0, hzhi = 0;  // the own row's halo keys at z = -1 and z = 8
     // 26 neighbours: the rows at y = 0 and y = 7 take their outer y neighbour from a halo row of zt (fixed
     // during the visit), the others from the neighbouring lane
-    const uint32_t hrow = ((x + 1u) * 10u + (y == 0u ? 0u : 9u)) * kSepStride;
+    const uint32_t hrow = ((y == 0u ? 20u : 28u) + x) * kSepStride;
     hzlo = tile[own] & ~3u;
     hzhi = tile[own + 9] & ~3u;
     // 6 neighbours: the halo row beside y = 0 or y = 7 in the tile (not rewritten during the visit)
@@ -395,16 +392,16 @@ __device__ inline uint32_t relax_brick(const RelaxJob& R, uint32_t brick, uint32
 #pragma unroll
             for (int o = 0; o < 10; ++o) r[o] = row[o];
 #pragma unroll
-            for (int z = 0; z < 8; ++z) zt[(hx * 10u + hy) * kSepStride + z] = min(min(r[z], r[z + 1]), r[z + 2]) & ~3u;
+            for (int z = 0; z < 8; ++z) zt[lane * kSepStride + z] = min(min(r[z], r[z + 1]), r[z + 2]) & ~3u;
         }
         __syncthreads();  // the tile is read for the last time above; yt may now overwrite it
         if (lane < 16u) {
-            const uint32_t sx = lane < 8u ? 0u : 9u, sy = lane & 7u;
+            const uint32_t sx = lane < 8u ? 0u : 9u, sy = lane & 7u, srow = lane < 8u ? 0u : 10u;
 #pragma unroll
             for (int z = 0; z < 8; ++z)
-                yt[(sx * 8u + sy) * kSepStride + z] = min(min(zt[(sx * 10u + sy) * kSepStride + z],
-                                                              zt[(sx * 10u + sy + 1u) * kSepStride + z]),
-                                                          zt[(sx * 10u + sy + 2u) * kSepStride + z]);
+                yt[(sx * 8u + sy) * kSepStride + z] = min(min(zt[(srow + sy) * kSepStride + z],
+                                                              zt[(srow + sy + 1u) * kSepStride + z]),
+                                                          zt[(srow + sy + 2u) * kSepStride + z]);
         }
     }
     uint32_t sweeps = 0;
@@ -506,38 +503,30 @@ __device__ inline uint32_t relax_brick(const RelaxJob& R, uint32_t brick, uint32
         }
     }
 
-    // neighbour bricks that see a dropped cell: bit (dx+1)*9 + (dy+1)*3 + (dz+1).  Lane x*8 + y holds row
+    // Neighbour bricks that see a dropped cell, one per lane: lane (dx+1)*9 + (dy+1)*3 + (dz+1).  Lane x*8 + y holds row
     // (x, y): a brick (dx, dy, dz) sees a dropped cell of a row with x = 0 (dx = -1) or 7 (dx = +1) or any
     // x (dx = 0), likewise for y, and a dropped end cell z = 0 (dz = -1) or 7 (dz = +1) or any cell
-    // (dz = 0); the 6-neighbour stencil sees faces only.  Built from three ballots with lane masks.
-    const uint64_t bzm[3] = { __ballot(changed && zlo), __ballot(changed), __ballot(changed && zhi) };
-    constexpr uint64_t kAll = ~0ull, kX0 = 0xFFull, kX7 = 0xFFull << 56, kY0 = 0x0101010101010101ull,
-                       kY7 = 0x8080808080808080ull;
-    const uint64_t mxs[3] = { kX0, kAll, kX7 }, mys[3] = { kY0, kAll, kY7 };
-    uint32_t dirs = 0;
-    if (R.n26) {
-#pragma unroll
-        for (uint32_t ix = 0; ix < 3; ++ix)
-#pragma unroll
-            for (uint32_t iy = 0; iy < 3; ++iy)
-#pragma unroll
-                for (uint32_t iz = 0; iz < 3; ++iz)
-                    if (ix * 9 + iy * 3 + iz != 13 && (bzm[iz] & mxs[ix] & mys[iy])) dirs |= 1u << (ix * 9 + iy * 3 + iz);
-    } else {
-        dirs = ((bzm[1] & kX0) ? 1u << 4 : 0u) | ((bzm[1] & kX7) ? 1u << 22 : 0u) | ((bzm[1] & kY0) ? 1u << 10 : 0u) |
-               ((bzm[1] & kY7) ? 1u << 16 : 0u) | (bzm[0] ? 1u << 12 : 0u) | (bzm[2] ? 1u << 14 : 0u);
-    }
-    dirs &= halo_live;  // a neighbour whose cells facing this brick are all EMPTY cannot take a drop from it
-    if (lane < 27u && (dirs & (1u << lane))) {
-        const int qx = (int)bx + (int)(lane / 9u) - 1, qy = (int)by + (int)((lane / 3u) % 3u) - 1,
-                  qz = (int)bz + (int)(lane % 3u) - 1;
-        if (qx >= 0 && qy >= 0 && qz >= 0 && (uint32_t)qx < R.nbx && (uint32_t)qy < R.nby && (uint32_t)qz < R.nbz)
-        {
-            const uint32_t id = ((uint32_t)qx * R.nby + (uint32_t)qy) * R.nbz + (uint32_t)qz;
-            R.nxt[id] = 1u;
+    // (dz = 0); the 6-neighbour stencil sees faces only.  And it can only take a drop from this brick through its halo
+    // cells of that direction (EMPTY keys never change): not where they are all EMPTY.
+    const uint64_t bz0 = __ballot(changed && zlo), bz1 = __ballot(changed), bz2 = __ballot(changed && zhi);
+    if (bz1 != 0ull) {
+        const uint32_t ix = lane / 9u, c = lane - ix * 9u, iy = c / 3u, iz = c - iy * 3u;
+        constexpr uint64_t kX0 = 0xFFull, kX7 = 0xFFull << 56, kY0 = 0x0101010101010101ull, kY7 = 0x8080808080808080ull;
+        const uint64_t rows = (ix == 0u ? kX0 : ix == 2u ? kX7 : ~0ull) & (iy == 0u ? kY0 : iy == 2u ? kY7 : ~0ull);
+        const uint64_t drops = (iz == 0u ? bz0 : iz == 2u ? bz2 : bz1) & rows;
+        const uint64_t halo = (pick3(b1, ix) & pick3(kHaloRows1, iy) & pick3(kHaloColumns1, iz)) |
+                              (pick3(b2, ix) & pick3(kHaloRows2, iy) & pick3(kHaloColumns2, iz));
+        const bool stencil = R.n26 ? lane != 13u : ((1u << 4 | 1u << 10 | 1u << 12 | 1u << 14 | 1u << 16 | 1u << 22) >> lane) & 1u;
+        const bool sees = lane < 27u && stencil && drops != 0ull && halo != 0ull;
+        if (sees) {
+            const int qx = (int)bx + (int)ix - 1, qy = (int)by + (int)iy - 1, qz = (int)bz + (int)iz - 1;
+            if (qx >= 0 && qy >= 0 && qz >= 0 && (uint32_t)qx < R.nbx && (uint32_t)qy < R.nby && (uint32_t)qz < R.nbz) {
+                const uint32_t id = ((uint32_t)qx * R.nby + (uint32_t)qy) * R.nbz + (uint32_t)qz;
+                R.nxt[id] = 1u;
+            }
         }
+        activated |= __ballot(sees) != 0ull;
     }
-    activated |= dirs != 0;
     __syncthreads();  // the tile is reused by the next brick
     return sweeps;
 }
@@ -737,6 +726,9 @@ __global__ __launch_bounds__(64) void k_flood_compact(Launch L, const uint32_t* 
 // visit's chain, and, before flags were bytes and the work counters spread, by same-address atomics at the
 // memory side.  Average of a flood's rounds: 256^3, 33 k visits, 20.3 -> 15.7 us; 512^3, 162 k visits, 34.5 ->
 // 23.8 us.
+// The neighbours to flag are found one per lane (27 + 27 scalar tests a visit before: 520 scalar instructions of a visit's
+// 1500), and the halo rows' minima take 1.3 KB of LDS instead of 3.6, so LDS no longer bounds the waves: 512^3, 26
+// neighbours 1.09 -> 1.05 ms.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_flood_relax(Launch L, const unsigned long long* lists, uint32_t list_cap,
                                                     const uint32_t* counts)
 {

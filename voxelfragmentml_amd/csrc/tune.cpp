@@ -22,15 +22,17 @@ namespace {
 std::mutex g_mu;
 // Defaults measured on MI355X with the mixed 64-job batch.  Cell kernels: 8192 workgroups of 4 waves
 // (8 waves per SIMD for the streaming kernels; 2048 left them at 2 and latency-bound).  Boundary
-// bricks: 16384.  Flood relaxation: 4096 one-wave workgroups (16 per CU), all resident at once, taking
-// short runs of their XCD's brick list round-robin (batch step on one box: 10.91-10.93 ms at 4096,
-// 10.95-10.98 at 4608, 11.02 at 3584, 11.30 at 5120).
-// Walker runs: 8 naive tiles, 4 boundary bricks.  Flood: chunks of 8 rounds, the first drain check after 3.
+// bricks: 16384.  Flood relaxation: one-wave workgroups, all resident at once, taking short runs of their XCD's brick
+// list round-robin: 4096 (16 per CU), and 5120 for edges above 256, whose lists are longer than that for most rounds
+// (relaxation of 64 mixed grids up to 384: 4.63 ms with 3072, 4.40 with 4096, 4.34 with 5120; a 256^3 flow is 1 %
+// slower with 5120).
+// Walker runs: 8 naive tiles, 8 boundary bricks (4 in tables of few bricks).  Flood: chunks of 8 rounds, the first drain
+// check after 3.
 LaunchShape g_shapes[kTuneBuckets] = {
     { 8192, 4096, 8192, 16384, 8, 8, 8, 3, 2048 },
     { 8192, 4096, 8192, 16384, 8, 8, 8, 3, 2048 },
     { 8192, 4096, 8192, 16384, 8, 8, 8, 3, 2048 },
-    { 8192, 4096, 8192, 16384, 8, 8, 8, 3, 2048 },
+    { 8192, 5120, 8192, 16384, 8, 8, 8, 3, 2048 },
 };
 uint64_t g_generation = 1;
 thread_local int t_bucket = kTuneBuckets - 1;
