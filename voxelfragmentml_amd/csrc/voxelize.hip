@@ -520,7 +520,7 @@ __device__ inline uint32_t wave_search(const unsigned long long* off, uint32_t n
     return lo + (63u - (uint32_t)__clzll((long long)m));
 }
 
-// A block takes chunks of kPairChunk consecutive pairs.  Two waves locate the chunk's first and last triangle, the
+// A block takes chunks of up to kPairChunk consecutive pairs.  Two waves locate the chunk's first and last triangle, the
 // block caches their offsets in LDS and each thread finds its triangle there.
 constexpr uint32_t kPairChunk = 4 * kVoxThreads;
 constexpr uint32_t kOffCache = 1024;
@@ -642,7 +642,7 @@ struct ShellWave {
 // instead of 33.7 M: 2.14 -> 1.82 ms there, 181 -> 136 us at 512^3 with a million triangles.
 // Parity: one lane per column of a triangle's column range.
 __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_vox_pairs(const JobDev* jobs, const TriSetup* setup,
-                                                           const unsigned long long* off, uint32_t ntris)
+                                                           const unsigned long long* off, uint32_t ntris, uint32_t chunk)
 {
     __shared__ uint32_t soff[kOffCache];
     __shared__ uint32_t sg[2];
@@ -652,11 +652,11 @@ __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))
     clear_table(W.table);
     // pairs [0, off[ntris]) are the shell's, [off[ntris], off[2 ntris]) the parity's
     const unsigned long long shell = off[ntris], total = off[2 * (size_t)ntris];
-    const unsigned long long ns = (shell + kPairChunk - 1) / kPairChunk, np = (total - shell + kPairChunk - 1) / kPairChunk;
+    const unsigned long long ns = (shell + chunk - 1) / chunk, np = (total - shell + chunk - 1) / chunk;
     for (unsigned long long c = blockIdx.x; c < ns + np; c += gridDim.x) {
         if (c < ns) {
-            const unsigned long long p0 = c * kPairChunk;
-            pair_chunk(off, ntris, p0, min(p0 + kPairChunk, shell), soff, sg, [&](uint32_t g, uint32_t col, bool valid) {
+            const unsigned long long p0 = c * chunk;
+            pair_chunk(off, ntris, p0, min(p0 + chunk, shell), soff, sg, [&](uint32_t g, uint32_t col, bool valid) {
                 const TriSetup Sg = load_setup(setup, ntris, g);
                 const TriSetup* S = &Sg;
                 const JobDev* J = jobs + (S->job & ~kWildTriangle);
@@ -718,8 +718,8 @@ __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))
                 combine_words<false>(W.table, J->shell_bits, (uint32_t)(((size_t)x * J->ny + (size_t)y) * J->wp + w), bits);
             });
         } else {
-            const unsigned long long p0 = shell + (c - ns) * kPairChunk;
-            pair_chunk(off + ntris, ntris, p0, min(p0 + kPairChunk, total), soff, sg, [&](uint32_t g, uint32_t local, bool valid) {
+            const unsigned long long p0 = shell + (c - ns) * chunk;
+            pair_chunk(off + ntris, ntris, p0, min(p0 + chunk, total), soff, sg, [&](uint32_t g, uint32_t local, bool valid) {
                 const TriSetup Sg = load_setup(setup, ntris, g);
                 const uint32_t nj = (uint32_t)(Sg.j1 - Sg.j0 + 1);
                 const JobDev* J = jobs + (Sg.job & ~kWildTriangle);
@@ -842,10 +842,13 @@ void launch_voxelize(const Launch& L, const VoxScratch& X, const uint32_t* col_p
         scan_exclusive_u32_to_u64(cnt_shell, X.shell_off, 2ull * X.total_tris, X.scan_tmp, L.s);
         // workgroups for as many pairs as a mesh of this size commonly leaves (a few surfaces across every column, a few
         // columns per triangle); more pairs take more steps
-        const uint32_t likely = ceil_div((uint64_t)total_groups * 256u * 4u + 8ull * X.total_tris, kPairChunk);
+        const uint64_t likely = (uint64_t)total_groups * 256u * 4u + 8ull * X.total_tris;
+        // few pairs: shorter chunks, so that no wave takes several steps while others have none (64^3 with 5 k triangles
+        // 22.6 -> 10.7 us, 128^3 with 20 k 30.8 -> 15.5; from 1024 chunks on the longer ones' one search for four steps pays)
+        const uint32_t chunk = (uint32_t)std::min<uint64_t>(kPairChunk, std::max<uint64_t>(1, likely / (1024u * kVoxThreads)) * kVoxThreads);
         TimedLaunch tl("vox_pairs", L.s);
-        k_vox_pairs<<<std::min(active_shape().pair_blocks, std::max(256u, likely)), kVoxThreads, 0, L.s>>>(L.jobs, X.setup,
-                                                                                                        X.shell_off, X.total_tris);
+        k_vox_pairs<<<std::min(active_shape().pair_blocks, std::max(256u, ceil_div(likely, chunk))), kVoxThreads, 0, L.s>>>(
+            L.jobs, X.setup, X.shell_off, X.total_tris, chunk);
         VF_CHECK_LAUNCH();
     }
     TimedLaunch tl("vox_fill", L.s);
