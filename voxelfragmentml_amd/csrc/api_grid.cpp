@@ -616,6 +616,7 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
         constexpr uint32_t kAhead = 6;
         volatile uint32_t* pr = g->pinned + kPinProgress;
         W.progress = g->pinned + kPinProgress;
+        W.job = &g->job;
         auto drain = [&]() -> uint32_t {
             pr[0] = pr[1] = pr[2] = 0;
             std::atomic_thread_fence(std::memory_order_seq_cst);

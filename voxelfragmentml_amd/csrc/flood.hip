@@ -531,6 +531,28 @@ __device__ inline uint32_t relax_brick(const RelaxJob& R, uint32_t brick, uint32
     return sweeps;
 }
 
+// The fields of a table's only job that rounds read, with the launch (keys null: read them from the table).
+struct RoundJob {
+    uint32_t nx, ny, nz, nb, b, n26;
+    uint32_t* keys;
+    uint32_t* ctl;
+    uint8_t* flags;
+    unsigned long long* sums;
+};
+__device__ inline void load_relax_fields(const JobDev* J, const RoundJob& A, RelaxJob& R)
+{
+    R.J = J;
+    R.nx = A.nx; R.ny = A.ny; R.nz = A.nz;
+    R.nbx = bdim(R.nx); R.nby = bdim(R.ny); R.nbz = bdim(R.nz);
+    R.nb = A.nb;
+    R.b = A.b;
+    R.keys = gcast<uint32_t>(A.keys);
+    R.ctl = gcast<uint32_t>(A.ctl);
+    R.flags = A.flags;
+    R.sums = A.sums;
+    R.nmask = gcast<const uint32_t>(reinterpret_cast<const uint32_t*>(live_base(R.flags, R.nb) + live_words(R.nbx, R.nby, R.nbz)));
+    R.n26 = A.n26 != 0u;
+}
 // The round-independent part of a flood job's relaxation state, in scalar registers, read in one batch of loads.
 __device__ inline void load_relax_fields(const JobDev* J, RelaxJob& R)
 {
@@ -593,12 +615,17 @@ __device__ inline uint32_t flood_job_active(const JobDev* J)
 // The loads come in two dependent batches: the job's fields, then its control words together with
 // both parities' flag group w (lane w of the task), of which *m receives the new round's bits.
 // progress (or null): host words told of it (FloodRoundScratch::progress).
-__device__ inline bool start_round(const Launch& L, uint32_t j, uint32_t i, uint32_t w, RelaxJob& R, uint64_t& m, uint32_t* progress)
+__device__ inline bool start_round(const Launch& L, const RoundJob& A, uint32_t j, uint32_t i, uint32_t w, RelaxJob& R, uint64_t& m,
+                                   uint32_t* progress)
 {
     const JobDev* J = L.jobs + j;
-    const uint32_t act = flood_job_active(J);
-    load_relax_fields(J, R);
-    if (!act) return false;
+    if (A.keys) {  // a running flood job
+        load_relax_fields(J, A, R);
+    } else {
+        const uint32_t act = flood_job_active(J);
+        load_relax_fields(J, R);
+        if (!act) return false;
+    }
     VF_AS_GLOBAL uint32_t* ctl = R.ctl;
     const uint32_t done = uni(ctl[1]), s0 = uni(ctl[4]), s1 = uni(ctl[5]), f0 = uni(ctl[2]), f1 = uni(ctl[3]);
     const uint32_t ng = relax_groups(R.nb), wc = min(w, ng - 1u);
@@ -648,13 +675,15 @@ __device__ inline bool start_round(const Launch& L, uint32_t j, uint32_t i, uint
 // i: the round's index in its chunk.
 __global__ __launch_bounds__(64) void k_flood_compact(Launch L, const uint32_t* prefix, uint32_t total_tasks,
                                                       unsigned long long* lists, uint32_t list_cap, uint32_t* counts,
-                                                      uint32_t* stale, uint32_t i, uint32_t* progress)
+                                                      uint32_t* stale, uint32_t i, uint32_t* progress, RoundJob A)
 {
     __shared__ uint32_t sp[kFloodMaxJobs + 1];
     const uint32_t lane = threadIdx.x;
     if (blockIdx.x == 0 && lane < kXcds) stale[lane] = 0u;
-    for (uint32_t i = lane; i <= L.njobs; i += 64u) sp[i] = prefix[i];
-    __syncthreads();
+    if (!A.keys) {
+        for (uint32_t i = lane; i <= L.njobs; i += 64u) sp[i] = prefix[i];
+        __syncthreads();
+    }
     const uint32_t xcd = blockIdx.x % kXcds, per_xcd = gridDim.x / kXcds, local = blockIdx.x / kXcds;
     if (local >= per_xcd) return;  // gridDim is a multiple of kXcds
     RelaxJob R{};
@@ -663,17 +692,20 @@ __global__ __launch_bounds__(64) void k_flood_compact(Launch L, const uint32_t* 
     for (uint32_t k = local;; k += per_xcd) {
         const uint32_t task = xcd + kXcds * k;
         if (task >= total_tasks) break;
-        uint32_t lo = 0, hi = L.njobs;  // job of the task: largest j with sp[j] <= task
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (sp[mid] <= task) lo = mid; else hi = mid;
+        uint32_t lo = 0, hi = L.njobs, t0 = 0;  // job of the task: largest j with sp[j] <= task
+        if (!A.keys) {
+            while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (sp[mid] <= task) lo = mid; else hi = mid;
+            }
+            t0 = sp[lo];
         }
         const uint32_t j = uni(lo);
-        const uint32_t w = (task - sp[j]) * 64u + lane;
+        const uint32_t w = (task - t0) * 64u + lane;
         uint64_t m = 0ull;
         if (j != cur_job) {
             cur_job = j;
-            running = start_round(L, j, i, w, R, m, progress);
+            running = start_round(L, A, j, i, w, R, m, progress);
         } else if (running) {
             m = w < relax_groups(R.nb) ? group_bits(load_group(parity_flags(R.flags, R.nb, R.par), w)) : 0ull;
         }
@@ -730,7 +762,7 @@ __global__ __launch_bounds__(64) void k_flood_compact(Launch L, const uint32_t* 
 // 1500), and the halo rows' minima take 1.3 KB of LDS instead of 3.6, so LDS no longer bounds the waves: 512^3, 26
 // neighbours 1.09 -> 1.05 ms.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_flood_relax(Launch L, const unsigned long long* lists, uint32_t list_cap,
-                                                    const uint32_t* counts)
+                                                    const uint32_t* counts, RoundJob A)
 {
     __shared__ uint32_t tile[kRelaxLdsWords];  // tile (yt reuses it), then zt
     const uint32_t lane = threadIdx.x;
@@ -746,7 +778,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
     uint32_t cur_job = 0xFFFFFFFFu;
     if (L.njobs == 1u) {
         cur_job = 0u;
-        load_relax_fields(L.jobs, R);
+        if (A.keys) load_relax_fields(L.jobs, A, R);
+        else load_relax_fields(L.jobs, R);
     }
     const uint32_t n = min(uni(cnt), list_cap);
     bool activated = false, error = false;
@@ -1231,16 +1264,22 @@ void launch_flood_rounds(const Launch& L, const FloodRoundScratch& W, uint32_t r
     const uint32_t cblocks = std::max(kXcds, std::min(blocks, (W.total_tasks + kXcds - 1) / kXcds * kXcds));
     unsigned long long* lists[2] = { W.lists, W.lists + (size_t)kXcds * W.list_cap };
     uint32_t* counts[2] = { W.counts, W.counts + kXcds };
+    // a round of a single grid is a chain of dependent loads in each launch: its job's fields save two of the compaction's
+    RoundJob A{};
+    if (W.job && L.njobs == 1 && W.job->active && W.job->algo == VF_FLOOD) {
+        const JobDev& J = *W.job;
+        A = RoundJob{ J.nx, J.ny, J.nz, J.nbricks, (uint32_t)J.key_bits, J.neighbourhood != 6 ? 1u : 0u, J.keys, J.fctl, J.bflags, J.sums };
+    }
     for (uint32_t i = 0; i < rounds; ++i) {
         const uint32_t p = i & 1u;  // round i lists into set p; set p ^ 1 (the previous round's) is cleared
         {
             TimedLaunch tl("flood_compact", L.s);
             k_flood_compact<<<cblocks, 64, 0, L.s>>>(L, W.task_prefix, W.total_tasks, lists[p], W.list_cap, counts[p],
-                                                     counts[p ^ 1u], i, W.progress);
+                                                     counts[p ^ 1u], i, W.progress, A);
             VF_CHECK_LAUNCH();
         }
         TimedLaunch tl("flood_relax", L.s);
-        k_flood_relax<<<blocks, 64, 0, L.s>>>(L, lists[p], W.list_cap, counts[p]);
+        k_flood_relax<<<blocks, 64, 0, L.s>>>(L, lists[p], W.list_cap, counts[p], A);
         VF_CHECK_LAUNCH();
     }
     if (W.progress) return;  // a compaction finds the drain and tells the host itself

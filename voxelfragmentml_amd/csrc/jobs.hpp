@@ -280,6 +280,7 @@ struct FloodRoundScratch {
     uint32_t* counts;              // 2 x kFloodXcds list lengths, zeroed with the seeds (a chunk leaves them zero)
     uint32_t* progress = nullptr;  // one job, or null: pinned host words that receive the last round started, the rounds
                                    // run once drained, and then the job's error flags
+    const JobDev* job = nullptr;  // host copy of the table's only job, where the caller has it: its fields go with the launches
 };
 constexpr uint32_t kFloodXcds = 8;
 uint32_t flood_list_cap(uint32_t total_tasks);  // entries per XCD list
