@@ -122,31 +122,70 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_down(const uint32_t* in, 
 
 // Up to kScanSmall items in one workgroup of 16 waves: three launches of a few blocks cost three launches' latency.
 constexpr uint32_t kSmallThreads = 1024, kScanSmall = kSmallThreads * kScanItems;
+// Rows of kSmallRow consecutive items, four a thread, so that loads and stores are whole lines (with 16 consecutive items a
+// thread, each of its stores touched a line of its own); every wave scans the waves' sums by itself.  14000 counts: 12.2 ->
+// 9.8 us, of which 6 are an empty launch's between two events.
+constexpr uint32_t kSmallRow = kSmallThreads * 4, kSmallRows = kScanSmall / kSmallRow;
+static_assert(kSmallRows * (kSmallThreads / 64) == 64, "a wave scans the waves' sums of all rows");
 __global__ __launch_bounds__(kSmallThreads) void k_scan_small(const uint32_t* in, uint32_t n, unsigned long long* out)
 {
-    __shared__ unsigned long long smem[kSmallThreads / 64];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, base = threadIdx.x * kScanItems;
-    uint32_t v[kScanItems];
-    load_items(in, base, n, vec_ok(in, in, base, n), v);
-    unsigned long long s = 0;
+    constexpr uint32_t kWaves = kSmallThreads / 64;
+    __shared__ unsigned long long smem[64];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, rows = (n + kSmallRow - 1) / kSmallRow;
+    const bool aligned = (((uintptr_t)in | (uintptr_t)out) & 15u) == 0;
+    if (threadIdx.x < 64u) smem[threadIdx.x] = 0ull;
+    uint4 v[kSmallRows];
 #pragma unroll
-    for (uint32_t k = 0; k < kScanItems; ++k) s += v[k];
-    unsigned long long x = s;
+    for (uint32_t r = 0; r < kSmallRows; ++r) {
+        const uint32_t b = r * kSmallRow + threadIdx.x * 4u;
+        v[r] = make_uint4(0u, 0u, 0u, 0u);
+        if (aligned && b + 4u <= n) {
+            v[r] = *reinterpret_cast<const uint4*>(in + b);
+        } else {
+            if (b < n) v[r].x = in[b];
+            if (b + 1u < n) v[r].y = in[b + 1u];
+            if (b + 2u < n) v[r].z = in[b + 2u];
+            if (b + 3u < n) v[r].w = in[b + 3u];
+        }
+    }
+    __syncthreads();
+    unsigned long long before[kSmallRows];  // in the wave's part of the row
+#pragma unroll
+    for (uint32_t r = 0; r < kSmallRows; ++r) {
+        before[r] = 0ull;
+        if (r >= rows) continue;  // uniform
+        const unsigned long long s = (unsigned long long)v[r].x + v[r].y + v[r].z + v[r].w;
+        unsigned long long x = s;
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned long long y = __shfl_up(x, o, 64);
+            if (lane >= (uint32_t)o) x += y;
+        }
+        if (lane == 63u) smem[r * kWaves + wave] = x;
+        before[r] = x - s;
+    }
+    __syncthreads();
+    const unsigned long long own = smem[lane];
+    unsigned long long x = own;
     for (int o = 1; o < 64; o <<= 1) {
         const unsigned long long y = __shfl_up(x, o, 64);
         if (lane >= (uint32_t)o) x += y;
     }
-    if (lane == 63u) smem[wave] = x;
-    __syncthreads();
-    unsigned long long e = x - s, total = 0;
-    for (uint32_t w = 0; w < kSmallThreads / 64; ++w) {
-        if (w < wave) e += smem[w];
-        total += smem[w];
-    }
+    const unsigned long long total = __shfl(x, 63, 64), first = x - own;
 #pragma unroll
-    for (uint32_t k = 0; k < kScanItems; ++k) {
-        if (base + k < n) out[base + k] = e;
-        e += v[k];
+    for (uint32_t r = 0; r < kSmallRows; ++r) {
+        if (r >= rows) continue;
+        const unsigned long long e0 = before[r] + __shfl(first, (int)(r * kWaves + wave), 64);
+        const unsigned long long e1 = e0 + v[r].x, e2 = e1 + v[r].y, e3 = e2 + v[r].z;
+        const uint32_t b = r * kSmallRow + threadIdx.x * 4u;
+        if (aligned && b + 4u <= n) {
+            reinterpret_cast<ulonglong2*>(out + b)[0] = make_ulonglong2(e0, e1);
+            reinterpret_cast<ulonglong2*>(out + b)[1] = make_ulonglong2(e2, e3);
+        } else {
+            if (b < n) out[b] = e0;
+            if (b + 1u < n) out[b + 1u] = e1;
+            if (b + 2u < n) out[b + 2u] = e2;
+            if (b + 3u < n) out[b + 3u] = e3;
+        }
     }
     if (threadIdx.x == 0) out[n] = total;
 }
