@@ -111,9 +111,10 @@ STAGES = {
     "voxelize": ["job_init", "vox_clear", "vox_setup", "scan", "vox_pairs", "vox_fill"],
     "seed": ["seed_count", "seed_pick"],
     "naive": ["naive", "naive64"],
-    "flood": ["flood_init", "flood_seed", "flood_compact", "flood_relax", "flood_plan", "flood_finish"],
+    # clear_labels writes the naive jobs' empty cells too
+    "flood": ["clear_labels", "flood_init", "flood_seed", "flood_compact", "flood_relax", "flood_plan", "flood_finish"],
     "boundaries+histogram": ["boundaries_hist", "hist_summary"],
-    "marching_cubes": ["mc_count", "mc_pairs", "mc_sort", "mc_emit", "mc_smooth"],
+    "marching_cubes": ["mc_count", "mc_pairs", "mc_sort", "mc_emit", "mc_smooth_prep", "mc_smooth"],
 }
 KERNELS = [k for ks in STAGES.values() for k in ks] + ["gather"]
 
@@ -224,9 +225,9 @@ def roofline(prof, specs, res, traffic_ok):
     if dom == "flood_relax":
         visits = sum(r["flood_bricks"] for r in res)
         out["limiter"] = ("latency of each visit's dependent chain (halo loads, then sweeps of LDS round trips) over "
-                          "dependent rounds: 13 of 18 waves per CU resident (4 x SQ_WAVE_CYCLES / SQ_BUSY_CYCLES per "
-                          "CU), waiting on results 42 % and on issue 30 % of their time (SQ_WAIT_ANY, SQ_WAIT_INST_ANY), "
-                          "VALU at 40 % of the rate the voxelizer sustains (SQ_INSTS_VALU); not HBM")
+                          "dependent rounds: 15 of 20 waves per CU resident (4 x SQ_WAVE_CYCLES / SQ_BUSY_CYCLES per "
+                          "CU), waiting on results 34 % and on issue 41 % of their time (SQ_WAIT_ANY, SQ_WAIT_INST_ANY), "
+                          "VALU at 58 % of the rate the voxelizer sustains (SQ_INSTS_VALU); not HBM")
         out["unit_work"] = {"brick_visits_per_step": visits, "visit_bytes_per_step": 4096 * visits,
                             "sweeps_per_step": sum(r["flood_sweeps"] for r in res),
                             "visit_gbs": round(4096 * visits / launches / (prof[dom]["avg_ms"] * 1e-3) / 1e9, 1)}
@@ -557,7 +558,7 @@ def main():
     out = {
         "metric": METRIC, "value": round(value, 4), "unit": "Gvoxels/s", "n_gpus": 1, "steps": a.steps,
         "warmup": a.warmup, "ms_per_step": round(ms_step, 3), "higher_is_better": True, "scaling": "weak",
-        "vs_baseline": None, "dtype": "u16 labels / u8 occupancy / int32 distances / fp32 SAT", "data": "synthetic",
+        "vs_baseline": None, "dtype": "u16 labels / 1-bit occupancy / int32 distances / fp32 SAT", "data": "synthetic",
         "config": {"workload": "mixed batch: 64 vessel jobs, edge U[64,384] (x4), 5k-300k triangles, 2-64 seeds, "
                                "distance uniform, naive/flood 50:50, flood noise 2, boundaries + histogram",
                    "jobs": len(specs), "voxels_per_step": voxels, "rng_seed": 4, "form": "batched (HIP graphs)"},

@@ -257,7 +257,7 @@ int vf_mesh_export_binm(vf_grid* g, uint32_t label_index, uint8_t* out, size_t c
  * relabels a grid; seeds, S and distance as for vf_fracture_naive (host
  * array); stream: a hipStream_t, or NULL for the default stream; the call
  * returns when the work on that stream has finished.  Everything beyond the
- * cells (the grid's occupancy bytes, the launch descriptor, the seeds) lives in
+ * cells (the grid's occupancy bits, the launch descriptor, the seeds) lives in
  * one static device array of VF_NOALLOC_SCRATCH_BYTES per GPU, held until the
  * process ends: grids of more than VF_NOALLOC_MAX_CELLS cells fail with
  * VF_ERR_INVALID_ARG.  Every call on a GPU shares that GPU's array, so calls
