@@ -55,6 +55,33 @@ def test_far_grid(vf):
         np.testing.assert_array_equal(g.read(), O.voxelize(xyz, tri, lo, hi, dims))
 
 
+@pytest.mark.parametrize("offset", [0.0, 1.0, 100.0, 1e4, 3e6])
+@pytest.mark.parametrize("dims", [(12, 18, 40), (40, 40, 33)])
+def test_grids_away_from_the_origin(vf, offset, dims):
+    # the further away, the coarser a cell's planes and offsets round, and the more cells lie too near an interval's end
+    print("offset", offset, dims, flush=True)
+    lo, hi = [offset - 1.0, 2 * offset - 1.0, 1.0 - offset], [offset + 1.0, 2 * offset + 1.0, 3.0 - offset]
+    xyz, tri = soup(int(offset) % 97 + dims[0], 250, 0.25)
+    xyz = (xyz + (np.array(lo) + np.array(hi)) / 2).astype(np.float32)
+    with vf.Grid(dims, lo, hi) as g:
+        g.voxelize(xyz, tri)
+        np.testing.assert_array_equal(g.read(), O.voxelize(xyz, tri, lo, hi, dims))
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_slivers_and_aligned_edges(vf, seed):
+    rng = np.random.default_rng(seed)
+    n, dims = 300, (33, 31, 64)
+    v = rng.uniform(-0.9, 0.9, (n, 1, 3)) + rng.uniform(-0.3, 0.3, (n, 3, 3)) * 10.0 ** rng.uniform(-6, 0, (n, 1, 3))
+    kind = rng.integers(0, 5, n)
+    v[kind == 1, 1] = v[kind == 1, 0] + np.array([0.3, 0, 0])  # an edge along each coordinate
+    v[kind == 2, 1] = v[kind == 2, 0] + np.array([0, 0.3, 0])
+    v[kind == 3, 1] = v[kind == 3, 0] + np.array([0, 0, 0.3])
+    v[kind == 4] = np.round(v[kind == 4] * 16) / 16  # corners of cells and of boxes
+    xyz = v.reshape(-1, 3).astype(np.float32)
+    check(vf, dims, xyz, np.arange(3 * n, dtype=np.uint32).reshape(-1, 3))
+
+
 def test_jobs_share_waves(vf):
     dims = [(6, 5, 40), (16, 16, 16), (3, 3, 3), (20, 9, 70), (8, 8, 8)]
     meshes = [soup(20 + i, 3 + 2 * i, 0.6) for i in range(len(dims))]

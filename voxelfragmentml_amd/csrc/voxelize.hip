@@ -160,37 +160,78 @@ __device__ __forceinline__ bool cell_passes(const Column& q, float lo, float hi)
     return !s.any();
 }
 
-// Narrows the cells z0..z1 of a column to those near the triangle's plane; every other cell fails the SAT's plane test.
-// Along the column the distance of a cell's centre from the plane, times the normal, is f(cz) = f0 + n2 (cz - a2) with
-// f0 = n0 (cx - ax) + n1 (cy - ay), and the plane test separates where |f| exceeds r = |n0| hx + |n1| hy + |n2| hz.  The test's
-// rounding, and this function's, stay below err: with m the triangle's extent plus a cell (no offset v or edge e of
-// the test is larger than a few m) and A the largest coordinate, an edge component is off by a few 2^-24 m, the
-// normal by a few 2^-24 m^2, the distances by a few 2^-24 m^3, and a cell's centre by a few 2^-24 A, which moves f by
-// m^2 times that; err takes 2^-18 of both, and the range a sixteenth of a cell more at each end.
-__device__ __forceinline__ void plane_range(const Column& q, float mnz, float csz, int& z0, int& z1)
+// The cells z0..z1 (inside one 32-cell word) of an open column of finite coordinates, from the z intervals in which the
+// tests that depend on z pass: `sure` are cells that pass every test, `maybe` those too near an interval's end to tell.
+// Along a column every such test is linear in the cell's number: with v_z = a - k cs an edge's projections are
+// c + k e cs, so the axis separates outside [(-rad - max c) / (e cs), (rad - min c) / (e cs)]; the plane's distance and
+// the z face likewise.  An interval is widened (to what may pass) and narrowed (to what surely does) by the rounding of
+// the FP32 tests and of this function.  With E the largest edge component, V a bound on the vertices' offsets, and S one on
+// the coordinates (|mn| + |a| + V), a cell's centre is off by less than 2^-21 S, an offset along z by 3 times that, an edge's
+// z component by 2^-22 V, so that
+//   an axis' projections and radius, here and there:  2^-20 V (V + E) + 2^-17.7 |e| S  <  2^-18 V (V + E) + 2^-15 |e| S,
+//   the plane's:  2^-18.4 E V^2 + 2^-18.8 E^2 V + 2^-17.7 |n_z| S  <  2^-17 E V (V + E) + 2^-15 |n_z| S,
+//   the z face's:  6 * 2^-21 S  <  2^-18 S.
+// A slope below 1/64 of the error is taken as that much: over a word's 32 cells it moves the projection by less than
+// half the error.
+struct ZCells {
+    uint32_t sure, maybe;
+};
+__device__ __forceinline__ ZCells z_cells(const Column& q, int z0, int z1, float mnz, float csz)
 {
-    const float e0x = q.v1x - q.v0x, e1x = q.v2x - q.v1x, e0y = q.v1y - q.v0y, e1y = q.v2y - q.v1y;
-    const float e0z = q.bz - q.az, e1z = q.cz - q.bz;
+    const float e0x = q.v1x - q.v0x, e1x = q.v2x - q.v1x, e2x = q.v0x - q.v2x;
+    const float e0y = q.v1y - q.v0y, e1y = q.v2y - q.v1y, e2y = q.v0y - q.v2y;
+    const float e0z = q.bz - q.az, e1z = q.cz - q.bz, e2z = q.az - q.cz;
+    const float base = mnz + ((float)z0 + 0.5f) * csz, hz = 0.5f * csz;
+    const float a = q.az - base, b = q.bz - base, c = q.cz - base;
+    auto max3 = [](float x, float y, float z) { return __builtin_fmaxf(__builtin_fmaxf(fabsf(x), fabsf(y)), fabsf(z)); };
+    const float E = max3(max3(e0x, e1x, e2x), max3(e0y, e1y, e2y), max3(e0z, e1z, e2z));
+    const float V = max3(max3(q.v0x, q.v1x, q.v2x), max3(q.v0y, q.v1y, q.v2y), E) + 2.0f * (csz + q.hx + q.hy);
+    const float S = fabsf(mnz) + fabsf(q.az) + V;
+    const float err = 0x1p-18f * V * (V + E), far = 0x1p-15f * S;
+    const float last = (float)(z1 - z0);
+    float olo = 0.0f, ohi = last, ilo = 0.0f, ihi = last;  // k of cells that may pass, that surely do
+    auto interval = [&](float lo, float hi, float e) {
+        olo = __builtin_fmaxf(olo, lo - e);
+        ohi = __builtin_fminf(ohi, hi + e);
+        ilo = __builtin_fmaxf(ilo, lo + e);
+        ihi = __builtin_fminf(ihi, hi - e);
+    };
+    // lower <= s k <= upper, both off by less than er
+    auto linear = [&](float s, float lower, float upper, float er) {
+        const float inv = __builtin_amdgcn_rcpf(__builtin_fmaxf(fabsf(s), er * 0x1p-6f));
+        const float lo = s < 0.0f ? -upper : lower, hi = s < 0.0f ? -lower : upper;
+        interval(lo * inv, hi * inv, er * inv + 0x1p-12f);
+    };
+    auto axis = [&](float ez, float ey, float py, float pz, float qy, float qz, float h) {
+        const float cp = __builtin_fmaf(ez, py, -(ey * pz)), cq = __builtin_fmaf(ez, qy, -(ey * qz));
+        const float er = __builtin_fmaf(far, fabsf(ey), err);
+        // an edge along the other coordinate separates nothing: all its products are 0
+        const float rad = ez == 0.0f && ey == 0.0f ? 4.0f * er : __builtin_fmaf(fabsf(ez), h, fabsf(ey) * hz);
+        linear(ey * csz, -rad - __builtin_fmaxf(cp, cq), rad - __builtin_fminf(cp, cq), er);
+    };
+    axis(e0z, e0y, q.v0y, a, q.v2y, c, q.hy);
+    axis(e0z, e0x, q.v0x, a, q.v2x, c, q.hx);
+    axis(e1z, e1y, q.v0y, a, q.v2y, c, q.hy);
+    axis(e1z, e1x, q.v0x, a, q.v2x, c, q.hx);
+    axis(e2z, e2y, q.v0y, a, q.v1y, b, q.hy);
+    axis(e2z, e2x, q.v0x, a, q.v1x, b, q.hx);
+    const float ic = __builtin_amdgcn_rcpf(csz);
+    interval((__builtin_fminf(__builtin_fminf(a, b), c) - hz) * ic, (__builtin_fmaxf(__builtin_fmaxf(a, b), c) + hz) * ic,
+             0x1p-18f * S * ic + 0x1p-12f);
     const float n0 = e0y * e1z - e1y * e0z, n1 = e0z * e1x - e1z * e0x, n2 = e0x * e1y - e1x * e0y;
-    const float v0x = q.v0x, v0y = q.v0y, hx = q.hx, hy = q.hy, az = q.az;
-    const float f0 = -(n0 * v0x + n1 * v0y);
-    // |v0x|, |v0y| are at most the extent plus a cell where the column lies in the candidate box
-    const float ex = __builtin_fmaxf(fabsf(e0x), __builtin_fmaxf(fabsf(e1x), fabsf(e0x + e1x)));
-    const float ey = __builtin_fmaxf(fabsf(e0y), __builtin_fmaxf(fabsf(e1y), fabsf(e0y + e1y)));
-    const float ez = __builtin_fmaxf(fabsf(e0z), __builtin_fmaxf(fabsf(e1z), fabsf(e0z + e1z)));
-    const float m = __builtin_fmaxf(ex, __builtin_fmaxf(ey, ez)) + 2.0f * (hx + hy + csz) + __builtin_fmaxf(fabsf(v0x), fabsf(v0y));
-    const float A = __builtin_fmaxf(fabsf(az), fabsf(mnz)) + m;
-    const float err = m * m * (m + A) * 0x1p-18f;
-    const float an2 = fabsf(n2);
-    const float w = fabsf(n0) * hx + fabsf(n1) * hy + an2 * csz * 0.5f + err;
-    // cells with |f0 + n2 ((z + 1/2) csz + mnz - az)| <= w, in cells from az
-    const float inv = __builtin_amdgcn_rcpf(an2 * csz);
-    const float at = (n2 > 0.0f ? -f0 : f0) * inv, half = w * inv + fabsf(at) * 0x1p-18f + 0.0625f;
-    const float base = (az - mnz) * __builtin_amdgcn_rcpf(csz) - 0.5f;
-    const float lo = __builtin_ceilf(base + at - half), hi = __builtin_floorf(base + at + half);
-    // NaN or infinity (a plane along z) leaves the range as it is
-    if (lo > (float)z0) z0 = lo > (float)z1 ? z1 + 1 : (int)lo;
-    if (hi < (float)z1) z1 = hi < (float)z0 ? z0 - 1 : (int)hi;
+    const float g = n0 * q.v0x + n1 * q.v0y + n2 * a;  // |g - n2 cs k| <= r
+    const float r = fabsf(n0) * q.hx + fabsf(n1) * q.hy + fabsf(n2) * hz;
+    const float errn = __builtin_fmaf(far, fabsf(n2), 0x1p-17f * E * V * (V + E));
+    linear(n2 * csz, g - r, g + r, errn);
+    // a triangle or cells so small or large that these lose their meaning: every cell by its tests
+    const bool good = err > 1e-30f && errn > 1e-30f && errn < 1e30f && csz > 1e-30f;
+    auto bits = [&](float lo, float hi) {
+        const int l = (int)__builtin_ceilf(lo), h = (int)__builtin_floorf(hi);  // both in -1 .. 32 where it matters
+        return l > h ? 0u : ((2u << (h & 31)) - 1u) & ~((1u << (l & 31)) - 1u);
+    };
+    const uint32_t all = bits(0.0f, last), may = good ? bits(__builtin_fminf(olo, 32.0f), ohi) : all;
+    const uint32_t sure = good ? bits(__builtin_fminf(ilo, 32.0f), __builtin_fmaxf(ihi, -1.0f)) : 0u;
+    return ZCells{ sure << (z0 & 31), (may & ~sure) << (z0 & 31) };
 }
 
 // z plane k of a grid (the lower face of cell k, the upper of cell k - 1), as cell_box has it
@@ -623,33 +664,24 @@ __device__ inline void combine_words(WordTable& T, uint32_t* words, uint32_t wor
     wave_lds_fence();
 }
 
-// A wave's column segments and the cells left of them.
-struct ShellWave {
-    float col[13][64];     // Column, then the grid's first z plane and cell size
-    uint32_t first[64];    // a segment's first cell in the wave's list | its z << 12
-    uint32_t word[64];     // its cells that pass
-    uint8_t owner[64 * 32];  // the segment of every cell of the list
-    WordTable table;
-};
-
 // The pairs left by the setup kernel, shell and parity in one launch (one after the other, each paid a launch of
 // thousands of workgroups and a tail).
 // Shell: one lane per column segment of a triangle's candidate box, the cells (x, y, z) with z in one 32-cell word: the
-// tests that do not depend on z, and the range of z near the triangle's plane.  The cells left, of very uneven
-// number, are listed over the wave and tested one per lane; the words found are combined and then merged by atomicOr.
-// Bound by FP32 instruction issue (81 % of the rate; about 140 of them a cell).  A lane that looped over its own cells
-// ran as long as the wave's longest column and merged every segment's word by itself, 50.3 M atomics on 64 mixed grids
-// instead of 33.7 M: 2.14 -> 1.82 ms there, 181 -> 136 us at 512^3 with a million triangles.
+// tests that do not depend on z, then the cells between the ends of the others' intervals (z_cells) at once and those
+// near an end one by one.  The words of a wave are combined and then merged by atomicOr.
+// Bound by FP32 instruction issue (91 % of the rate).  Testing cell after cell, about 140 instructions each, a lane ran as
+// long as the wave's longest column and merged every segment's word by itself: 2.14 ms for 64 mixed grids, 181 us
+// at 512^3 with a million triangles; with the cells listed over the wave and the words combined (50.3 -> 33.7 M
+// atomics) 1.82 ms and 135 us; by intervals 1.61 ms and 124 us, 256^3 with 200 k triangles 52 -> 39 us.
 // Parity: one lane per column of a triangle's column range.
 __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_vox_pairs(const JobDev* jobs, const TriSetup* setup,
                                                            const unsigned long long* off, uint32_t ntris, uint32_t chunk)
 {
     __shared__ uint32_t soff[kOffCache];
     __shared__ uint32_t sg[2];
-    __shared__ ShellWave sw[kVoxThreads / 64];
-    ShellWave& W = sw[threadIdx.x >> 6];
-    const uint32_t lane = threadIdx.x & 63u;
-    clear_table(W.table);
+    __shared__ WordTable tables[kVoxThreads / 64];
+    WordTable& table = tables[threadIdx.x >> 6];
+    clear_table(table);
     // pairs [0, off[ntris]) are the shell's, [off[ntris], off[2 ntris]) the parity's
     const unsigned long long shell = off[ntris], total = off[2 * (size_t)ntris];
     const unsigned long long ns = (shell + chunk - 1) / chunk, np = (total - shell + chunk - 1) / chunk;
@@ -674,48 +706,22 @@ __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))
                 float cx, hx, cy, hy;
                 cell_box(x, J->mn[0], J->cs[0], &cx, &hx);
                 cell_box(y, J->mn[1], J->cs[1], &cy, &hy);
-                int z0 = max(lo2, (int)(32 * w)), z1 = min(hi2, (int)(32 * w + 31));
+                const int z0 = max(lo2, (int)(32 * w)), z1 = min(hi2, (int)(32 * w + 31));
                 const Column q = make_column(S->P[0], S->P[1], S->P[2], cx, hx, cy, hy);
-                uint32_t bits = 0, n = 0;
+                uint32_t bits = 0;
                 if (valid) {
                     if (S->job & kWildTriangle) {
                         bits = sat_column<false>(q, z0, z1, mnz, csz);
                     } else if (column_open<true>(q)) {
-                        plane_range(q, mnz, csz, z0, z1);
-                        n = (uint32_t)max(z1 - z0 + 1, 0);
+                        const ZCells z = z_cells(q, z0, z1, mnz, csz);
+                        bits = z.sure;
+                        for (uint32_t m = z.maybe; m; m &= m - 1u) {
+                            const int k = (int)(32 * w) + (int)__builtin_ctz(m);
+                            if (cell_passes<true>(q, z_plane(k, mnz, csz), z_plane(k + 1, mnz, csz))) bits |= m & -m;
+                        }
                     }
                 }
-                uint32_t inc = n;  // wave inclusive scan
-#pragma unroll
-                for (int o = 1; o < 64; o <<= 1) {
-                    const uint32_t t = __shfl_up(inc, o, 64);
-                    if (lane >= (uint32_t)o) inc += t;
-                }
-                const uint32_t cells = __shfl(inc, 63, 64), start = inc - n;
-                if (n) {
-                    const float f[13] = { q.v0x, q.v1x, q.v2x, q.v0y, q.v1y, q.v2y, q.hx, q.hy, q.az, q.bz, q.cz, mnz, csz };
-#pragma unroll
-                    for (int k = 0; k < 13; ++k) W.col[k][lane] = f[k];
-                    W.first[lane] = start | (uint32_t)z0 << 12;
-                    W.word[lane] = 0u;
-                    for (uint32_t k = 0; k < n; ++k) W.owner[start + k] = (uint8_t)lane;
-                }
-                wave_lds_fence();
-                for (uint32_t i0 = 0; i0 < cells; i0 += 64u) {
-                    const uint32_t i = i0 + lane;
-                    if (i < cells) {
-                        const uint32_t o = W.owner[i], first = W.first[o];
-                        const int z = (int)(first >> 12) + (int)(i - (first & 0xFFFu));
-                        const Column r{ W.col[0][o], W.col[1][o], W.col[2][o], W.col[3][o], W.col[4][o], W.col[5][o],
-                                        W.col[6][o], W.col[7][o], W.col[8][o], W.col[9][o], W.col[10][o] };
-                        const float rmn = W.col[11][o], rcs = W.col[12][o];
-                        if (cell_passes<true>(r, z_plane(z, rmn, rcs), z_plane(z + 1, rmn, rcs)))
-                            atomicOr(&W.word[o], 1u << (z & 31));
-                    }
-                }
-                wave_lds_fence();
-                if (n) bits = W.word[lane];
-                combine_words<false>(W.table, J->shell_bits, (uint32_t)(((size_t)x * J->ny + (size_t)y) * J->wp + w), bits);
+                combine_words<false>(table, J->shell_bits, (uint32_t)(((size_t)x * J->ny + (size_t)y) * J->wp + w), bits);
             });
         } else {
             const unsigned long long p0 = shell + (c - ns) * chunk;
@@ -725,7 +731,7 @@ __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))
                 const JobDev* J = jobs + (Sg.job & ~kWildTriangle);
                 uint32_t word = 0, bit = 0;
                 if (valid) parity_column(J, Sg, Sg.i0 + (int)(local / nj), Sg.j0 + (int)(local % nj), word, bit);
-                combine_words<true>(W.table, J->toggle_bits, word, bit);
+                combine_words<true>(table, J->toggle_bits, word, bit);
             });
         }
     }
