@@ -830,7 +830,8 @@ void launch_boundaries_tiled(const Launch& L, bool any_wide, bool table)
         };
         // long runs look at many bricks at once, but leave workgroups idle where there are few bricks: a 256^3 grid (8192)
         // takes 26 us with runs of 4 and 30 with 8, a 512^3 grid (65536) 99 and 81, 64 mixed grids 1010 and 945; a 64^3 grid
-        // (128) 15 with runs of 4 and 7.5 brick by brick, a 160^3 one (2000) 16 and 11
+        // (128) 15 with runs of 4 and 7.5 brick by brick, a 160^3 one (2000) 16 and 11.  Without a table, which reads every
+        // label: 512^3 102 with runs of 4 and 95 with 8, 256^3 18.7 with 4 and 22 brick by brick, 128^3 12.3 and 7.7
         const uint32_t run = L.total_bricks < 4096u ? 1u : L.total_bricks < 32768u ? std::min(sh.brick_run, 4u) : sh.brick_run;
         if (run == 1) go(std::integral_constant<uint32_t, 1>{});
         else if (run == 2) go(std::integral_constant<uint32_t, 2>{});

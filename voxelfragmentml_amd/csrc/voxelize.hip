@@ -338,9 +338,10 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_setup(const JobDev* jobs, u
     // shared by the lanes of a wave: each lane stashes its triangle in the wave's slots and lists its
     // columns as (lane << kColBits | column) in an owner table; the wave then takes the listed columns 64 at a
     // time, instead of every lane looping over its own (as many steps as its largest triangle).
-    // Bound by the memory side's atomics, 13 M for 9.2 M triangles of 64 grids: of 0.93 ms, 0.42 go to them, 0.31 to the
-    // parity tests, 0.19 to the shell's and 0.17 to the record stores.  Most change a word that no other triangle nearby
-    // changes, so combining them in LDS first gains nothing here.
+    // Bound by the memory side's atomics first: 0.93 ms for the 9.2 M triangles of 64 mixed grids, with 13 M atomics.
+    // Timed with one part left out each: 0.51 ms without the atomics, 0.62 without the parity columns, 0.74 without the
+    // shell's cells, 0.76 without the record stores, 0.26 with neither columns, cells nor stores.  Combining the
+    // words in LDS before their atomics, as the pairs do, was 0.91 ms here and at 64^3 15.7 us instead of 13.4.
     constexpr uint32_t kWaves = kVoxThreads / 64;
     // 16-bit pairs hold cell indices (< 2048) and extents: lo0 | lo1 << 16, lo2 | hi2 << 16, ey | nj << 16, i0 | j0 << 16
     enum { kLo01, kLo2Hi2, kEyNj, kI0J0, kJob, kX, kY = kX + 3, kZ = kY + 3, kAreaLo = kZ + 3, kAreaHi, kFields };
