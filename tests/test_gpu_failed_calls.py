@@ -1,0 +1,50 @@
+"""Single-grid calls that end in an error, and the grid afterwards."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+BOX = ([-1.03, -1.03, -1.03], [1.03, 1.03, 1.03])
+EUC, MAN, CHE = 0, 1, 2
+
+
+def winding_path(dims):
+    """One corridor, a cell wide, through the whole grid: along x, row after row, layer after layer."""
+    nx, ny, nz = dims
+    g = np.zeros(dims, np.uint16)
+    g[:, ::2, ::2] = 1
+    rows, layers = (ny + 1) // 2, (nz + 1) // 2
+    for k in range(layers):
+        for r in range(rows - 1):  # the ends of the rows, in turn
+            g[-1 if (k * rows + r) % 2 == 0 else 0, 2 * r + 1, 2 * k] = 1
+        if k + 1 < layers:  # a layer ends where the next begins
+            g[-1 if (k * rows + rows - 1) % 2 == 0 else 0, 2 * (rows - 1) if k % 2 == 0 else 0, 2 * k + 1] = 1
+    return g
+
+
+def overlong_flood(g):
+    """A flood whose distances do not fit its keys: 4096 seeds take 12 bits, which leaves a distance 18, and the path of
+    about 190000 cells of weight 2 on average is longer than 2^18."""
+    seeds = np.zeros((4096, 4), np.uint32)
+    seeds[:, 3] = 2 + np.arange(4096) % 250
+    g.fracture_flood(seeds, MAN, noise_seed=5, noise_amp=2)
+
+
+LONG = (96, 88, 88)
+
+
+def test_flood_after_one_that_failed(vf):
+    # rounds are queued ahead: none of the failed flood's may be left when the next one on the grid begins
+    path = winding_path(LONG)
+    seeds = np.array([[0, 0, 0, 2], [50, 40, 44, 3], [95, 44, 20, 4]], np.uint32)
+    want = O.flood(path, seeds, 6, 3, 1)
+    with vf.Grid(LONG, *BOX) as g:
+        g.write(path)
+        for _ in range(3):
+            with pytest.raises(vf.VfError, match="VF_ERR_OVERFLOW"):
+                overlong_flood(g)
+            for _ in range(2):
+                g.fracture_flood(seeds, MAN, noise_seed=3, noise_amp=1)
+                np.testing.assert_array_equal(g.read(), want)

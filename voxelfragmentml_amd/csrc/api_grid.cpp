@@ -617,6 +617,15 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
         volatile uint32_t* pr = g->pinned + kPinProgress;
         W.progress = g->pinned + kPinProgress;
         W.job = &g->job;
+        // on every way out by an exception: the rounds still queued store to the pinned words that the next call resets
+        struct WaitOnFailure {
+            hipStream_t s;
+            bool armed = true;
+            ~WaitOnFailure()
+            {
+                if (armed) (void)hipStreamSynchronize(s);
+            }
+        } rounds_queued{ g->stream };
         auto drain = [&]() -> uint32_t {
             pr[0] = pr[1] = pr[2] = 0;
             std::atomic_thread_fence(std::memory_order_seq_cst);
@@ -658,6 +667,7 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
         g->labels_from_occ = false;
         g->mc.valid = false;
         VF_HIP(hipStreamSynchronize(g->stream));
+        rounds_queued.armed = false;
     });
 }
 
