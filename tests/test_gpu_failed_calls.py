@@ -48,3 +48,25 @@ def test_flood_after_one_that_failed(vf):
             for _ in range(2):
                 g.fracture_flood(seeds, MAN, noise_seed=3, noise_amp=1)
                 np.testing.assert_array_equal(g.read(), want)
+
+
+def test_a_failed_flood_leaves_the_labels(vf):
+    path = winding_path(LONG)
+    path[10:20, ::2, ::2] = 0x8007  # cells of a fragment, flagged
+    path[:, 0, 0] = 5
+    seeds = np.array([[0, 0, 0, 2], [50, 40, 44, 3]], np.uint32)
+    with vf.Grid(LONG, *BOX) as g:
+        g.write(path)
+        mesh = g.marching_cubes(7)
+        with pytest.raises(vf.VfError, match="VF_ERR_OVERFLOW"):
+            overlong_flood(g)
+        np.testing.assert_array_equal(g.read(), path)
+        np.testing.assert_array_equal(g.occupancy(), (path != 0).astype(np.uint8))
+        np.testing.assert_array_equal(g.histogram(), O.histogram(path))
+        np.testing.assert_array_equal(g.read_mesh()["xyz"], mesh["xyz"])
+        g.homogenize()  # labels of one flood, kept by a failed one after it
+        g.fracture_flood(seeds, MAN, noise_seed=3, noise_amp=1)
+        want = O.flood((path != 0).astype(np.uint16), seeds, 6, 3, 1)
+        with pytest.raises(vf.VfError, match="VF_ERR_OVERFLOW"):
+            overlong_flood(g)
+        np.testing.assert_array_equal(g.read(), want)

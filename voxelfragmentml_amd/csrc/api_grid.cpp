@@ -607,7 +607,6 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
         g->flood_lists.ensure(2ull * kFloodXcds * W.list_cap * 8);
         W.lists = g->flood_lists.as<unsigned long long>();
         W.counts = g->fctl.as<uint32_t>() + 48;
-        launch_clear_labels(L);
         launch_flood_init(L, W);
         launch_flood_seed(L, W);
         // Rounds are queued kAhead ahead of the one running, whose number the device stores to pinned memory, so the
@@ -663,6 +662,7 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
             VF_HIP(hipStreamSynchronize(g->stream));
             if (ctl[1] == 0) g->last_flood_levels += drain();  // regions were freed: second growth
         }
+        launch_clear_labels(L);  // not before the flood is known to end well: a failed one leaves the labels
         launch_flood_finish(L);
         g->labels_from_occ = false;
         g->mc.valid = false;
