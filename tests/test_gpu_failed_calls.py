@@ -70,3 +70,31 @@ def test_a_failed_flood_leaves_the_labels(vf):
         with pytest.raises(vf.VfError, match="VF_ERR_OVERFLOW"):
             overlong_flood(g)
         np.testing.assert_array_equal(g.read(), want)
+
+
+@pytest.mark.parametrize("read_first", [False, True])
+def test_a_failed_voxelization_of_a_new_box_leaves_it_empty(vf, read_first):
+    dims = (40, 33, 50)
+    xyz, tri = vf.vessel_mesh(5, *vf.vessel_segments(3000))
+    bad = tri.copy()
+    bad[len(tri) // 2, 1] = len(xyz)  # found on the device only
+    good, broken = vf.DeviceMesh(xyz, tri), vf.DeviceMesh(xyz, bad)
+    empty = np.zeros(dims, np.uint16)
+    want = O.voxelize(xyz, tri, *BOX, dims)
+    with vf.Grid(dims, *BOX) as g:
+        for _ in range(2):
+            if read_first:
+                np.testing.assert_array_equal(g.read(), empty)
+            with pytest.raises(vf.VfError, match="VF_ERR_INVALID_ARG"):
+                g.voxelize_device(broken)
+            np.testing.assert_array_equal(g.read(), empty)
+            np.testing.assert_array_equal(g.histogram(), np.zeros(65536, np.uint32))
+            g.voxelize_device(good)
+            np.testing.assert_array_equal(g.read(), want)
+            with pytest.raises(vf.VfError, match="VF_ERR_INVALID_ARG"):  # a grid with values keeps them
+                g.voxelize_device(broken)
+            np.testing.assert_array_equal(g.read(), want)
+            np.testing.assert_array_equal(g.occupancy(), want)
+            g.set_aabb(*BOX, dims)
+    good.close()
+    broken.close()

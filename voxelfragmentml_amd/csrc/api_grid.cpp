@@ -369,6 +369,10 @@ int vf_voxelize_device(vf_grid* g, const float* d_xyz, uint32_t nv, const uint32
         X.scan_tmp_bytes = g->scan_tmp.bytes;
         launch_voxelize(L, X, pre + kHeadGroups, groups, nullptr);
         grid_report(g);
+        if (reported_stat(g, kStatError) && g->labels_from_occ) {  // a new box: its cells stay EMPTY
+            launch_clear_labels(L);
+            g->labels_from_occ = false;
+        }
         check_device_error(g, "voxelize", reported_stat(g, kStatError));
         if (merge) {
             // labels = new ? FREE : old, occupancy as the labels then say
