@@ -1,0 +1,51 @@
+"""Counts of grids with many labels: below, at and above the ends of the ranges that are counted in one place or another,
+in every workgroup of the kernel and in few."""
+import time
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+BOX = ([-1.03, -1.03, -1.03], [1.03, 1.03, 1.03])
+
+
+def counts(g):
+    return np.bincount((g & 0x7FFF)[g > 1].ravel(), minlength=65536).astype(np.uint32)
+
+
+@pytest.mark.parametrize("dims", [(5, 6, 7), (64, 64, 64), (130, 120, 139)])
+@pytest.mark.parametrize("lo,hi", [(2, 1024), (1020, 1030), (2, 4000), (12280, 12300), (1023, 12288), (17400, 17408), (17400, 17409), (2, 32768)])
+def test_many_labels(vf, dims, lo, hi):
+    print("histogram", dims, lo, hi, flush=True)
+    rng = np.random.default_rng(hi)
+    noise = rng.integers(lo, hi, dims).astype(np.uint16)
+    noise[rng.random(dims) < 0.3] = 0
+    noise[rng.random(dims) < 0.1] |= 0x8000
+    last = np.zeros(dims, np.uint16)  # one cell of the largest label, in the last workgroup
+    last[-1, -1, -1] = hi - 1
+    with vf.Grid(dims, *BOX) as grid:
+        for g in (noise, last, noise):
+            grid.write(g)
+            for n in (65536, hi, hi - 1, 1025):
+                np.testing.assert_array_equal(grid.histogram(n), counts(g)[:n])
+
+
+def test_many_labels_take_no_longer_than_few(vf):
+    # fragments of 8^3 cells with 1500 labels: 5 to 14 times the time of 900 where those above 1023 were counted in HBM
+    rng = np.random.default_rng(0)
+    out = np.zeros(65536, np.uint32)
+    took = []
+    with vf.Grid((256, 256, 256), *BOX) as grid:
+        for labels in (900, 1500):
+            g = np.kron(rng.integers(2, 2 + labels, (32, 32, 32)), np.ones((8, 8, 8), np.int64)).astype(np.uint16)
+            grid.write(g)
+            best = 1.0
+            for _ in range(8):
+                t0 = time.perf_counter()
+                vf.check(vf.lib().vf_histogram(grid._h, out.ctypes.data, 65536))
+                best = min(best, time.perf_counter() - t0)
+            np.testing.assert_array_equal(out, counts(g))
+            took.append(best)
+    print("900 and 1500 labels:", took, flush=True)
+    assert took[1] < 3 * took[0] + 50e-6

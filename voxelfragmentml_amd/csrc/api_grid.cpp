@@ -769,13 +769,19 @@ int vf_histogram(vf_grid* g, uint32_t* counts, uint32_t ncounts)
         grid_materialize(g);
         Launch L = grid_launch(g);
         launch_histogram(L, g->hist.as<uint32_t>(), g->hist.as<uint32_t>() + 65536, g->pinned + kPinHist);
-        // most grids have labels below kHistBins only: the other counts are cleared while the device counts
+        // the counts come through pinned memory up to the largest label (beyond its room there by a copy); the others are
+        // cleared while the device counts
         const uint32_t n = std::min<uint32_t>(ncounts, 65536), head = std::min(n, kHistBins);
         if (ncounts > head) std::memset(counts + head, 0, (size_t)(ncounts - head) * 4);
         VF_HIP(hipStreamSynchronize(g->stream));
-        std::memcpy(counts, g->pinned + kPinHist, (size_t)head * 4);
-        if (n > head && g->pinned[kPinHist + kHistBins]) {
-            VF_HIP(hipMemcpyAsync(counts, g->hist.p, (size_t)n * 4, hipMemcpyDeviceToHost, g->stream));
+        const uint32_t* host = g->pinned + kPinHist;
+        if (head) std::memcpy(counts, host, (size_t)head * 4);
+        const uint32_t top = host[kHistBins], end = std::min(n, top + 1);
+        if (n <= head || !top) return;
+        if (top < kHistBins + kHistLargeHost) {
+            if (end > head) std::memcpy(counts + head, host + kPinLarge, (size_t)(end - head) * 4);
+        } else {
+            VF_HIP(hipMemcpyAsync(counts, g->hist.p, (size_t)end * 4, hipMemcpyDeviceToHost, g->stream));
             VF_HIP(hipStreamSynchronize(g->stream));
         }
     });

@@ -128,26 +128,29 @@ __global__ void k_report(const unsigned long long* stats, const uint4* seeds, ui
     for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) reinterpret_cast<uint4*>(host + kPinSeeds)[i] = seeds[i];
 }
 
-// The histogram of a single grid.  Labels below kHistBins are counted in LDS by kHistBlocks workgroups of 16 waves,
-// which then store their counts (1 MiB) for k_hist_sum; larger ones go to the counts in HBM.  Bound by HBM: 2 bytes
+// The histogram of a single grid.  Labels below kHistLds are counted in LDS by kHistBlocks workgroups of 16 waves,
+// which then store the counts of those below kHistBins (1 MiB) for k_hist_sum and add the others, where there are any, to
+// the counts in HBM; still larger labels go there cell by cell.  Bound by HBM: 2 bytes
 // per cell.  A lane adds the cells of one label among its 8 with one LDS atomic; lanes of a wave that hold the same label
 // follow each other at one a cycle, which costs less than counting them over the wave first (110 us for a 512^3 grid).
 // 8192 workgroups that added their counts to the same few addresses in HBM took 98 us for a 512^3 grid and 57 us for a
-// 256^3 one; now 75 and 20 us, of which clearing and summing take 10.  The word after the partial counts is set when a
-// larger label occurs.
-constexpr uint32_t kHistThreads = 1024;
+// 256^3 one; now 75 and 20 us, of which clearing and summing take 10.  The word after the partial counts receives the largest
+// label of kHistBins or more.  With those counted in HBM alone, 1500 labels in 8^3 blocks of a 256^3 grid took 400 us.
+constexpr uint32_t kHistThreads = 1024, kHistLds = 12288;  // 48 KiB of counts; a workgroup has its CU to itself
 __global__ __launch_bounds__(kHistThreads) void k_histogram(Launch L, uint32_t* part)
 {
-    __shared__ uint32_t bins[kHistBins];
+    __shared__ __attribute__((aligned(16))) uint32_t bins[kHistLds];
+    __shared__ uint32_t largest;  // label, 0 where all are below kHistBins
     const JobDev& J = L.jobs[0];
     const uint16_t* labels = J.labels;
     const uint64_t V = J.V;
-    for (uint32_t i = threadIdx.x; i < kHistBins; i += kHistThreads) bins[i] = 0;
+    for (uint32_t i = threadIdx.x; i < kHistLds / 4; i += kHistThreads) reinterpret_cast<uint4*>(bins)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (threadIdx.x == 0) largest = 0;
+    uint32_t top = 0;
     __syncthreads();
     constexpr uint64_t kStep = (uint64_t)kHistThreads * kCellsPerThread;
     constexpr uint32_t kRun = 4;  // steps whose loads are issued together
     const uint64_t steps = (V + kStep - 1) / kStep;
-    const uint32_t lane = threadIdx.x & 63u;
     // steps are dealt round-robin: a vessel's cells lie in some slabs of the box and not in others
     for (uint64_t s = blockIdx.x; s < steps; s += (uint64_t)kRun * gridDim.x) {
         uint4 q[kRun];
@@ -180,23 +183,33 @@ __global__ __launch_bounds__(kHistThreads) void k_histogram(Launch L, uint32_t* 
                 for (uint32_t k = 0; k < 8u; ++k) eq |= m[k] == l ? 1u << k : 0u;
                 eq &= rest;
                 rest &= ~eq;
-                if (l < kHistBins) {
-                    atomicAdd(&bins[l], (uint32_t)__popc(eq));
-                } else {
-                    atomicAdd(J.hist + l, (uint32_t)__popc(eq));
-                    part[kHistBlocks * kHistBins] = 1u;
-                }
+                top = max(top, l);
+                if (l < kHistLds) atomicAdd(&bins[l], (uint32_t)__popc(eq));
+                else atomicAdd(J.hist + l, (uint32_t)__popc(eq));
             }
         }
     }
+    if (top >= kHistBins) atomicMax(&largest, top);
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < kHistBins; i += kHistThreads) part[blockIdx.x * kHistBins + i] = bins[i];
+    if (!largest) return;
+    for (uint32_t i = kHistBins + threadIdx.x; i < kHistLds; i += kHistThreads) {
+        const uint32_t c = bins[i];
+        if (c) atomicAdd(J.hist + i, c);
+    }
+    if (threadIdx.x == 0) atomicMax(part + kHistBlocks * kHistBins, largest);
 }
 
-// Sums nparts partial counts of 64 bins per workgroup into hist and, where given, host memory.
+// Sums nparts partial counts of 64 bins per workgroup into hist and, where given, host memory; the workgroups after those
+// store the counts of larger labels there, where they occur.
 __global__ __launch_bounds__(256) void k_hist_sum(const uint32_t* part, uint32_t nparts, uint32_t* hist, uint32_t* host)
 {
     __shared__ uint32_t sum[4][64];
+    if (blockIdx.x >= kHistBins / 64) {
+        const uint32_t i = (blockIdx.x - kHistBins / 64) * 256u + threadIdx.x;
+        if (kHistBins + i <= part[kHistBlocks * kHistBins]) host[kPinLarge + i] = hist[kHistBins + i];
+        return;
+    }
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, bin = blockIdx.x * 64u + lane;
     uint32_t n = 0;
 #pragma unroll 8
@@ -805,7 +818,8 @@ void launch_histogram(const Launch& L, uint32_t* hist, uint32_t* part, uint32_t*
     VF_CHECK_LAUNCH();
     k_histogram<<<blocks, kHistThreads, 0, L.s>>>(L, part);
     VF_CHECK_LAUNCH();
-    k_hist_sum<<<kHistBins / 64, 256, 0, L.s>>>(part, blocks, hist, host);
+    static_assert(kHistLargeHost % 256 == 0, "whole workgroups");
+    k_hist_sum<<<kHistBins / 64 + (host ? kHistLargeHost / 256 : 0u), 256, 0, L.s>>>(part, blocks, hist, host);
     VF_CHECK_LAUNCH();
 }
 

@@ -210,12 +210,14 @@ void launch_homogenize(const Launch& L);
 void launch_clear_labels(const Launch& L);
 void launch_undo_mask(const Launch& L, uint16_t keep_mask);
 // job 0's histogram of labels above FREE into its hist (given again; cleared first); part: kHistPartBytes of scratch; host (or
-// null): pinned memory for the first kHistBins counts and a flag, not 0 when a larger label occurs
+// null): pinned memory for the first kHistBins counts, the largest label of kHistBins or more (0: none) and, from kPinLarge
+// on, the kHistLargeHost counts after the first as far as that label
 constexpr uint32_t kHistBins = 1024, kHistBlocks = 256;
 // pinned words of a grid that kernels report to: statistics, flood progress (three words), a histogram's first counts
-// and its flag, seeds
+// and largest label, seeds
 constexpr uint32_t kPinStats = 0, kPinProgress = 2 * kStatCount, kPinHist = 64, kPinSeeds = kPinHist + kHistBins + 64,
                    kPinWords = kPinSeeds + 4 * 4096;
+constexpr uint32_t kPinLarge = kPinSeeds - kPinHist, kHistLargeHost = kPinWords - kPinSeeds;  // in the seeds' place
 constexpr size_t kHistPartBytes = ((size_t)kHistBlocks * kHistBins + 64) * 4;
 void launch_hist_heads(const Launch& L, uint32_t* host);  // every job's first kHistBins counts to pinned host memory
 void launch_histogram(const Launch& L, uint32_t* hist, uint32_t* part, uint32_t* host);
