@@ -726,10 +726,10 @@ int vf_erode(vf_grid* g, int convolution, uint32_t size, uint32_t iterations, fl
         Launch L = grid_launch(g);
         for (uint32_t it = 0; it < iterations; ++it) {
             launch_boundaries_tiled(L, false, false);
-            launch_erode_step(L, g->erode_bits.as<uint8_t>(), g->erode_mask.as<uint8_t>(), (uint32_t)side, limit,
+            launch_erode_step(L, g->V, g->erode_bits.as<uint8_t>(), g->erode_mask.as<uint8_t>(), (uint32_t)side, limit,
                               probability, noise_seed);
         }
-        launch_isolated_cells(L, g->erode_bits.as<uint8_t>());
+        launch_isolated_cells(L, g->V, g->erode_bits.as<uint8_t>());
         launch_labels_to_occ(L);
         g->mc.valid = false;
         VF_HIP(hipStreamSynchronize(g->stream));
@@ -743,7 +743,7 @@ int vf_remove_isolated_cells(vf_grid* g)
         grid_materialize(g);
         g->erode_bits.ensure(erode_bytes(g->dims));
         Launch L = grid_launch(g);
-        launch_isolated_cells(L, g->erode_bits.as<uint8_t>());
+        launch_isolated_cells(L, g->V, g->erode_bits.as<uint8_t>());
         launch_labels_to_occ(L);
         g->mc.valid = false;
         VF_HIP(hipStreamSynchronize(g->stream));

@@ -552,10 +552,10 @@ void Engine::erode(Table& t)
         one.total_bricks = brick_count(e.d.nx, e.d.ny, e.d.nz);
         for (uint32_t it = 0; it < e.spec.erosion_iterations; ++it) {
             launch_boundaries_tiled(one, false, false);
-            launch_erode_step(one, e.erode_bits, e.erode_mask, e.erode_side, e.erode_limit, e.spec.erosion_probability,
+            launch_erode_step(one, e.d.V, e.erode_bits, e.erode_mask, e.erode_side, e.erode_limit, e.spec.erosion_probability,
                               e.spec.erosion_seed);
         }
-        launch_isolated_cells(one, e.erode_bits);
+        launch_isolated_cells(one, e.d.V, e.erode_bits);
     }
 }
 

@@ -9,8 +9,8 @@
 // The step's noise gate is the reference's uniform float noise buffer as a
 // counter-based draw per cell: (hash32(seed, cell) >> 8) / 2^24.
 //
-// Both stencils find the cells that become EMPTY first (a byte of bits per 8 cells of a brick) and empty them in the
-// grid in a second pass over those bits: the grid is read and written where there is something, never copied.
+// Both stencils find the cells that become EMPTY first (a bit per cell) and empty them in the grid in a second
+// pass over those bits: the grid is read and written where there is something, never copied.
 #include "cellops.hpp"
 
 #include <cmath>
@@ -148,10 +148,82 @@ __global__ __launch_bounds__(kCellThreads) void k_empty_cells(const JobDev* Jg, 
     store_group(Jg->labels, g, make_uint4(w[0], w[1], w[2], w[3]));
 }
 
+// The same by a thread per cell in linear order that reads its window from memory: cell c's bit is bit c % 64 of word
+// c / 64.  For grids where bricks do not pay (by_cells).
+template <bool kErode>
+__global__ __launch_bounds__(kCellThreads) void k_stencil_cells(const JobDev* Jg, unsigned long long* kill, const uint8_t* mask,
+                                                                uint32_t side, float limit, float probability, uint64_t noise_seed)
+{
+    __shared__ uint8_t smask[kErode ? kMaxErosionSide * kMaxErosionSide * kMaxErosionSide : 1];
+    if (kErode) {
+        for (uint32_t i = threadIdx.x; i < side * side * side; i += kCellThreads) smask[i] = mask[i];
+        __syncthreads();
+    }
+    const JobDev& J = *Jg;
+    const auto* in = gcast<const uint16_t>(J.labels);
+    const int nx = (int)J.nx, ny = (int)J.ny, nz = (int)J.nz, h = (int)side / 2;
+    const uint64_t c = (uint64_t)blockIdx.x * kCellThreads + threadIdx.x;
+    const uint32_t v = c < J.V ? in[c] : 0u;
+    const bool test = kErode ? v > kFree && (v & 0x7FFFu) != 0 &&
+                                   (float)(hash32(noise_seed, (uint32_t)c) >> 8) * (1.0f / 16777216.0f) < probability
+                             : v != 0;
+    bool gone = false;
+    if (test) {
+        uint32_t cx, cy, cz;
+        decompose(c, &J, cx, cy, cz);
+        const int x = (int)cx, y = (int)cy, z = (int)cz;
+        const int x0 = max(x - h, 0), x1 = min(x + h, nx - 1), y0 = max(y - h, 0), y1 = min(y + h, ny - 1),
+                  z0 = max(z - h, 0), z1 = min(z + h, nz - 1);
+        uint32_t count = 0;
+        for (int xx = x0; xx <= x1; ++xx)
+            for (int yy = y0; yy <= y1; ++yy) {
+                const auto* row = in + ((size_t)xx * ny + yy) * nz;
+                const int m0 = kErode ? ((xx - x + h) * (int)side + (yy - y + h)) * (int)side - z + h : 0;
+                for (int zz = z0; zz <= z1; ++zz) count += row[zz] == v && (!kErode || smask[m0 + zz]) ? 1u : 0u;
+            }
+        gone = kErode ? (float)count / (float)((x1 - x0 + 1) * (y1 - y0 + 1) * (z1 - z0 + 1)) < limit : count < 7u;
+    }
+    const uint64_t m = __ballot(gone);
+    if ((threadIdx.x & 63u) == 0 && c < J.V) kill[c / 64u] = m;
+}
+
+__global__ __launch_bounds__(kCellThreads) void k_empty_linear(const JobDev* Jg, const uint8_t* kill)
+{
+    const uint64_t g = (uint64_t)blockIdx.x * kCellThreads + threadIdx.x;
+    if (8u * g >= Jg->V) return;
+    const uint32_t bits = kill[g];
+    if (!bits) return;
+    uint16_t v[8];
+    load8(Jg->labels, 8u * g, Jg->V, v);
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; ++k)
+        if ((bits >> k) & 1u) v[k] = kEmpty;
+    store8(Jg->labels, 8u * g, Jg->V, v);
+}
+
+// Thin grids, whose cells are less than a third of their bricks' (2048 x 2048 x 1, window 3: 824 us a step by bricks, 159 by
+// cells; 600 x 600 x 9, where they are 0.28: 98 and 80; x 12, 0.38: 102 and 96; x 16, 0.5: 106 and 119), and grids of too
+// few bricks for the chip, which a brick's steps one after another take longer: isolated cells 27.1 us by bricks and 21.5 by
+// cells at 64^3 (128 bricks), 34.7 and 30.7 at 96^3 (432), 38.8 and 40.6 at 128^3 (1024); window 3 17.2 and 15.2 at 64^3,
+// 19.3 and 18.2 at 80^3 (300), 20.6 and 23.1 at 96^3; larger windows are even up to 50 bricks (40^3: 32 and 30 for 5, 221
+// and 191 for 15) and then better by bricks (64^3: 52 and 60 for 7).
+bool by_cells(uint64_t V, uint32_t bricks, uint32_t side, bool erode)
+{
+    return V * 3u < (uint64_t)bricks * kTileCells || bricks < (!erode ? 1000u : side <= 3u ? 320u : 64u);
+}
+
 template <uint32_t SIDE, bool kErode>
-void launch_stencil(const Launch& L, uint8_t* kill, const uint8_t* mask, uint32_t side, float limit, float probability,
+void launch_stencil(const Launch& L, uint64_t V, uint8_t* kill, const uint8_t* mask, uint32_t side, float limit, float probability,
                     uint64_t noise_seed)
 {
+    if (by_cells(V, L.total_bricks, side, kErode)) {
+        k_stencil_cells<kErode><<<ceil_div(V, kCellThreads), kCellThreads, 0, L.s>>>(L.jobs, reinterpret_cast<unsigned long long*>(kill), mask, side,
+                                                                                     limit, probability, noise_seed);
+        VF_CHECK_LAUNCH();
+        k_empty_linear<<<ceil_div(V, 8u * kCellThreads), kCellThreads, 0, L.s>>>(L.jobs, kill);
+        VF_CHECK_LAUNCH();
+        return;
+    }
     const size_t wide = kBrickX + 2 * (side / 2), lds = wide * wide * (kBrickZ + 2 * (side / 2)) * 2 + side * side * 4;
     k_stencil<SIDE, kErode><<<L.total_bricks, kCellThreads, lds, L.s>>>(L.jobs, kill, mask, side, limit, probability, noise_seed);
     VF_CHECK_LAUNCH();
@@ -199,19 +271,19 @@ size_t erode_bytes(const uint32_t dims[3])
     return (size_t)brick_count(dims[0], dims[1], dims[2]) * kCellThreads;
 }
 
-void launch_erode_step(const Launch& L, uint8_t* kill, const uint8_t* mask, uint32_t side, float limit, float probability,
-                       uint64_t noise_seed)
+void launch_erode_step(const Launch& L, uint64_t V, uint8_t* kill, const uint8_t* mask, uint32_t side, float limit,
+                       float probability, uint64_t noise_seed)
 {
     if (side > kMaxErosionSide || side % 2 == 0) fail(VF_ERR_INVALID_ARG, "erosion window side %u", side);
     TimedLaunch tl("erode_step", L.s);
-    if (side == 3) launch_stencil<3, true>(L, kill, mask, side, limit, probability, noise_seed);
-    else launch_stencil<0, true>(L, kill, mask, side, limit, probability, noise_seed);
+    if (side == 3) launch_stencil<3, true>(L, V, kill, mask, side, limit, probability, noise_seed);
+    else launch_stencil<0, true>(L, V, kill, mask, side, limit, probability, noise_seed);
 }
 
-void launch_isolated_cells(const Launch& L, uint8_t* kill)
+void launch_isolated_cells(const Launch& L, uint64_t V, uint8_t* kill)
 {
     TimedLaunch tl("isolated_cells", L.s);
-    launch_stencil<3, false>(L, kill, nullptr, 3, 0.0f, 0.0f, 0);
+    launch_stencil<3, false>(L, V, kill, nullptr, 3, 0.0f, 0.0f, 0);
 }
 
 }  // namespace vf

@@ -303,9 +303,10 @@ void launch_flood_finish(const Launch& L);
 constexpr uint32_t kMaxErosionSide = 15;
 int erosion_mask(int type, uint32_t size, std::vector<uint8_t>& mask, float& activations);
 size_t erode_bytes(const uint32_t dims[3]);
-void launch_erode_step(const Launch& L, uint8_t* kill, const uint8_t* mask, uint32_t side, float limit, float probability,
+// V: the grid's cells
+void launch_erode_step(const Launch& L, uint64_t V, uint8_t* kill, const uint8_t* mask, uint32_t side, float limit, float probability,
                        uint64_t noise_seed);
-void launch_isolated_cells(const Launch& L, uint8_t* kill);
+void launch_isolated_cells(const Launch& L, uint64_t V, uint8_t* kill);
 
 // Sub-seed pass after the first drain (jobs with a non-null sub): merge touching
 // same-fragment seed regions, keep each fragment's smallest-id component, and,
