@@ -279,6 +279,7 @@ int vf_grid_write(vf_grid* g, const uint16_t* in)
         g->labels_from_occ = false;
         g->clean = false;
         g->mc.valid = false;
+        g->occ_unset = false;  // written below
         launch_labels_to_occ(grid_launch(g));
         VF_HIP(hipStreamSynchronize(g->stream));
     });
