@@ -147,7 +147,8 @@ constexpr uint32_t kPruneSeeds = 16;
 // whose occupancy loads are issued together (a launch shape the tuner picks).
 // 512^3, 128 seeds, Chebyshev: 442 us applying every seed in linear tiles, 84 us by bricks and 34 us of clearing, 68 us
 // since a run's bricks are looked at by occupancy words together (live_bricks) instead of a byte a thread.
-template <typename K, uint32_t RUN>
+// LINEAR: tiles of 2048 cells in linear order in place of bricks, for grids that fill little of their bricks (launch_naive).
+template <typename K, uint32_t RUN, bool LINEAR>
 __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(sizeof(K) == 4 ? 5 : 4))) void k_naive(Launch L)
 {
     __shared__ __attribute__((aligned(16))) uint2 seeds[kSeedChunk];
@@ -211,8 +212,8 @@ __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(si
         return m;
     };
     constexpr uint32_t kRun = RUN;
-    walk_tile_runs_strided<kRun>(L, L.bt_prefix, L.total_bricks, &sJ, sp, [&](const JobDev& J, uint32_t j, uint32_t first,
-                                                                             uint32_t nrun) {
+    walk_tile_runs_strided<kRun>(L, LINEAR ? L.tile_prefix : L.bt_prefix, LINEAR ? L.total_tiles : L.total_bricks, &sJ, sp,
+                                 [&](const JobDev& J, uint32_t j, uint32_t first, uint32_t nrun) {
         if (!J.active || J.algo != VF_NAIVE || J.naive_key64 != kWant || J.S == 0) return;
         const uint32_t S = J.S;
         const bool one_chunk = S <= kSeedChunk;
@@ -221,9 +222,24 @@ __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(si
             staged = j;
         }
         auto brick = [&](uint32_t id) {
-        const BrickAt at = brick_at(J, id);
-        const CellGroup grp = cell_group(J, at);
-        const uint32_t occ = group_occ(J, grp);
+        BrickAt at;
+        CellGroup grp;
+        uint32_t occ = 0;
+        const uint32_t c0 = id * kTileCells + tid * kCellsPerThread;  // LINEAR: the thread's first cell
+        if constexpr (LINEAR) {
+            if (c0 < J.V) {
+                uint32_t x, y, z;
+                decompose(c0, &J, x, y, z);
+                for (uint32_t k = 0; k < kCellsPerThread && c0 + k < J.V; ++k) {
+                    occ |= occ_bit(J, x, y, z) ? 1u << k : 0u;
+                    advance(x, y, z, &J);
+                }
+            }
+        } else {
+            at = brick_at(J, id);
+            grp = cell_group(J, at);
+            occ = group_occ(J, grp);
+        }
         // block-wide exclusive scan of the occupied counts -> compacted positions
         const uint32_t n = (uint32_t)__popc(occ);
         uint32_t inc = n;
@@ -241,10 +257,29 @@ __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(si
             total += wsum[w];
         }
         for (int k = 0; k < 8; ++k)
-            if ((occ >> k) & 1u) cells[pos++] = (uint16_t)(tid * 8 + k);  // row of the brick * 32 + z
+            if ((occ >> k) & 1u) cells[pos++] = (uint16_t)(tid * 8 + k);  // row of the brick * 32 + z; place in the tile
         __syncthreads();
-        const uint32_t lo[3] = { at.x, at.y, at.z },
-                       hi[3] = { min(at.x + kBrickX, J.nx) - 1u, min(at.y + kBrickY, J.ny) - 1u, min(at.z + kBrickZ, J.nz) - 1u };
+        if (LINEAR && total == 0) return;  // block-uniform
+        uint32_t lo[3], hi[3];  // the box of the brick or tile
+        if constexpr (LINEAR) {
+            decompose((uint64_t)id * kTileCells, &J, lo[0], lo[1], lo[2]);
+            decompose(min((uint64_t)(id + 1u) * kTileCells, J.V) - 1u, &J, hi[0], hi[1], hi[2]);
+            if (lo[0] != hi[0]) {
+                lo[1] = 0;
+                hi[1] = J.ny - 1u;
+            }
+            if (lo[0] != hi[0] || lo[1] != hi[1]) {
+                lo[2] = 0;
+                hi[2] = J.nz - 1u;
+            }
+        } else {
+            lo[0] = at.x;
+            lo[1] = at.y;
+            lo[2] = at.z;
+            hi[0] = min(at.x + kBrickX, J.nx) - 1u;
+            hi[1] = min(at.y + kBrickY, J.ny) - 1u;
+            hi[2] = min(at.z + kBrickZ, J.nz) - 1u;
+        }
         const int dist = J.dist;
         const bool drop = S > kPruneSeeds;
         uint32_t bound = 0xFFFFFFFFu;
@@ -276,8 +311,14 @@ __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(si
 #pragma unroll
             for (uint32_t q = 0; q < 4; ++q) {
                 const uint32_t c = q < gq ? cells[tid + (q0 + q) * kCellThreads] : 0u, row = c >> 5;
-                cxy[q] = (at.x + row / kBrickY) | (at.y + row % kBrickY) << 16;
-                cz[q] = at.z + (c & 31u);
+                if constexpr (LINEAR) {
+                    uint32_t x, y;
+                    decompose((uint64_t)id * kTileCells + c, &J, x, y, cz[q]);
+                    cxy[q] = x | y << 16;
+                } else {
+                    cxy[q] = (at.x + row / kBrickY) | (at.y + row % kBrickY) << 16;
+                    cz[q] = at.z + (c & 31u);
+                }
             }
             K best[4];
 #pragma unroll
@@ -303,12 +344,28 @@ __global__ __launch_bounds__(kCellThreads) __attribute__((amdgpu_waves_per_eu(si
             }
         }
         __syncthreads();
-        if (occ) store_group(J.labels, grp, lab4[tid]);
+        if (occ) {
+            const uint4 out = lab4[tid];
+            if constexpr (LINEAR) {
+                const uint32_t w[4] = { out.x, out.y, out.z, out.w };
+                uint16_t v[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) v[k] = (uint16_t)(w[k >> 1] >> (16 * (k & 1)));
+                store8(J.labels, c0, J.V, v);
+            } else {
+                store_group(J.labels, grp, out);
+            }
+        }
         __syncthreads();  // lab and cells are reused by the next brick
         };
         // the bricks of the run with an occupied cell; the others (most of a vessel's box) stay EMPTY
+        if constexpr (LINEAR) {
 #pragma unroll 1
-        for (uint32_t any = live_bricks<kRun>(J, first, nrun); any; any &= any - 1u) brick(first + (uint32_t)__builtin_ctz(any));
+            for (uint32_t r = 0; r < nrun; ++r) brick(first + r);
+        } else {
+#pragma unroll 1
+            for (uint32_t any = live_bricks<kRun>(J, first, nrun); any; any &= any - 1u) brick(first + (uint32_t)__builtin_ctz(any));
+        }
     });
 }
 
@@ -374,20 +431,27 @@ __global__ void k_ri_reset(uint32_t* counters, uint32_t idx) { counters[idx] = 0
 void launch_naive(const Launch& L, bool key64)
 {
     if (L.njobs > kWalkMaxJobs) fail(VF_ERR_INVALID_ARG, "naive launch with %u jobs (max %u)", L.njobs, kWalkMaxJobs);
-    const uint32_t blocks = std::max(1u, std::min(L.total_bricks, active_shape().cell_blocks));
     TimedLaunch tl(key64 ? "naive64" : "naive", L.s);
     // grids of few bricks: one brick per run, so that they spread over the device (in runs of 8 a 64^3 grid's 128
     // bricks kept 16 workgroups busy)
-    const uint32_t run = L.total_bricks < kNaiveSmall ? 1u : active_shape().naive_run;
-    auto go = [&](auto r) {
+    // Many bricks with few cells each (2048 x 2048 x 1: 64 of 2048): tiles of cells in linear order, 2.0 to 5.0 times as fast
+    // as bricks there with 4 to 128 seeds (272 -> 54 us for 32 seeds and every 20th cell occupied), 1.2 to 2.4 at
+    // 2048 x 1500 x 4; at a quarter of the cells it depends on the seeds (2 x 2048 x 2048: 0.5 to 1.3), and with few bricks
+    // they are even (300 x 300 x 2, 1444 bricks: 0.8 to 1.1)
+    const bool thin = L.total_bricks >= kNaiveSmall && (uint64_t)L.total_tiles * 6u < L.total_bricks;
+    const uint32_t run = thin || L.total_bricks < kNaiveSmall ? 1u : active_shape().naive_run;
+    const uint32_t blocks = std::max(1u, std::min(thin ? L.total_tiles : L.total_bricks, active_shape().cell_blocks));
+    auto go = [&](auto r, auto linear) {
         constexpr uint32_t R = decltype(r)::value;
-        if (key64) k_naive<unsigned long long, R><<<blocks, kCellThreads, 0, L.s>>>(L);
-        else k_naive<uint32_t, R><<<blocks, kCellThreads, 0, L.s>>>(L);
+        constexpr bool LINEAR = decltype(linear)::value;
+        if (key64) k_naive<unsigned long long, R, LINEAR><<<blocks, kCellThreads, 0, L.s>>>(L);
+        else k_naive<uint32_t, R, LINEAR><<<blocks, kCellThreads, 0, L.s>>>(L);
     };
-    if (run == 1) go(std::integral_constant<uint32_t, 1>{});
-    else if (run == 4) go(std::integral_constant<uint32_t, 4>{});
-    else if (run == 16) go(std::integral_constant<uint32_t, 16>{});
-    else go(std::integral_constant<uint32_t, 8>{});
+    if (thin) go(std::integral_constant<uint32_t, 1>{}, std::true_type{});
+    else if (run == 1) go(std::integral_constant<uint32_t, 1>{}, std::false_type{});
+    else if (run == 4) go(std::integral_constant<uint32_t, 4>{}, std::false_type{});
+    else if (run == 16) go(std::integral_constant<uint32_t, 16>{}, std::false_type{});
+    else go(std::integral_constant<uint32_t, 8>{}, std::false_type{});
     VF_CHECK_LAUNCH();
 }
 
