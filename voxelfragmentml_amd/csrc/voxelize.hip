@@ -621,14 +621,9 @@ __device__ inline void clear_table(WordTable& T)
     }
     wave_lds_fence();
 }
-// XOR (parity) or OR of bits into words[word], by all lanes of a wave; words: the lane's job's array (bits 0: nothing)
-template <bool XOR>
+// OR of bits into words[word], by all lanes of a wave; words: the lane's job's array (bits 0: nothing)
 __device__ inline void combine_words(WordTable& T, uint32_t* words, uint32_t word, uint32_t bits)
 {
-    auto change = [](uint32_t* p, uint32_t b) {
-        if (XOR) atomicXor(p, b);
-        else atomicOr(p, b);
-    };
     const uint64_t with = __ballot(bits != 0u);
     if (with == 0ull) return;
     // lanes of one job share the table; a wave across two jobs changes its words one by one
@@ -638,7 +633,7 @@ __device__ inline void combine_words(WordTable& T, uint32_t* words, uint32_t wor
                    hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(w0 >> 32), (int)first);
     uint32_t* const base = (uint32_t*)(((uint64_t)hi << 32) | lo);
     if (__ballot(bits != 0u && words != base)) {
-        if (bits) change(words + word, bits);
+        if (bits) atomicOr(words + word, bits);
         return;
     }
     bool pending = bits != 0u;
@@ -647,8 +642,7 @@ __device__ inline void combine_words(WordTable& T, uint32_t* words, uint32_t wor
         if (pending) {
             const uint32_t old = atomicCAS(&T.key[h], 0xFFFFFFFFu, word);
             if (old == 0xFFFFFFFFu || old == word) {
-                if (XOR) atomicXor(&T.bits[h], bits);
-                else atomicOr(&T.bits[h], bits);
+                atomicOr(&T.bits[h], bits);
                 pending = false;
             } else {
                 h = (h + 1u) & 127u;
@@ -660,7 +654,7 @@ __device__ inline void combine_words(WordTable& T, uint32_t* words, uint32_t wor
     for (uint32_t e = threadIdx.x & 63u; e < 128u; e += 64u) {
         const uint32_t k = T.key[e], b = T.bits[e];
         if (k != 0xFFFFFFFFu) {
-            if (b) change(base + k, b);
+            if (b) atomicOr(base + k, b);
             T.key[e] = 0xFFFFFFFFu;
             T.bits[e] = 0u;
         }
@@ -672,12 +666,15 @@ __device__ inline void combine_words(WordTable& T, uint32_t* words, uint32_t wor
 // thousands of workgroups and a tail).
 // Shell: one lane per column segment of a triangle's candidate box, the cells (x, y, z) with z in one 32-cell word: the
 // tests that do not depend on z, then the cells between the ends of the others' intervals (z_cells) at once and those
-// near an end one by one.  The words of a wave are combined and then merged by atomicOr.
+// near an end one by one (all of them where no lane of the wave has more than two).  The words of a wave are combined and
+// then merged by atomicOr, where it has many triangles; those of one triangle are all different, and of two or three hardly the same
+// (600 x 600 x 16 with 50 k triangles: 123 us combining all, 91; 2048 x 2048 x 1 with 20 k: 550 and 434).
 // Bound by FP32 instruction issue (91 % of the rate).  Testing cell after cell, about 140 instructions each, a lane ran as
 // long as the wave's longest column and merged every segment's word by itself: 2.14 ms for 64 mixed grids, 181 us
 // at 512^3 with a million triangles; with the cells listed over the wave and the words combined (50.3 -> 33.7 M
 // atomics) 1.82 ms and 135 us; by intervals 1.61 ms and 124 us, 256^3 with 200 k triangles 52 -> 39 us.
-// Parity: one lane per column of a triangle's column range.
+// Parity: one lane per column of a triangle's column range, one atomicXor each (combining them too gained nothing at any size,
+// 512^3 with a million triangles 141 us either way, and cost up to 8 % on flat grids).
 __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_vox_pairs(const JobDev* jobs, const TriSetup* setup,
                                                            const unsigned long long* off, uint32_t ntris, uint32_t chunk)
 {
@@ -713,9 +710,12 @@ __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))
                 const int z0 = max(lo2, (int)(32 * w)), z1 = min(hi2, (int)(32 * w + 31));
                 const Column q = make_column(S->P[0], S->P[1], S->P[2], cx, hx, cy, hy);
                 uint32_t bits = 0;
+                const bool few = __ballot(valid && z1 - z0 >= 2) == 0ull;
                 if (valid) {
                     if (S->job & kWildTriangle) {
                         bits = sat_column<false>(q, z0, z1, mnz, csz);
+                    } else if (few) {
+                        bits = sat_column<true>(q, z0, z1, mnz, csz);
                     } else if (column_open<true>(q)) {
                         const ZCells z = z_cells(q, z0, z1, mnz, csz);
                         bits = z.sure;
@@ -725,7 +725,11 @@ __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))
                         }
                     }
                 }
-                combine_words<false>(table, J->shell_bits, (uint32_t)(((size_t)x * J->ny + (size_t)y) * J->wp + w), bits);
+                const uint32_t word = (uint32_t)(((size_t)x * J->ny + (size_t)y) * J->wp + w);
+                // lanes of a wave have ascending triangles
+                const uint32_t triangles = (uint32_t)__builtin_amdgcn_readlane((int)g, 63) - (uint32_t)__builtin_amdgcn_readfirstlane((int)g) + 1u;
+                if (triangles > 3u) combine_words(table, J->shell_bits, word, bits);
+                else if (bits) atomicOr(J->shell_bits + word, bits);
             });
         } else {
             const unsigned long long p0 = shell + (c - ns) * chunk;
@@ -735,7 +739,7 @@ __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))
                 const JobDev* J = jobs + (Sg.job & ~kWildTriangle);
                 uint32_t word = 0, bit = 0;
                 if (valid) parity_column(J, Sg, Sg.i0 + (int)(local / nj), Sg.j0 + (int)(local % nj), word, bit);
-                combine_words<true>(table, J->toggle_bits, word, bit);
+                if (bit) atomicXor(J->toggle_bits + word, bit);
             });
         }
     }
