@@ -50,3 +50,19 @@ def test_waves_of_two_grids(vf):
         assert [r["status"] for r in b.run(jobs)] == [0, 0]
     for (xyz, tri), d, out in zip(meshes, dims, outs):
         np.testing.assert_array_equal(out != 0, O.voxelize(xyz, tri, *BOX, d) != 0)
+
+
+def test_columns_far_outside_an_axis(vf):
+    # steep slivers beside columns of many cells: an axis excludes the whole column by quotients far below or above any
+    # cell's number, which are clamped before they become integers
+    rng = np.random.default_rng(3)
+    n = 400
+    a = rng.uniform(-0.9, 0.9, (n, 1, 3))
+    v = a + rng.uniform(-1, 1, (n, 3, 3)) * np.array([0.6, 0.6, 1e-6])
+    v[::2, 2] = v[::2, 1] + [1e-7, 0.4, 1e-7]
+    v[::3, :, 2] += rng.uniform(-0.5, 0.5, (len(v[::3]), 3))
+    xyz, tri = v.reshape(-1, 3).astype(np.float32), np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+    for dims in ((40, 50, 64), (30, 30, 200), (300, 20, 33)):
+        with vf.Grid(dims, *BOX) as g:
+            g.voxelize(xyz, tri)
+            np.testing.assert_array_equal(g.read(), O.voxelize(xyz, tri, *BOX, dims))

@@ -229,7 +229,7 @@ __device__ __forceinline__ ZCells z_cells(const Column& q, int z0, int z1, float
         const int l = (int)__builtin_ceilf(lo), h = (int)__builtin_floorf(hi);  // both in -1 .. 32 where it matters
         return l > h ? 0u : ((2u << (h & 31)) - 1u) & ~((1u << (l & 31)) - 1u);
     };
-    const uint32_t all = bits(0.0f, last), may = good ? bits(__builtin_fminf(olo, 32.0f), ohi) : all;
+    const uint32_t all = bits(0.0f, last), may = good ? bits(__builtin_fminf(olo, 32.0f), __builtin_fmaxf(ohi, -1.0f)) : all;
     const uint32_t sure = good ? bits(__builtin_fminf(ilo, 32.0f), __builtin_fmaxf(ihi, -1.0f)) : 0u;
     return ZCells{ sure << (z0 & 31), (may & ~sure) << (z0 & 31) };
 }
