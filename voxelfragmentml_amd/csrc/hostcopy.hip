@@ -272,7 +272,8 @@ bool device_reaches(const void* p)
 
 void HostCopies::run(hipStream_t s)
 {
-    if (start(s)) VF_HIP(hipStreamSynchronize(s));
+    const bool none = list_.empty();
+    if (start(s) || none) VF_HIP(hipStreamSynchronize(s));
 }
 
 bool HostCopies::start(hipStream_t s)
@@ -285,7 +286,7 @@ bool HostCopies::start(hipStream_t s)
     if (total >= kStagedMin)
         for (const Part& p : list)
             if (!device_reaches(p.dst)) staged.push_back(p);
-    bool direct = staged.size() < list.size();
+    bool direct = staged.size() < list.size();  // false for an empty list
     if (direct)
         for (const Part& p : list)
             if (staged.empty() || device_reaches(p.dst)) VF_HIP(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s));
@@ -296,7 +297,7 @@ bool HostCopies::start(hipStream_t s)
             for (const Part& p : staged) VF_HIP(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s));
         }
     }
-    return direct || total == 0;
+    return direct;
 }
 
 }  // namespace vf
