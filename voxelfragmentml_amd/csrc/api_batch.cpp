@@ -378,26 +378,6 @@ void vf_server::loop()
             peak_device_bytes = std::max(peak_device_bytes, dev);
             if (in_use > reserved) max_unreserved = std::max(max_unreserved, in_use - reserved);
         };
-        // marching cubes of a group of finished jobs: its buffers are sized only once the surfaces are
-        // counted, so they are reserved then (cached blocks give way first); a group that cannot fit the
-        // budget fails with VF_ERR_BUDGET.  The meshes leave with the results, the buffers go back.
-        size_t mc_reserved = 0;
-        auto extract = [&](std::vector<EJob*>& group) {
-            auto reserve = [&](size_t bytes) {
-                E.make_room(bytes, budget);
-                std::lock_guard<std::mutex> lk(mu);
-                if (reserved + bytes > budget) return false;
-                reserved += bytes;
-                mc_reserved += bytes;
-                return true;
-            };
-            E.extract(group, reserve);
-            audit();
-            E.release_extract();
-            std::lock_guard<std::mutex> lk(mu);
-            reserved -= mc_reserved;
-            mc_reserved = 0;
-        };
         std::vector<EJob*> leveling;  // flood jobs between front and drain
         Table* lev = nullptr;
         bool lev_dirty = false;
@@ -452,6 +432,33 @@ void vf_server::loop()
                 (void)hipEventDestroy(g.done);
                 leaving.pop_front();
             }
+        };
+        // marching cubes of a group of finished jobs: its buffers are sized only once the surfaces are
+        // counted, so they are reserved then (cached blocks give way first); a group that cannot fit the
+        // budget fails with VF_ERR_BUDGET.  The meshes leave with the results, the buffers go back.
+        size_t mc_reserved = 0;
+        auto extract = [&](std::vector<EJob*>& group) {
+            auto reserve = [&](size_t bytes) {
+                for (;;) {
+                    E.make_room(bytes, budget);
+                    {
+                        std::lock_guard<std::mutex> lk(mu);
+                        if (reserved + bytes <= budget) {
+                            reserved += bytes;
+                            mc_reserved += bytes;
+                            return true;
+                        }
+                    }
+                    if (leaving.empty()) return false;
+                    retire(true);  // finished jobs return what they hold when their grids have left
+                }
+            };
+            E.extract(group, reserve);
+            audit();
+            E.release_extract();
+            std::lock_guard<std::mutex> lk(mu);
+            reserved -= mc_reserved;
+            mc_reserved = 0;
         };
         for (;;) {
             std::vector<EJob*> admitted;
