@@ -78,3 +78,37 @@ def test_meshes_fit_once_the_grids_before_them_have_left(vf):
         np.testing.assert_array_equal(counts, first)
     grid.free()
     dev.close()
+
+
+def test_smoothing_stays_within_the_reservation(vf):
+    # a box of many fragments: nearly all of the job's memory is its meshes' and their smoothing's
+    corner = np.array([[x, y, z] for x in (-0.95, 0.95) for y in (-0.95, 0.95) for z in (-0.95, 0.95)], np.float32)
+    face = np.array([[0, 1, 3], [0, 3, 2], [4, 6, 7], [4, 7, 5], [0, 4, 5], [0, 5, 1], [2, 3, 7], [2, 7, 6], [0, 2, 6], [0, 6, 4],
+                     [1, 5, 7], [1, 7, 3]], np.uint32)
+    dev = vf.DeviceMesh(corner, face)
+    dims = (100, 96, 104)
+    buf = vf.MeshBuffers(1500000, 3000000)
+
+    def job(smooth):
+        j = dev.job(dims, *BOX, 250, 3, vf.NAIVE, vf.EUCLIDEAN, marching_cubes=1, smooth=(3, 0.8, 2, 0.3) if smooth else (0, 0, 0, 0))
+        buf.attach(j)
+        return j
+
+    with vf.Batch() as b:
+        assert b.run([job(True)])[0]["status"] == 0
+    want = {k: v.copy() for k, v in buf.mesh().items()}
+    assert len(want["xyz"]) > 300000
+    tight = least_budget(vf, lambda: job(True)) + (1 << 16)
+    print("vertices", len(want["xyz"]), "budgets", tight, least_budget(vf, lambda: job(False)), flush=True)
+    for budget in (tight, 8 << 30):
+        s = vf.Server(budget, 3)
+        for _ in range(2):
+            buf.xyz[:] = 0
+            for smooth in (False, True):
+                assert s.wait(s.submit(job(smooth)))["status"] == 0
+            for k, v in buf.mesh().items():
+                np.testing.assert_array_equal(v, want[k])
+        m = s.memory()
+        s.close()
+        assert m["max_unreserved_bytes"] == 0 and m["reserved_bytes"] == 0 and m["peak_device_bytes"] <= budget, (budget, m)
+    dev.close()

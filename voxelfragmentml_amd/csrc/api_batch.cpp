@@ -453,7 +453,7 @@ void vf_server::loop()
                     retire(true);  // finished jobs return what they hold when their grids have left
                 }
             };
-            E.extract(group, reserve);
+            E.extract(group, reserve, [&](size_t bytes) { E.make_room(bytes, budget); });
             audit();
             E.release_extract();
             std::lock_guard<std::mutex> lk(mu);

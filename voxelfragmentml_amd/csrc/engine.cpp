@@ -630,7 +630,7 @@ void Engine::finish(EJob& e, const uint32_t* w, const uint32_t* hist)
     }
 }
 
-void Engine::extract(const std::vector<EJob*>& js, const std::function<bool(size_t)>& reserve)
+void Engine::extract(const std::vector<EJob*>& js, const std::function<bool(size_t)>& reserve, const std::function<void(size_t)>& room)
 {
     std::vector<EJob*> mj;
     for (EJob* e : js)
@@ -660,9 +660,9 @@ void Engine::extract(const std::vector<EJob*>& js, const std::function<bool(size
         smooth |= sm[i].nb_iters || sm[i].b_iters;
         outs[i] = e.spec.mesh_out;
     }
-    mc_run_jobs(mc_, s, spec.data(), n, res.data(), reserve);
+    mc_run_jobs(mc_, s, spec.data(), n, res.data(), reserve, smooth);
     // smoothing moves vertices only: triangles, flags and labels leave beside it
-    if (mc_.valid && smooth) mc_smooth_jobs(mc_, s, sm.data(), n, false);
+    if (mc_.valid && smooth) mc_smooth_jobs(mc_, s, sm.data(), n, false, room);
     mc_read_jobs(mc_, s, smooth ? side : s, res.data(), outs.data(), n);
     for (uint32_t i = 0; i < n; ++i) {
         vf_result& r = mj[i]->res;

@@ -115,8 +115,10 @@ public:
     bool collect(Table& t, bool later = false);
     hipStream_t copies = nullptr;
     // marching cubes (and smoothing) of every listed job with marching_cubes set and no error, in one
-    // launch set: counts into the results, meshes into the jobs' mesh_out.  reserve: see mc_run_jobs.
-    void extract(const std::vector<EJob*>& js, const std::function<bool(size_t)>& reserve = nullptr);
+    // launch set: counts into the results, meshes into the jobs' mesh_out.  reserve: see mc_run_jobs, room:
+    // mc_smooth_jobs.
+    void extract(const std::vector<EJob*>& js, const std::function<bool(size_t)>& reserve = nullptr,
+                 const std::function<void(size_t)>& room = nullptr);
     void release_extract();  // the meshes and their scratch back to the block cache
 
     uint32_t* pinned = nullptr;     // gathered stats staging (16 words x kMaxTableJobs)

@@ -368,9 +368,10 @@ struct McJobResult {
     int status;            // VF_ERR_INVALID_ARG: more labels than marching cubes supports
 };
 // reserve (optional): asked for the bytes of each of the two phases' buffers before they are taken; a
-// refusal ends the run with every grid's status VF_ERR_BUDGET
+// refusal ends the run with every grid's status VF_ERR_BUDGET; smooth: they are to be smoothed, for which the second
+// phase's bytes are enough too
 void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* jobs, uint32_t n, McJobResult* out,
-                 const std::function<bool(size_t)>& reserve);
+                 const std::function<bool(size_t)>& reserve, bool smooth = false);
 // copies each grid's mesh of the last run to its vf_mesh_out (NULL entries skipped) when it fits
 // fixed: a stream that does not wait for a smoothing still running on s (or s): all but the positions is copied on it
 void mc_read_jobs(McScratch& W, hipStream_t s, hipStream_t fixed, const McJobResult* res, vf_mesh_out* const* outs, uint32_t n);
@@ -390,8 +391,10 @@ struct McSmooth {
     float b_weight;
 };
 void mc_smooth(McScratch& W, hipStream_t s, uint32_t nb_iters, float nb_weight, uint32_t b_iters, float b_weight);
-// wait: until the positions are final
-void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32_t njobs, bool wait = true);
+// wait: until the positions are final; room (optional): told the bytes of the buffers before they are taken, in place of the
+// pairs', which go back to the cache first
+void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32_t njobs, bool wait = true,
+                    const std::function<void(size_t)>& room = nullptr);
 
 // scan (scan.hip): exclusive prefix sums, graph-capturable, no host sync
 size_t scan_tmp_bytes(uint64_t n);

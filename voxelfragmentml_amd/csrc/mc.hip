@@ -1143,8 +1143,14 @@ hipError_t sort_pairs(void* tmp, size_t& bytes, const uint32_t* keys, uint32_t* 
     return rocprim::radix_sort_pairs<Config>(tmp, bytes, keys, skeys, vals, svals, n, 0u, (unsigned)bits, s);
 }
 
+// What smoothing takes (the buffers of mc_smooth_jobs).
+size_t smooth_bytes(uint64_t nv, uint64_t nt, uint32_t njobs)
+{
+    return (size_t)(std::max(nt * 16, nv * 32) + nv * 12 + nt * 24 + (nv + 1) * 8 + scan_tmp_bytes(nv) + njobs * sizeof(uint4) + 6 * 64);
+}
+
 void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n, McJobResult* out,
-                 const std::function<bool(size_t)>& reserve)
+                 const std::function<bool(size_t)>& reserve, bool smooth)
 {
     if (n == 0) return;
     auto refuse = [&] {
@@ -1251,12 +1257,12 @@ void mc_run_jobs(McScratch& W, hipStream_t s, const McJobSpec* spec, uint32_t n,
     std::vector<uint32_t> sjob((size_t)base[n] + 1, 0);
     for (uint32_t j = 0; j < n; ++j)
         for (uint32_t g = base[j]; g < base[j + 1]; ++g) sjob[g] = j;
-    if (reserve) {  // the second phase's buffers: pairs (double-buffered, counts, prefixes) and the meshes
+    if (reserve) {  // the second phase's buffers: pairs (double-buffered, counts, prefixes), then smoothing's in their place, and the meshes
         size_t sort_bytes = 0;
         if (npairs) VF_HIP(sort_pairs(nullptr, sort_bytes, nullptr, nullptr, nullptr, nullptr, (size_t)npairs, 32, s));
-        const size_t phase2 = (size_t)npairs * (4 + 4 + 8 + 8 + 4 + 4 + 8 + 8) + sort_bytes + scan_tmp_bytes(npairs) +
-                              (size_t)NT * (12 + 1) + (size_t)NV * 12 + 3 * ((size_t)S + 1) * 8 + ((size_t)S + 1) * 4 +
-                              13 * 320;
+        const size_t pairs = (size_t)npairs * (4 + 4 + 8 + 8 + 4 + 4 + 8 + 8) + sort_bytes + scan_tmp_bytes(npairs);
+        const size_t phase2 = std::max(pairs, smooth ? smooth_bytes(NV, NT, n) : 0) + (size_t)NT * (12 + 1) + (size_t)NV * 12 + 3 * ((size_t)S + 1) * 8 + ((size_t)S + 1) * 4 +
+                              13 * 320;  // as many blocks as the pairs and the meshes have
         if (!reserve(phase2 + phase2 / 8)) {
             refuse();
             return;
@@ -1433,7 +1439,8 @@ void mc_read(McScratch& W, hipStream_t s, float* xyz, uint32_t* tri, uint8_t* tr
     mc_read_range(W, s, 0, W.nl, xyz, tri, tri_flag, labels, voff, toff);
 }
 
-void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32_t njobs, bool wait)
+void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32_t njobs, bool wait,
+                    const std::function<void(size_t)>& room)
 {
     if (!W.valid) fail(VF_ERR_INVALID_ARG, "no marching-cubes mesh to smooth");
     if (njobs + 1 != W.label_base.size()) fail(VF_ERR_INVALID_ARG, "smoothing parameters for %u grids, mesh of %zu", njobs,
@@ -1466,6 +1473,11 @@ void mc_smooth_jobs(McScratch& W, hipStream_t s, const McSmooth* per_job, uint32
     D.njobs = njobs;
     // (such a mesh, its pairs and these buffers would not fit 288 GB)
     if (W.nv >= kNoVertex) fail(VF_ERR_OVERFLOW, "smoothing of 2^31 vertices or more");
+    if (room) {  // the pairs have become meshes
+        for (int b : { kBKeys0, kBKeys1, kBVals0, kBVals1, kBSort, kBCntT, kBCntV, kBTpre, kBVpre, kBScan }) B[b].release(*W.cache);
+        const size_t bytes = smooth_bytes(W.nv, W.nt, njobs);
+        room(bytes + bytes / 8 + 6 * 256);
+    }
     W.ensure(kBSmTmp, std::max((size_t)W.nt * 16, (size_t)W.nv * 32) + 64);  // corners, then truncated positions, twice
     W.ensure(kBSmFlag, (size_t)W.nv * 12 + 64);  // info, deg, vjob
     W.ensure(kBSmScan, scan_tmp_bytes(W.nv) + 64);
