@@ -1,0 +1,51 @@
+"""Objects that live for one model: grids that are made, read once and dropped cost no more than their copies, whether a
+longer-lived object shares the copies' ring of pinned memory with them or not.  Cells equal those written."""
+import time
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+BOX = ([-1.03, -1.03, -1.03], [1.03, 1.03, 1.03])
+
+
+def read_once(vf, cells, out):
+    t0 = time.perf_counter()
+    with vf.Grid(cells.shape, *BOX) as g:
+        g.write(cells)
+        vf.check(vf.lib().vf_grid_read(g._h, out.ctypes.data))
+    return time.perf_counter() - t0
+
+
+@pytest.mark.parametrize("edge", [64, 82, 100, 128, 140, 200])
+def test_one_read_of_a_grid(vf, edge):
+    cells = np.random.default_rng(edge).integers(0, 0x7FFF, (edge,) * 3, np.uint16)
+    out = np.zeros_like(cells)
+    alone = []
+    for _ in range(12):
+        out[:] = 0
+        alone.append(read_once(vf, cells, out))
+        np.testing.assert_array_equal(out, cells)
+    with vf.Grid((256, 256, 64), *BOX) as other:  # 8 MiB: makes the ring and holds it
+        big = np.ones((256, 256, 64), np.uint16)
+        other.write(big)
+        np.testing.assert_array_equal(other.read(), big)
+        shared = []
+        for _ in range(12):
+            out[:] = 0
+            shared.append(read_once(vf, cells, out))
+            np.testing.assert_array_equal(out, cells)
+    alone, shared = sorted(alone)[3], sorted(shared)[3]
+    print("a grid of", edge, "alone", alone, "beside another", shared, flush=True)
+    if edge < 128:  # below 4 MiB: no ring of its own, which took 110 to 150 us more
+        assert alone < shared + 100e-6
+
+
+def test_reads_of_one_grid_add_up(vf):
+    # 1.1 MB a read: the runtime's copies first, then the ring that they have paid for
+    cells = np.random.default_rng(1).integers(0, 0x7FFF, (82, 82, 82), np.uint16)
+    with vf.Grid(cells.shape, *BOX) as g:
+        g.write(cells)
+        for _ in range(8):
+            np.testing.assert_array_equal(g.read(), cells)

@@ -23,6 +23,10 @@ constexpr uint32_t kStagePart = 1u << 15;    // bytes of a workgroup
 constexpr uint32_t kStageBlocks = kChunk / kStagePart;
 constexpr uint32_t kHelpers = 3;
 constexpr size_t kStagedMin = 1u << 20;      // fewer bytes: the runtime's copy (512 KiB take it 30 us, this one 33; 1.7 MiB 97 and 75)
+// Bytes an object has to copy before it makes a pool (one that is there is used from kStagedMin on): making and dropping it takes
+// 120 to 150 us, and a MiB by it 33 us less than by the runtime.  A program that makes a grid, reads it and drops it took 427 us
+// for one of 82^3 cells with a pool each time, 323 without.
+constexpr size_t kPoolPays = 4u << 20;
 
 // Chunk blockIdx.y: bytes of src to dst, equally aligned; workgroup b's flag is set to seq when its part is in host
 // memory.  A launch takes kGroup chunks: the gap between two launches and the wait for the last store of one cost 7 us,
@@ -247,13 +251,14 @@ private:
 };
 
 namespace {
-std::shared_ptr<CopyPool> shared_pool()
+// The pool that some object holds; make: or a new one.
+std::shared_ptr<CopyPool> shared_pool(bool make)
 {
     static std::mutex mu;
     static std::weak_ptr<CopyPool> pool;
     std::lock_guard<std::mutex> lk(mu);
     std::shared_ptr<CopyPool> p = pool.lock();
-    if (!p) {
+    if (!p && make) {
         p = std::make_shared<CopyPool>();
         pool = p;
     }
@@ -291,8 +296,9 @@ bool HostCopies::start(hipStream_t s)
         for (const Part& p : list)
             if (staged.empty() || device_reaches(p.dst)) VF_HIP(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s));
     if (!staged.empty()) {
-        if (!pool_) pool_ = shared_pool();
-        if (!pool_->run(staged, s)) {  // in use by another thread
+        for (const Part& p : staged) asked_ += p.bytes;
+        if (!pool_) pool_ = shared_pool(asked_ >= kPoolPays);
+        if (!pool_ || !pool_->run(staged, s)) {  // not worth one, or in use by another thread
             direct = true;
             for (const Part& p : staged) VF_HIP(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s));
         }

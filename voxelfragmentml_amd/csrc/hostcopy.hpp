@@ -30,6 +30,7 @@ public:
 private:
     std::vector<Part> list_;
     std::shared_ptr<CopyPool> pool_;
+    uint64_t asked_ = 0;  // bytes that a pool would have copied so far, and copied
 };
 
 }  // namespace vf
