@@ -579,23 +579,25 @@ bool Engine::collect(Table& t, bool later)
     const uint32_t n = t.L.njobs;
     uint32_t counted = 0;
     for (const EJob* e : t.jobs) counted += e->spec.histogram_out != nullptr;
-    if (counted) {
-        if (hist_jobs_ < n) {
-            if (hist_pinned_) VF_HIP(hipHostFree(hist_pinned_));
-            hist_pinned_ = nullptr;
-            hist_jobs_ = 0;
-            uint32_t room = 16;
-            while (room < n) room *= 2;
-            VF_HIP(hipHostMalloc(reinterpret_cast<void**>(&hist_pinned_), (size_t)room * kHistBins * 4));
+    if (counted && hist_jobs_ < n) {
+        if (hist_pinned_) VF_HIP(hipHostFree(hist_pinned_));
+        hist_pinned_ = nullptr;
+        hist_jobs_ = 0;
+        uint32_t room = 16;
+        while (room < n) room *= 2;
+        if (hipHostMalloc(reinterpret_cast<void**>(&hist_pinned_), (size_t)room * kHistBins * 4) == hipSuccess) {
             hist_jobs_ = room;
+        } else {  // without pinned memory all counts are copied
+            (void)hipGetLastError();
+            hist_pinned_ = nullptr;
         }
-        launch_hist_heads(t.L, hist_pinned_);
     }
+    if (counted && hist_jobs_) launch_hist_heads(t.L, hist_pinned_);
     VF_HIP(hipMemcpyAsync(pinned, t.gather, 16 * 4 * (size_t)n, hipMemcpyDeviceToHost, s));
     for (EJob* e : t.jobs)
         if (e->spec.histogram_out) std::memset(e->spec.histogram_out + kHistBins, 0, (65536 - kHistBins) * 4);
     VF_HIP(hipStreamSynchronize(s));
-    for (uint32_t i = 0; i < n; ++i) finish(*t.jobs[i], pinned + 16 * i, hist_pinned_ + (size_t)i * kHistBins);
+    for (uint32_t i = 0; i < n; ++i) finish(*t.jobs[i], pinned + 16 * i, hist_jobs_ ? hist_pinned_ + (size_t)i * kHistBins : nullptr);
     if (later) return to_host_.start(copies);  // s is drained: its work is visible to the other stream
     to_host_.run(s);
     return false;
@@ -622,8 +624,8 @@ void Engine::finish(EJob& e, const uint32_t* w, const uint32_t* hist)
     if (e.spec.labels_out) to_host_.add(e.spec.labels_out, e.d.labels, e.d.V * 2);
     if (e.spec.histogram_out) {
         uint32_t labels = 0;
-        for (uint32_t k = 2; k < kHistBins; ++k) labels += hist[k] != 0;
-        if (r.status == VF_OK && e.d.active && labels == r.num_labels)
+        for (uint32_t k = 2; hist && k < kHistBins; ++k) labels += hist[k] != 0;
+        if (hist && r.status == VF_OK && e.d.active && labels == r.num_labels)
             std::memcpy(e.spec.histogram_out, hist, kHistBins * 4);
         else
             to_host_.add(e.spec.histogram_out, e.d.hist, 65536 * 4);

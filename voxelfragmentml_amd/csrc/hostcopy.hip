@@ -251,7 +251,7 @@ private:
 };
 
 namespace {
-// The pool that some object holds; make: or a new one.
+// The pool that some object holds; make: or a new one.  None where there is no pinned memory for it.
 std::shared_ptr<CopyPool> shared_pool(bool make)
 {
     static std::mutex mu;
@@ -259,7 +259,11 @@ std::shared_ptr<CopyPool> shared_pool(bool make)
     std::lock_guard<std::mutex> lk(mu);
     std::shared_ptr<CopyPool> p = pool.lock();
     if (!p && make) {
-        p = std::make_shared<CopyPool>();
+        try {
+            p = std::make_shared<CopyPool>();
+        } catch (const Exception&) {
+            return nullptr;
+        }
         pool = p;
     }
     return p;
@@ -298,7 +302,7 @@ bool HostCopies::start(hipStream_t s)
     if (!staged.empty()) {
         for (const Part& p : staged) asked_ += p.bytes;
         if (!pool_) pool_ = shared_pool(asked_ >= kPoolPays);
-        if (!pool_ || !pool_->run(staged, s)) {  // not worth one, or in use by another thread
+        if (!pool_ || !pool_->run(staged, s)) {  // no pool, or in use by another thread
             direct = true;
             for (const Part& p : staged) VF_HIP(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s));
         }
