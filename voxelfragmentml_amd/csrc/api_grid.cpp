@@ -639,6 +639,7 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
             uint64_t queued = 0;
             uint32_t seen = 0;
             auto moved = std::chrono::steady_clock::now();
+            HostPause pause;
             while (pr[1] == 0) {
                 const uint32_t at = pr[0];
                 if (queued < (uint64_t)at + kAhead) {
@@ -650,7 +651,7 @@ int vf_fracture_flood(vf_grid* g, const vf_seed* seeds, uint32_t S, int distance
                 } else if (at != seen) {
                     seen = at;
                     moved = std::chrono::steady_clock::now();
-                } else if (std::chrono::steady_clock::now() - moved > std::chrono::milliseconds(20)) {
+                } else if (pause(); std::chrono::steady_clock::now() - moved > std::chrono::milliseconds(20)) {
                     // a long round, or no word will come: wait for what is queued, then there is progress or an error
                     VF_HIP(hipStreamSynchronize(g->stream));
                     if (pr[1] == 0 && pr[0] == at) fail(VF_ERR_DEVICE, "flood rounds stopped");

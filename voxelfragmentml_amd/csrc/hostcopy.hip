@@ -137,11 +137,15 @@ public:
                     launched_.store(queued += k, std::memory_order_release);
                 }
             };
+            HostPause pause;
             for (;;) {
                 queue();
                 uint32_t i = next_.load(std::memory_order_relaxed);
                 if (i >= n) break;
-                if (i >= queued) continue;  // its slot is still being copied by a helper
+                if (i >= queued) {  // its slot is still being copied by a helper
+                    pause();
+                    continue;
+                }
                 if (!filled(i)) {
                     wait(i, s, queue);
                     continue;
@@ -151,7 +155,7 @@ public:
                     {
                         std::lock_guard<std::mutex> lk(mu_);
                         ++round_;
-                        active_ = (uint32_t)helpers_.size();
+                        open_ = true;
                     }
                     cv_.notify_all();
                 }
@@ -195,8 +199,10 @@ private:
     void wait(uint32_t i, hipStream_t s, F&& queue)
     {
         auto since = std::chrono::steady_clock::now();
+        HostPause pause;
         while (!filled(i) && next_.load(std::memory_order_relaxed) == i) {
             queue();
+            pause();
             if (std::chrono::steady_clock::now() - since > std::chrono::milliseconds(20)) {
                 // the work before the copies takes longer, or the device failed
                 VF_HIP(hipStreamSynchronize(s));
@@ -205,10 +211,12 @@ private:
             }
         }
     }
+    // until no helper looks at the chunks any more: those that have not woken up yet miss the round
     void settle(bool awake)
     {
         if (!awake) return;
         std::unique_lock<std::mutex> lk(mu_);
+        open_ = false;
         done_.wait(lk, [&] { return active_ == 0; });
     }
     void help(uint64_t seen)
@@ -216,16 +224,20 @@ private:
         for (;;) {
             {
                 std::unique_lock<std::mutex> lk(mu_);
-                cv_.wait(lk, [&] { return stop_ || (round_ != seen && active_); });
+                cv_.wait(lk, [&] { return stop_ || (round_ != seen && open_); });
                 if (stop_) return;
                 seen = round_;
+                ++active_;
             }
             const uint32_t n = (uint32_t)chunks_.size();
+            HostPause pause;
             for (;;) {
                 uint32_t i = next_.load();
                 if (i >= n || failed_.load()) break;
                 if (i < launched_.load(std::memory_order_acquire) && filled(i)) {
                     if (next_.compare_exchange_strong(i, i + 1)) copy(i);
+                } else {
+                    pause();
                 }
             }
             {
@@ -240,7 +252,8 @@ private:
     std::condition_variable cv_, done_;
     std::vector<std::thread> helpers_;
     uint64_t round_ = 0;
-    uint32_t active_ = 0;
+    uint32_t active_ = 0;  // helpers in the round
+    bool open_ = false;    // helpers may still join it
     bool stop_ = false;
     uint8_t* base_ = nullptr;
     uint32_t* flags_ = nullptr;

@@ -1,11 +1,26 @@
 // Copies of device memory to a caller's host memory.
 #pragma once
 #include <memory>
+#include <thread>
 #include <vector>
 
 #include "common.hpp"
 
 namespace vf {
+
+// Between two looks at a word that the device or another thread will change: a few pauses of the core, for waits of a
+// microsecond or two, then the core goes to any other thread that wants it.
+class HostPause {
+public:
+    void operator()()
+    {
+        if (++looks_ > 64) std::this_thread::yield();
+        else __builtin_ia32_pause();
+    }
+
+private:
+    uint32_t looks_ = 0;
+};
 
 class CopyPool;
 
