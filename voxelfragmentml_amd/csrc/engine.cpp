@@ -170,7 +170,6 @@ Engine::Engine()
     VF_HIP(hipGetDevice(&device));
     VF_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     VF_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
-    VF_HIP(hipStreamCreateWithFlags(&copies, hipStreamNonBlocking));
     VF_HIP(hipEventCreateWithFlags(&side_go, hipEventDisableTiming));
     VF_HIP(hipEventCreateWithFlags(&side_done, hipEventDisableTiming));
     VF_HIP(hipHostMalloc(reinterpret_cast<void**>(&pinned), 16 * 4 * kMaxTableJobs));
@@ -598,7 +597,10 @@ bool Engine::collect(Table& t, bool later)
         if (e->spec.histogram_out) std::memset(e->spec.histogram_out + kHistBins, 0, (65536 - kHistBins) * 4);
     VF_HIP(hipStreamSynchronize(s));
     for (uint32_t i = 0; i < n; ++i) finish(*t.jobs[i], pinned + 16 * i, hist_jobs_ ? hist_pinned_ + (size_t)i * kHistBins : nullptr);
-    if (later) return to_host_.start(copies);  // s is drained: its work is visible to the other stream
+    if (later) {
+        if (!copies && !to_host_.empty()) VF_HIP(hipStreamCreateWithFlags(&copies, hipStreamNonBlocking));
+        return to_host_.start(copies);  // s is drained: its work is visible to the other stream
+    }
     to_host_.run(s);
     return false;
 }
