@@ -173,17 +173,21 @@ static void validate_seeds(const vf_grid* g, const vf_seed* seeds, uint32_t S)
                  seeds[s].z, g->dims[0], g->dims[1], g->dims[2]);
 }
 
+// Up to this many seeds ride in launches' arguments (128 each, one launch after another), more by a copy and a wait: a 20^3 grid's
+// labels take 27 and 37 us with 8 seeds, 88 and 93 with 512, 125 and 121 with 768, 544 and 494 with 4096.
+constexpr uint32_t kSeedsByLaunch = 512;
+
 static void upload_seeds(vf_grid* g, const vf_seed* seeds, uint32_t S)
 {
     g->seeds.ensure((size_t)std::max<uint32_t>(S, 1) * sizeof(uint4));
-    if (S <= kMaxDeviceSeeds) launch_put_seeds(g->seeds.as<uint4>(), seeds, S, g->stream);
+    if (S <= kSeedsByLaunch) launch_put_seeds(g->seeds.as<uint4>(), seeds, S, g->stream);
     else VF_HIP(hipMemcpyAsync(g->seeds.p, seeds, (size_t)S * sizeof(uint4), hipMemcpyHostToDevice, g->stream));
     if (g->job.seeds != g->seeds.as<uint4>() || g->job.S != S || g->job.S_draw != S) {
         g->job.seeds = g->seeds.as<uint4>();
         g->job.S = g->job.S_draw = S;
         g->job_dirty = true;
     }
-    if (S > kMaxDeviceSeeds) VF_HIP(hipStreamSynchronize(g->stream));  // the caller's list may go
+    if (S > kSeedsByLaunch) VF_HIP(hipStreamSynchronize(g->stream));  // the caller's list may go
 }
 
 static vf_grid* checked(vf_grid* g)
