@@ -368,7 +368,7 @@ void vf_server::loop()
     (void)hipSetDevice(device);
     ServerTrace tr;
     try {
-        Engine E;
+        Engine E(true);
         // engine allocations never exceed the bytes reserved by admitted jobs: checked after every step
         // that allocates (job blocks, tables, worklists, front scratch)
         auto audit = [&] {

@@ -75,7 +75,8 @@ struct Table {
 
 class Engine {
 public:
-    Engine();
+    // with_copies: with a stream for copies that collect() leaves in flight
+    explicit Engine(bool with_copies = false);
     ~Engine();
     Engine(const Engine&) = delete;
     Engine& operator=(const Engine&) = delete;
@@ -113,7 +114,7 @@ public:
     // after post(t): waits for it, fills the jobs' results and makes their optional grid and histogram copies.
     // later: copies that the device makes by itself may be left in flight on the stream `copies`; true if they are.
     bool collect(Table& t, bool later = false);
-    hipStream_t copies = nullptr;  // made when it is first used
+    hipStream_t copies = nullptr;
     // marching cubes (and smoothing) of every listed job with marching_cubes set and no error, in one
     // launch set: counts into the results, meshes into the jobs' mesh_out.  reserve: see mc_run_jobs, room:
     // mc_smooth_jobs.

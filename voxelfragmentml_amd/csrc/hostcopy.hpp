@@ -32,7 +32,6 @@ public:
     {
         if (bytes) list_.push_back(Part{ static_cast<uint8_t*>(dst), static_cast<const uint8_t*>(src), bytes });
     }
-    bool empty() const { return list_.empty(); }
     void run(hipStream_t s);
     // as run, but copies that the device makes by itself (to pinned memory) may be left in flight: true if they are, and
     // without copies it waits for nothing
