@@ -53,10 +53,6 @@ constexpr uint32_t kCellThreads = 256;
 constexpr uint32_t kCellsPerThread = 8;
 static_assert(kCellThreads * kCellsPerThread == kTileCells, "tile shape");
 
-struct Cell8 {
-    uint16_t v[8];
-};
-
 __device__ inline void load8(const uint16_t* p, uint64_t c0, uint64_t V, uint16_t v[8])
 {
     if (c0 + 8 <= V) {

@@ -157,11 +157,6 @@ __device__ inline uint4 gload4(const void* p)
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 __device__ inline void gstore4(void* p, uint4 q) { *(VF_AS_GLOBAL vf_u32x4*)p = vf_u32x4{ q.x, q.y, q.z, q.w }; }
-__device__ inline uint2 gload2(const void* p)
-{
-    const vf_u32x2 v = *(const VF_AS_GLOBAL vf_u32x2*)p;
-    return make_uint2(v.x, v.y);
-}
 // the same at any cell's address: rows of uint16 cells start on 2-byte, of keys on 4-byte, of bytes on any boundaries where
 // nz is odd (global accesses need no alignment on gfx950)
 typedef vf_u32x4 vf_u32x4_a2 __attribute__((aligned(2)));
@@ -186,7 +181,6 @@ __device__ inline void gstore4_words(VF_AS_GLOBAL uint32_t* p, uint4 q)
 }
 typedef vf_u32x2 vf_u32x2_a1 __attribute__((aligned(1)));
 __device__ inline void gstore2_bytes(uint8_t* p, uint2 q) { *(VF_AS_GLOBAL vf_u32x2_a1*)p = vf_u32x2_a1{ q.x, q.y }; }
-__device__ inline void gstore2(void* p, uint2 q) { *(VF_AS_GLOBAL vf_u32x2*)p = vf_u32x2{ q.x, q.y }; }
 
 __host__ __device__ inline uint32_t fmix32(uint32_t h)
 {

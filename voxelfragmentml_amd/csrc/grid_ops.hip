@@ -407,7 +407,7 @@ __global__ __launch_bounds__(kCellThreads) void k_cells_post(Launch L, int bsize
 // 16-byte load per thread and bricks without a label stop there; live bricks
 // load the halo and run separable max/min passes z, y, x in LDS.
 constexpr int kBTX = 8, kBTY = 8, kBTZ = 32;
-constexpr int kBHX = kBTX + 2, kBHY = kBTY + 2, kBHZ = kBTZ + 2;
+constexpr int kBHX = kBTX + 2, kBHY = kBTY + 2;
 // z-pass row stride (words): a multiple of 4, so a thread's 8-value segment is two 16-byte LDS accesses;
 // 36 = 9 groups of 4 banks per row, so the 16-byte accesses of 8 consecutive lanes (2 rows x 4 segments)
 // fall on distinct bank groups
@@ -415,7 +415,7 @@ constexpr int kAZ = kBTZ + 4;
 
 // TABLE: the jobs of a table, whose labels follow their occupancy; also accumulate
 // the histogram and the grid checksum of the final cells (jobs with a window size <= 1; the others
-// get theirs from k_checksum<true>).
+// get theirs from k_checksum).
 //
 // Each thread owns an 8-cell z segment of one of the brick's 64 rows and loads
 // it with its two z neighbours (clamped coordinates = replicate padding), so
@@ -668,17 +668,15 @@ __global__ __launch_bounds__(256) void k_boundaries_tiled(Launch L, uint32_t per
     }, flush);
 }
 
-// Order-independent grid checksum: sum over the non-EMPTY cells of checksum_term.
-// ONLY_WIDE: only jobs whose boundary window is wider than 1 (the tiled
-// boundary kernel sums the others).
-template <bool ONLY_WIDE>
+// Order-independent grid checksum, the sum over the non-EMPTY cells of checksum_term, of the jobs whose boundary
+// window is wider than 1 (the tiled boundary kernel sums the others).
 __global__ __launch_bounds__(kCellThreads) void k_checksum(Launch L)
 {
     __shared__ BlockSum bs;
     __shared__ JobDev sJ;
     unsigned long long acc = 0;
     walk_tiles(L, L.tile_prefix, L.total_tiles, &sJ, [&](const JobDev& J, uint32_t, uint32_t local, uint32_t) {
-        if (!J.active || (ONLY_WIDE && J.bsize <= 1)) return;
+        if (!J.active || J.bsize <= 1) return;
         const uint64_t c0 = (uint64_t)local * kTileCells + threadIdx.x * kCellsPerThread;
         if (c0 >= J.V) return;
         uint16_t v[8];
@@ -895,17 +893,10 @@ void launch_boundaries_tiled(const Launch& L, bool any_wide, bool table)
         VF_CHECK_LAUNCH();
         if (table) {
             TimedLaunch tc("checksum", L.s);
-            k_checksum<true><<<grid_for(L), kCellThreads, 0, L.s>>>(L);
+            k_checksum<<<grid_for(L), kCellThreads, 0, L.s>>>(L);
             VF_CHECK_LAUNCH();
         }
     }
-}
-
-void launch_checksum(const Launch& L)
-{
-    TimedLaunch tl("checksum", L.s);
-    k_checksum<false><<<grid_for(L), kCellThreads, 0, L.s>>>(L);
-    VF_CHECK_LAUNCH();
 }
 
 void launch_job_init(const Launch& L)

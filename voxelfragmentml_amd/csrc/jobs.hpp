@@ -144,16 +144,6 @@ __device__ inline uint32_t find_job(const uint32_t* prefix, uint32_t njobs, uint
     return lo;
 }
 
-__device__ inline uint64_t find_job64(const unsigned long long* prefix, uint32_t n, unsigned long long t)
-{
-    uint32_t lo = 0, hi = n;
-    while (hi - lo > 1) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (prefix[mid] <= t) lo = mid; else hi = mid;
-    }
-    return lo;
-}
-
 // --------------------------------------------------------------- launchers
 // All launchers enqueue on stream s; none synchronises.  `jobs` and the
 // prefix tables are device pointers.
@@ -228,7 +218,6 @@ void launch_boundaries(const Launch& L, int size /* < 0: per-job bsize */);
 void launch_boundaries_tiled(const Launch& L, bool any_wide, bool table);
 void launch_job_init(const Launch& L);     // zero stats, histogram and flood control of every job
 void launch_gather(const Launch& L, uint32_t* out);  // 16 words per job: stats (low 32 bits) + flood state
-void launch_checksum(const Launch& L);
 void launch_count_occupied(const Launch& L);
 void launch_hist_summary(const Launch& L);  // kStatLabels of every job (added: zeroed by job_init)
 
@@ -287,8 +276,8 @@ struct FloodRoundScratch {
 constexpr uint32_t kFloodXcds = 8;
 uint32_t flood_list_cap(uint32_t total_tasks);  // entries per XCD list
 // Key init and brick liveness, then seed stamping and the bricks' neighbour liveness (W's task prefix
-// deals the work: a task is 4096 bricks of a job).  Both brick flag parities of every flood job must be
-// zero before launch_flood_seed (launch_job_init clears them).
+// deals the work: a task is 4096 bricks of a job).  The init also clears both brick flag parities of every flood job, on
+// which launch_flood_seed sets the first round's flags: one follows the other for every growth.
 void launch_flood_init(const Launch& L, const FloodRoundScratch& W);
 void launch_flood_seed(const Launch& L, const FloodRoundScratch& W);
 // `rounds` (rounded up to an even count) relaxation rounds for every running flood job of L.  Each job

@@ -25,7 +25,7 @@ constexpr uint32_t kNaiveSmall = 8192;  // bricks of a launch below which runs a
 
 // (d << b) | i.  32-bit keys: d < 2^24 (at most 3 * 2047^2) and b <= 17, so it is one 24-bit
 // multiply-add, d * 2^b + i.
-template <int DIST, typename K>
+template <typename K>
 __device__ inline K pack_key(uint32_t d, uint32_t i, uint32_t b)
 {
     if constexpr (sizeof(K) == 4) return (K)(__umul24(d, 1u << b) + i);
@@ -60,7 +60,7 @@ __device__ inline K seed_key(uint32_t xy, uint32_t z, uint32_t sxy, uint32_t sz,
         const uint32_t ax = sad16(xy & 0xFFFFu, sxy & 0xFFFFu, 0u), ay = sad16(xy >> 16, sxy >> 16, 0u), az = sad16(z, sz, 0u);
         d = offset_dist<DIST>(ax, ay, az);
     }
-    return pack_key<DIST, K>(d, id, b);
+    return pack_key<K>(d, id, b);
 }
 
 // Seeds in LDS: x | y << 16, then z | (index in the chunk) << 16.
