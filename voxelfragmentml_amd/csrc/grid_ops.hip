@@ -172,7 +172,7 @@ __global__ void k_report(const unsigned long long* stats, const uint4* seeds, ui
 // 8192 workgroups that added their counts to the same few addresses in HBM took 98 us for a 512^3 grid and 57 us for a
 // 256^3 one; now 75 and 20 us, of which clearing and summing take 10.  The word after the partial counts receives the largest
 // label of kHistBins or more.  With those counted in HBM alone, 1500 labels in 8^3 blocks of a 256^3 grid took 400 us.
-constexpr uint32_t kHistThreads = 1024, kHistLds = 12288;  // 48 KiB of counts; a workgroup has its CU to itself
+constexpr uint32_t kHistThreads = 1024, kHistLds = 4096;
 __global__ __launch_bounds__(kHistThreads) void k_histogram(Launch L, uint32_t* part)
 {
     __shared__ __attribute__((aligned(16))) uint32_t bins[kHistLds];
@@ -219,31 +219,40 @@ __global__ __launch_bounds__(kHistThreads) void k_histogram(Launch L, uint32_t* 
                 for (uint32_t k = 0; k < 8u; ++k) eq |= m[k] == l ? 1u << k : 0u;
                 eq &= rest;
                 rest &= ~eq;
-                top = max(top, l);
-                if (l < kHistLds) atomicAdd(&bins[l], (uint32_t)__popc(eq));
-                else atomicAdd(J.hist + l, (uint32_t)__popc(eq));
+                if (l < kHistLds) {
+                    atomicAdd(&bins[l], (uint32_t)__popc(eq));
+                } else {
+                    atomicAdd(J.hist + l, (uint32_t)__popc(eq));
+                    top = max(top, l);
+                }
             }
         }
     }
-    if (top >= kHistBins) atomicMax(&largest, top);
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < kHistBins; i += kHistThreads) part[blockIdx.x * kHistBins + i] = bins[i];
-    if (!largest) return;
+#pragma unroll
     for (uint32_t i = kHistBins + threadIdx.x; i < kHistLds; i += kHistThreads) {
         const uint32_t c = bins[i];
-        if (c) atomicAdd(J.hist + i, c);
+        if (c) {
+            atomicAdd(J.hist + i, c);
+            top = max(top, i);
+        }
     }
-    if (threadIdx.x == 0) atomicMax(part + kHistBlocks * kHistBins, largest);
+    if (top) atomicMax(&largest, top);
+    __syncthreads();
+    if (threadIdx.x == 0 && largest) atomicMax(part + kHistBlocks * kHistBins, largest);
 }
 
 // Sums nparts partial counts of 64 bins per workgroup into hist and, where given, host memory; the workgroups after those
 // store the counts of larger labels there, where they occur.
+constexpr uint32_t kLargeBlocks = 8;
 __global__ __launch_bounds__(256) void k_hist_sum(const uint32_t* part, uint32_t nparts, uint32_t* hist, uint32_t* host)
 {
     __shared__ uint32_t sum[4][64];
     if (blockIdx.x >= kHistBins / 64) {
-        const uint32_t i = (blockIdx.x - kHistBins / 64) * 256u + threadIdx.x;
-        if (kHistBins + i <= part[kHistBlocks * kHistBins]) host[kPinLarge + i] = hist[kHistBins + i];
+        const uint32_t top = part[kHistBlocks * kHistBins];  // 0: no larger label
+        for (uint32_t i = (blockIdx.x - kHistBins / 64) * 256u + threadIdx.x; i < kHistLargeHost && kHistBins + i <= top; i += kLargeBlocks * 256u)
+            host[kPinLarge + i] = hist[kHistBins + i];
         return;
     }
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, bin = blockIdx.x * 64u + lane;
@@ -852,8 +861,7 @@ void launch_histogram(const Launch& L, uint32_t* hist, uint32_t* part, uint32_t*
     VF_CHECK_LAUNCH();
     k_histogram<<<blocks, kHistThreads, 0, L.s>>>(L, part);
     VF_CHECK_LAUNCH();
-    static_assert(kHistLargeHost % 256 == 0, "whole workgroups");
-    k_hist_sum<<<kHistBins / 64 + (host ? kHistLargeHost / 256 : 0u), 256, 0, L.s>>>(part, blocks, hist, host);
+    k_hist_sum<<<kHistBins / 64 + (host ? kLargeBlocks : 0u), 256, 0, L.s>>>(part, blocks, hist, host);
     VF_CHECK_LAUNCH();
 }
 

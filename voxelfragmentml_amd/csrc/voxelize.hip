@@ -714,10 +714,9 @@ __global__ __launch_bounds__(kVoxThreads) __attribute__((amdgpu_waves_per_eu(5))
                 if (valid) {
                     if (S->job & kWildTriangle) {
                         bits = sat_column<false>(q, z0, z1, mnz, csz);
-                    } else if (few) {
-                        bits = sat_column<true>(q, z0, z1, mnz, csz);
                     } else if (column_open<true>(q)) {
-                        const ZCells z = z_cells(q, z0, z1, mnz, csz);
+                        ZCells z{ 0u, ((2u << (z1 - z0)) - 1u) << (z0 & 31) };
+                        if (!few) z = z_cells(q, z0, z1, mnz, csz);
                         bits = z.sure;
                         for (uint32_t m = z.maybe; m; m &= m - 1u) {
                             const int k = (int)(32 * w) + (int)__builtin_ctz(m);
