@@ -9,9 +9,9 @@ from test_gpu_stencils import labelled
 pytestmark = pytest.mark.gpu
 
 BOX = ([-1.03, -1.03, -1.03], [1.03, 1.03, 1.03])
-# bricks of 8 x 8 x 32: 72 and 100 (windows above 3 from 64 on), 300 and 336 (window 3 from 320), 975 and 1020 (isolated
-# cells from 1000); then grids whose cells are less than a third of their bricks'
-DIMS = [(47, 48, 41), (80, 80, 31), (80, 80, 70), (90, 60, 97), (100, 115, 130), (136, 117, 97), (61, 65, 3), (1, 130, 200), (150, 2, 90),
+# bricks of 8 x 8 x 32: 72 and 100 (windows above 3 from 64 on), 300 and 336 (window 3 from 320), 605 and 660 (isolated
+# cells from 640), 975 and 1020; then grids whose cells are less than a third of their bricks'
+DIMS = [(47, 48, 41), (80, 80, 31), (80, 80, 70), (90, 60, 97), (88, 83, 130), (88, 90, 130), (100, 115, 130), (136, 117, 97), (61, 65, 3), (1, 130, 200), (150, 2, 90),
         (300, 70, 10), (300, 70, 11)]
 
 

@@ -204,12 +204,13 @@ __global__ __launch_bounds__(kCellThreads) void k_empty_linear(const JobDev* Jg,
 // Thin grids, whose cells are less than a third of their bricks' (2048 x 2048 x 1, window 3: 824 us a step by bricks, 159 by
 // cells; 600 x 600 x 9, where they are 0.28: 98 and 80; x 12, 0.38: 102 and 96; x 16, 0.5: 106 and 119), and grids of too
 // few bricks for the chip, which a brick's steps one after another take longer: isolated cells 27.1 us by bricks and 21.5 by
-// cells at 64^3 (128 bricks), 34.7 and 30.7 at 96^3 (432), 38.8 and 40.6 at 128^3 (1024); window 3 17.2 and 15.2 at 64^3,
-// 19.3 and 18.2 at 80^3 (300), 20.6 and 23.1 at 96^3; larger windows are even up to 50 bricks (40^3: 32 and 30 for 5, 221
-// and 191 for 15) and then better by bricks (64^3: 52 and 60 for 7).
+// cells at 64^3 (128 bricks), 34.7 and 30.7 at 96^3 (432), 38.8 and 40.6 at 128^3 (1024; six jobs of 120^3 with 900 bricks
+// each take 739 us by bricks, 756 by cells); window 3 17.2 and 15.2 at 64^3, 19.3 and 18.2 at 80^3 (300), 20.6 and 23.1 at
+// 96^3; larger windows are even up to 50 bricks (40^3: 32 and 30 for 5, 221 and 191 for 15) and then better by bricks (64^3:
+// 52 and 60 for 7).
 bool by_cells(uint64_t V, uint32_t bricks, uint32_t side, bool erode)
 {
-    return V * 3u < (uint64_t)bricks * kTileCells || bricks < (!erode ? 1000u : side <= 3u ? 320u : 64u);
+    return V * 3u < (uint64_t)bricks * kTileCells || bricks < (!erode ? 640u : side <= 3u ? 320u : 64u);
 }
 
 template <uint32_t SIDE, bool kErode>
