@@ -11,7 +11,8 @@
 // so ties go to the lowest index exactly as the reference's strict '<' does.
 // Work goes by bricks of 8 x 8 x 32 cells: a brick's occupied cells are
 // compacted, the seeds that cannot be nearest to any of its cells are dropped,
-// and a thread applies the rest to its few cells in registers.
+// and a thread applies the rest to its few cells in registers.  Flat grids of
+// many bricks go by tiles of cells in linear order instead.
 #include <type_traits>
 
 #include "cellops.hpp"
